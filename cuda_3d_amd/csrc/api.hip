@@ -455,7 +455,10 @@ int32_t gca_ctx_create(int32_t device, gca_ctx *out)
     if (hipDeviceGetAttribute(&c->wall_khz, hipDeviceAttributeWallClockRate, device) != hipSuccess) c->wall_khz = 0;
     if (hipStreamCreateWithFlags(&c->stream, hipStreamNonBlocking) != hipSuccess ||
         hipEventCreate(&c->ev_a) != hipSuccess || hipEventCreate(&c->ev_b) != hipSuccess ||
-        hipHostMalloc((void **)&c->dev_err, sizeof(uint32_t), hipHostMallocDefault) != hipSuccess) {
+        hipHostMalloc((void **)&c->dev_err, sizeof(uint32_t), hipHostMallocDefault) != hipSuccess ||
+        hipHostMalloc((void **)&c->pinned, sizeof(double) * gca_ctx_s::kPinnedDoubles, hipHostMallocDefault) !=
+            hipSuccess) {
+        if (c->dev_err) hipHostFree(c->dev_err);
         if (c->stream) hipStreamDestroy(c->stream);
         if (c->ev_a) hipEventDestroy(c->ev_a);
         if (c->ev_b) hipEventDestroy(c->ev_b);
@@ -485,6 +488,7 @@ int32_t gca_ctx_destroy(gca_ctx c)
     hipEventDestroy(c->ev_b);
     hipStreamDestroy(c->stream);
     hipHostFree(c->dev_err);
+    hipHostFree(c->pinned);
     delete c;
     return GCA_OK;
 }

@@ -112,6 +112,10 @@ struct gca_ctx_s {
     // device-raised error word in mapped host memory (a bounded wait that gave up); read and
     // cleared at synchronisation points
     uint32_t *dev_err = nullptr;
+    // pinned host memory (kPinnedDoubles) that a launch's last block stores its sums into; read
+    // after the stream has been synchronised
+    static constexpr int kPinnedDoubles = 32;
+    double *pinned = nullptr;
     int n_cu = 0;         // compute units of the device (persistent launch sizing)
     int wall_khz = 0;     // rate of the device wall clock (wall_clock64)
     // persistent bitmap of the voxel downsampler (kept all-zero between calls)

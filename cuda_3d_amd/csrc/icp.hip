@@ -104,9 +104,8 @@ struct PairDesc {
     const float4 *sgrad;
     double *partials;    // one FP64 partial (kPartStride doubles) per work unit
     int32_t *nnprev;     // matched target slot of each source point in the previous iteration
-    IcpState *st;        // single-pair kernels (Gauss-Newton build, residuals, objective)
     float sl, sc;        // sqrt(lambda), sqrt(1 - lambda)
-    int32_t nblk;        // single-pair kernels: workgroups
+    int32_t nblk;        // single-pair kernels (Gauss-Newton build, residuals, objective): workgroups
     int32_t unit_cap;    // cap on work units per iteration
     int32_t lanes[3];    // lanes per query for n < 16384, n < 49152, larger
 };
@@ -1176,11 +1175,19 @@ static void launch_build_gn(gca_ctx ctx, const PairDesc &P, const float4 *tgt_xy
 }
 
 // ---- generic FP64 block sums with last-block finish (residuals, objective) -----------------
+// A block's sums go out write-through and wavefront 0, which stored them, takes the ticket with a
+// release, so no other wavefront's stores are flushed for it.  The last block reads kFinishRows
+// blocks' sums at a time with all its threads, then one thread per value adds them from LDS in
+// block order: the adjoint of 100k points 105 -> 19 us, the residuals of 92k 105 -> 16 us (one
+// thread per value reading them from memory as well: a round trip per block).
+constexpr int kFinishRows = 128;
+
 template <int NV>
 __device__ __forceinline__ void sum_finish(double (&v)[NV], double *partials, int nblk, uint32_t *ticket,
                                            double *result)
 {
     __shared__ double wv[kIcpBlock / kWave][NV];
+    __shared__ double rows[kFinishRows][NV];
     __shared__ bool last;
 #pragma unroll
     for (int k = 0; k < NV; ++k) v[k] = wave_sum(v[k]);
@@ -1190,29 +1197,45 @@ __device__ __forceinline__ void sum_finish(double (&v)[NV], double *partials, in
     if (threadIdx.x < NV) {
         double a = 0.0;
         for (int w = 0; w < kIcpBlock / kWave; ++w) a += wv[w][threadIdx.x];
-        partials[(int64_t)blockIdx.x * kPartStride + threadIdx.x] = a;
+        store_coherent(&partials[(int64_t)blockIdx.x * kPartStride + threadIdx.x], a);
     }
-    fence_release_agent();
-    __syncthreads();
-    if (threadIdx.x == 0) last = atomicAdd(ticket, 1u) == (uint32_t)(nblk - 1);
+    static_assert(NV <= kWave, "the ticket's release covers wavefront 0's stores");
+    if (threadIdx.x == 0)
+        last = __hip_atomic_fetch_add(ticket, 1u, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_AGENT) == (uint32_t)(nblk - 1);
     __syncthreads();
     if (!last) return;
     fence_acquire_agent();
-    if (threadIdx.x < NV) {
-        double a = 0.0;
-        for (int b = 0; b < nblk; ++b) a += partials[(int64_t)b * kPartStride + threadIdx.x];
-        result[threadIdx.x] = a;
+    double a = 0.0;
+    for (int b0 = 0; b0 < nblk; b0 += kFinishRows) {
+        const int nr = min(kFinishRows, nblk - b0);
+        for (int e = threadIdx.x; e < nr * NV; e += kIcpBlock)
+            rows[e / NV][e % NV] = partials[(int64_t)(b0 + e / NV) * kPartStride + e % NV];
+        __syncthreads();
+        if (threadIdx.x < NV) {
+#pragma unroll 8
+            for (int r = 0; r < nr; ++r) a += rows[r][threadIdx.x];
+        }
+        __syncthreads();
     }
+    if (threadIdx.x < NV) result[threadIdx.x] = a;
     if (threadIdx.x == 0) *ticket = 0u;
 }
 
+// Pose of the residual kernel (the first three rows) and parameters of the objective's adjoint,
+// passed by value: a copy to the device before each launch cost more than the launch.
+struct Pose34 {
+    double m[12];
+};
+struct ObjectiveParams {
+    double T[16], dT[16], RzRy[9], Rx[9], M[9];
+};
+
 __global__ __launch_bounds__(kIcpBlock) void k_residuals(PairDesc P, const float4 *__restrict__ tgt_xyzi,
-                                                         const int32_t *__restrict__ nn, const double *__restrict__ Tm,
-                                                         float lam, float sl, float sc, int kind,
-                                                         float *__restrict__ out, double *__restrict__ result)
+                                                         const int32_t *__restrict__ nn, Pose34 Tm, float lam,
+                                                         float sl, float sc, int kind, float *__restrict__ out,
+                                                         uint32_t *ticket, double *__restrict__ result)
 {
-    double T[12];
-    for (int k = 0; k < 12; ++k) T[k] = Tm[k];
+    const double *T = Tm.m;
     const int n = P.src_hdr->n;
     double v[1] = {0.0};
     for (int i = blockIdx.x * kIcpBlock + threadIdx.x; i < n; i += P.nblk * kIcpBlock) {
@@ -1248,20 +1271,17 @@ __global__ __launch_bounds__(kIcpBlock) void k_residuals(PairDesc P, const float
             v[0] += a;
         }
     }
-    sum_finish<1>(v, P.partials, P.nblk, &P.st->ticket, result);
+    sum_finish<1>(v, P.partials, P.nblk, ticket, result);
 }
 
 // Objective E and its adjoint at pose dT(xi) * T with frozen correspondences, all in FP64.
 __global__ __launch_bounds__(kIcpBlock) void k_objective_grad(PairDesc P, const float4 *__restrict__ tgt_xyzi,
                                                               const int32_t *__restrict__ nn,
-                                                              const double *__restrict__ prm, double lam,
-                                                              float4 *__restrict__ dpts, double *__restrict__ result)
+                                                              ObjectiveParams prm, double lam,
+                                                              float4 *__restrict__ dpts, uint32_t *ticket,
+                                                              double *__restrict__ result)
 {
-    // prm: T[16] | dT[16] | RzRy[9] | Rx[9] | M[9]
-    __shared__ double s[59];
-    if (threadIdx.x < 59) s[threadIdx.x] = prm[threadIdx.x];
-    __syncthreads();
-    const double *T = s, *dT = s + 16, *RzRy = s + 32, *Rx = s + 41, *M = s + 50;
+    const double *T = prm.T, *dT = prm.dT, *RzRy = prm.RzRy, *Rx = prm.Rx, *M = prm.M;
     const int n = P.src_hdr->n;
     double v[7] = {0, 0, 0, 0, 0, 0, 0};
     for (int i = blockIdx.x * kIcpBlock + threadIdx.x; i < n; i += P.nblk * kIcpBlock) {
@@ -1306,7 +1326,7 @@ __global__ __launch_bounds__(kIcpBlock) void k_objective_grad(PairDesc P, const 
             dpts[i] = o;
         }
     }
-    sum_finish<7>(v, P.partials, P.nblk, &P.st->ticket, result);
+    sum_finish<7>(v, P.partials, P.nblk, ticket, result);
 }
 
 // ---------------------------------------------------------------------------------------------
@@ -1355,17 +1375,6 @@ __global__ void k_state_init(IcpState *states, const PairDesc *__restrict__ pair
     }
     s.ticket = 0u;
     s.bar_top = 0u;
-}
-
-// State of the single-pair kernels (Gauss-Newton build, residuals, objective).
-__global__ void k_state_simple(IcpState *st, const double *__restrict__ T0)
-{
-    if (threadIdx.x != 0) return;
-    for (int k = 0; k < 16; ++k) st->T[k] = T0[k];
-    for (int k = 0; k < kNSys; ++k) st->sys[k] = 0.0;
-    st->iter = 0;
-    st->done = 0;
-    st->ticket = 0u;
 }
 
 // ---------------------------------------------------------------------------------------------
@@ -1889,27 +1898,22 @@ int32_t icp_plan_results(gca_ctx ctx, const IcpPlan *p, double *T_out, gca_icp_r
     return GCA_OK;
 }
 
-// Set-up of the single-pair kernels over given correspondences.
-static int32_t single_pair(gca_ctx ctx, gca_cloud src, gca_cloud tgt, IcpWork &w, PairDesc &P, int64_t &n)
+// Set-up of the single-pair kernels over given correspondences: no launch and no copy.  The ticket
+// is zero from its allocation on and left at zero by every launch; a launch's last block stores
+// the sums into the ctx's pinned memory, so a stream synchronisation is all it takes to read them.
+static int32_t single_pair(gca_ctx ctx, gca_cloud src, gca_cloud tgt, PairDesc &P, uint32_t **ticket)
 {
     GCA_TRY(cloud_sync_header(src));
-    n = src->host_hdr.n;
-    const int32_t nb = icp_blocks(n);
-    GCA_TRY(icp_work(ctx, 1, 1, nb, 1, 0, w));
     P = PairDesc{};
     P.src = src->xyzi;
     P.src_hdr = src->hdr;
     P.tgt_hdr = tgt->hdr;
     P.nrm = tgt->nrm;
     P.grad = tgt->grad;
-    P.partials = w.partials;
-    P.st = w.states;
-    P.nblk = nb;
-    static const double I[16] = {1, 0, 0, 0, 0, 1, 0, 0, 0, 0, 1, 0, 0, 0, 0, 1};
-    GCA_HIP(hipMemcpyAsync(w.T0, I, sizeof(I), hipMemcpyHostToDevice, ctx->stream));
-    hipLaunchKernelGGL(k_state_simple, dim3(1), dim3(64), 0, ctx->stream, w.states, (const double *)w.T0);
-    GCA_HIP(hipGetLastError());
-    return GCA_OK;
+    P.nblk = icp_blocks(src->host_hdr.n);
+    P.partials = (double *)ctx_scratch(ctx, 14, sizeof(double) * kPartStride * P.nblk, false);
+    *ticket = (uint32_t *)ctx_scratch(ctx, 9, 256, true);
+    return P.partials && *ticket ? GCA_OK : GCA_ERR_OUT_OF_MEMORY;
 }
 
 }  // namespace gca
@@ -1925,16 +1929,13 @@ int32_t gca_build_gauss_newton(gca_ctx ctx, gca_cloud src, gca_cloud tgt, const 
     if (!ctx || !src || !tgt || !nn_dev || !T || !out) return GCA_ERR_INVALID_VALUE;
     if (lambda > 1.0f || !(lambda >= 0.0f) || mode < 0 || mode > 2) return GCA_ERR_INVALID_VALUE;  // .cu:438-441
     if (!tgt->has_normals || !tgt->has_gradient) return GCA_ERR_NOT_READY;                       // .cu:449-452
-    IcpWork w;
     PairDesc P;
-    int64_t n;
-    GCA_TRY(single_pair(ctx, src, tgt, w, P, n));
-    launch_build_gn(ctx, P, tgt->xyzi, nn_dev, T, lambda, mode, &w.states->ticket, w.states->sys);
+    uint32_t *ticket;
+    GCA_TRY(single_pair(ctx, src, tgt, P, &ticket));
+    launch_build_gn(ctx, P, tgt->xyzi, nn_dev, T, lambda, mode, ticket, ctx->pinned);
     GCA_HIP(hipGetLastError());
-    IcpState S;
-    GCA_HIP(hipMemcpyAsync(&S, w.states, offsetof(IcpState, q), hipMemcpyDeviceToHost, ctx->stream));
     GCA_HIP(hipStreamSynchronize(ctx->stream));
-    memcpy(out, S.sys, sizeof(double) * kNSys);
+    memcpy(out, ctx->pinned, sizeof(double) * kNSys);
     return GCA_OK;
 }
 
@@ -1971,20 +1972,17 @@ int32_t gca_compute_residuals(gca_ctx ctx, gca_cloud src, gca_cloud tgt, const i
     if (!ctx || !src || !tgt || !nn_dev || !T || kind < 0 || kind > 2) return GCA_ERR_INVALID_VALUE;
     if (lambda > 1.0f || !(lambda >= 0.0f)) return GCA_ERR_INVALID_VALUE;
     if (!tgt->has_normals || !tgt->has_gradient) return GCA_ERR_NOT_READY;
-    IcpWork w;
     PairDesc P;
-    int64_t n;
-    GCA_TRY(single_pair(ctx, src, tgt, w, P, n));
-    GCA_HIP(hipMemcpyAsync(w.T0 + 16, T, sizeof(double) * 16, hipMemcpyHostToDevice, ctx->stream));
-    double *res = w.T0 + 32;
+    uint32_t *ticket;
+    GCA_TRY(single_pair(ctx, src, tgt, P, &ticket));
+    Pose34 pose;
+    memcpy(pose.m, T, sizeof(pose.m));
     const float sl = sqrtf(lambda), sc = sqrtf(1.0f - lambda);
-    hipLaunchKernelGGL(k_residuals, dim3((unsigned)P.nblk), dim3(kIcpBlock), 0, ctx->stream, P, tgt->xyzi, nn_dev,
-                       (const double *)(w.T0 + 16), lambda, sl, sc, kind, out_dev, res);
+    hipLaunchKernelGGL(k_residuals, dim3((unsigned)P.nblk), dim3(kIcpBlock), 0, ctx->stream, P, tgt->xyzi, nn_dev, pose,
+                       lambda, sl, sc, kind, out_dev, ticket, ctx->pinned);
     GCA_HIP(hipGetLastError());
-    double s = 0.0;
-    GCA_HIP(hipMemcpyAsync(&s, res, sizeof(double), hipMemcpyDeviceToHost, ctx->stream));
     GCA_HIP(hipStreamSynchronize(ctx->stream));
-    if (sum) *sum = s;
+    if (sum) *sum = ctx->pinned[0];
     return GCA_OK;
 }
 
@@ -2264,38 +2262,30 @@ int32_t gca_color_icp_objective_grad(gca_ctx ctx, gca_cloud src, gca_cloud tgt, 
     if (!ctx || !src || !tgt || !nn_dev || !T || !xi) return GCA_ERR_INVALID_VALUE;
     if (lambda > 1.0f || !(lambda >= 0.0f)) return GCA_ERR_INVALID_VALUE;
     if (!tgt->has_normals || !tgt->has_gradient) return GCA_ERR_NOT_READY;
-    IcpWork w;
     PairDesc P;
-    int64_t n;
-    GCA_TRY(single_pair(ctx, src, tgt, w, P, n));
-    double prm[59];
-    memcpy(prm, T, sizeof(double) * 16);
+    uint32_t *ticket;
+    GCA_TRY(single_pair(ctx, src, tgt, P, &ticket));
+    ObjectiveParams prm;
+    memcpy(prm.T, T, sizeof(prm.T));
     const double ca = cos(xi[0]), sa = sin(xi[0]), cb = cos(xi[1]), sb = sin(xi[1]), cc = cos(xi[2]), sc = sin(xi[2]);
-    double *dT = prm + 16;
     const double dTv[16] = {cc * cb, cc * sb * sa - sc * ca, cc * sb * ca + sc * sa, xi[3],
                             sc * cb, sc * sb * sa + cc * ca, sc * sb * ca - cc * sa, xi[4],
                             -sb,     cb * sa,                cb * ca,                xi[5],
                             0.0,     0.0,                    0.0,                    1.0};
-    memcpy(dT, dTv, sizeof(dTv));
+    memcpy(prm.dT, dTv, sizeof(dTv));
     const double RzRy[9] = {cc * cb, -sc, cc * sb, sc * cb, cc, sc * sb, -sb, 0.0, cb};
     const double Rx[9] = {1, 0, 0, 0, ca, -sa, 0, sa, ca};
-    memcpy(prm + 32, RzRy, sizeof(RzRy));
-    memcpy(prm + 41, Rx, sizeof(Rx));
+    memcpy(prm.RzRy, RzRy, sizeof(RzRy));
+    memcpy(prm.Rx, Rx, sizeof(Rx));
     for (int i = 0; i < 3; ++i)
         for (int j = 0; j < 3; ++j)
-            prm[50 + 3 * i + j] = (dT[4 * i] * T[j] + dT[4 * i + 1] * T[4 + j]) + dT[4 * i + 2] * T[8 + j];
-    double *dprm = (double *)ctx_scratch(ctx, 10, sizeof(double) * 80, false);
-    if (!dprm) return GCA_ERR_OUT_OF_MEMORY;
-    GCA_HIP(hipMemcpyAsync(dprm, prm, sizeof(prm), hipMemcpyHostToDevice, ctx->stream));
-    double *res = dprm + 64;
-    hipLaunchKernelGGL(k_objective_grad, dim3((unsigned)P.nblk), dim3(kIcpBlock), 0, ctx->stream, P, tgt->xyzi, nn_dev,
-                       (const double *)dprm, (double)lambda, (float4 *)dpts_dev, res);
+            prm.M[3 * i + j] = (dTv[4 * i] * T[j] + dTv[4 * i + 1] * T[4 + j]) + dTv[4 * i + 2] * T[8 + j];
+    hipLaunchKernelGGL(k_objective_grad, dim3((unsigned)P.nblk), dim3(kIcpBlock), 0, ctx->stream, P, tgt->xyzi, nn_dev, prm,
+                       (double)lambda, (float4 *)dpts_dev, ticket, ctx->pinned);
     GCA_HIP(hipGetLastError());
-    double r[7];
-    GCA_HIP(hipMemcpyAsync(r, res, sizeof(r), hipMemcpyDeviceToHost, ctx->stream));
     GCA_HIP(hipStreamSynchronize(ctx->stream));
-    if (E) *E = r[0];
-    if (dE_dxi) memcpy(dE_dxi, r + 1, sizeof(double) * 6);
+    if (E) *E = ctx->pinned[0];
+    if (dE_dxi) memcpy(dE_dxi, ctx->pinned + 1, sizeof(double) * 6);
     return GCA_OK;
 }
 
