@@ -372,6 +372,7 @@ void grid_params(const float bmin[3], const float bmax[3], float r, GridDesc *d,
     d->ncells = (int64_t)d->dims[0] * d->dims[1] * d->dims[2];
     d->cell_q = cell_quarters > 4 ? cell_quarters : 0;
     d->pad = 0;
+    d->inv_cell = 1.0 / (double)s;
 }
 
 int32_t grid_build(gca_ctx ctx, gca_cloud c, float radius, bool exact)

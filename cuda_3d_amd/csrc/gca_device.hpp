@@ -289,7 +289,13 @@ __device__ __forceinline__ int32_t grid_cell(double p, float o, float s, int32_t
     return (int32_t)c;
 }
 
-// Cell range overlapped by the box [q - r, q + r] (r in FP64); false if empty or q not finite.
+// Cells [lo, hi] that hold every point within r (FP64) of q along each axis; false if none or q not
+// finite.  Positions in cells come from the reciprocal of the cell edge, where a point's own cell
+// (grid_cell) is a division; kCellSlack (in cells) covers the difference: both are within a few
+// units of the last place of at most 2^25 cells (4e-9 each), so a bound may only take in one cell
+// too many, and the walk's distances decide.  (Six divisions a query took a sixth of the
+// instructions of a neighbourhood walk.)
+constexpr double kCellSlack = 1e-6;
 __device__ __forceinline__ bool grid_range_r(const GridDesc &g, float qx, float qy, float qz, double r,
                                              int32_t lo[3], int32_t hi[3])
 {
@@ -297,8 +303,9 @@ __device__ __forceinline__ bool grid_range_r(const GridDesc &g, float qx, float 
 #pragma unroll
     for (int a = 0; a < 3; ++a) {
         if (!isfinite(q[a])) return false;
-        double l = floor(((double)q[a] - r - (double)g.origin[a]) / (double)g.cell);
-        double h = floor(((double)q[a] + r - (double)g.origin[a]) / (double)g.cell);
+        const double c = (double)q[a] - (double)g.origin[a];
+        double l = floor((c - r) * g.inv_cell - kCellSlack);
+        double h = floor((c + r) * g.inv_cell + kCellSlack);
         l = fmax(l, 0.0);
         h = fmin(h, (double)(g.dims[a] - 1));
         if (l > h) return false;

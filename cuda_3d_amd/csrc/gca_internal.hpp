@@ -63,6 +63,7 @@ struct GridDesc {
     int32_t cell_q;  // 0: canonical cell (the radius, doubled while too many cells); else the tuned
                      // edge in quarters of the radius
     int32_t pad;
+    double inv_cell;  // 1 / cell
 };
 
 struct Grid {

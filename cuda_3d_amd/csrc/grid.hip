@@ -20,6 +20,7 @@
 
 #include "gca_device.hpp"
 #include "gca_internal.hpp"
+#include "neighbours.hpp"
 
 namespace gca {
 
@@ -202,96 +203,13 @@ int32_t grid_gather_attributes(gca_ctx ctx, gca_cloud c)
 
 // ---- queries ---------------------------------------------------------------------------------
 
-struct GridView {
-    GridDesc g;
-    const uint32_t *start;
-    const int32_t *order;
-    const float4 *sxyzi;
-};
+constexpr int kQUnroll = 4;  // candidates in flight per lane
 
-__device__ __forceinline__ GridView make_view(const GridDesc &g, const uint32_t *start, const int32_t *order,
-                                              const float4 *sxyzi)
+// The query's own column of cells, kept within box b.
+__device__ __forceinline__ void own_column(const GridDesc &g, float4 q, const Box &b, int &ix, int &iy)
 {
-    GridView v;
-    v.g = g;
-    v.start = start;
-    v.order = order;
-    v.sxyzi = sxyzi;
-    return v;
-}
-
-// ---- candidate walk of a lane group --------------------------------------------------------
-// A query's candidates are the z-runs of cells of its box, at most nine when the cell is at least
-// the radius (ten or more only where rounding widens the box by a cell: the walk then goes on in
-// further sets of nine).  A group of gs lanes (a power of two, lanes g = 0 .. gs - 1 of one
-// wavefront) walks each set as one flattened range, kQUnroll loads in flight per lane: one thread
-// per query spent its time waiting for one candidate after another.
-constexpr int kQRuns = 9;
-constexpr int kQUnroll = 4;
-
-struct Box {
-    int32_t lo[3], hi[3];
-};
-
-// Calls f(slot, point, valid) kQUnroll times per round on every lane of the group (valid: the lane
-// has a candidate), then more(): false ends the walk (the same answer on the group's lanes).  Run
-// `skip` (its number in the box's (x, y) order, -1: none) is left out.
-template <class F, class M>
-__device__ __forceinline__ void group_walk_runs(const GridView &v, const Box &b, int g, int gs, int skip, F &&f, M &&more)
-{
-    const int nry = b.hi[1] - b.lo[1] + 1;
-    const int nruns = (b.hi[0] - b.lo[0] + 1) * nry;
-    for (int r0 = 0; r0 < nruns; r0 += kQRuns) {
-        uint32_t rs[kQRuns], cum[kQRuns + 1];
-        cum[0] = 0;
-#pragma unroll
-        for (int r = 0; r < kQRuns; ++r) {
-            uint32_t s0 = 0, s1 = 0;
-            if (r0 + r < nruns && r0 + r != skip) {
-                const int ix = b.lo[0] + (r0 + r) / nry, iy = b.lo[1] + (r0 + r) % nry;
-                const int64_t row = ((int64_t)ix * v.g.dims[1] + iy) * v.g.dims[2];
-                s0 = v.start[row + b.lo[2]];
-                s1 = v.start[row + b.hi[2] + 1];
-            }
-            rs[r] = s0;
-            cum[r + 1] = s1 > s0 ? s1 - s0 : 0u;
-        }
-#pragma unroll
-        for (int r = 0; r < kQRuns; ++r) cum[r + 1] += cum[r];
-        const uint32_t total = cum[kQRuns];
-        for (uint32_t f0 = 0; f0 < total; f0 += gs * kQUnroll) {
-            float4 c[kQUnroll];
-            uint32_t sl[kQUnroll];
-#pragma unroll
-            for (int u = 0; u < kQUnroll; ++u) {
-                const uint32_t fi = f0 + u * gs + g;
-                sl[u] = 0;
-                c[u] = make_float4(0.f, 0.f, 0.f, 0.f);
-                if (fi < total) {
-                    uint32_t t = rs[0] + fi;
-#pragma unroll
-                    for (int r = 1; r < kQRuns; ++r)
-                        if (fi >= cum[r]) t = rs[r] + (fi - cum[r]);
-                    sl[u] = t;
-                    c[u] = v.sxyzi[t];
-                }
-            }
-#pragma unroll
-            for (int u = 0; u < kQUnroll; ++u) f(sl[u], c[u], f0 + u * gs + g < total);
-            if (!more()) return;
-        }
-    }
-}
-
-// The query's own column of cells within box b, as a box of one run, and its run number in b.
-__device__ __forceinline__ int own_column(const GridDesc &g, float4 q, const Box &b, Box &col)
-{
-    const int ix = min(max(grid_cell(q.x, g.origin[0], g.cell, g.dims[0]), b.lo[0]), b.hi[0]);
-    const int iy = min(max(grid_cell(q.y, g.origin[1], g.cell, g.dims[1]), b.lo[1]), b.hi[1]);
-    col = b;
-    col.lo[0] = col.hi[0] = ix;
-    col.lo[1] = col.hi[1] = iy;
-    return (ix - b.lo[0]) * (b.hi[1] - b.lo[1] + 1) + (iy - b.lo[1]);
+    ix = min(max(grid_cell(q.x, g.origin[0], g.cell, g.dims[0]), b.lo[0]), b.hi[0]);
+    iy = min(max(grid_cell(q.y, g.origin[1], g.cell, g.dims[1]), b.lo[1]), b.hi[1]);
 }
 
 // Points within the radius of q, counted by a group of lanes (the count is on all of them); the
@@ -299,7 +217,8 @@ __device__ __forceinline__ int own_column(const GridDesc &g, float4 q, const Box
 // exceeds `limit`.
 __device__ __forceinline__ uint32_t group_count(const GridView &v, float4 q, int g, int gs, uint32_t limit)
 {
-    Box b, col;
+    Box b;
+    int ix, iy;
     if (!grid_range(v.g, q.x, q.y, q.z, b.lo, b.hi)) return 0;
     const double r2 = (double)v.g.radius * (double)v.g.radius;
     uint32_t k = 0, all = 0;
@@ -311,9 +230,9 @@ __device__ __forceinline__ uint32_t group_count(const GridView &v, float4 q, int
         for (int m = 1; m < gs; m <<= 1) all += __shfl_xor(all, m, kWave);
         return all <= limit;
     };
-    const int own = own_column(v.g, q, b, col);
-    group_walk_runs(v, col, g, gs, -1, test, sum);
-    if (all <= limit) group_walk_runs(v, b, g, gs, own, test, sum);
+    own_column(v.g, q, b, ix, iy);
+    group_walk_column<kQUnroll>(v, b, ix, iy, g, gs, test, sum);
+    if (all <= limit) group_walk_box<kQUnroll>(v, b, g, gs, ix, iy, test, sum);
     return all;
 }
 
@@ -360,21 +279,16 @@ __global__ __launch_bounds__(256) void k_nn(const float4 *__restrict__ q, const 
             }
         };
         auto go = [] { return true; };
-        Box b, col;
+        Box b;
+        int ix, iy;
         if (grid_range(g, p.x, p.y, p.z, b.lo, b.hi)) {
-            own_column(g, p, b, col);
-            group_walk_runs(v, col, gl, kNnLanes, -1, test, go);
+            own_column(g, p, b, ix, iy);
+            group_walk_column<kQUnroll>(v, b, ix, iy, gl, kNnLanes, test, go);
             reduce();
-            bool rest = true;
-            if (bi >= 0)
-                rest = grid_range_r(g, p.x, p.y, p.z, fmin((double)g.radius, sqrt(bd) * (1.0 + kBoxRel) + kBoxAbs),
-                                    b.lo, b.hi);
-            if (rest) {
-                // the column was searched over the full box's cells, a superset of this box's
-                const int own = col.lo[0] >= b.lo[0] && col.lo[0] <= b.hi[0] && col.lo[1] >= b.lo[1] && col.lo[1] <= b.hi[1]
-                                    ? (col.lo[0] - b.lo[0]) * (b.hi[1] - b.lo[1] + 1) + (col.lo[1] - b.lo[1])
-                                    : -1;
-                group_walk_runs(v, b, gl, kNnLanes, own, test, go);
+            // the column was searched over the full box's cells, a superset of what is left of it
+            if (bi < 0 || grid_range_r(g, p.x, p.y, p.z, fmin((double)g.radius, sqrt(bd) * (1.0 + kBoxRel) + kBoxAbs),
+                                       b.lo, b.hi)) {
+                group_walk_box<kQUnroll>(v, b, gl, kNnLanes, ix, iy, test, go);
                 reduce();
             }
         }
@@ -420,112 +334,16 @@ __global__ __launch_bounds__(256) void k_radius_count(const float4 *__restrict__
     }
 }
 
-// The fill keeps a query's candidates (those within the radius) in an LDS buffer.  When the buffer
-// is nearly full, only the `want` smallest keys stay: a threshold with exactly that many keys below
-// it is found by bisection, each step one compare and one ballot per 64 keys, and later candidates
-// above it are dropped at once.  So the work is one pass over the candidates whatever their
-// number, where an insertion sort in global memory grew with the square of the neighbourhood
+// The fill collects a query's keys in LDS (wave_collect): one pass over the candidates whatever
+// their number, where an insertion sort in global memory grew with the square of the neighbourhood
 // (11k queries of a 424x240 frame, 3 cm, 30 nearest: 81 us, 134 ms before; the counts 14 us with 16
-// lanes per query, 364 us with one).  A list
-// longer than the buffer comes out in blocks of kFillBlock, each pass taking the keys after the
-// last one written.
+// lanes per query, 364 us with one).  A list longer than the buffer comes out in blocks of
+// kSelBlock, each pass taking the keys after the last one written.
 constexpr int kFillWaves = 4;
-constexpr int kFillCap = 512;               // buffered keys per wavefront (6 KB of LDS)
-constexpr int kFillPer = kFillCap / kWave;  // keys per lane
-constexpr int kFillBlock = kFillCap - kWave;
-constexpr int kFillRank = 2 * kWave;        // up to here lists are ordered by counting ranks
-
-struct FillBuf {
-    double d2[kFillCap];
-    int32_t idx[kFillCap];
-};
-
-__device__ __forceinline__ void fill_sync()
-{
-    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-    __builtin_amdgcn_wave_barrier();
-    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-}
-
-// Keeps the `want` smallest of the buffer's m keys (want < m) and sets (td, ti) so that exactly the
-// kept keys are below it in (d2, index) order.  Run by a whole wavefront; every d2 is in [0, r2).
-__device__ __forceinline__ void fill_prune(FillBuf &buf, int m, int want, double r2, double &td, int32_t &ti)
-{
-    const int lane = lane_id();
-    double d[kFillPer];
-    int32_t x[kFillPer];
-#pragma unroll
-    for (int j = 0; j < kFillPer; ++j) {
-        const int e = lane + kWave * j;
-        d[j] = e < m ? buf.d2[e] : DBL_MAX;
-        x[j] = e < m ? buf.idx[e] : INT_MAX;
-    }
-    auto below = [&](double t) {
-        int c = 0;
-#pragma unroll
-        for (int j = 0; j < kFillPer; ++j) c += __popcll(__ballot(d[j] < t));
-        return c;
-    };
-    // lo has fewer than `want` keys below it, hi more; non-negative doubles order as their bits.
-    // Steps alternate between the place a uniform spread of d2 (points on a surface) would give and
-    // the middle of the bits, which bounds their number.
-    double lo = 0.0, hi = r2;
-    int clo = 0, chi = m;
-    td = -1.0;
-    ti = -1;
-    for (int step = 0;; ++step) {
-        const long long bl = __double_as_longlong(lo), bh = __double_as_longlong(hi);
-        if (bh - bl <= 1) break;  // the keys in question all equal lo
-        double t = __longlong_as_double(bl + ((bh - bl) >> 1));
-        if ((step & 1) == 0) {
-            const double s = lo + (hi - lo) * ((double)(want - clo) / (double)(chi - clo));
-            if (s > lo && s < hi) t = s;
-        }
-        const int c = below(t);
-        if (c == want) {
-            td = t;  // everything below t, whatever its index
-            break;
-        }
-        if (c < want) {
-            lo = t;
-            clo = c;
-        } else {
-            hi = t;
-            chi = c;
-        }
-    }
-    if (td < 0.0) {
-        // ties at lo: of the keys equal to lo, those of the want - clo lowest indices
-        int a = -1, z = INT_MAX - 1;  // count(index <= a) < need <= count(index <= z)
-        while (z - a > 1) {
-            const int mid = a + (z - a) / 2;
-            int c = 0;
-#pragma unroll
-            for (int j = 0; j < kFillPer; ++j) c += __popcll(__ballot(d[j] == lo && x[j] <= mid));
-            if (c < want - clo) a = mid;
-            else z = mid;
-        }
-        td = lo;
-        ti = z + 1;
-    }
-    int pos = 0;
-    fill_sync();
-#pragma unroll
-    for (int j = 0; j < kFillPer; ++j) {
-        const bool keep = key_less(d[j], x[j], td, ti);
-        const uint64_t k = __ballot(keep);
-        if (keep) {
-            const int e = pos + __popcll(k & ((1ull << lane) - 1ull));
-            buf.d2[e] = d[j];
-            buf.idx[e] = x[j];
-        }
-        pos += __popcll(k);
-    }
-    fill_sync();
-}
+constexpr int kFillRank = 2 * kWave;  // up to here lists are ordered by counting ranks
 
 // Writes the buffer's m keys' indices to out in (d2, index) order; the last key goes to (ld, li).
-__device__ __forceinline__ void fill_write(FillBuf &buf, int m, int32_t *__restrict__ out, double &ld, int32_t &li)
+__device__ __forceinline__ void fill_write(SelBuf<false> &buf, int m, int32_t *__restrict__ out, double &ld, int32_t &li)
 {
     const int lane = lane_id();
     if (m <= kFillRank) {
@@ -549,7 +367,7 @@ __device__ __forceinline__ void fill_write(FillBuf &buf, int m, int32_t *__restr
         buf.d2[e] = DBL_MAX;
         buf.idx[e] = INT_MAX;
     }
-    fill_sync();
+    wave_lds_sync();
     for (int k = 2; k <= n2; k *= 2)  // bitonic
         for (int j = k / 2; j > 0; j /= 2) {
             for (int t = lane; t < n2 / 2; t += kWave) {
@@ -563,7 +381,7 @@ __device__ __forceinline__ void fill_write(FillBuf &buf, int m, int32_t *__restr
                     buf.idx[b] = xa;
                 }
             }
-            fill_sync();
+            wave_lds_sync();
         }
     for (int e = lane; e < m; e += kWave) out[e] = buf.idx[e];
     ld = buf.d2[m - 1];
@@ -577,10 +395,9 @@ __global__ __launch_bounds__(kWave *kFillWaves) void k_radius_fill(const float4 
                                                                    const uint32_t *__restrict__ off,
                                                                    int32_t *__restrict__ out)
 {
-    __shared__ FillBuf bufs[kFillWaves];
+    __shared__ SelBuf<false> bufs[kFillWaves];
     const int w = __builtin_amdgcn_readfirstlane((int)threadIdx.x / kWave);
-    const int lane = lane_id();
-    FillBuf &buf = bufs[w];
+    SelBuf<false> &buf = bufs[w];
     const GridView v = make_view(g, start, order, sxyzi);
     const double r2 = (double)g.radius * (double)g.radius;
     for (int i = (int)blockIdx.x * kFillWaves + w; i < n; i += (int)gridDim.x * kFillWaves) {
@@ -592,40 +409,8 @@ __global__ __launch_bounds__(kWave *kFillWaves) void k_radius_fill(const float4 
         double ld = -1.0;  // the last key written
         int32_t li = -1;
         for (int done = 0; done < total;) {
-            const int want = min(total - done, kFillBlock);
-            double td = DBL_MAX;  // keys at or above this are not among the `want` smallest
-            int32_t ti = INT_MAX;
-            int m = 0;
-            fill_sync();
-            group_walk_runs(
-                v, b, lane, kWave, -1,
-                [&](uint32_t s, float4 c, bool valid) {
-                    const double d2 = dist2(c.x, c.y, c.z, p.x, p.y, p.z);
-                    bool in = valid && d2 < r2 && d2 <= td && d2 >= ld;
-                    int32_t ix = 0;
-                    if (in) {
-                        ix = order[s];
-                        in = key_less(d2, ix, td, ti) && key_less(ld, li, d2, ix);
-                    }
-                    const uint64_t k = __ballot(in);
-                    if (in) {
-                        const int e = m + __popcll(k & ((1ull << lane) - 1ull));
-                        buf.d2[e] = d2;
-                        buf.idx[e] = ix;
-                    }
-                    m += __popcll(k);
-                    if (m > kFillBlock) {  // the next 64 might not fit (m > want, too)
-                        fill_sync();
-                        fill_prune(buf, m, want, r2, td, ti);
-                        m = want;
-                    }
-                },
-                [] { return true; });
-            fill_sync();
-            if (m > want) {
-                fill_prune(buf, m, want, r2, td, ti);
-                m = want;
-            }
+            const int want = min(total - done, kSelBlock);
+            const int m = wave_collect(v, b, p, r2, want, ld, li, buf);
             fill_write(buf, m, out + first + done, ld, li);
             done += want;
         }

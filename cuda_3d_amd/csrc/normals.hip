@@ -5,17 +5,16 @@
 //
 // The reference materialises every (query, neighbour) pair, reduces 36-byte raw-moment
 // records by key in FP32 and solves the 3x3 eigenproblem with an FP32 trigonometric closed
-// form.  Here a group of G lanes walks the query's grid runs (all run bounds loaded first, then
-// one flattened candidate walk with several loads in flight per lane), and the neighbourhood
-// sums are accumulated in 2^-40 fixed point scaled by the radius, centred on the query point:
-// integer adds are exact, so neither G nor the reduction order changes the result, which equals
-// the FP64 oracle's.  The colour gradient's sums are the raw ones (sum u u^T, sum u dI); its
+// form.  Here a group of eight lanes walks the query's grid runs (all run bounds loaded first,
+// then one flattened candidate walk), and the neighbourhood sums are accumulated in 2^-40 fixed
+// point scaled by the radius, centred on the query point: integer adds are exact, so the order of
+// the reduction does not change the result, which equals the FP64 oracle's.  The colour gradient's sums are the raw ones (sum u u^T, sum u dI); its
 // tangent projection is applied to the sums in the solve, so they need no normal and can be
-// gathered in the same walk as the normals' (k_moments_pair) when the gradient radius is the
-// smaller one.  A query with more than K > 0 points within the radius is finished by one
-// wavefront that buffers the in-radius candidates in LDS and keeps a candidate iff fewer than K
-// others precede it in (d2, index) order.  The covariance is then diagonalised per point with a
-// cyclic Jacobi iteration in FP64 (only +, -, *, /, sqrt: identical on host and device).
+// gathered in the same walk as the normals' when the gradient radius is the smaller one.  Where
+// the K nearest are wanted the walk keeps the in-radius candidates in LDS and a threshold with
+// exactly K of them below it is bisected by the group; the few queries with more candidates than
+// fit there are finished by one wavefront each.  The covariance is then diagonalised per point with
+// a cyclic Jacobi iteration in FP64 (only +, -, *, /, sqrt: identical on host and device).
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
@@ -24,176 +23,9 @@
 
 #include "gca_device.hpp"
 #include "gca_internal.hpp"
+#include "neighbours.hpp"
 
 namespace gca {
-
-constexpr int kNbCap = 256;          // LDS candidates per wave
-constexpr int kWavesPerBlock = 4;
-
-struct NbBuf {
-    double d2[kNbCap];
-    int32_t idx[kNbCap];
-    int32_t slot[kNbCap];
-    float4 p[kNbCap];
-};
-
-__device__ __forceinline__ void wave_lds_sync()
-{
-    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-    __builtin_amdgcn_wave_barrier();
-    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-}
-
-struct GridRefs {
-    GridDesc g;
-    const uint32_t *start;
-    const int32_t *order;
-    const float4 *sxyzi;
-};
-
-constexpr int kNbRuns = 9;      // grid runs per query when the cell is at least the radius
-constexpr int kOvfUnroll = 2;   // 64-candidate steps in flight per wave in the K-selection walk
-
-// Calls f(slot, idx, point) on the lanes for every selected neighbour of q; returns the
-// number of selected neighbours (wave-uniform).  K == 0: all within radius.  With at most
-// kNbRuns runs (every grid grid_build makes) all run bounds are loaded at once and the runs are
-// walked as one flattened candidate range, kOvfUnroll x 64 candidates in flight; the in-radius
-// candidates go to LDS with their points.  The selection (the K smallest (d2, index) keys) and
-// the count depend only on the candidate set, not on the visiting order.
-template <class F>
-__device__ __forceinline__ int32_t for_each_neighbour(const GridRefs &G, float4 q, int32_t K, NbBuf &buf, F &&f)
-{
-    int32_t lo[3], hi[3];
-    if (!grid_range(G.g, q.x, q.y, q.z, lo, hi)) return 0;
-    const double r2 = (double)G.g.radius * (double)G.g.radius;
-    const int lane = lane_id();
-    const int nry = hi[1] - lo[1] + 1;
-    const int nruns = (hi[0] - lo[0] + 1) * nry;
-    int32_t count = 0;
-    wave_lds_sync();
-    // stores one in-radius candidate per flagged lane at the next free LDS positions
-    auto keep = [&](bool in, uint32_t s, double d2, int32_t ix, float4 p) {
-        const uint64_t m = __ballot(in);
-        if (in) {
-            const int32_t pos = count + __popcll(m & ((1ull << lane) - 1ull));
-            if (K == 0) {
-                f(s, ix, p);
-            } else if (pos < kNbCap) {
-                buf.d2[pos] = d2;
-                buf.idx[pos] = ix;
-                buf.slot[pos] = (int32_t)s;
-                buf.p[pos] = p;
-            }
-        }
-        count += __popcll(m);
-    };
-    if (nruns <= kNbRuns) {
-        uint32_t rs[kNbRuns], cum[kNbRuns + 1];
-#pragma unroll
-        for (int r = 0; r < kNbRuns; ++r) {
-            uint32_t a = 0, b = 0;
-            if (r < nruns) {
-                const int ix = lo[0] + r / nry, iy = lo[1] + r % nry;
-                const int64_t row = ((int64_t)ix * G.g.dims[1] + iy) * G.g.dims[2];
-                a = G.start[row + lo[2]];
-                b = G.start[row + hi[2] + 1];
-            }
-            rs[r] = a;
-            cum[r + 1] = b - a;
-        }
-        cum[0] = 0;
-#pragma unroll
-        for (int r = 0; r < kNbRuns; ++r) cum[r + 1] += cum[r];
-        const uint32_t total = cum[kNbRuns];
-        for (uint32_t f0 = 0; f0 < total; f0 += kWave * kOvfUnroll) {
-            float4 c[kOvfUnroll];
-            int32_t ci[kOvfUnroll];
-            uint32_t cs[kOvfUnroll];
-#pragma unroll
-            for (int u = 0; u < kOvfUnroll; ++u) {
-                const uint32_t fi = f0 + u * kWave + lane;
-                cs[u] = 0;
-                if (fi < total) {
-                    uint32_t sl = rs[0] + fi;
-#pragma unroll
-                    for (int r = 1; r < kNbRuns; ++r)
-                        if (fi >= cum[r]) sl = rs[r] + (fi - cum[r]);
-                    cs[u] = sl;
-                    c[u] = G.sxyzi[sl];
-                    ci[u] = G.order[sl];
-                }
-            }
-#pragma unroll
-            for (int u = 0; u < kOvfUnroll; ++u) {
-                const bool valid = f0 + u * kWave + lane < total;
-                const double d2 = valid ? dist2(c[u].x, c[u].y, c[u].z, q.x, q.y, q.z) : 0.0;
-                keep(valid && d2 < r2, cs[u], d2, valid ? ci[u] : 0, valid ? c[u] : make_float4(0.f, 0.f, 0.f, 0.f));
-            }
-        }
-    } else {
-        // cell smaller than the radius (not produced by grid_build): run by run
-        for (int32_t ix = lo[0]; ix <= hi[0]; ++ix)
-            for (int32_t iy = lo[1]; iy <= hi[1]; ++iy) {
-                const int64_t row = ((int64_t)ix * G.g.dims[1] + iy) * G.g.dims[2];
-                const uint32_t s0 = G.start[row + lo[2]], s1 = G.start[row + hi[2] + 1];
-                for (uint32_t b = s0; b < s1; b += kWave) {
-                    const uint32_t s = b + lane;
-                    bool in = false;
-                    double d2 = 0.0;
-                    float4 p = make_float4(0.f, 0.f, 0.f, 0.f);
-                    int32_t id = 0;
-                    if (s < s1) {
-                        p = G.sxyzi[s];
-                        id = G.order[s];
-                        d2 = dist2(p.x, p.y, p.z, q.x, q.y, q.z);
-                        in = d2 < r2;
-                    }
-                    keep(in, s, d2, id, p);
-                }
-            }
-    }
-    if (K == 0) return count;
-    wave_lds_sync();
-    if (count <= K) {
-        for (int32_t e = lane; e < count; e += kWave) f(buf.slot[e], buf.idx[e], buf.p[e]);
-        return count;
-    }
-    if (count <= kNbCap) {
-        for (int32_t e = lane; e < count; e += kWave) {
-            const double de = buf.d2[e];
-            const int32_t ie = buf.idx[e];
-            int32_t rank = 0;
-            for (int32_t j = 0; j < count; ++j) rank += key_less(buf.d2[j], buf.idx[j], de, ie) ? 1 : 0;
-            if (rank < K) f(buf.slot[e], ie, buf.p[e]);
-        }
-        return K;
-    }
-    // Overflow of the LDS buffer (very dense neighbourhood): rank each candidate against a
-    // rescan of the runs.  Slow but exact; only reached with > kNbCap points within radius.
-    for (int32_t ix = lo[0]; ix <= hi[0]; ++ix)
-        for (int32_t iy = lo[1]; iy <= hi[1]; ++iy) {
-            const int64_t row = ((int64_t)ix * G.g.dims[1] + iy) * G.g.dims[2];
-            const uint32_t s0 = G.start[row + lo[2]], s1 = G.start[row + hi[2] + 1];
-            for (uint32_t s = s0 + lane; s < s1; s += kWave) {
-                const float4 p = G.sxyzi[s];
-                const double de = dist2(p.x, p.y, p.z, q.x, q.y, q.z);
-                if (!(de < r2)) continue;
-                const int32_t ie = G.order[s];
-                int32_t rank = 0;
-                for (int32_t jx = lo[0]; jx <= hi[0] && rank < K; ++jx)
-                    for (int32_t jy = lo[1]; jy <= hi[1] && rank < K; ++jy) {
-                        const int64_t rw = ((int64_t)jx * G.g.dims[1] + jy) * G.g.dims[2];
-                        for (uint32_t t = G.start[rw + lo[2]]; t < G.start[rw + hi[2] + 1]; ++t) {
-                            const float4 c = G.sxyzi[t];
-                            const double dc = dist2(c.x, c.y, c.z, q.x, q.y, q.z);
-                            if (dc < r2 && key_less(dc, G.order[t], de, ie)) ++rank;
-                        }
-                    }
-                if (rank < K) f(s, ie, p);
-            }
-        }
-    return K;
-}
 
 // Cyclic Jacobi for a symmetric 3x3 (same operation sequence as the oracle's orc_eigen3).
 __host__ __device__ inline void jacobi3(double A[3][3], double v[3][3])
@@ -265,13 +97,11 @@ __host__ __device__ inline float4 normal_from_moments(int32_t cnt, const long lo
     return out;
 }
 
-// ---- group walk ------------------------------------------------------------------------------
-// The common case (no K cap, or at most K points within the radius) runs G lanes per query:
-// every lane visits its share of the query's flattened candidate space with kNbUnroll loads in
-// flight and accumulates integer moments; the group then sums them with shuffles.  Integer
-// sums are exact, so the result does not depend on G or on the visiting order.
+// ---- neighbourhood sums ----------------------------------------------------------------------
 constexpr int kNbBlock = 256;
-constexpr int kNbUnroll = 4;
+constexpr int kNbLanes = 8;     // lanes per query
+constexpr int kNbUnroll = 2;    // candidates in flight per lane
+constexpr int kOvfWaves = 4;    // wavefronts per workgroup of the overflow kernel
 
 struct Moments {
     long long S[9];
@@ -279,244 +109,312 @@ struct Moments {
     int32_t pad;
 };
 
-// Calls f(p, d2) on the lane for every candidate of its share with d2 < r^2; returns the
-// group's in-radius count (on every lane of the group).
-template <class F>
-__device__ __forceinline__ int32_t group_walk(const GridRefs &G, float4 q, int g, int gs, F &&f)
-{
-    int32_t lo[3], hi[3];
-    int32_t cnt = 0;
-    if (grid_range(G.g, q.x, q.y, q.z, lo, hi)) {
-        const double r2 = (double)G.g.radius * (double)G.g.radius;
-        const int nry = hi[1] - lo[1] + 1;
-        const int nruns = (hi[0] - lo[0] + 1) * nry;
-        if (nruns <= kNbRuns) {
-            uint32_t rs[kNbRuns], cum[kNbRuns + 1];
+// Neighbourhood sums (2^-40 fixed point) of the neighbours p of a query q, u = (p - q) / r:
+//   KIND 0, normals:  sum u, sum u u^T (xx xy xz yy yz zz)
+//   KIND 1, gradient: sum u u^T, sum u dI with dI = I_p - I_q (raw: the projection onto the query's
+//                     tangent plane is applied to the sums, gradient_from_moments)
+// The query itself contributes exactly zero to every sum (and one to the count).
+// |u_a| <= 1 (to rounding), so the u and u u^T terms are integers up to 2^40, rounded to nearest
+// even by one instruction, and sums of up to kExactTerms of them are exact in FP64: two operations
+// a term, where the 64-bit integer path takes five.  The scale 2^40 is applied as 2^20 per factor:
+// powers of two, so every rounding is that of the plain expressions.  The u dI terms have no such
+// bound and use the general conversion and integer sums; so do all terms of larger neighbourhoods.
+constexpr double kFx20 = 1048576.0;
+constexpr int32_t kExactTerms = 4096;
+
+template <int KIND>
+struct MomentSum {
+    static constexpr int ND = KIND == 0 ? 9 : 6;  // terms bounded by 2^40
+    double d[ND];
+    long long x[9 - ND + 1];  // the u dI terms
+    __device__ __forceinline__ void zero()
+    {
 #pragma unroll
-            for (int r = 0; r < kNbRuns; ++r) {
-                uint32_t a = 0, b = 0;
-                if (r < nruns) {
-                    const int ix = lo[0] + r / nry, iy = lo[1] + r % nry;
-                    const int64_t row = ((int64_t)ix * G.g.dims[1] + iy) * G.g.dims[2];
-                    a = G.start[row + lo[2]];
-                    b = G.start[row + hi[2] + 1];
-                }
-                rs[r] = a;
-                cum[r + 1] = b - a;
-            }
-            cum[0] = 0;
+        for (int k = 0; k < ND; ++k) d[k] = 0.0;
 #pragma unroll
-            for (int r = 0; r < kNbRuns; ++r) cum[r + 1] += cum[r];
-            const uint32_t total = cum[kNbRuns];
-            for (uint32_t f0 = g; f0 < total; f0 += gs * kNbUnroll) {
-                float4 c[kNbUnroll];
-                bool ok[kNbUnroll];
-#pragma unroll
-                for (int u = 0; u < kNbUnroll; ++u) {
-                    const uint32_t fi = f0 + u * gs;
-                    ok[u] = fi < total;
-                    if (ok[u]) {
-                        uint32_t sl = rs[0] + fi;
-#pragma unroll
-                        for (int r = 1; r < kNbRuns; ++r)
-                            if (fi >= cum[r]) sl = rs[r] + (fi - cum[r]);
-                        c[u] = G.sxyzi[sl];
-                    }
-                }
-#pragma unroll
-                for (int u = 0; u < kNbUnroll; ++u) {
-                    if (!ok[u]) continue;
-                    const double d2 = dist2(c[u].x, c[u].y, c[u].z, q.x, q.y, q.z);
-                    if (d2 < r2) {
-                        f(c[u], d2);
-                        ++cnt;
-                    }
-                }
-            }
-        } else {
-            // cell smaller than the radius (not produced by grid_build): plain run walk
-            for (int32_t ix = lo[0]; ix <= hi[0]; ++ix)
-                for (int32_t iy = lo[1]; iy <= hi[1]; ++iy) {
-                    const int64_t row = ((int64_t)ix * G.g.dims[1] + iy) * G.g.dims[2];
-                    const uint32_t s0 = G.start[row + lo[2]], s1 = G.start[row + hi[2] + 1];
-                    for (uint32_t sl = s0 + g; sl < s1; sl += gs) {
-                        const float4 c = G.sxyzi[sl];
-                        const double d2 = dist2(c.x, c.y, c.z, q.x, q.y, q.z);
-                        if (d2 < r2) {
-                            f(c, d2);
-                            ++cnt;
-                        }
-                    }
-                }
+        for (int k = 0; k < 9 - ND; ++k) x[k] = 0;
+    }
+    // inv: 2^20 / radius
+    __device__ __forceinline__ void add(float4 q, float px, float py, float pz, float pw, double inv)
+    {
+        const double w0 = ((double)px - (double)q.x) * inv;
+        const double w1 = ((double)py - (double)q.y) * inv;
+        const double w2 = ((double)pz - (double)q.z) * inv;
+        int k = 0;
+        if constexpr (KIND == 0) {
+            d[0] += __builtin_rint(w0 * kFx20);
+            d[1] += __builtin_rint(w1 * kFx20);
+            d[2] += __builtin_rint(w2 * kFx20);
+            k = 3;
+        }
+        d[k] += __builtin_rint(w0 * w0);
+        d[k + 1] += __builtin_rint(w0 * w1);
+        d[k + 2] += __builtin_rint(w0 * w2);
+        d[k + 3] += __builtin_rint(w1 * w1);
+        d[k + 4] += __builtin_rint(w1 * w2);
+        d[k + 5] += __builtin_rint(w2 * w2);
+        if constexpr (KIND == 1) {
+            const double dI = (double)pw - (double)q.w;
+            x[0] += fx((w0 * dI) * kFx20);
+            x[1] += fx((w1 * dI) * kFx20);
+            x[2] += fx((w2 * dI) * kFx20);
         }
     }
-    for (int m = 1; m < gs; m <<= 1) cnt += __shfl_xor(cnt, m, kWave);
+    // The sums as integers.
+    __device__ __forceinline__ void take(long long S[9]) const
+    {
+#pragma unroll
+        for (int k = 0; k < ND; ++k) S[k] = (long long)d[k];
+#pragma unroll
+        for (int k = ND; k < 9; ++k) S[k] = x[k - ND];
+    }
+};
+
+// The sums over all neighbours within the radius (no K cap) by the gs lanes of a group: the lane's
+// part; returns its part of the count.
+template <int KIND>
+__device__ __forceinline__ int32_t walk_moments(const GridView &v, const Box &b, float4 q, int gl, int gs, double r2,
+                                                double inv, MomentSum<KIND> &A)
+{
+    A.zero();
+    int32_t cnt = 0;
+    group_walk_box<kNbUnroll>(
+        v, b, gl, gs,
+        [&](uint32_t, float4 c, bool valid) {
+            if (valid && dist2(c.x, c.y, c.z, q.x, q.y, q.z) < r2) {
+                A.add(q, c.x, c.y, c.z, c.w, inv);
+                ++cnt;
+            }
+        });
     return cnt;
 }
 
-// Neighbourhood moments (2^-40 fixed point) of one neighbour p of query q, u = (p - q) / r.
-// Every neighbour is within the radius, so |u_a| <= 1 (to rounding) and the u and u u^T terms
-// are below 2^41 in fixed point: fx_small converts them; the u dI terms use the general fx.
-//
-//   normals:  S = sum u, sum u u^T (xx xy xz yy yz zz)
-//   gradient: S = sum u u^T, sum u dI with dI = I_p - I_q (raw: the projection onto the query's
-//             tangent plane is applied to the sums, gradient_from_moments)
-// The query itself contributes exactly zero to every sum (and one to the count).
+// The same with integer sums, for neighbourhoods beyond kExactTerms: term by term.
 template <int KIND>
-__device__ __forceinline__ void add_moments(long long S[9], float4 q, float4 p, double inv_r)
+__device__ __forceinline__ void walk_moments_wide(const GridView &v, const Box &b, float4 q, int gl, int gs, double r2,
+                                                  double inv, long long S[9])
 {
-    if (KIND == 0) {
-        const double u0 = ((double)p.x - (double)q.x) * inv_r;
-        const double u1 = ((double)p.y - (double)q.y) * inv_r;
-        const double u2 = ((double)p.z - (double)q.z) * inv_r;
-        S[0] += fx_small(u0 * kFx40);
-        S[1] += fx_small(u1 * kFx40);
-        S[2] += fx_small(u2 * kFx40);
-        S[3] += fx_small((u0 * u0) * kFx40);
-        S[4] += fx_small((u0 * u1) * kFx40);
-        S[5] += fx_small((u0 * u2) * kFx40);
-        S[6] += fx_small((u1 * u1) * kFx40);
-        S[7] += fx_small((u1 * u2) * kFx40);
-        S[8] += fx_small((u2 * u2) * kFx40);
-    } else {
-        const double u0 = ((double)p.x - (double)q.x) * inv_r;
-        const double u1 = ((double)p.y - (double)q.y) * inv_r;
-        const double u2 = ((double)p.z - (double)q.z) * inv_r;
-        const double dI = (double)p.w - (double)q.w;
-        S[0] += fx_small((u0 * u0) * kFx40);
-        S[1] += fx_small((u0 * u1) * kFx40);
-        S[2] += fx_small((u0 * u2) * kFx40);
-        S[3] += fx_small((u1 * u1) * kFx40);
-        S[4] += fx_small((u1 * u2) * kFx40);
-        S[5] += fx_small((u2 * u2) * kFx40);
-        S[6] += fx((u0 * dI) * kFx40);
-        S[7] += fx((u1 * dI) * kFx40);
-        S[8] += fx((u2 * dI) * kFx40);
-    }
+#pragma unroll
+    for (int k = 0; k < 9; ++k) S[k] = 0;
+    group_walk_box<1>(
+        v, b, gl, gs,
+        [&](uint32_t, float4 c, bool valid) {
+            if (valid && dist2(c.x, c.y, c.z, q.x, q.y, q.z) < r2) {
+                MomentSum<KIND> A;
+                long long t[9];
+                A.zero();
+                A.add(q, c.x, c.y, c.z, c.w, inv);
+                A.take(t);
+#pragma unroll
+                for (int k = 0; k < 9; ++k) S[k] += t[k];
+            }
+        });
 }
 
-// Pass 1: moments of every query whose neighbourhood needs no K selection; queries with more
-// than K > 0 points within the radius are appended to the overflow list instead.
-template <int KIND>
-__global__ __launch_bounds__(kNbBlock) void k_moments(const float4 *__restrict__ xyzi, const float4 *__restrict__ nrm,
-                                                      const CloudHdr *__restrict__ hdr, GridDesc g,
-                                                      const uint32_t *__restrict__ start,
-                                                      const int32_t *__restrict__ order,
-                                                      const float4 *__restrict__ sxyzi, int32_t K, int gs,
-                                                      Moments *__restrict__ mom, int32_t *__restrict__ ovf,
-                                                      uint32_t *__restrict__ ovf_n)
+// The wavefront's sums and a count, stored by its first lane.
+__device__ __forceinline__ void wave_store(long long S[9], int32_t cnt, Moments &M)
 {
-    const GridRefs G{g, start, order, sxyzi};
+#pragma unroll
+    for (int c = 0; c < 9; ++c) S[c] = wave_sum(S[c]);
+    if (lane_id() != 0) return;
+#pragma unroll
+    for (int c = 0; c < 9; ++c) M.S[c] = S[c];
+    M.cnt = cnt;
+}
+
+// The group's sums and a count, stored by its first lane.
+template <int KIND>
+__device__ __forceinline__ void group_store(MomentSum<KIND> &A, int32_t cnt, int gl, Moments &M)
+{
+    constexpr int ND = MomentSum<KIND>::ND;
+#pragma unroll
+    for (int k = 0; k < ND; ++k) A.d[k] = group_sum<kNbLanes>(A.d[k]);
+#pragma unroll
+    for (int k = 0; k < 9 - ND; ++k) A.x[k] = group_sum<kNbLanes>(A.x[k]);
+    if (gl != 0) return;
+#pragma unroll
+    for (int k = 0; k < ND; ++k) M.S[k] = (long long)A.d[k];
+#pragma unroll
+    for (int k = ND; k < 9; ++k) M.S[k] = A.x[k - ND];
+    M.cnt = cnt;
+}
+
+// Sums without a K cap: 27 us for the gradient of those points at 2 cm (32 us with 64-bit integer
+// sums and a division per cell bound).  Eight lanes per query: 4 and 16 measured 1-2 % and 5 % slower on a 640x480 target at 1 cm, and
+// 2 and 4 % on the overlapped odometry of such frames.
+template <int KIND>
+__global__ __launch_bounds__(kNbBlock) void k_moments(const float4 *__restrict__ xyzi, const CloudHdr *__restrict__ hdr,
+                                                      GridDesc g, const uint32_t *__restrict__ start,
+                                                      const float4 *__restrict__ sxyzi, Moments *__restrict__ mom)
+{
+    const GridView v = make_view(g, start, nullptr, sxyzi);
     const int n = hdr->n;
-    const int lg = __builtin_ctz((unsigned)gs);
-    const int gl = (int)threadIdx.x & (gs - 1);
-    const int per_block = kNbBlock >> lg;
-    const double inv_r = 1.0 / (double)g.radius;
-    for (int base = blockIdx.x * per_block; base < n; base += gridDim.x * per_block) {
-        const int qi = base + ((int)threadIdx.x >> lg);
-        if (qi >= n) break;  // whole groups leave together
-        const float4 q = xyzi[qi];
-        long long S[9] = {0, 0, 0, 0, 0, 0, 0, 0, 0};
-        const int32_t cnt = group_walk(G, q, gl, gs, [&](float4 p, double) { add_moments<KIND>(S, q, p, inv_r); });
-        if (K > 0 && cnt > K) {
-            if (gl == 0) ovf[atomicAdd(ovf_n, 1u)] = qi;
-            continue;
-        }
+    const int gl = (int)threadIdx.x & (kNbLanes - 1);
+    const double r2 = (double)g.radius * (double)g.radius;
+    const double inv = kFx20 * (1.0 / (double)g.radius);
+    for (int i = (int)(blockIdx.x * kNbBlock + threadIdx.x) / kNbLanes; i < n; i += (int)(gridDim.x * kNbBlock) / kNbLanes) {
+        const float4 q = xyzi[i];
+        MomentSum<KIND> A;
+        Box b;
+        int32_t cnt = 0;
+        A.zero();
+        if (grid_range(g, q.x, q.y, q.z, b.lo, b.hi)) cnt = walk_moments<KIND>(v, b, q, gl, kNbLanes, r2, inv, A);
+        cnt = (int32_t)group_sum<kNbLanes>((uint32_t)cnt);
+        if (cnt <= kExactTerms) {
+            group_store<KIND>(A, cnt, gl, mom[i]);
+        } else {
+            long long S[9];
+            walk_moments_wide<KIND>(v, b, q, gl, kNbLanes, r2, inv, S);
 #pragma unroll
-        for (int c = 0; c < 9; ++c)
-            for (int m = 1; m < gs; m <<= 1) S[c] += __shfl_xor(S[c], m, kWave);
-        if (gl == 0) {
-            Moments &M = mom[qi];
+            for (int k = 0; k < 9; ++k) S[k] = group_sum<kNbLanes>(S[k]);
+            if (gl == 0) {
+                Moments &M = mom[i];
 #pragma unroll
-            for (int c = 0; c < 9; ++c) M.S[c] = S[c];
-            M.cnt = cnt;
+                for (int k = 0; k < 9; ++k) M.S[k] = S[k];
+                M.cnt = cnt;
+            }
         }
     }
 }
 
-// Pass 1, normals and colour gradient together (gradient radius rg <= the normals' radius, no K
-// cap for the gradient): the walk covers the normals' radius and the candidates within rg also
-// add the gradient's raw sums, with the same d2 < rg^2 test as the gradient's own walk, so both
-// moment sets equal those of separate walks.  A query with more than K > 0 points within the
-// normals' radius goes to the overflow list for its normal moments; its gradient sums are
-// complete here.
-struct PairArgs {
+// Sums over the K > 0 nearest neighbours within the radius (KIND), and with PAIR (KIND 0) also the
+// colour gradient's over all neighbours within rg <= the radius, from one walk.
+//   1. the walk puts the in-radius candidates into the group's part of LDS, packed;
+//   2. if there are more than K, the group bisects a threshold with exactly K distances below it:
+//      each lane counts among its own candidates (in registers), the counts are added across the
+//      group by data-parallel moves;
+//   3. every lane adds its selected candidates: packed, so the lanes are busy, where adding in the
+//      walk runs at the share of candidates that are in the radius (about a third).
+// Ties at the threshold are settled by index.  A query with more than kSelCandidates in-radius
+// candidates goes to the overflow list.  Bound half by instruction issue (the walk's tests), half by
+// the latency of the cell bounds and candidates.  110k points of a raw 640x480 frame at 1 cm, the 30
+// nearest of about 50 within 2.5 cm: 37 us and 5 us for the (empty) overflow launch, where adding in
+// the walk and ranking every larger neighbourhood by a wavefront of its own took 81 and 75 us.
+// LDS: 32 groups x 96 candidates x 12 bytes (36 KB, four workgroups per CU), 16 bytes with PAIR.
+constexpr int kSelCandidates = 96;
+
+struct SelArgs {
     const float4 *xyzi;
     const CloudHdr *hdr;
     GridDesc g;
     const uint32_t *start;
     const int32_t *order;
     const float4 *sxyzi;
-    int32_t K, gs;
-    double rg;
+    int32_t K, pad;
+    double rg;  // PAIR
     Moments *mom, *mom_g;
     int32_t *ovf;
     uint32_t *ovf_n;
 };
 
-template <int N>
-__global__ __launch_bounds__(kNbBlock) void k_moments_pair(Jobs<PairArgs, N> J)
+template <int KIND, bool PAIR, int N>
+__global__ __launch_bounds__(kNbBlock) void k_moments_sel(Jobs<SelArgs, N> J)
 {
-    const PairArgs &A = J.a[N == 1 ? 0 : blockIdx.y];
-    const float4 *__restrict__ xyzi = A.xyzi;
+    constexpr int PER = kSelCandidates / kNbLanes;
+    constexpr int WORDS = KIND == 1 || PAIR ? 4 : 3;  // the gradient's candidates carry their intensity
+    __shared__ float cand[kNbBlock / kNbLanes][WORDS][kSelCandidates];
+    const SelArgs &A = J.a[N == 1 ? 0 : blockIdx.y];
     const GridDesc &g = A.g;
-    const int32_t K = A.K;
-    const int gs = A.gs;
-    const double rg = A.rg;
-    Moments *__restrict__ mom = A.mom;
-    Moments *__restrict__ mom_g = A.mom_g;
-    int32_t *__restrict__ ovf = A.ovf;
-    uint32_t *__restrict__ ovf_n = A.ovf_n;
-    const GridRefs G{g, A.start, A.order, A.sxyzi};
+    const GridView v = make_view(g, A.start, nullptr, A.sxyzi);
     const int n = A.hdr->n;
-    const int lg = __builtin_ctz((unsigned)gs);
-    const int gl = (int)threadIdx.x & (gs - 1);
-    const int per_block = kNbBlock >> lg;
-    const double inv_r = 1.0 / (double)g.radius;
-    const double inv_rg = 1.0 / rg;
-    const double rg2 = rg * rg;
-    for (int base = blockIdx.x * per_block; base < n; base += gridDim.x * per_block) {
-        const int qi = base + ((int)threadIdx.x >> lg);
-        if (qi >= n) break;  // whole groups leave together
-        const float4 q = xyzi[qi];
-        long long S[9] = {0, 0, 0, 0, 0, 0, 0, 0, 0}, Sg[9] = {0, 0, 0, 0, 0, 0, 0, 0, 0};
-        int32_t cg = 0;
-        const int32_t cnt = group_walk(G, q, gl, gs, [&](float4 p, double d2) {
-            add_moments<0>(S, q, p, inv_r);
-            if (d2 < rg2) {
-                add_moments<1>(Sg, q, p, inv_rg);
-                ++cg;
+    const int32_t K = A.K;
+    const int gl = (int)threadIdx.x & (kNbLanes - 1);
+    const int base = lane_id() & ~(kNbLanes - 1);  // the group's first lane in its wavefront
+    auto &C = cand[(int)threadIdx.x / kNbLanes];
+    const double r2 = (double)g.radius * (double)g.radius;
+    const double inv = kFx20 * (1.0 / (double)g.radius);
+    const double rg2 = PAIR ? A.rg * A.rg : 0.0, inv_g = PAIR ? kFx20 * (1.0 / A.rg) : 0.0;
+    for (int i = (int)(blockIdx.x * kNbBlock + threadIdx.x) / kNbLanes; i < n; i += (int)(gridDim.x * kNbBlock) / kNbLanes) {
+        const float4 q = A.xyzi[i];
+        Box b;
+        int32_t cnt = 0;
+        const bool box = grid_range(g, q.x, q.y, q.z, b.lo, b.hi);
+        wave_lds_sync();
+        if (box)
+            group_walk_box<kNbUnroll>(
+                v, b, gl, kNbLanes,
+                [&](uint32_t, float4 c, bool valid) {
+                    const bool in = valid && dist2(c.x, c.y, c.z, q.x, q.y, q.z) < r2;
+                    const uint32_t m = (uint32_t)(__ballot(in) >> base) & ((1u << kNbLanes) - 1u);
+                    const int pos = cnt + __popc(m & ((1u << gl) - 1u));
+                    if (in && pos < kSelCandidates) {
+                        C[0][pos] = c.x;
+                        C[1][pos] = c.y;
+                        C[2][pos] = c.z;
+                        if (WORDS == 4) C[WORDS - 1][pos] = c.w;
+                    }
+                    cnt += __popc(m);
+                });
+        wave_lds_sync();
+        const bool over = cnt > kSelCandidates;
+        if (!over) {
+            double d[PER];
+#pragma unroll
+            for (int j = 0; j < PER; ++j) {
+                const int e = gl + kNbLanes * j;
+                d[j] = e < cnt ? dist2(C[0][e], C[1][e], C[2][e], q.x, q.y, q.z) : DBL_MAX;
             }
-        });
-        for (int m = 1; m < gs; m <<= 1) cg += __shfl_xor(cg, m, kWave);
+            double thr = r2;  // all of them
+            int below = K;    // of the K, how many are below thr: fewer only for a tie at thr
+            if (cnt > K) {
+                const bool plain = find_threshold(
+                    cnt, K, r2, thr, below,
+                    [&](double t) {
+                        uint32_t c = 0;
 #pragma unroll
-        for (int c = 0; c < 9; ++c)
-            for (int m = 1; m < gs; m <<= 1) Sg[c] += __shfl_xor(Sg[c], m, kWave);
-        if (gl == 0) {
-            Moments &M = mom_g[qi];
+                        for (int j = 0; j < PER; ++j) c += d[j] < t ? 1u : 0u;
+                        return (int)group_sum<kNbLanes>(c);
+                    },
+                    [&](double t) {
+                        double v = DBL_MAX;
 #pragma unroll
-            for (int c = 0; c < 9; ++c) M.S[c] = Sg[c];
-            M.cnt = cg;
+                        for (int j = 0; j < PER; ++j) v = d[j] >= t ? fmin(v, d[j]) : v;
+                        return group_min<kNbLanes>(v);
+                    });
+                if (plain) below = K;
+            }
+            MomentSum<KIND> M;
+            MomentSum<1> Mg;
+            uint32_t cg = 0;
+            M.zero();
+            Mg.zero();
+#pragma unroll
+            for (int j = 0; j < PER; ++j) {
+                const int e = gl + kNbLanes * j;
+                if (!(d[j] < r2)) continue;
+                const float x = C[0][e], y = C[1][e], z = C[2][e], w = WORDS == 4 ? C[WORDS - 1][e] : 0.f;
+                if (d[j] < thr) M.add(q, x, y, z, w, inv);
+                if (PAIR && d[j] < rg2) {
+                    Mg.add(q, x, y, z, w, inv_g);
+                    ++cg;
+                }
+            }
+            // a tie (rare): of the points at that distance, those of the lowest indices, one a walk
+            for (uint32_t last = 0; below < K; ++below) {
+                uint32_t first = UINT_MAX;  // index + 1
+                float4 p = q;
+                group_walk_box<1>(v, b, gl, kNbLanes, [&](uint32_t s, float4 c, bool valid) {
+                    if (!valid || dist2(c.x, c.y, c.z, q.x, q.y, q.z) != thr) return;
+                    const uint32_t ix = (uint32_t)A.order[s] + 1u;
+                    if (ix > last && ix < first) {
+                        first = ix;
+                        p = c;
+                    }
+                });
+                last = group_min<kNbLanes>(first);
+                if (first == last) M.add(q, p.x, p.y, p.z, p.w, inv);
+            }
+            group_store<KIND>(M, min(cnt, K), gl, A.mom[i]);
+            if (PAIR) group_store<1>(Mg, (int32_t)group_sum<kNbLanes>(cg), gl, A.mom_g[i]);
         }
-        if (K > 0 && cnt > K) {
-            if (gl == 0) ovf[atomicAdd(ovf_n, 1u)] = qi;
-            continue;
-        }
-#pragma unroll
-        for (int c = 0; c < 9; ++c)
-            for (int m = 1; m < gs; m <<= 1) S[c] += __shfl_xor(S[c], m, kWave);
-        if (gl == 0) {
-            Moments &M = mom[qi];
-#pragma unroll
-            for (int c = 0; c < 9; ++c) M.S[c] = S[c];
-            M.cnt = cnt;
-        }
+        if (over && gl == 0) A.ovf[atomicAdd(A.ovf_n, 1u)] = i;
     }
 }
 
-// Pass 2: the overflow queries, one wavefront each, with exact K-nearest selection.
+// The overflow queries, one wavefront each: the K smallest (d2, index) keys by wave_collect; with
+// mom_g, then the gradient's sums over all neighbours within rg.
 struct OvfArgs {
-    const float4 *xyzi, *nrm;
+    const float4 *xyzi;
     const CloudHdr *hdr;
     GridDesc g;
     const uint32_t *start;
@@ -525,39 +423,76 @@ struct OvfArgs {
     int32_t K, pad;
     const int32_t *ovf;
     const uint32_t *ovf_n;
-    Moments *mom;
+    Moments *mom, *mom_g;
+    double rg;
 };
 
 template <int KIND, int N>
-__global__ __launch_bounds__(kWave *kWavesPerBlock) void k_moments_overflow(Jobs<OvfArgs, N> J)
+__global__ __launch_bounds__(kWave *kOvfWaves) void k_moments_overflow(Jobs<OvfArgs, N> J)
 {
     const OvfArgs &A = J.a[N == 1 ? 0 : blockIdx.y];
-    const float4 *__restrict__ xyzi = A.xyzi;
     const GridDesc &g = A.g;
     const int32_t K = A.K;
-    const int32_t *__restrict__ ovf = A.ovf;
-    Moments *__restrict__ mom = A.mom;
-    __shared__ NbBuf bufs[kWavesPerBlock];
-    const int w = threadIdx.x / kWave;
-    NbBuf &buf = bufs[w];
-    const GridRefs G{g, A.start, A.order, A.sxyzi};
+    __shared__ SelBuf<true> bufs[kOvfWaves];
+    const int w = __builtin_amdgcn_readfirstlane((int)threadIdx.x / kWave);
+    const int lane = lane_id();
+    SelBuf<true> &buf = bufs[w];
+    const GridView v = make_view(g, A.start, A.order, A.sxyzi);
     const int n = A.hdr->n;
     const uint32_t m = *A.ovf_n;
-    const double inv_r = 1.0 / (double)g.radius;
-    for (uint32_t e = blockIdx.x * kWavesPerBlock + w; e < m; e += gridDim.x * kWavesPerBlock) {
-        const int qi = ovf[e];
+    const double r2 = (double)g.radius * (double)g.radius;
+    const double inv = kFx20 * (1.0 / (double)g.radius);
+    for (uint32_t e = blockIdx.x * kOvfWaves + w; e < m; e += gridDim.x * kOvfWaves) {
+        const int qi = A.ovf[e];
         if (qi < 0 || qi >= n) continue;
-        const float4 q = xyzi[qi];
-        long long S[9] = {0, 0, 0, 0, 0, 0, 0, 0, 0};
-        const int32_t cnt = for_each_neighbour(G, q, K, buf, [&](uint32_t, int32_t, float4 p) {
-            add_moments<KIND>(S, q, p, inv_r);
-        });
+        const float4 q = A.xyzi[qi];  // in reach of the grid, or it would have no candidates
+        long long S[9] = {0, 0, 0, 0, 0, 0, 0, 0, 0}, t[9];
+        int32_t cnt = 0;
+        Box b;
+        if (!grid_range(g, q.x, q.y, q.z, b.lo, b.hi)) continue;
+        {
+            MomentSum<KIND> M;
+            double ld = -1.0;  // the largest key taken (K beyond one collection: several)
+            int32_t li = -1;
+            while (cnt < K) {
+                const int want = min(K - cnt, kSelBlock);
+                const int got = wave_collect(v, b, q, r2, want, ld, li, buf);
+                double md = -1.0;
+                int32_t mi = -1;
+                M.zero();
+                for (int k = lane; k < got; k += kWave) {
+                    const float4 p = v.sxyzi[buf.slot[k]];
+                    M.add(q, p.x, p.y, p.z, p.w, inv);
+                    if (key_less(md, mi, buf.d2[k], buf.idx[k])) {
+                        md = buf.d2[k];
+                        mi = buf.idx[k];
+                    }
+                }
+                M.take(t);
 #pragma unroll
-        for (int c = 0; c < 9; ++c) S[c] = wave_sum(S[c]);
-        if (lane_id() == 0) {
-            Moments &M = mom[qi];
-            for (int c = 0; c < 9; ++c) M.S[c] = S[c];
-            M.cnt = cnt;
+                for (int k = 0; k < 9; ++k) S[k] += t[k];
+                cnt += got;
+                if (got < want || cnt >= K) break;
+                for (int s = 1; s < kWave; s <<= 1) {
+                    const double od = __shfl_xor(md, s, kWave);
+                    const int32_t oi = __shfl_xor(mi, s, kWave);
+                    if (key_less(md, mi, od, oi)) {
+                        md = od;
+                        mi = oi;
+                    }
+                }
+                ld = md;
+                li = mi;
+            }
+        }
+        wave_store(S, cnt, A.mom[qi]);
+        if (KIND == 0 && A.mom_g) {
+            const double rg2 = A.rg * A.rg, inv_g = kFx20 * (1.0 / A.rg);
+            MomentSum<1> M;
+            const int32_t cg = wave_sum(walk_moments<1>(v, b, q, lane, kWave, rg2, inv_g, M));
+            if (cg <= kExactTerms) M.take(S);
+            else walk_moments_wide<1>(v, b, q, lane, kWave, rg2, inv_g, S);
+            wave_store(S, cg, A.mom_g[qi]);
         }
     }
 }
@@ -683,13 +618,17 @@ static unsigned grid_for(int64_t items, int per_block, int64_t cap)
     return (unsigned)std::min<int64_t>(cap, std::max<int64_t>(1, (items + per_block - 1) / per_block));
 }
 
-static int normals_lanes(gca_ctx ctx) { return ctx->tune[GCA_TUNE_NORMALS_LANES] ? ctx->tune[GCA_TUNE_NORMALS_LANES] : 8; }
+// The sums without a K cap of the cloud of A, on grid d.
+template <int KIND>
+static void launch_all(dim3 grid, hipStream_t stream, const SelArgs &A, const GridDesc &d, Moments *mom)
+{
+    hipLaunchKernelGGL(k_moments<KIND>, grid, dim3(kNbBlock), 0, stream, A.xyzi, A.hdr, d, A.start, A.sxyzi, mom);
+}
 
 template <int KIND>
 static int32_t launch_moments_pipeline(gca_ctx ctx, gca_cloud c, float radius, int32_t K, float4 *out)
 {
     const Grid &G = c->grid;
-    const int gs = normals_lanes(ctx);
     const int64_t cap = std::max<int64_t>(c->cap, 1);
     Moments *mom = (Moments *)ctx_scratch(ctx, 17, sizeof(Moments) * cap, false);
     int32_t *ovf = (int32_t *)ctx_scratch(ctx, 18, sizeof(int32_t) * cap, false);
@@ -697,12 +636,15 @@ static int32_t launch_moments_pipeline(gca_ctx ctx, gca_cloud c, float radius, i
     if (!mom || !ovf || !ovf_n) return GCA_ERR_OUT_OF_MEMORY;
     const GridDesc d = query_desc(G, radius);
     StageTimer timer(ctx, KIND == 0 ? GCA_STAGE_NORMALS : GCA_STAGE_GRADIENT);
-    hipLaunchKernelGGL(k_moments<KIND>, dim3(grid_for(cap, kNbBlock / gs, 4096)), dim3(kNbBlock), 0, ctx->stream,
-                       c->xyzi, c->nrm, c->hdr, d, G.start, G.order, G.sxyzi, K, gs, mom, ovf, ovf_n);
+    const dim3 grid(grid_for(cap, kNbBlock / kNbLanes, 4096));
+    const Jobs<SelArgs, 1> sj{{{c->xyzi, c->hdr, d, G.start, G.order, G.sxyzi, K, 0, 0.0, mom, nullptr, ovf, ovf_n}}};
     if (K > 0) {
-        const Jobs<OvfArgs, 1> oj{{{c->xyzi, c->nrm, c->hdr, d, G.start, G.order, G.sxyzi, K, 0, ovf, ovf_n, mom}}};
-        hipLaunchKernelGGL((k_moments_overflow<KIND, 1>), dim3(grid_for(cap, kWavesPerBlock, 1024)),
-                           dim3(kWave * kWavesPerBlock), 0, ctx->stream, oj);
+        hipLaunchKernelGGL((k_moments_sel<KIND, false, 1>), grid, dim3(kNbBlock), 0, ctx->stream, sj);
+        const Jobs<OvfArgs, 1> oj{{{c->xyzi, c->hdr, d, G.start, G.order, G.sxyzi, K, 0, ovf, ovf_n, mom, nullptr, 0.0}}};
+        hipLaunchKernelGGL((k_moments_overflow<KIND, 1>), dim3(grid_for(cap, kOvfWaves, 1024)), dim3(kWave * kOvfWaves),
+                           0, ctx->stream, oj);
+    } else {
+        launch_all<KIND>(grid, ctx->stream, sj.a[0], d, mom);
     }
     hipLaunchKernelGGL(k_solve<KIND>, dim3(grid_for(cap, kNbBlock, 2048)), dim3(kNbBlock), 0, ctx->stream, c->hdr,
                        (const Moments *)mom, (const float4 *)c->nrm, (double)radius, out, ovf_n);
@@ -722,7 +664,7 @@ int32_t launch_gradient(gca_ctx ctx, gca_cloud c, float radius, int32_t K)
 
 // The three kernels of one joint normals + gradient call, as jobs.
 struct PairJobs {
-    PairArgs pair;
+    SelArgs pair;
     OvfArgs ovf;
     SolveArgs solve;
     unsigned nb_pair, nb_ovf, nb_solve;
@@ -737,7 +679,6 @@ static int32_t pair_prepare(gca_ctx ctx, gca_cloud c, float radius, int32_t K, f
         GCA_HIP(hipMalloc(&G.snrm, sizeof(float4) * G.cap_pts));
         GCA_HIP(hipMalloc(&G.sgrad, sizeof(float4) * G.cap_pts));
     }
-    const int gs = normals_lanes(ctx);
     const int64_t cap = std::max<int64_t>(c->cap, 1);
     Moments *mom = (Moments *)ctx_scratch(ctx, 17, sizeof(Moments) * cap, false);
     int32_t *ovf = (int32_t *)ctx_scratch(ctx, 18, sizeof(int32_t) * cap, false);
@@ -746,39 +687,46 @@ static int32_t pair_prepare(gca_ctx ctx, gca_cloud c, float radius, int32_t K, f
     if (!mom || !ovf || !ovf_n || !mom_g) return GCA_ERR_OUT_OF_MEMORY;
     const GridDesc d = query_desc(G, radius);
     const double rg = (double)gradient_radius;
-    pj->pair = PairArgs{c->xyzi, c->hdr, d, G.start, G.order, G.sxyzi, K, gs, rg, mom, mom_g, ovf, ovf_n};
-    pj->ovf = OvfArgs{c->xyzi, c->nrm, c->hdr, d, G.start, G.order, G.sxyzi, K, 0, ovf, ovf_n, mom};
+    pj->pair = SelArgs{c->xyzi, c->hdr, d, G.start, G.order, G.sxyzi, K, 0, rg, mom, mom_g, ovf, ovf_n};
+    pj->ovf = OvfArgs{c->xyzi, c->hdr, d, G.start, G.order, G.sxyzi, K, 0, ovf, ovf_n, mom, mom_g, rg};
     pj->solve = SolveArgs{c->hdr, mom, mom_g, rg, c->nrm, c->grad, grid_attrs ? (const int32_t *)G.order : nullptr,
                           grid_attrs ? G.snrm : nullptr, grid_attrs ? G.sgrad : nullptr, ovf_n};
-    pj->nb_pair = grid_for(cap, kNbBlock / gs, 4096);
-    pj->nb_ovf = K > 0 ? grid_for(cap, kWavesPerBlock, 1024) : 0;
+    pj->nb_pair = grid_for(cap, kNbBlock / kNbLanes, 4096);
+    pj->nb_ovf = grid_for(cap, kOvfWaves, 1024);
     pj->nb_solve = grid_for(cap, kNbBlock, 2048);
     return GCA_OK;
 }
 
-// moments (one walk), overflow K-selection (jobs with K > 0), solve: each kernel once for all nj
-// calls (blockIdx.y = call), on stream.  A job without K selection contributes no overflow
-// workgroups' work: its overflow list stays empty (count zero), so its rows of the overflow
-// launch find nothing.
+// moments, overflow K-selection, solve: each kernel once for all nj calls (blockIdx.y = call), on
+// stream.  A call without a K cap has no selection to share a walk with, so its two sums come from
+// a walk each.
 template <int N>
 static int32_t pair_launch(hipStream_t stream, const PairJobs *pj, int nj)
 {
-    Jobs<PairArgs, N> pair{};
+    Jobs<SelArgs, N> pair{};
     Jobs<OvfArgs, N> ovf{};
     Jobs<SolveArgs, N> solve{};
-    unsigned nb_pair = 1, nb_ovf = 0, nb_solve = 1;
+    unsigned nb_pair = 1, nb_ovf = 1, nb_solve = 1, nsel = 0;
     for (int j = 0; j < nj; ++j) {
-        pair.a[j] = pj[j].pair;
-        ovf.a[j] = pj[j].ovf;
+        const SelArgs &A = pj[j].pair;
+        if (A.K > 0) {
+            pair.a[nsel] = A;
+            ovf.a[nsel++] = pj[j].ovf;
+            nb_pair = std::max(nb_pair, pj[j].nb_pair);
+            nb_ovf = std::max(nb_ovf, pj[j].nb_ovf);
+        } else {
+            GridDesc dg = A.g;
+            dg.radius = (float)A.rg;
+            launch_all<0>(dim3(pj[j].nb_pair), stream, A, A.g, A.mom);
+            launch_all<1>(dim3(pj[j].nb_pair), stream, A, dg, A.mom_g);
+        }
         solve.a[j] = pj[j].solve;
-        nb_pair = std::max(nb_pair, pj[j].nb_pair);
-        nb_ovf = std::max(nb_ovf, pj[j].nb_ovf);
         nb_solve = std::max(nb_solve, pj[j].nb_solve);
     }
-    hipLaunchKernelGGL(k_moments_pair<N>, dim3(nb_pair, (unsigned)nj), dim3(kNbBlock), 0, stream, pair);
-    if (nb_ovf > 0)
-        hipLaunchKernelGGL((k_moments_overflow<0, N>), dim3(nb_ovf, (unsigned)nj), dim3(kWave * kWavesPerBlock), 0,
-                           stream, ovf);
+    if (nsel > 0) {
+        hipLaunchKernelGGL((k_moments_sel<0, true, N>), dim3(nb_pair, nsel), dim3(kNbBlock), 0, stream, pair);
+        hipLaunchKernelGGL((k_moments_overflow<0, N>), dim3(nb_ovf, nsel), dim3(kWave * kOvfWaves), 0, stream, ovf);
+    }
     hipLaunchKernelGGL(k_solve_pair<N>, dim3(nb_solve, (unsigned)nj), dim3(kNbBlock), 0, stream, solve);
     GCA_HIP(hipGetLastError());
     return GCA_OK;

@@ -55,3 +55,57 @@ def test_neighbour_queries(ctx, kind, n, r):
     count = (_dist2(ref, ref) < r2).sum(1)
     for m in (-1, 0, 1, 8, int(np.median(count)), n):
         np.testing.assert_array_equal(cr.radius_outlier_removal(r, m).download()[0], ref[count > m], err_msg=f"min {m}")
+
+
+@pytest.mark.parametrize("kind,n,r", [
+    ("uniform", 2, 0.05), ("uniform", 65, 0.1), ("uniform", 1200, 0.09), ("plane", 2500, 0.02), ("plane", 2500, 0.04),
+    ("lattice", 1900, 0.03), ("lattice", 1900, 0.08), ("place", 30, 0.01), ("place", 97, 0.01), ("place", 600, 0.01),
+    ("uniform", 4200, 0.5)])
+def test_normals_and_gradient(ctx, kind, n, r):
+    """Normals and gradients with neighbourhoods around the group's buffer (96), the wavefront's
+    (448) and the exact sums' bound (4096), and with ties: the oracle's FP64 operations on the
+    same integer sums, so the same bits."""
+    import cuda_3d_amd as g
+    import oracle as O
+
+    rng = np.random.default_rng(n)
+    x = _cloud(kind, n, rng)
+    pc = g.PointCloud.from_numpy(x, rng.uniform(0, 1, x.shape).astype(np.float32), ctx=ctx)
+    xyzi = pc.download_xyzi()
+    for K in ((0, 30, 1000) if n > 4000 else (0, 1, 3, 30, 95, 96, 97, 448, 449, 1000)):
+        assert pc.estimate_normals(r, K)
+        nrm = O.estimate_normals(xyzi, r, K)
+        np.testing.assert_array_equal(pc.download_normals(), nrm[:, :3], err_msg=f"normals, {K} nearest")
+        assert pc.compute_color_gradient(r, K)
+        np.testing.assert_array_equal(pc.download_gradient(), O.color_gradient(xyzi, nrm, r, K)[:, :3],
+                                      err_msg=f"gradient, {K} nearest")
+
+
+@pytest.mark.parametrize("K", [0, 1, 30, 90, 500])
+def test_pipeline_wide_normals(ctx, K):
+    """The pipeline's joint walk (normals and gradient) with neighbourhoods on both sides of the
+    group's buffer, against the separate calls: two frames, the same pose bit for bit."""
+    import ctypes as C
+
+    import cuda_3d_amd as g
+    from cuda_3d_amd import _lib as L
+    from cuda_3d_amd import scene
+    from cuda_3d_amd.core import _ptr
+
+    (td, tc), (sd, sc), _, cm = scene.frame_pair(5, 320, 240)
+    cam, bil = g.make_camera(320, 240, cm.fx, cm.fy, cm.cx, cm.cy), g.bilateral(g.BILATERAL_FIXED, 2, 2.0, 30.0)
+    dev = [(g.device_tensor(d.view(np.int16)), g.device_tensor(c)) for d, c in ((td, tc), (sd, sc))]
+    lv = [g.level_params(v, 5.0 * v, K, 2.0 * v, 0, g.icp_params(5, 2.5 * v)) for v in (0.04, 0.02)]
+    h, valid, T, reps = C.c_void_p(), C.c_int32(), np.zeros(16), (L.IcpReport * 2)()
+    L.check(L.lib.gca_pipeline_create(ctx.handle, C.byref(cam), C.byref(bil), 0.2, 3.5, 2, (L.LevelParams * 2)(*lv),
+                                      C.byref(h)), "create")
+    try:
+        for d, c in dev:
+            L.check(L.lib.gca_pipeline_step(h, C.c_void_p(d.data_ptr()), C.c_void_p(c.data_ptr())), "step")
+        L.check(L.lib.gca_pipeline_result(h, _ptr(T), reps, C.byref(valid)), "result")
+    finally:
+        L.lib.gca_pipeline_destroy(h)
+    full = [g.PointCloud.create_from_rgbd(d, c, cam, bil, 0.2, 3.5, ctx=ctx) for d, c in dev]
+    want, wreps = g.multiscale_icp(full[1], full[0], lv)
+    np.testing.assert_array_equal(T.reshape(4, 4), want)
+    assert [r.n_correspondences for r in reps] == [r.n_correspondences for r in wreps]
