@@ -239,9 +239,9 @@ __device__ __forceinline__ void group_store(MomentSum<KIND> &A, int32_t cnt, int
     M.cnt = cnt;
 }
 
-// Sums without a K cap: 27 us for the gradient of those points at 2 cm (32 us with 64-bit integer
-// sums and a division per cell bound).  Eight lanes per query: 4 and 16 measured 1-2 % and 5 % slower on a 640x480 target at 1 cm, and
-// 2 and 4 % on the overlapped odometry of such frames.
+// Sums without a K cap: 27 us for the gradient of 110k points at 2 cm (32 us with 64-bit integer
+// sums and a division per cell bound).  Eight lanes per query: 4 and 16 measured 1-2 % and 5 %
+// slower on a 640x480 target at 1 cm, 2 and 4 % on the overlapped odometry of such frames.
 template <int KIND>
 __global__ __launch_bounds__(kNbBlock) void k_moments(const float4 *__restrict__ xyzi, const CloudHdr *__restrict__ hdr,
                                                       GridDesc g, const uint32_t *__restrict__ start,

@@ -134,22 +134,31 @@ __global__ __launch_bounds__(256) void k_voxel_mark(Jobs<MarkArgs, N> J)
 // kVoxChunk consecutive points (raster order: a few image rows, whose points share few voxels)
 // and sums their fixed-point values per voxel in an LDS hash table keyed by the voxel's rank
 // (open addressing, linear probing); it then hands each distinct voxel's sums to global memory
-// once.  Device-scope 64-bit
-// atomics bound this kernel, so the hand-over takes one compare-and-swap on the voxel's claim
-// word: the workgroup that wins it stores its sums plainly into the voxel's "A" record, the
-// others add theirs atomically into the "B" record (a point whose probe sequence found no slot
-// does the same with its own values).  Raster chunks of 2048 points meet 1.3 / 1.9 / 3.0
-// workgroups per voxel at 1 / 2 / 4 cm on a 640x480 frame, so most voxels take one CAS instead
-// of seven atomics.  Integer sums are exact, so neither the arrival order nor the split into A
-// and B changes the result.  Every voxel's A record is written by its claimant, so only B and
-// the claim need clearing after use.
+// once: the workgroup whose compare-and-swap wins the voxel's claim word stores its sums plainly
+// into the voxel's "A" record, the others add theirs atomically into the "B" record (a point whose
+// probe sequence found no slot does the same with its own values).  Integer sums are exact, so
+// neither the arrival order nor the split into A and B changes the result.  Every voxel's A record
+// is written by its claimant, so only B and the claim need clearing after use.
+//
+// Device-scope atomics are paid per cache line an instruction touches, so the hand-over is
+// transposed: each lane claims one voxel, then eight lanes together store or add the eight words of
+// a record, a line at a time (adding 7 words to 131k records: 42 us with a record per lane, 9 us
+// with eight lanes per record).  With the hand-over that cheap, small chunks pay: they spread over
+// the chip and end together, where chunks of 2048 points (135 for a 640x480 frame) left half of it
+// idle and the ones with most voxels, their tables full, ran twice as long as the rest.
+// 277k points of a raw frame at 1 cm 38 -> 22 us; of a filtered one at 1 / 2 / 4 cm 30 / 20 / 17 ->
+// 20 / 13 / 13 us; 1.5M points of a map at 8 mm 155 -> 72 us (chunks of 256 and 1024 points measured
+// within 3 % of 512 at one size or another and worse at the next).
 // Per-voxel record (kVoxRec words): A sums [0, 7), lattice key [7], B sums [8, 15), claim [15].
 constexpr int kVoxRec = 16;
-constexpr int kVoxChunk = 2048;
-constexpr int kVoxBlock = 1024;  // 2 points per thread: short per-thread chains, many waves per chunk
-constexpr int kVoxTableBits = 10;
+constexpr int kVoxBlock = 512;
+constexpr int kVoxChunk = kVoxBlock;  // a point per thread
+constexpr int kVoxTableBits = 9;      // an entry per point: a chunk of distinct voxels still fits
 constexpr int kVoxTable = 1 << kVoxTableBits;
 constexpr int kVoxProbe = 16;
+// LDS entry: sums [0, 7), key [7], rank in the low half of [8] (-1: free).  Nine words: neighbouring
+// entries start two banks apart, and the hand-over reads an entry's words side by side.
+constexpr int kVoxEntry = 9;
 
 struct AccumArgs {
     const float4 *xyzi, *rgb;
@@ -168,28 +177,25 @@ __global__ __launch_bounds__(kVoxBlock) void k_voxel_accum(Jobs<AccumArgs, N> J)
     const uint32_t *__restrict__ bitmap = A.bitmap;
     const uint32_t *__restrict__ word_pre = A.word_pre;
     unsigned long long *__restrict__ acc = A.acc;
-    __shared__ int32_t t_rank[kVoxTable];
-    __shared__ long long t_key[kVoxTable];
-    __shared__ unsigned long long t_sum[7][kVoxTable];
+    __shared__ unsigned long long tab[kVoxTable][kVoxEntry];
     __shared__ VoxelParams s_vp;
+    auto rank_of = [&](int h) { return reinterpret_cast<int32_t *>(&tab[h][8]); };
     if (threadIdx.x == 0) s_vp = *A.vpp;
-    for (int h = threadIdx.x; h < kVoxTable; h += blockDim.x) {
-        t_rank[h] = -1;
-#pragma unroll
-        for (int k = 0; k < 7; ++k) t_sum[k][h] = 0ull;
-    }
+    for (int w = threadIdx.x; w < kVoxTable * kVoxEntry; w += kVoxBlock)
+        (&tab[0][0])[w] = w % kVoxEntry == 8 ? ~0ull : 0ull;
     __syncthreads();
     const VoxelParams vp = s_vp;
     const int n = vp.bad ? 0 : A.hdr->n;
+    const int lane = lane_id(), k = lane & 7;  // the word of a record this lane hands over
     for (int base = blockIdx.x * kVoxChunk; base < n; base += gridDim.x * kVoxChunk) {  // block-uniform
-        __syncthreads();  // table clear (initial, or by the previous chunk's flush)
-        const int end = min(base + kVoxChunk, n);
-        for (int i = base + (int)threadIdx.x; i < end; i += blockDim.x) {
-            const float4 p = xyzi[i], c = rgb[i];
-            const int64_t L = voxel_key(vp, p);  // the marking pass's key, recomputed
-            const uint32_t w = bitmap[L >> 5];
-            const uint32_t below = w & ((1u << (uint32_t)(L & 31)) - 1u);
-            const int32_t r = (int32_t)(word_pre[L >> 5] + (uint32_t)__popc(below));
+        const int i = base + (int)threadIdx.x;
+        const bool on = i < n;
+        const float4 p = xyzi[on ? i : n - 1], c = rgb[on ? i : n - 1];
+        const int64_t L = voxel_key(vp, p);  // the marking pass's key, recomputed
+        const uint32_t below = bitmap[L >> 5] & ((1u << (uint32_t)(L & 31)) - 1u);
+        const int32_t r = (int32_t)(word_pre[L >> 5] + (uint32_t)__popc(below));
+        __syncthreads();  // table clear (initial, or by the previous chunk's hand-over)
+        if (on) {
             unsigned long long v[7];
             v[0] = (unsigned long long)fx((double)p.x * kFx30);
             v[1] = (unsigned long long)fx((double)p.y * kFx30);
@@ -201,8 +207,8 @@ __global__ __launch_bounds__(kVoxBlock) void k_voxel_accum(Jobs<AccumArgs, N> J)
             uint32_t h = ((uint32_t)r * 2654435761u) >> (32 - kVoxTableBits);  // multiplicative hash
             int slot = -1;
             for (int t = 0; t < kVoxProbe; ++t) {
-                const int32_t old = atomicCAS(&t_rank[h], -1, r);
-                if (old == -1) t_key[h] = L;  // same value from every point of the voxel
+                const int32_t old = atomicCAS(rank_of((int)h), -1, r);
+                if (old == -1) tab[h][7] = (unsigned long long)L;
                 if (old == -1 || old == r) {
                     slot = (int)h;
                     break;
@@ -211,32 +217,35 @@ __global__ __launch_bounds__(kVoxBlock) void k_voxel_accum(Jobs<AccumArgs, N> J)
             }
             if (slot >= 0) {
 #pragma unroll
-                for (int k = 0; k < 7; ++k) atomicAdd(&t_sum[k][slot], v[k]);
+                for (int q = 0; q < 7; ++q) atomicAdd(&tab[slot][q], v[q]);
             } else {
                 unsigned long long *a = acc + kVoxRec * (int64_t)r;
                 const bool own = atomicCAS(&a[15], 0ull, 1ull) == 0ull;
 #pragma unroll
-                for (int k = 0; k < 7; ++k) {
-                    if (own) a[k] = v[k];
-                    else atomicAdd(&a[8 + k], v[k]);
+                for (int q = 0; q < 7; ++q) {
+                    if (own) a[q] = v[q];
+                    else atomicAdd(&a[8 + q], v[q]);
                 }
-                a[7] = (unsigned long long)L;
+                if (own) a[7] = (unsigned long long)L;
             }
         }
         __syncthreads();
-        for (int h = threadIdx.x; h < kVoxTable; h += blockDim.x) {
-            const int32_t r = t_rank[h];
-            if (r < 0) continue;
-            unsigned long long *a = acc + kVoxRec * (int64_t)r;
-            const bool own = atomicCAS(&a[15], 0ull, 1ull) == 0ull;
+        for (int h0 = (int)threadIdx.x - k; h0 < kVoxTable; h0 += kVoxBlock) {
+            const int32_t r = *rank_of(h0 + k);  // this lane claims entry h0 + k
+            bool own = false;
+            if (r >= 0) own = atomicCAS(&acc[kVoxRec * (int64_t)r + 15], 0ull, 1ull) == 0ull;
+            const int32_t mine = r < 0 ? -1 : 2 * r + (own ? 1 : 0);
 #pragma unroll
-            for (int k = 0; k < 7; ++k) {
-                if (own) a[k] = t_sum[k][h];
-                else atomicAdd(&a[8 + k], t_sum[k][h]);
-                t_sum[k][h] = 0ull;
+            for (int j = 0; j < 8; ++j) {  // the group's entry h0 + j, word k
+                const int32_t e = __shfl(mine, (lane & ~7) + j, kWave);
+                if (e < 0) continue;
+                unsigned long long *a = acc + kVoxRec * (int64_t)(e >> 1);
+                const unsigned long long v = tab[h0 + j][k];
+                if (e & 1) a[k] = v;
+                else if (k < 7) atomicAdd(&a[8 + k], v);
+                tab[h0 + j][k] = 0ull;
             }
-            a[7] = (unsigned long long)t_key[h];
-            t_rank[h] = -1;
+            *rank_of(h0 + k) = -1;
         }
     }
 }
