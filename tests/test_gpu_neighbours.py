@@ -109,3 +109,34 @@ def test_pipeline_wide_normals(ctx, K):
     want, wreps = g.multiscale_icp(full[1], full[0], lv)
     np.testing.assert_array_equal(T.reshape(4, 4), want)
     assert [r.n_correspondences for r in reps] == [r.n_correspondences for r in wreps]
+
+
+@pytest.mark.parametrize("kind,n,r", [("uniform", 1, 0.05), ("uniform", 64, 0.05), ("uniform", 65, 0.05), ("uniform", 900, 0.02),
+                                      ("uniform", 2600, 0.02), ("plane", 2500, 0.006), ("plane", 2500, 0.02),
+                                      ("lattice", 700, 0.02), ("place", 200, 0.01)])
+def test_components(ctx, kind, n, r):
+    """Clusters and residual segments where most points are in one component, in many, or in runs of
+    neighbouring indices that end at a wavefront's edge; labels are whole numbers, so equal."""
+    import cuda_3d_amd as g
+    import oracle as O
+
+    rng = np.random.default_rng(n)
+    x = _cloud(kind, n, rng)
+    x[: n // 5] += np.float32(0.5)   # a second region, and indices sorted in half of the cases
+    if n % 2 == 0:
+        x = x[np.lexsort(x.T)]
+    if n > 100:
+        x[n // 2] = 1.0  # far from everything
+    pc = g.PointCloud.from_numpy(x, np.zeros_like(x), ctx=ctx)
+    pc.set_normals(np.zeros_like(x))
+    xyzi = pc.download_xyzi()
+    res = rng.uniform(0, 0.02, n).astype(np.float32)
+    res[: n // 2] = 0.001
+    for residual in (None, res):
+        for least in (1, 4):
+            want = O.euclidean_clustering(xyzi, r, least, max(n, least), residual=residual)
+            got = (pc.euclidean_clustering(r, least, max(n, least)) if residual is None else
+                   pc.icp_residual_segmentation(r, residual, least, max(n, least)))
+            assert len(got) == len(want)
+            for a, b in zip(got, want):
+                np.testing.assert_array_equal(a, np.sort(b))
