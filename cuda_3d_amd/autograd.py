@@ -14,7 +14,7 @@ import numpy as np
 import torch
 
 from . import _lib as L
-from .core import PointCloud, objective_grad
+from .core import PointCloud, _objective_grad
 
 
 class ColoredICPObjective(torch.autograd.Function):
@@ -23,14 +23,14 @@ class ColoredICPObjective(torch.autograd.Function):
         if src_xyzi.dtype != torch.float32 or not src_xyzi.is_cuda or src_xyzi.shape[-1] != 4:
             raise ValueError("src_xyzi must be a float32 cuda tensor of shape (N, 4)")
         pts = src_xyzi.detach().contiguous()
+        xi64 = np.asarray(xi.detach().cpu().numpy(), np.float64)
         torch.cuda.synchronize()  # torch's writes before the library's stream reads
         L.check(L.lib.gca_cloud_upload_device(work.ctx.handle, work.handle, C.c_void_p(pts.data_ptr()),
                                               None, pts.shape[0]), "gca_cloud_upload_device")
-        xi64 = np.asarray(xi.detach().cpu().numpy(), np.float64)
-        E, dxi, dpts = objective_grad(work, target, nn, T, xi64, lam, want_points=True)
-        ctx.save_for_backward(torch.as_tensor(dxi, dtype=torch.float64, device=xi.device),
-                              dpts.clone())
-        return torch.tensor(E, dtype=torch.float64, device=xi.device)
+        E, dxi, dpts = _objective_grad(work, target, nn, T, xi64, lam, pts.shape[0])
+        ctx.save_for_backward(torch.as_tensor(dxi, dtype=torch.float64, device=xi.device), dpts)
+        # (a fill does not wait for the device, as the copy of a host scalar does)
+        return torch.full((), E, dtype=torch.float64, device=xi.device)
 
     @staticmethod
     def backward(ctx, gE):

@@ -276,7 +276,7 @@ class PointCloud:
 
     # ---- operations ---------------------------------------------------------------------------
     def copy(self) -> "PointCloud":
-        out = PointCloud(self.ctx, 1)
+        out = PointCloud(self.ctx)
         check(lib.gca_cloud_copy(self.ctx.handle, self.handle, out.handle), "gca_cloud_copy")
         return out
 
@@ -573,9 +573,13 @@ def solve_gauss_newton(JTJ, JTr):
 def objective_grad(src: PointCloud, tgt: PointCloud, nn, T, xi, lambda_geometric=0.968,
                    want_points=True):
     """Colored-ICP objective at dT(xi) T and its adjoint: (E, dE/dxi, dE/d(xyz,I) or None)."""
+    return _objective_grad(src, tgt, nn, T, xi, lambda_geometric, src.points_number(), want_points)
+
+
+def _objective_grad(src, tgt, nn, T, xi, lambda_geometric, n, want_points=True):
+    """objective_grad of a source known to hold n points."""
     t = _torch()
     nn_t = nn if isinstance(nn, t.Tensor) else device_tensor(np.asarray(nn, np.int32))
-    n = src.points_number()
     dp = t.empty((max(n, 1), 4), dtype=t.float32, device="cuda") if want_points else None
     E = C.c_double()
     dxi = np.zeros(6)

@@ -29,6 +29,191 @@ int32_t ctx_take_device_error(gca_ctx ctx)
     return GCA_ERR_DEVICE;
 }
 
+// Gives blocks back to the runtime, the oldest first, until at most `keep` bytes are held.
+static void pool_drop_locked(BufferPool &P, size_t keep)
+{
+    int k = 0;
+    while (k < P.n && P.bytes > keep) {
+        P.bytes -= P.block[k].bytes;
+        hipFree(P.block[k++].p);
+    }
+    for (int j = k; j < P.n; ++j) P.block[j - k] = P.block[j];
+    P.n -= k;
+}
+
+static void pool_drop(gca_ctx ctx, size_t keep)
+{
+    std::lock_guard<std::mutex> lock(ctx->pool.m);
+    pool_drop_locked(ctx->pool, keep);
+}
+
+// Steps of an eighth of the power of two below, so at most an eighth of a buffer is slack.
+static size_t pool_class(size_t bytes)
+{
+    size_t step = BufferPool::kSmall / 8;
+    while (bytes > 16 * step) step *= 2;
+    return (bytes + step - 1) / step * step;
+}
+
+int32_t dev_alloc(gca_ctx ctx, void **p, size_t bytes)
+{
+    *p = nullptr;
+    if (bytes >= BufferPool::kSmall) {
+        bytes = pool_class(bytes);
+        BufferPool &P = ctx->pool;
+        std::lock_guard<std::mutex> lock(P.m);
+        for (int k = P.n - 1; k >= 0; --k)
+            if (P.block[k].bytes == bytes) {
+                *p = P.block[k].p;
+                P.bytes -= bytes;
+                for (int j = k + 1; j < P.n; ++j) P.block[j - 1] = P.block[j];
+                --P.n;
+                return GCA_OK;
+            }
+    }
+    int dev = ctx->device;
+    GCA_HIP(hipGetDevice(&dev));
+    if (dev != ctx->device) GCA_HIP(hipSetDevice(ctx->device));
+    hipError_t e = hipMalloc(p, bytes);
+    if (e == hipErrorOutOfMemory) {
+        pool_drop(ctx, 0);
+        e = hipMalloc(p, bytes);
+    }
+    if (dev != ctx->device) hipSetDevice(dev);
+    if (e != hipSuccess) *p = nullptr;
+    GCA_HIP(e);
+    return GCA_OK;
+}
+
+void dev_free(gca_ctx ctx, void *p, size_t bytes, bool idle)
+{
+    if (!p) return;
+    BufferPool &P = ctx->pool;
+    const size_t cls = pool_class(bytes);
+    if (!idle || bytes < BufferPool::kSmall || cls > BufferPool::kLimit / 4) {
+        hipFree(p);
+        return;
+    }
+    std::lock_guard<std::mutex> lock(P.m);
+    if (P.n == BufferPool::kMax) pool_drop_locked(P, P.bytes - P.block[0].bytes);
+    P.block[P.n++] = BufferPool::Block{p, cls};
+    P.bytes += cls;
+    pool_drop_locked(P, BufferPool::kLimit);
+}
+
+// The release of any allocation waits for all streams of the device, so that of a small one
+// (0.8 us with its allocation when the device is idle) stands in for the releases saved; unlike
+// a device synchronisation it is allowed while a stream is captured in relaxed mode.
+bool device_idle(gca_ctx ctx)
+{
+    int dev = ctx->device;
+    if (hipGetDevice(&dev) != hipSuccess) return false;
+    if (dev != ctx->device && hipSetDevice(ctx->device) != hipSuccess) return false;
+    void *p = nullptr;
+    const bool ok = hipMalloc(&p, 256) == hipSuccess && hipFree(p) == hipSuccess;
+    if (dev != ctx->device) hipSetDevice(dev);
+    return ok;
+}
+
+void *ctx_host_buf(gca_ctx ctx, size_t bytes)
+{
+    if (ctx->host_buf_bytes < bytes) {
+        if (ctx->host_buf) {
+            hipStreamSynchronize(ctx->stream);
+            hipHostFree(ctx->host_buf);
+        }
+        ctx->host_buf = nullptr;
+        ctx->host_buf_bytes = 0;
+        const size_t want = (bytes + bytes / 2 + 4095) & ~size_t(4095);
+        if (hipHostMalloc(&ctx->host_buf, want, hipHostMallocDefault) != hipSuccess) {
+            ctx->host_buf = nullptr;
+            return nullptr;
+        }
+        ctx->host_buf_bytes = want;
+    }
+    return ctx->host_buf;
+}
+
+static CloudHdr empty_hdr()
+{
+    CloudHdr h{};
+    for (int a = 0; a < 3; ++a) {
+        h.bmin_key[a] = float_to_key(FLT_MAX);
+        h.bmax_key[a] = float_to_key(FLT_MIN);
+    }
+    return h;
+}
+
+struct HdrBatch {
+    CloudHdr *h[HdrPool::kPer];
+};
+
+__global__ __launch_bounds__(HdrPool::kPer) void k_hdrs_reset(HdrBatch b, CloudHdr h)
+{
+    if (b.h[threadIdx.x]) *b.h[threadIdx.x] = h;
+}
+
+// A header that holds an empty cloud's.
+static int32_t hdr_take(gca_ctx ctx, HdrRef *out)
+try {
+    HdrPool &P = ctx->hdrs;
+    std::lock_guard<std::mutex> lock(P.m);
+    if (P.ready.empty() && P.used.size() >= HdrPool::kPer / 2) {
+        hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
+        GCA_HIP(hipStreamIsCapturing(ctx->stream, &cap));
+        if (cap == hipStreamCaptureStatusNone) {
+            const size_t n = std::min<size_t>(P.used.size(), HdrPool::kPer);
+            HdrBatch b{};
+            for (size_t k = 0; k < n; ++k) b.h[k] = &P.used[P.used.size() - 1 - k].dev->h;
+            P.ready.reserve(n);
+            hipLaunchKernelGGL(k_hdrs_reset, dim3(1), dim3(HdrPool::kPer), 0, ctx->stream, b, empty_hdr());
+            GCA_HIP(hipGetLastError());
+            GCA_HIP(hipStreamSynchronize(ctx->stream));
+            for (size_t k = 0; k < n; ++k) {
+                P.ready.push_back(P.used.back());
+                P.used.pop_back();
+            }
+        }
+    }
+    if (P.ready.empty()) {
+        std::vector<HdrSlot> init(HdrPool::kPer);
+        for (auto &s : init) s.h = empty_hdr();
+        P.ready.reserve(HdrPool::kPer);
+        P.slabs.reserve(P.slabs.size() + 1);
+        P.host_slabs.reserve(P.host_slabs.size() + 1);
+        P.used.reserve((P.slabs.size() + 1) * HdrPool::kPer);
+        HdrSlot *d = nullptr;
+        CloudHdr *h = nullptr;
+        int32_t st = dev_alloc(ctx, (void **)&d, sizeof(HdrSlot) * HdrPool::kPer);
+        if (st == GCA_OK && hipHostMalloc((void **)&h, sizeof(CloudHdr) * HdrPool::kPer, hipHostMallocDefault) != hipSuccess)
+            st = GCA_ERR_OUT_OF_MEMORY;
+        if (st == GCA_OK &&
+            hipMemcpy(d, init.data(), sizeof(HdrSlot) * HdrPool::kPer, hipMemcpyHostToDevice) != hipSuccess) {
+            hipHostFree(h);
+            st = GCA_ERR_DEVICE;
+        }
+        if (st != GCA_OK) {
+            hipFree(d);
+            return st;
+        }
+        P.slabs.push_back(d);
+        P.host_slabs.push_back(h);
+        for (int k = 0; k < HdrPool::kPer; ++k) P.ready.push_back(HdrRef{d + k, h + k});
+    }
+    *out = P.ready.back();
+    P.ready.pop_back();
+    return GCA_OK;
+} catch (...) {
+    return GCA_ERR_OUT_OF_MEMORY;
+}
+
+// (used has room for every slot of every slab, so this does not allocate)
+static void hdr_give(gca_ctx ctx, const HdrRef &r)
+{
+    std::lock_guard<std::mutex> lock(ctx->hdrs.m);
+    ctx->hdrs.used.push_back(r);
+}
+
 void *ctx_scratch(gca_ctx ctx, int slot, size_t bytes, bool zeroed)
 {
     if (slot < 0 || slot >= gca_ctx_s::kScratchSlots) return nullptr;
@@ -41,10 +226,14 @@ void *ctx_scratch(gca_ctx ctx, int slot, size_t bytes, bool zeroed)
         }
         size_t want = bytes + bytes / 2;
         want = (want + 255) & ~size_t(255);
+        ctx->scratch_bytes[slot] = 0;
         if (hipMalloc(&ctx->scratch[slot], want) != hipSuccess) {
             ctx->scratch[slot] = nullptr;
-            ctx->scratch_bytes[slot] = 0;
-            return nullptr;
+            pool_drop(ctx, 0);
+            if (hipMalloc(&ctx->scratch[slot], want) != hipSuccess) {
+                ctx->scratch[slot] = nullptr;
+                return nullptr;
+            }
         }
         ctx->scratch_bytes[slot] = want;
         ctx->scratch_zeroed[slot] = false;
@@ -281,22 +470,33 @@ int32_t exclusive_scan_u32(gca_ctx ctx, const uint32_t *in, uint32_t *out, int64
 
 // ---------------------------------------------------------------------------------------
 
+// The arrays (those in the header's slot stay with it).
+static void cloud_arrays_free(gca_cloud c, bool idle)
+{
+    if (c->xyzi && c->xyzi != c->ref.dev->one) {
+        dev_array_free(c->ctx, c->xyzi, c->cap, idle);
+        dev_array_free(c->ctx, c->rgb, c->cap, idle);
+        dev_array_free(c->ctx, c->nrm, c->cap, idle);
+        dev_array_free(c->ctx, c->grad, c->cap, idle);
+    }
+    c->xyzi = c->rgb = c->nrm = c->grad = nullptr;
+    c->cap = 0;
+}
+
 int32_t cloud_reserve(gca_cloud c, int64_t cap)
 {
     if (cap <= c->cap) return GCA_OK;
     if (cap > (int64_t)INT_MAX / 2) return GCA_ERR_INVALID_VALUE;
-    GCA_HIP(hipStreamSynchronize(c->ctx->stream));
-    hipFree(c->xyzi);
-    hipFree(c->rgb);
-    hipFree(c->nrm);
-    hipFree(c->grad);
-    c->xyzi = c->rgb = c->nrm = c->grad = nullptr;
-    c->cap = 0;
-    size_t b = sizeof(float4) * (size_t)cap;
-    GCA_HIP(hipMalloc(&c->xyzi, b));
-    GCA_HIP(hipMalloc(&c->rgb, b));
-    GCA_HIP(hipMalloc(&c->nrm, b));
-    GCA_HIP(hipMalloc(&c->grad, b));
+    bool idle = false;
+    if (c->xyzi != c->ref.dev->one) {
+        GCA_HIP(hipStreamSynchronize(c->ctx->stream));
+        idle = device_idle(c->ctx);
+    }
+    cloud_arrays_free(c, idle);
+    GCA_TRY(dev_array(c->ctx, &c->xyzi, cap));
+    GCA_TRY(dev_array(c->ctx, &c->rgb, cap));
+    GCA_TRY(dev_array(c->ctx, &c->nrm, cap));
+    GCA_TRY(dev_array(c->ctx, &c->grad, cap));
     c->cap = cap;
     return GCA_OK;
 }
@@ -304,12 +504,19 @@ int32_t cloud_reserve(gca_cloud c, int64_t cap)
 int32_t cloud_sync_header(gca_cloud c)
 {
     if (c->host_valid) return GCA_OK;
-    GCA_HIP(hipMemcpyAsync(&c->host_hdr, c->hdr, sizeof(CloudHdr), hipMemcpyDeviceToHost,
-                           c->ctx->stream));
+    GCA_HIP(hipMemcpyAsync(c->ref.host, c->hdr, sizeof(CloudHdr), hipMemcpyDeviceToHost, c->ctx->stream));
     GCA_HIP(hipStreamSynchronize(c->ctx->stream));
     GCA_TRY(ctx_take_device_error(c->ctx));  // a header behind a failed scan is not valid
+    c->host_hdr = *c->ref.host;
     c->host_valid = true;
     return GCA_OK;
+}
+
+int32_t cloud_sync_count(gca_ctx ctx, gca_cloud c)
+{
+    // (on another ctx's stream the read-back is also what orders that stream's work first)
+    if ((c->host_valid || c->n_valid) && c->ctx == ctx) return GCA_OK;
+    return cloud_sync_header(c);
 }
 
 void cloud_host_bounds(gca_cloud c, float mn[3], float mx[3])
@@ -323,17 +530,23 @@ void cloud_host_bounds(gca_cloud c, float mn[3], float mx[3])
 void cloud_points_changed(gca_cloud c)
 {
     c->host_valid = false;
+    c->n_valid = false;
     c->grid.valid = false;
     c->grid.attrs_valid = false;
 }
 
+hipError_t bounds_enqueue(gca_ctx ctx, const float4 *xyzi, int64_t cap, CloudHdr *hdr)
+{
+    hipLaunchKernelGGL(k_bounds_init, dim3(1), dim3(1), 0, ctx->stream, hdr);
+    // few blocks: each issues six atomics on the same header words
+    int64_t nb = std::min<int64_t>(64, std::max<int64_t>(1, (cap + 255) / 256));
+    hipLaunchKernelGGL(k_bounds_reduce, dim3((unsigned)nb), dim3(256), 0, ctx->stream, xyzi, hdr);
+    return hipGetLastError();
+}
+
 int32_t launch_bounds(gca_ctx ctx, gca_cloud c)
 {
-    hipLaunchKernelGGL(k_bounds_init, dim3(1), dim3(1), 0, ctx->stream, c->hdr);
-    // few blocks: each issues six atomics on the same header words
-    int64_t nb = std::min<int64_t>(64, std::max<int64_t>(1, (c->cap + 255) / 256));
-    hipLaunchKernelGGL(k_bounds_reduce, dim3((unsigned)nb), dim3(256), 0, ctx->stream, c->xyzi, c->hdr);
-    GCA_HIP(hipGetLastError());
+    GCA_HIP(bounds_enqueue(ctx, c->xyzi, c->cap, c->hdr));
     return GCA_OK;
 }
 
@@ -480,6 +693,10 @@ int32_t gca_ctx_destroy(gca_ctx c)
     for (int i = 0; i < 16; ++i)
         if (c->level_clouds[i]) gca_cloud_destroy(c->level_clouds[i]);
     for (int i = 0; i < gca_ctx_s::kScratchSlots; ++i) hipFree(c->scratch[i]);
+    pool_drop(c, 0);
+    for (void *p : c->hdrs.slabs) hipFree(p);
+    for (void *p : c->hdrs.host_slabs) hipHostFree(p);
+    if (c->host_buf) hipHostFree(c->host_buf);
     for (hipEvent_t e : c->prof_pool) hipEventDestroy(e);
     hipFree(c->bitmap);
     hipFree(c->lut);
@@ -572,24 +789,20 @@ int32_t gca_cloud_create(gca_ctx ctx, int64_t capacity, gca_cloud *out)
     gca_cloud c = new (std::nothrow) gca_cloud_s();
     if (!c) return GCA_ERR_OUT_OF_MEMORY;
     c->ctx = ctx;
-    if (hipMalloc(&c->hdr, sizeof(CloudHdr)) != hipSuccess) {
+    int32_t s = hdr_take(ctx, &c->ref);
+    if (s != GCA_OK) {
         delete c;
-        return GCA_ERR_OUT_OF_MEMORY;
+        return s;
     }
-    CloudHdr h{};
-    h.n = 0;
-    for (int a = 0; a < 3; ++a) {
-        h.bmin_key[a] = float_to_key(FLT_MAX);
-        h.bmax_key[a] = float_to_key(FLT_MIN);
-    }
-    if (hipMemcpy(c->hdr, &h, sizeof(h), hipMemcpyHostToDevice) != hipSuccess) {
-        hipFree(c->hdr);
-        delete c;
-        return GCA_ERR_DEVICE;
-    }
-    c->host_hdr = h;
+    c->hdr = &c->ref.dev->h;
+    c->host_hdr = empty_hdr();
     c->host_valid = true;
-    int32_t s = cloud_reserve(c, std::max<int64_t>(capacity, 1));
+    c->xyzi = &c->ref.dev->one[0];
+    c->rgb = &c->ref.dev->one[1];
+    c->nrm = &c->ref.dev->one[2];
+    c->grad = &c->ref.dev->one[3];
+    c->cap = 1;
+    s = cloud_reserve(c, capacity);
     if (s != GCA_OK) {
         gca_cloud_destroy(c);
         return s;
@@ -598,28 +811,15 @@ int32_t gca_cloud_create(gca_ctx ctx, int64_t capacity, gca_cloud *out)
     return GCA_OK;
 }
 
-static void grid_free(Grid &g)
-{
-    hipFree(g.count);
-    hipFree(g.start);
-    hipFree(g.order);
-    hipFree(g.sxyzi);
-    hipFree(g.cell_of);
-    hipFree(g.snrm);
-    hipFree(g.sgrad);
-    g = Grid();
-}
-
 int32_t gca_cloud_destroy(gca_cloud c)
 {
     if (!c) return GCA_ERR_INVALID_VALUE;
     hipStreamSynchronize(c->ctx->stream);
-    hipFree(c->xyzi);
-    hipFree(c->rgb);
-    hipFree(c->nrm);
-    hipFree(c->grad);
-    hipFree(c->hdr);
-    grid_free(c->grid);
+    const bool idle = device_idle(c->ctx);
+    cloud_arrays_free(c, idle);
+    grid_free_cells(c->ctx, c->grid, idle);
+    grid_free_points(c->ctx, c->grid, idle);
+    if (idle) hdr_give(c->ctx, c->ref);  // (else the slot is left unused until the ctx goes)
     delete c;
     return GCA_OK;
 }
@@ -668,6 +868,8 @@ int32_t gca_cloud_upload(gca_cloud c, const float *xyz, const float *rgb, int64_
     c->has_normals = c->has_gradient = false;
     cloud_points_changed(c);
     GCA_TRY(launch_bounds(c->ctx, c));
+    c->host_hdr.n = n32;
+    c->n_valid = true;
     return GCA_OK;
 }
 
@@ -689,6 +891,8 @@ int32_t gca_cloud_upload_device(gca_ctx ctx, gca_cloud c, const void *xyzi, cons
     c->has_normals = c->has_gradient = false;
     cloud_points_changed(c);
     GCA_TRY(launch_bounds(ctx, c));
+    c->host_hdr.n = (int32_t)n;
+    c->n_valid = true;
     return GCA_OK;
 }
 
@@ -776,74 +980,110 @@ int32_t gca_cloud_bounds(gca_cloud c, float mn[3], float mx[3])
     return GCA_OK;
 }
 
+// A cloud's points and header in one launch (the four copies and the header's took 5 launches, and
+// copied the whole capacity).
+static __global__ __launch_bounds__(256) void k_cloud_copy(const CloudHdr *__restrict__ h, const float4 *__restrict__ xyzi,
+                                                           const float4 *__restrict__ rgb, const float4 *__restrict__ nrm,
+                                                           const float4 *__restrict__ grad, CloudHdr *__restrict__ dh,
+                                                           float4 *__restrict__ dxyzi, float4 *__restrict__ drgb,
+                                                           float4 *__restrict__ dnrm, float4 *__restrict__ dgrad)
+{
+    const CloudHdr hdr = *h;
+    for (int i = blockIdx.x * blockDim.x + threadIdx.x; i < hdr.n; i += gridDim.x * blockDim.x) {
+        dxyzi[i] = xyzi[i];
+        drgb[i] = rgb[i];
+        if (nrm) dnrm[i] = nrm[i];
+        if (grad) dgrad[i] = grad[i];
+    }
+    if (blockIdx.x == 0 && threadIdx.x == 0) *dh = hdr;
+}
+
 int32_t gca_cloud_copy(gca_ctx ctx, gca_cloud src, gca_cloud dst)
 {
     if (!ctx || !src || !dst || src == dst) return GCA_ERR_INVALID_VALUE;
     GCA_TRY(cloud_reserve(dst, src->cap));
-    size_t b = sizeof(float4) * (size_t)src->cap;
-    GCA_HIP(hipMemcpyAsync(dst->xyzi, src->xyzi, b, hipMemcpyDeviceToDevice, ctx->stream));
-    GCA_HIP(hipMemcpyAsync(dst->rgb, src->rgb, b, hipMemcpyDeviceToDevice, ctx->stream));
-    if (src->has_normals)
-        GCA_HIP(hipMemcpyAsync(dst->nrm, src->nrm, b, hipMemcpyDeviceToDevice, ctx->stream));
-    if (src->has_gradient)
-        GCA_HIP(hipMemcpyAsync(dst->grad, src->grad, b, hipMemcpyDeviceToDevice, ctx->stream));
-    GCA_HIP(hipMemcpyAsync(dst->hdr, src->hdr, sizeof(CloudHdr), hipMemcpyDeviceToDevice, ctx->stream));
+    const unsigned nb = (unsigned)std::min<int64_t>(2048, std::max<int64_t>(1, (src->cap + 255) / 256));
+    hipLaunchKernelGGL(k_cloud_copy, dim3(nb), dim3(256), 0, ctx->stream, src->hdr, src->xyzi, src->rgb,
+                       src->has_normals ? src->nrm : nullptr, src->has_gradient ? src->grad : nullptr, dst->hdr,
+                       dst->xyzi, dst->rgb, dst->nrm, dst->grad);
+    GCA_HIP(hipGetLastError());
     dst->has_normals = src->has_normals;
     dst->has_gradient = src->has_gradient;
     cloud_points_changed(dst);
+    dst->host_hdr.n = src->host_hdr.n;
+    dst->n_valid = src->host_valid || src->n_valid;
     return GCA_OK;
+}
+
+// dst += src in one launch: the points below nd stay where they are (moved = 0) or are copied to
+// the grown arrays, those from nd on are src's.  nrm null: no normals survive.
+static __global__ __launch_bounds__(256) void k_cloud_append(const float4 *xyzi, const float4 *rgb, const float4 *nrm,
+                                                             const float4 *more_xyzi, const float4 *more_rgb,
+                                                             const float4 *more_nrm, int nd, int total, int moved,
+                                                             float4 *to_xyzi, float4 *to_rgb, float4 *to_nrm,
+                                                             CloudHdr *__restrict__ h)
+{
+    const int step = gridDim.x * blockDim.x;
+    for (int i = (moved ? 0 : nd) + blockIdx.x * blockDim.x + threadIdx.x; i < total; i += step) {
+        const bool own = i < nd;
+        const int k = own ? i : i - nd;
+        to_xyzi[i] = (own ? xyzi : more_xyzi)[k];
+        to_rgb[i] = (own ? rgb : more_rgb)[k];
+        if (nrm) to_nrm[i] = (own ? nrm : more_nrm)[k];
+    }
+    if (blockIdx.x == 0 && threadIdx.x == 0) h->n = total;
 }
 
 int32_t gca_cloud_append(gca_ctx ctx, gca_cloud dst, gca_cloud src)
 {
     // point_cloud::operator+= (point_cloud.cu:55-73)
     if (!ctx || !dst || !src) return GCA_ERR_INVALID_VALUE;
-    GCA_TRY(cloud_sync_header(dst));
-    GCA_TRY(cloud_sync_header(src));
-    GCA_HIP(hipStreamSynchronize(ctx->stream));
+    GCA_TRY(cloud_sync_count(ctx, dst));
+    GCA_TRY(cloud_sync_count(ctx, src));
     const int64_t nd = dst->host_hdr.n, ns = src->host_hdr.n, total = nd + ns;
     if (total > (int64_t)INT_MAX / 2) return GCA_ERR_INVALID_VALUE;
     const bool normals = dst->has_normals && src->has_normals;
-    if (total > dst->cap) {
-        // grow, keeping dst's points (and normals when they survive)
-        const int64_t cap = std::max<int64_t>(total, dst->cap + dst->cap / 2);
-        const size_t b = sizeof(float4) * (size_t)cap;
-        float4 *a[4] = {nullptr, nullptr, nullptr, nullptr};
-        for (int k = 0; k < 4; ++k)
-            if (hipMalloc(&a[k], b) != hipSuccess) {
-                for (int j = 0; j < k; ++j) hipFree(a[j]);
-                return GCA_ERR_OUT_OF_MEMORY;
+    // the arrays that are read: dst's own unless they grow, src's (dst's own when src is dst)
+    float4 *from[3] = {dst->xyzi, dst->rgb, dst->nrm};
+    const float4 *more[3] = {src->xyzi, src->rgb, src->nrm};
+    float4 *to[4] = {dst->xyzi, dst->rgb, dst->nrm, dst->grad};
+    const int64_t cap = total > dst->cap ? std::max<int64_t>(total, dst->cap + dst->cap / 2) : dst->cap;
+    if (cap > dst->cap)
+        for (int k = 0; k < 4; ++k) {
+            const int32_t st = dev_array(dst->ctx, &to[k], cap);
+            if (st != GCA_OK) {
+                for (int j = 0; j < k; ++j) dev_array_free(dst->ctx, to[j], cap, true);
+                return st;
             }
-        const size_t keep = sizeof(float4) * (size_t)nd;
-        if (keep) {
-            GCA_HIP(hipMemcpyAsync(a[0], dst->xyzi, keep, hipMemcpyDeviceToDevice, ctx->stream));
-            GCA_HIP(hipMemcpyAsync(a[1], dst->rgb, keep, hipMemcpyDeviceToDevice, ctx->stream));
-            if (normals) GCA_HIP(hipMemcpyAsync(a[2], dst->nrm, keep, hipMemcpyDeviceToDevice, ctx->stream));
         }
-        GCA_HIP(hipStreamSynchronize(ctx->stream));
-        hipFree(dst->xyzi);
-        hipFree(dst->rgb);
-        hipFree(dst->nrm);
-        hipFree(dst->grad);
-        dst->xyzi = a[0];
-        dst->rgb = a[1];
-        dst->nrm = a[2];
-        dst->grad = a[3];
-        dst->cap = cap;  // (when src is dst, its arrays are these new ones: the first nd entries)
+    const unsigned nb = (unsigned)std::min<int64_t>(2048, std::max<int64_t>(1, (total + 255) / 256));
+    hipLaunchKernelGGL(k_cloud_append, dim3(nb), dim3(256), 0, ctx->stream, from[0], from[1], normals ? from[2] : nullptr,
+                       more[0], more[1], more[2], (int)nd, (int)total, cap > dst->cap ? 1 : 0, to[0], to[1], to[2],
+                       dst->hdr);
+    hipError_t e = hipGetLastError();
+    // get_min_bound / get_max_bound recompute the bounds (point_cloud.cu:107-132)
+    if (e == hipSuccess) e = bounds_enqueue(ctx, to[0], cap, dst->hdr);
+    const hipError_t es = hipStreamSynchronize(ctx->stream);
+    if (e == hipSuccess) e = es;
+    if (cap > dst->cap) {
+        const bool idle = device_idle(dst->ctx);
+        if (e != hipSuccess) {
+            for (auto &a : to) dev_array_free(dst->ctx, a, cap, idle);
+        } else {
+            cloud_arrays_free(dst, idle);
+            dst->xyzi = to[0];
+            dst->rgb = to[1];
+            dst->nrm = to[2];
+            dst->grad = to[3];
+            dst->cap = cap;
+        }
     }
-    if (ns > 0) {
-        const size_t b = sizeof(float4) * (size_t)ns;
-        GCA_HIP(hipMemcpyAsync(dst->xyzi + nd, src->xyzi, b, hipMemcpyDeviceToDevice, ctx->stream));
-        GCA_HIP(hipMemcpyAsync(dst->rgb + nd, src->rgb, b, hipMemcpyDeviceToDevice, ctx->stream));
-        if (normals) GCA_HIP(hipMemcpyAsync(dst->nrm + nd, src->nrm, b, hipMemcpyDeviceToDevice, ctx->stream));
-    }
-    dst->host_hdr.n = (int32_t)total;
-    GCA_HIP(hipMemcpyAsync(&dst->hdr->n, &dst->host_hdr.n, sizeof(int32_t), hipMemcpyHostToDevice, ctx->stream));
-    GCA_TRY(launch_bounds(ctx, dst));  // get_min_bound / get_max_bound recompute them (point_cloud.cu:107-132)
-    GCA_HIP(hipStreamSynchronize(ctx->stream));
+    GCA_HIP(e);
     dst->has_normals = normals;
     dst->has_gradient = false;
     cloud_points_changed(dst);
+    dst->host_hdr.n = (int32_t)total;
+    dst->n_valid = true;
     return GCA_OK;
 }
 
@@ -907,8 +1147,8 @@ int32_t gca_euclidean_clustering(gca_ctx ctx, gca_cloud c, float tolerance, int3
     if (!counts) return GCA_ERR_OUT_OF_MEMORY;
     GCA_TRY(launch_euclidean_clustering(ctx, c, tolerance, (uint32_t)min_cluster_size,
                                         (uint32_t)max_cluster_size, labels_dev, counts));
-    uint32_t h[2] = {0, 0};
-    GCA_HIP(hipMemcpyAsync(h, counts, sizeof(h), hipMemcpyDeviceToHost, ctx->stream));
+    const uint32_t *h = (const uint32_t *)ctx->pinned;
+    GCA_HIP(hipMemcpyAsync(ctx->pinned, counts, 2 * sizeof(uint32_t), hipMemcpyDeviceToHost, ctx->stream));
     GCA_HIP(hipStreamSynchronize(ctx->stream));
     *n_clusters = (int32_t)h[0];
     if (n_cut) *n_cut = (int32_t)h[1];
@@ -933,8 +1173,8 @@ int32_t gca_residual_segmentation(gca_ctx ctx, gca_cloud c, float tolerance, con
     if (!counts) return GCA_ERR_OUT_OF_MEMORY;
     GCA_TRY(launch_euclidean_clustering(ctx, c, tolerance, (uint32_t)min_cluster_size, (uint32_t)max_cluster_size,
                                         labels_dev, counts, abs_residual_dev));
-    uint32_t h[2] = {0, 0};
-    GCA_HIP(hipMemcpyAsync(h, counts, sizeof(h), hipMemcpyDeviceToHost, ctx->stream));
+    const uint32_t *h = (const uint32_t *)ctx->pinned;
+    GCA_HIP(hipMemcpyAsync(ctx->pinned, counts, 2 * sizeof(uint32_t), hipMemcpyDeviceToHost, ctx->stream));
     GCA_HIP(hipStreamSynchronize(ctx->stream));
     *n_clusters = (int32_t)h[0];
     if (n_cut) *n_cut = (int32_t)h[1];
@@ -1062,8 +1302,10 @@ int32_t gca_transform(gca_ctx ctx, gca_cloud c, const double T[16])
 {
     if (!ctx || !c || !T) return GCA_ERR_INVALID_VALUE;
     GCA_TRY(launch_transform(ctx, c, T));
+    const bool n_valid = c->host_valid || c->n_valid;
     cloud_points_changed(c);
     GCA_TRY(launch_bounds(ctx, c));  // point_cloud.cu:96-100 recomputes the bounds
+    c->n_valid = n_valid;
     return GCA_OK;
 }
 

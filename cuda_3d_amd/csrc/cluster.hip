@@ -553,9 +553,9 @@ int32_t launch_euclidean_clustering(gca_ctx ctx, gca_cloud c, float tolerance, u
     hipLaunchKernelGGL(k_cc_compress, wide, dim3(kCcWide), 0, ctx->stream, c->hdr, label, size, (const int32_t *)big);
     hipLaunchKernelGGL(k_cc_over, grid, block, 0, ctx->stream, c->hdr, label, size, max_size, jobs, counts_dev + 1);
     GCA_HIP(hipGetLastError());
-    uint32_t n_jobs = 0;
-    GCA_HIP(hipMemcpyAsync(&n_jobs, counts_dev + 1, sizeof(uint32_t), hipMemcpyDeviceToHost, ctx->stream));
+    GCA_HIP(hipMemcpyAsync(ctx->pinned, counts_dev + 1, sizeof(uint32_t), hipMemcpyDeviceToHost, ctx->stream));
     GCA_HIP(hipStreamSynchronize(ctx->stream));
+    const uint32_t n_jobs = *(const uint32_t *)ctx->pinned;
     if (n_jobs > 0) {
         // Components above max_size are cut as the reference's searches cut them.  Their
         // neighbour lists (radius search of the cloud against itself, canonical order) and a

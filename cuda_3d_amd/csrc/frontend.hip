@@ -424,6 +424,14 @@ static int32_t build_lut(gca_ctx ctx, const gca_bilateral *f, FrontParams *fp)
     if (same && f->mode == GCA_BILATERAL_FIXED)
         same = ctx->lut_key_radius == f->radius && ctx->lut_key_ss == f->sigma_space &&
                ctx->lut_key_sd == f->sigma_depth;
+    if (same) {
+        for (int s = 0; s < 6; ++s) {
+            fp->ws_off[s] = ctx->lut_ws_off[s];
+            fp->wr_off[s] = ctx->lut_wr_off[s];
+            fp->wr_len[s] = ctx->lut_wr_len[s];
+        }
+        return GCA_OK;
+    }
     std::vector<double> tab;
     int nsteps = (f->mode == GCA_BILATERAL_REFERENCE_ADAPTIVE) ? 6 : 1;
     for (int s = 0; s < nsteps; ++s) {
@@ -451,23 +459,26 @@ static int32_t build_lut(gca_ctx ctx, const gca_bilateral *f, FrontParams *fp)
         }
         fp->wr_len[s] = len;
     }
-    if (!same) {
-        size_t bytes = tab.size() * sizeof(double);
-        if (ctx->lut_bytes < bytes) {
-            GCA_HIP(hipStreamSynchronize(ctx->stream));
-            hipFree(ctx->lut);
-            ctx->lut = nullptr;
-            ctx->lut_bytes = 0;
-            GCA_HIP(hipMalloc(&ctx->lut, bytes));
-            ctx->lut_bytes = bytes;
-        }
-        GCA_HIP(hipStreamSynchronize(ctx->stream));
-        GCA_HIP(hipMemcpy(ctx->lut, tab.data(), bytes, hipMemcpyHostToDevice));
-        ctx->lut_key_mode = f->mode;
-        ctx->lut_key_radius = f->radius;
-        ctx->lut_key_ss = f->sigma_space;
-        ctx->lut_key_sd = f->sigma_depth;
+    size_t bytes = tab.size() * sizeof(double);
+    GCA_HIP(hipStreamSynchronize(ctx->stream));
+    ctx->lut_key_mode = -1;  // until the tables are there
+    if (ctx->lut_bytes < bytes) {
+        hipFree(ctx->lut);
+        ctx->lut = nullptr;
+        ctx->lut_bytes = 0;
+        GCA_TRY(dev_alloc(ctx, (void **)&ctx->lut, bytes));
+        ctx->lut_bytes = bytes;
     }
+    GCA_HIP(hipMemcpy(ctx->lut, tab.data(), bytes, hipMemcpyHostToDevice));
+    for (int s = 0; s < 6; ++s) {
+        ctx->lut_ws_off[s] = fp->ws_off[s];
+        ctx->lut_wr_off[s] = fp->wr_off[s];
+        ctx->lut_wr_len[s] = fp->wr_len[s];
+    }
+    ctx->lut_key_mode = f->mode;
+    ctx->lut_key_radius = f->radius;
+    ctx->lut_key_ss = f->sigma_space;
+    ctx->lut_key_sd = f->sigma_depth;
     return GCA_OK;
 }
 

@@ -13,6 +13,7 @@
 
 #include <cstdint>
 #include <cstring>
+#include <mutex>
 #include <vector>
 
 #include "../../include/gca/gca.h"
@@ -99,6 +100,44 @@ struct Jobs {
     A a[N];
 };
 
+// Device buffers given back by clouds and grids, kept for the next ones of the same size class.
+// A HIP allocation of 2 MiB or more takes 17-25 us and its release 60-230 us (below 64 KiB: 0.4 us
+// each), so a call that makes and drops a cloud spends more on them than on its kernels (a copy,
+// transform, append and 1 cm downsample of 0.8 M points: 2280 us with them, 232 us here).  Blocks enter the pool only once the
+// device has been idle since their last use, so the next owner may use them on any stream.
+struct BufferPool {
+    static constexpr size_t kSmall = 64 << 10;   // smaller buffers are not kept
+    static constexpr size_t kLimit = 512 << 20;  // bytes kept per ctx; the oldest go first
+    static constexpr int kMax = 192;
+    std::mutex m;
+    struct Block {
+        void *p;
+        size_t bytes;
+    } block[kMax];  // in the order they came back
+    int n = 0;
+    size_t bytes = 0;
+};
+
+// One cloud's header on the device, with the arrays of a cloud of one point behind it (a cloud
+// that is made before its size is known owns no other memory), and where it is read back to.
+struct HdrSlot {
+    CloudHdr h;
+    float4 one[4];
+    char pad[32];
+};
+struct HdrRef {
+    HdrSlot *dev;
+    CloudHdr *host;  // pinned
+};
+// Headers by slabs of kPer: ready ones carry an empty cloud's header, used ones are reset together
+// by one launch once kPer / 2 of them have come back.
+struct HdrPool {
+    static constexpr int kPer = 64;
+    std::mutex m;
+    std::vector<HdrRef> ready, used;
+    std::vector<void *> slabs, host_slabs;
+};
+
 }  // namespace gca
 
 struct gca_ctx_s {
@@ -117,6 +156,12 @@ struct gca_ctx_s {
     // after the stream has been synchronised
     static constexpr int kPinnedDoubles = 32;
     double *pinned = nullptr;
+    // pinned host memory for a call's uploads and read-backs, grown on demand (ctx_host_buf); a
+    // small read-back into it takes 12 us, into pageable memory 21
+    void *host_buf = nullptr;
+    size_t host_buf_bytes = 0;
+    gca::BufferPool pool;
+    gca::HdrPool hdrs;
     int n_cu = 0;         // compute units of the device (persistent launch sizing)
     int wall_khz = 0;     // rate of the device wall clock (wall_clock64)
     // persistent bitmap of the voxel downsampler (kept all-zero between calls)
@@ -128,7 +173,7 @@ struct gca_ctx_s {
     size_t lut_bytes = 0;
     int32_t lut_key_mode = -1, lut_key_radius = -1;
     float lut_key_ss = -1.f, lut_key_sd = -1.f;
-    int32_t lut_len = 0;
+    int32_t lut_ws_off[6] = {0}, lut_wr_off[6] = {0}, lut_wr_len[6] = {0};
     // ICP device state
     void *icp_state = nullptr;
     size_t icp_state_bytes = 0;
@@ -179,10 +224,12 @@ struct gca_cloud_s {
     int64_t cap = 0;
     float4 *xyzi = nullptr, *rgb = nullptr, *nrm = nullptr, *grad = nullptr;
     gca::CloudHdr *hdr = nullptr;
+    gca::HdrRef ref{};  // hdr's slot; with cap 1 the four arrays may lie in it too
     bool has_normals = false, has_gradient = false;
     // host copy of the header (valid when host_valid)
     bool host_valid = false;
     gca::CloudHdr host_hdr{};
+    bool n_valid = false;  // host_hdr.n alone is current (the bounds may not be)
     // cached neighbour grid (built for grid.desc.radius); invalidated when points change
     gca::Grid grid;
 };
@@ -192,10 +239,33 @@ namespace gca {
 // Internal helpers implemented in api.hip -------------------------------------------------
 int32_t hip_status(hipError_t e);
 void *ctx_scratch(gca_ctx ctx, int slot, size_t bytes, bool zeroed);
+// Pinned host memory of the ctx; its content is the calling entry point's until that returns.
+void *ctx_host_buf(gca_ctx ctx, size_t bytes);
+// Buffers of clouds and grids (BufferPool).  dev_free: bytes as allocated; idle = device_idle()
+// succeeded after the last work that may use p was enqueued (else p goes back to the runtime,
+// which waits for the device itself).
+int32_t dev_alloc(gca_ctx ctx, void **p, size_t bytes);
+void dev_free(gca_ctx ctx, void *p, size_t bytes, bool idle);
+void grid_free_cells(gca_ctx ctx, Grid &g, bool idle);   // count, start
+void grid_free_points(gca_ctx ctx, Grid &g, bool idle);  // the arrays of cap_pts entries
+bool device_idle(gca_ctx ctx);  // waits until all work of all streams of the device is done
+template <class T>
+int32_t dev_array(gca_ctx ctx, T **p, int64_t n)
+{
+    return dev_alloc(ctx, (void **)p, sizeof(T) * (size_t)n);
+}
+template <class T>
+void dev_array_free(gca_ctx ctx, T *&p, int64_t n, bool idle)
+{
+    dev_free(ctx, p, sizeof(T) * (size_t)n, idle);
+    p = nullptr;
+}
 // GCA_ERR_DEVICE (and clears it) when a kernel raised the ctx's device error word.
 int32_t ctx_take_device_error(gca_ctx ctx);
 int32_t cloud_reserve(gca_cloud c, int64_t cap);
 int32_t cloud_sync_header(gca_cloud c);  // copies hdr to host (synchronises the stream)
+// host_hdr.n current for a call on ctx's stream: no read-back where the host set the count itself.
+int32_t cloud_sync_count(gca_ctx ctx, gca_cloud c);
 void cloud_host_bounds(gca_cloud c, float mn[3], float mx[3]);
 void cloud_points_changed(gca_cloud c);
 // (Re)builds c->grid so that it serves queries of `radius`.  A cached grid whose cell edge lies
@@ -270,6 +340,8 @@ int32_t launch_normals_gradient(gca_ctx ctx, gca_cloud c, float radius, int32_t 
                                 bool grid_attrs = false);
 int32_t launch_transform(gca_ctx ctx, gca_cloud c, const double T[16]);
 int32_t launch_bounds(gca_ctx ctx, gca_cloud c);
+// The bounds of hdr->n points (at most cap) into hdr.
+hipError_t bounds_enqueue(gca_ctx ctx, const float4 *xyzi, int64_t cap, CloudHdr *hdr);
 int32_t launch_copy_cloud(gca_ctx ctx, gca_cloud src, gca_cloud dst);
 int32_t launch_upload_finish(gca_ctx ctx, gca_cloud c, int64_t n);
 

@@ -81,37 +81,42 @@ __global__ __launch_bounds__(256) void k_grid_scatter(Jobs<ScatterArgs, N> J)
     }
 }
 
+void grid_free_cells(gca_ctx ctx, Grid &g, bool idle)
+{
+    dev_array_free(ctx, g.count, g.cap_cells, idle);
+    dev_array_free(ctx, g.start, g.cap_cells + 1, idle);
+    g.cap_cells = 0;
+}
+
+void grid_free_points(gca_ctx ctx, Grid &g, bool idle)
+{
+    dev_array_free(ctx, g.order, g.cap_pts, idle);
+    dev_array_free(ctx, g.sxyzi, g.cap_pts, idle);
+    dev_array_free(ctx, g.cell_of, g.cap_pts, idle);
+    dev_array_free(ctx, g.snrm, g.cap_pts, idle);
+    dev_array_free(ctx, g.sgrad, g.cap_pts, idle);
+    g.cap_pts = 0;
+}
+
 int32_t grid_prepare(gca_ctx ctx, gca_cloud c, const GridDesc &d)
 {
     Grid &G = c->grid;
     G.valid = false;
     if (G.cap_cells < d.ncells) {
-        GCA_HIP(hipStreamSynchronize(ctx->stream));
-        hipFree(G.count);
-        hipFree(G.start);
-        G.count = G.start = nullptr;
-        G.cap_cells = 0;
+        if (G.count) GCA_HIP(hipStreamSynchronize(ctx->stream));
+        grid_free_cells(c->ctx, G, G.count && device_idle(c->ctx));
         int64_t want = std::min<int64_t>(kGridCellCap, d.ncells + d.ncells / 4 + 1024);
-        GCA_HIP(hipMalloc(&G.count, sizeof(uint32_t) * want));
-        GCA_HIP(hipMalloc(&G.start, sizeof(uint32_t) * (want + 1)));
+        GCA_TRY(dev_array(c->ctx, &G.count, want));
+        GCA_TRY(dev_array(c->ctx, &G.start, want + 1));
         GCA_HIP(hipMemsetAsync(G.count, 0, sizeof(uint32_t) * want, ctx->stream));
         G.cap_cells = want;
     }
     if (G.cap_pts < c->cap) {
-        GCA_HIP(hipStreamSynchronize(ctx->stream));
-        hipFree(G.order);
-        hipFree(G.sxyzi);
-        hipFree(G.cell_of);
-        hipFree(G.snrm);
-        hipFree(G.sgrad);
-        G.order = nullptr;
-        G.sxyzi = nullptr;
-        G.cell_of = nullptr;
-        G.snrm = G.sgrad = nullptr;
-        G.cap_pts = 0;
-        GCA_HIP(hipMalloc(&G.order, sizeof(int32_t) * c->cap));
-        GCA_HIP(hipMalloc(&G.sxyzi, sizeof(float4) * c->cap));
-        GCA_HIP(hipMalloc(&G.cell_of, sizeof(uint32_t) * c->cap));
+        if (G.order) GCA_HIP(hipStreamSynchronize(ctx->stream));
+        grid_free_points(c->ctx, G, G.order && device_idle(c->ctx));
+        GCA_TRY(dev_array(c->ctx, &G.order, c->cap));
+        GCA_TRY(dev_array(c->ctx, &G.sxyzi, c->cap));
+        GCA_TRY(dev_array(c->ctx, &G.cell_of, c->cap));
         G.cap_pts = c->cap;
     }
     return GCA_OK;
@@ -190,8 +195,8 @@ int32_t grid_gather_attributes(gca_ctx ctx, gca_cloud c)
     if (!G.valid) return GCA_ERR_NOT_READY;
     if (G.attrs_valid) return GCA_OK;
     if (!G.snrm) {
-        GCA_HIP(hipMalloc(&G.snrm, sizeof(float4) * G.cap_pts));
-        GCA_HIP(hipMalloc(&G.sgrad, sizeof(float4) * G.cap_pts));
+        GCA_TRY(dev_array(c->ctx, &G.snrm, G.cap_pts));
+        GCA_TRY(dev_array(c->ctx, &G.sgrad, G.cap_pts));
     }
     const unsigned nb = (unsigned)std::min<int64_t>(4096, std::max<int64_t>(1, (c->cap + 255) / 256));
     hipLaunchKernelGGL(k_gather_sorted, dim3(nb), dim3(256), 0, ctx->stream, c->hdr, G.order, c->nrm, c->grad,
@@ -431,9 +436,9 @@ int32_t launch_radius(gca_ctx ctx, gca_cloud q, gca_cloud ref, float radius, int
                        d, G.start, G.sxyzi, (uint32_t)max_nn, cnt);
     GCA_HIP(hipGetLastError());
     GCA_TRY(exclusive_scan_u32(ctx, cnt, (uint32_t *)offsets, nq, tot_dev));
-    uint32_t capped = 0;
-    GCA_HIP(hipMemcpyAsync(&capped, tot_dev, sizeof(uint32_t), hipMemcpyDeviceToHost, ctx->stream));
+    GCA_HIP(hipMemcpyAsync(ctx->pinned, tot_dev, sizeof(uint32_t), hipMemcpyDeviceToHost, ctx->stream));
     GCA_HIP(hipStreamSynchronize(ctx->stream));
+    const uint32_t capped = *(const uint32_t *)ctx->pinned;
     *total = capped;
     if (!idx) return GCA_OK;  // count-only query
     if ((int64_t)capped > idx_cap) return GCA_ERR_INVALID_VALUE;

@@ -1411,6 +1411,7 @@ struct IcpWork {
     int32_t *unit_state = nullptr;
     int32_t *unit_first = nullptr;
     uint32_t *err = nullptr;
+    size_t init_off = 0, t0_off = 0;  // from pairs on, in bytes
 };
 
 static size_t align256(size_t b) { return (b + 255) & ~size_t(255); }
@@ -1418,21 +1419,22 @@ static size_t align256(size_t b) { return (b + 255) & ~size_t(255); }
 static int32_t icp_work(gca_ctx ctx, int n_states, int n_t0, int64_t partial_slots, int64_t nnprev_n,
                         int64_t table_units, IcpWork &w)
 {
-    w.states = (IcpState *)ctx_scratch(ctx, 13, sizeof(IcpState) * n_states, false);
+    w.states = (IcpState *)ctx_scratch(ctx, 13, sizeof(IcpState) * n_states + 256, false);
     w.partials = (double *)ctx_scratch(ctx, 14, sizeof(double) * kPartStride * std::max<int64_t>(partial_slots, 1), false);
     w.nnprev = (int32_t *)ctx_scratch(ctx, 16, sizeof(int32_t) * std::max<int64_t>(nnprev_n, 1), false);
     if (!w.states || !w.partials || !w.nnprev) return GCA_ERR_OUT_OF_MEMORY;
     const size_t b_pairs = align256(sizeof(PairDesc) * n_states), b_init = align256(sizeof(StateInit) * n_states),
                  b_t0 = align256(sizeof(double) * 16 * std::max(n_t0, 4)),
                  b_us = align256(sizeof(int32_t) * std::max<int64_t>(table_units, 1)),
-                 b_uf = align256(sizeof(int32_t) * n_states), b_err = 256;
-    const size_t need = b_pairs + b_init + b_t0 + b_us + b_uf + b_err;
+                 b_uf = align256(sizeof(int32_t) * n_states);
+    const size_t need = b_pairs + b_init + b_t0 + b_us + b_uf;
     if (!ctx->icp_state || ctx->icp_state_bytes < need) {
         GCA_HIP(hipStreamSynchronize(ctx->stream));
         hipFree(ctx->icp_state);
         ctx->icp_state = nullptr;
+        ctx->icp_state_bytes = 0;
         size_t want = need * 2 + 4096;
-        GCA_HIP(hipMalloc(&ctx->icp_state, want));
+        GCA_TRY(dev_alloc(ctx, &ctx->icp_state, want));
         ctx->icp_state_bytes = want;
     }
     char *base = (char *)ctx->icp_state;
@@ -1441,12 +1443,13 @@ static int32_t icp_work(gca_ctx ctx, int n_states, int n_t0, int64_t partial_slo
     w.init = (StateInit *)base;
     base += b_init;
     w.T0 = (double *)base;
+    w.init_off = b_pairs;
+    w.t0_off = b_pairs + b_init;
     base += b_t0;
     w.unit_state = (int32_t *)base;
     base += b_us;
     w.unit_first = (int32_t *)base;
-    base += b_uf;
-    w.err = (uint32_t *)base;
+    w.err = (uint32_t *)(w.states + n_states);  // read back with the states
     return GCA_OK;
 }
 
@@ -1660,9 +1663,15 @@ static int32_t run_states(gca_ctx ctx, int n_pairs, int n_levels, const gca_clou
     std::vector<StateInit> I;
     std::vector<int32_t> tail;
     states_describe(n_pairs, n_levels, srcs, tgts, params, lanes, unit_cap, w.partials, w.nnprev, nn_off, P, I, tail);
-    GCA_HIP(hipMemcpyAsync(w.pairs, P.data(), sizeof(PairDesc) * n_states, hipMemcpyHostToDevice, ctx->stream));
-    GCA_HIP(hipMemcpyAsync(w.init, I.data(), sizeof(StateInit) * n_states, hipMemcpyHostToDevice, ctx->stream));
-    GCA_HIP(hipMemcpyAsync(w.T0, T0, sizeof(double) * 16 * n_pairs, hipMemcpyHostToDevice, ctx->stream));
+    // one upload and one read-back, from and to pinned memory (free here: a call that uses it ends
+    // with the stream synchronised)
+    const size_t up = w.t0_off + sizeof(double) * 16 * n_pairs, down = sizeof(IcpState) * n_states + sizeof(uint32_t);
+    char *host = (char *)ctx_host_buf(ctx, align256(up) + down);
+    if (!host) return GCA_ERR_OUT_OF_MEMORY;
+    memcpy(host, P.data(), sizeof(PairDesc) * n_states);
+    memcpy(host + w.init_off, I.data(), sizeof(StateInit) * n_states);
+    memcpy(host + w.t0_off, T0, sizeof(double) * 16 * n_pairs);
+    GCA_HIP(hipMemcpyAsync(w.pairs, host, up, hipMemcpyHostToDevice, ctx->stream));
     hipLaunchKernelGGL(k_state_init, dim3((n_states + 63) / 64), dim3(64), 0, ctx->stream, w.states,
                        (const PairDesc *)w.pairs, (const StateInit *)w.init, (const double *)w.T0, n_states, w.err);
     GCA_HIP(hipGetLastError());
@@ -1704,14 +1713,13 @@ static int32_t run_states(gca_ctx ctx, int n_pairs, int n_levels, const gca_clou
         GCA_HIP(hipGetLastError());
     }
 
-    std::vector<IcpState> S(n_states);
-    uint32_t err = 0;
-    // one contiguous copy (a strided copy into pageable memory costs a transfer per row)
-    GCA_HIP(hipMemcpyAsync(S.data(), w.states, sizeof(IcpState) * n_states, hipMemcpyDeviceToHost, ctx->stream));
-    GCA_HIP(hipMemcpyAsync(&err, w.err, sizeof(err), hipMemcpyDeviceToHost, ctx->stream));
+    const IcpState *S = (const IcpState *)(host + align256(up));
+    GCA_HIP(hipMemcpyAsync(host + align256(up), w.states, down, hipMemcpyDeviceToHost, ctx->stream));
     GCA_HIP(hipStreamSynchronize(ctx->stream));
+    uint32_t err;
+    memcpy(&err, S + n_states, sizeof(err));
     if (err) return GCA_ERR_DEVICE;
-    states_report(ctx, S.data(), n_pairs, n_states, tail, T0, T_out, reps);
+    states_report(ctx, S, n_pairs, n_states, tail, T0, T_out, reps);
     return GCA_OK;
 }
 
@@ -1903,7 +1911,7 @@ int32_t icp_plan_results(gca_ctx ctx, const IcpPlan *p, double *T_out, gca_icp_r
 // the sums into the ctx's pinned memory, so a stream synchronisation is all it takes to read them.
 static int32_t single_pair(gca_ctx ctx, gca_cloud src, gca_cloud tgt, PairDesc &P, uint32_t **ticket)
 {
-    GCA_TRY(cloud_sync_header(src));
+    GCA_TRY(cloud_sync_count(ctx, src));
     P = PairDesc{};
     P.src = src->xyzi;
     P.src_hdr = src->hdr;

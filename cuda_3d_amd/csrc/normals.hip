@@ -676,8 +676,8 @@ static int32_t pair_prepare(gca_ctx ctx, gca_cloud c, float radius, int32_t K, f
     if (!(gradient_radius <= radius)) return GCA_ERR_INVALID_VALUE;
     Grid &G = c->grid;
     if (grid_attrs && !G.snrm) {
-        GCA_HIP(hipMalloc(&G.snrm, sizeof(float4) * G.cap_pts));
-        GCA_HIP(hipMalloc(&G.sgrad, sizeof(float4) * G.cap_pts));
+        GCA_TRY(dev_array(c->ctx, &G.snrm, G.cap_pts));
+        GCA_TRY(dev_array(c->ctx, &G.sgrad, G.cap_pts));
     }
     const int64_t cap = std::max<int64_t>(c->cap, 1);
     Moments *mom = (Moments *)ctx_scratch(ctx, 17, sizeof(Moments) * cap, false);

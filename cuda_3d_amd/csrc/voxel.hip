@@ -492,7 +492,7 @@ static int32_t voxel_prepare(gca_ctx ctx, gca_cloud in, float voxel, gca_cloud o
             ctx->bitmap = nullptr;
             ctx->bitmap_words = 0;
             int64_t want = std::max<int64_t>(words + words / 4, 1 << 16);
-            GCA_HIP(hipMalloc(&ctx->bitmap, sizeof(uint32_t) * want));
+            GCA_TRY(dev_array(ctx, &ctx->bitmap, want));
             ctx->bitmap_words = want;
         }
         GCA_HIP(hipMemsetAsync(ctx->bitmap, 0, sizeof(uint32_t) * ctx->bitmap_words, ctx->stream));
