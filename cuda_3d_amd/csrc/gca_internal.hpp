@@ -360,7 +360,8 @@ bool icp_plan_clouds_current(const IcpPlan *plan, const gca_cloud *srcs, const i
 // The same launch in parts (state set-up; one state's persistent launch, which takes the
 // state's sizes from its clouds' headers, so it may be enqueued before they are final; results),
 // for overlapping state s's registration with the building of state s + 1's source.
-int32_t icp_plan_init(gca_ctx ctx, IcpPlan *plan);
+// sizes_later: icp_plan_persist will take the states' sizes (else icp_plan_run's launches).
+int32_t icp_plan_init(gca_ctx ctx, IcpPlan *plan, bool sizes_later);
 // Whether state s's target cloud still has the grid (geometry and arrays) the plan was made
 // with: a plan reads the target's grid through pointers and a geometry fixed at its creation.
 bool icp_plan_target_current(const IcpPlan *plan, int s, gca_cloud tgt);

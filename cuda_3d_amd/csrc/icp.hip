@@ -75,6 +75,14 @@ __host__ __device__ inline int subq_unit(int nvb, int x, int c)
     return x * q + (x < r ? x : r) + c;
 }
 
+// A state's open word: epoch << 32 | mask of the sub-queues with unclaimed units (epochs kEpochWait
+// and kEpochDone with an empty mask).  The words of a launch's states lie side by side, so a
+// workgroup looks for work with one coalesced read.
+__host__ __device__ inline unsigned long long open_word(uint32_t epoch, int nvb)
+{
+    return (unsigned long long)epoch << 32 | (nvb >= kSubQ ? (1u << kSubQ) - 1u : (1u << nvb) - 1u);
+}
+
 struct IcpState {
     double T[16];
     double sys[kNSys];
@@ -458,7 +466,7 @@ __device__ __forceinline__ void sum_partials(const double *partials, int n, doub
 // result is exactly that of the full search.  Ties in d2 compare original indices, which are
 // loaded only then.
 constexpr int kMaxRuns = 9;
-constexpr int kUnroll = 4;
+constexpr int kUnroll = 4, kPersistUnroll = 8;  // candidates in flight per lane
 constexpr double kWarmRel = 1e-9, kWarmAbs = 1e-9;
 
 __device__ __forceinline__ void nn_consider(const PairDesc &P, double d2, int32_t s, double r2, double &bd,
@@ -473,6 +481,7 @@ __device__ __forceinline__ void nn_consider(const PairDesc &P, double d2, int32_
     }
 }
 
+template <int U>
 __device__ __forceinline__ int32_t nn_group(const PairDesc &P, float qx, float qy, float qz, int g, int G,
                                             int32_t sp)
 {
@@ -494,7 +503,7 @@ __device__ __forceinline__ int32_t nn_group(const PairDesc &P, float qx, float q
         const int nry = hi[1] - lo[1] + 1;
         const int nruns = (hi[0] - lo[0] + 1) * nry;
         if (nruns <= kMaxRuns) {
-            // bounds of all (ix, iy) runs up front, then one flattened walk with kUnroll
+            // bounds of all (ix, iy) runs up front, then one flattened walk with U
             // independent loads in flight per lane
             uint32_t rs[kMaxRuns], cum[kMaxRuns + 1];
 #pragma unroll
@@ -513,11 +522,11 @@ __device__ __forceinline__ int32_t nn_group(const PairDesc &P, float qx, float q
 #pragma unroll
             for (int r = 0; r < kMaxRuns; ++r) cum[r + 1] += cum[r];
             const uint32_t total = cum[kMaxRuns];
-            for (uint32_t f0 = g; f0 < total; f0 += G * kUnroll) {
-                uint32_t sl[kUnroll];
-                float4 c[kUnroll];
+            for (uint32_t f0 = g; f0 < total; f0 += G * U) {
+                uint32_t sl[U];
+                float4 c[U];
 #pragma unroll
-                for (int u = 0; u < kUnroll; ++u) {
+                for (int u = 0; u < U; ++u) {
                     const uint32_t f = f0 + u * G;
                     uint32_t s = 0xffffffffu;
                     if (f < total) {
@@ -530,7 +539,7 @@ __device__ __forceinline__ int32_t nn_group(const PairDesc &P, float qx, float q
                     sl[u] = s;
                 }
 #pragma unroll
-                for (int u = 0; u < kUnroll; ++u) {
+                for (int u = 0; u < U; ++u) {
                     if (sl[u] == 0xffffffffu) continue;
                     nn_consider(P, dist2(c[u].x, c[u].y, c[u].z, qx, qy, qz), (int32_t)sl[u], r2, bd, bs);
                 }
@@ -571,7 +580,7 @@ __device__ __forceinline__ int32_t nn_group(const PairDesc &P, float qx, float q
 // No accumulator is live during the search, which keeps register use (and so the number of
 // resident wavefronts hiding the search's load latency) in check.  Leaves the unit's partial in
 // sys[0..28] (LDS; entry k written by thread k).
-template <int MODE>
+template <int MODE, int U = kUnroll>
 __device__ __forceinline__ void icp_unit(const PairDesc &P, int n, int G, int nvb, int ntgt, int vb, bool warm,
                                          const double *T, double *sys)
 {
@@ -594,7 +603,7 @@ __device__ __forceinline__ void icp_unit(const PairDesc &P, int n, int G, int nv
             }
             // the warm-start slot is only a bound: any in-range value is safe, stale or not
             if ((uint32_t)sp >= (uint32_t)ntgt) sp = -1;
-            const int32_t s = nn_group(P, x, y, z, g, G, sp);
+            const int32_t s = nn_group<U>(P, x, y, z, g, G, sp);
             if (g == 0) slot[j] = s;
         }
         __syncthreads();
@@ -655,10 +664,11 @@ __device__ __forceinline__ double euler_elem(int t, const double *trig, const do
 // Epoch finish of state p (whole workgroup, run by the workgroup that took the last ticket):
 // fixed-order FP64 sum of the unit partials, LDL^T solve, Euler increment, T <- dT T, the
 // stopping rule of color_icp.cu:216-228, then the hand-over: the next epoch of this state, or
-// the pose to the next level of the chain.  A failed solve takes the identity step (which also
+// the pose to the next level of the chain (all_queues: its sizes are not known yet, the launch that
+// runs it masks the open word).  A failed solve takes the identity step (which also
 // satisfies the stopping rule), as the reference does.
-__device__ __noinline__ void icp_finish(IcpState *states, int p, uint32_t epoch, const double *partials, int nvb, double *sys,
-                                        bool naive)
+__device__ __noinline__ void icp_finish(IcpState *states, unsigned long long *open, int p, uint32_t epoch,
+                                        const double *partials, int nvb, bool all_queues, double *sys, bool naive)
 {
     IcpState *st = states + p;
     __shared__ double Tc[16], Tn[16], dT[16], xi[6], trig[6];
@@ -731,6 +741,15 @@ __device__ __noinline__ void icp_finish(IcpState *states, int p, uint32_t epoch,
                 __hip_atomic_store(&states[f_next].q[t].w, 0ull, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
         }
     }
+    // A workgroup that sees an open word before the claim words only loses a claim.
+    if (t == kSubQ) {
+        const unsigned long long w =
+            f_done ? (unsigned long long)kEpochDone << 32 : open_word(epoch + 1, nvb);
+        __hip_atomic_store(&open[p], w, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        if (f_done && f_next >= 0)
+            __hip_atomic_store(&open[f_next], open_word(0, all_queues ? kSubQ : states[f_next].nvb), __ATOMIC_RELAXED,
+                               __HIP_MEMORY_SCOPE_AGENT);
+    }
 }
 
 // Unit partial -> global, ticket, and the epoch finish by the workgroup completing the epoch.
@@ -740,8 +759,8 @@ __device__ __noinline__ void icp_finish(IcpState *states, int p, uint32_t epoch,
 // whichever XCD it runs.  The partial and the matched slots are written through, so the
 // release has little left to write back.
 template <int MODE>
-__device__ __forceinline__ void unit_commit(const PairDesc &P, IcpState *states, int p, int vb, int nvb,
-                                            uint32_t epoch, double *sys)
+__device__ __forceinline__ void unit_commit(const PairDesc &P, IcpState *states, unsigned long long *open, int p, int vb,
+                                            int nvb, bool all_queues, uint32_t epoch, double *sys)
 {
     __shared__ bool last;
     if (threadIdx.x < kNSys) store_coherent(&P.partials[(int64_t)vb * kPartStride + threadIdx.x], sys[threadIdx.x]);
@@ -751,29 +770,38 @@ __device__ __forceinline__ void unit_commit(const PairDesc &P, IcpState *states,
     __syncthreads();
     if (!last) return;
     fence_acquire_agent();
-    icp_finish(states, p, epoch, P.partials, nvb, sys, MODE == GCA_ACCUM_NAIVE_FP32);
+    icp_finish(states, open, p, epoch, P.partials, nvb, all_queues, sys, MODE == GCA_ACCUM_NAIVE_FP32);
 }
 
 // ---- persistent launch: every iteration of every state --------------------------------------
-// Scheduling loop of one workgroup: read the claim words (one coherent load per state and
-// sub-queue, a window at a time), pick the first state with unclaimed units in round-robin order
-// from the state last served and, in it, the sub-queue nearest to the workgroup's own, claim a
-// unit with one atomic, run it.  A workgroup only waits (sleep + re-poll)
+// Scheduling loop of one workgroup: read the open words (a coalesced coherent read of kIcpBlock
+// states at a time), pick the first state with unclaimed units in round-robin order from the state
+// last served and, in it, the sub-queue nearest to the workgroup's own, claim a unit with one
+// atomic, run it.  The claim of a sub-queue's last unit takes its bit out of the open word before
+// the unit runs, so before the epoch can end.  A workgroup only waits (sleep + re-poll)
 // when every unit of every open epoch is claimed, i.e. held by running workgroups, so progress
 // never depends on how many workgroups are resident.  Exits when every state is done.
-// (Claiming first and scanning only on failure was measured slower: every workgroup that ends
-// a unit after the epoch is drained adds a failing atomic on a hot claim word.)
-// 4 wavefronts per SIMD (<= 128 VGPRs): resident wavefronts are what hides the latency of the
-// neighbour search's dependent loads.
+// (Reading the claim words themselves, 64 of them at a time, took a workgroup without work 24
+// dependent reads for the 192 states of 64 pairs on three levels: a lone state's iteration then
+// lasted 57 us, most of it the wait until somebody came past its open epoch again.  Claiming first
+// and scanning only on failure was measured slower: every workgroup that ends a unit after the
+// epoch is drained adds a failing atomic on a hot claim word.)
+// 4 wavefronts per SIMD (<= 128 VGPRs) for the launches below that need their workgroups resident, so
+// that two of them fit the device at once.  The persistent launch needs none of its workgroups
+// resident and takes the registers (144) that 8 candidates in flight need: three workgroups per CU,
+// and as many are launched.  64 pairs of 5k to 200k points, three levels: 8.25 ms with the claim
+// words scanned; 6.57 with the open words, 6.41 with 8 candidates in flight (4: 6.5), 5.92 with three
+// workgroups per CU (four, of which one waits for its turn: 5.92).
 #define GCA_ICP_OCCUPANCY __attribute__((amdgpu_waves_per_eu(4, 8)))
-constexpr int kScanWindow = 64;  // claim words read per scan round (one wavefront's loads)
-
+#define GCA_PERSIST_OCCUPANCY __attribute__((amdgpu_waves_per_eu(3, 8)))
+constexpr int kPersistPerCu = 3;
 // refresh (launches over one state only): the state's sizes are taken from its clouds' headers
 // at the start, by every workgroup for itself (workgroup 0 also stores them in the state), for a
 // launch enqueued before its source cloud's size was final.
 template <int MODE>
-__global__ __launch_bounds__(kIcpBlock) GCA_ICP_OCCUPANCY void k_icp_persist(const PairDesc *__restrict__ pairs, IcpState *states,
-                                                           int s_first, int n_states, int refresh, uint32_t *err)
+__global__ __launch_bounds__(kIcpBlock) GCA_PERSIST_OCCUPANCY void k_icp_persist(const PairDesc *__restrict__ pairs, IcpState *states,
+                                                           unsigned long long *open, int s_first, int n_states,
+                                                           int refresh, uint32_t *err)
 {
     __shared__ double T[12];
     __shared__ double sys[kPartStride];
@@ -812,36 +840,30 @@ __global__ __launch_bounds__(kIcpBlock) GCA_ICP_OCCUPANCY void k_icp_persist(con
     int home = (int)(blockIdx.x % (unsigned)n_states);
     const int myq = (int)(blockIdx.x % (unsigned)kSubQ);  // workgroups are dealt to XCDs round-robin
     uint32_t idle = 0;
-    const int n_words = n_states * kSubQ;
     for (;;) {
-        // The claim words are read a window of kScanWindow words at a time, from the state last
-        // served on; the next window is read only when this one has no unclaimed unit.  (Reading
-        // every word for every claim put so much polling traffic on a few hot lines that it
-        // bounded a launch with many states: 64 words per round run the 64-pair batch 17 %
-        // faster than all 1536, 256 words 12 % faster.)
         int my_rot = INT_MAX;
         uint32_t my_epoch = 0;
         int pick = INT_MAX, alive = 0;
-        for (int w0 = 0; w0 < n_words; w0 += kScanWindow) {
+        for (int w0 = 0; w0 < n_states; w0 += kIcpBlock) {
             if (threadIdx.x == 0) {
                 s_pick = INT_MAX;
                 s_alive = 0;
             }
             __syncthreads();
-            const int r = w0 + (int)threadIdx.x;  // rotation index: state (home + r / kSubQ), slot r % kSubQ
-            if ((int)threadIdx.x < kScanWindow && r < n_words) {
-                const int p = s_first + (home + r / kSubQ) % n_states, x = (myq + r % kSubQ) % kSubQ;
-                const unsigned long long w =
-                    __hip_atomic_load(&states[p].q[x].w, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-                const uint32_t e = (uint32_t)(w >> 32), c = (uint32_t)w;
+            const int r = w0 + (int)threadIdx.x;  // rotation index: state home + r
+            if (r < n_states) {
+                const int p = s_first + (home + r < n_states ? home + r : home + r - n_states);
+                const unsigned long long w = __hip_atomic_load(&open[p], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+                const uint32_t e = (uint32_t)(w >> 32);
+                uint32_t mask = (uint32_t)w;
+                if (refresh) mask &= (uint32_t)open_word(0, s_nvb);
                 if (e != kEpochDone) {
                     s_alive = 1;
-                    // first state in round-robin order from the last one served, then the
-                    // sub-queue nearest to this workgroup's own
-                    if (e != kEpochWait && c < subq_units(refresh ? s_nvb : states[p].nvb, x)) {
-                        my_rot = r;
+                    if (mask) {
+                        const uint32_t turned = (mask >> myq) | (mask << (kSubQ - myq));
+                        my_rot = r * kSubQ + __builtin_ctz(turned);
                         my_epoch = e;
-                        atomicMin(&s_pick, r);
+                        atomicMin(&s_pick, my_rot);
                     }
                 }
             }
@@ -880,6 +902,8 @@ __global__ __launch_bounds__(kIcpBlock) GCA_ICP_OCCUPANCY void k_icp_persist(con
             const bool ok = e < kEpochWait && c < subq_units(refresh ? s_nvb : st->nvb, x);
             s_vb = ok ? subq_unit(refresh ? s_nvb : st->nvb, x, (int)c) : -1;
             s_epoch = e;
+            if (ok && c + 1 == subq_units(refresh ? s_nvb : st->nvb, x))
+                __hip_atomic_fetch_and(&open[p], ~(1ull << x), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
             if (ok && e == 0 && c == 0 && x == 0) st->t_start = wall_clock64();  // unit 0 of the first epoch
         } else if (threadIdx.x >= kWave && threadIdx.x < kWave + 12) {
             T[threadIdx.x - kWave] = load_coherent(&st->T[threadIdx.x - kWave]);
@@ -897,10 +921,10 @@ __global__ __launch_bounds__(kIcpBlock) GCA_ICP_OCCUPANCY void k_icp_persist(con
         const PairDesc &P = pairs[p];
         const int nvb = refresh ? s_nvb : st->nvb;
         if (refresh)
-            icp_unit<MODE>(P, s_nsrc, s_G, nvb, s_ntgt, vb, epoch > 0, T, sys);
+            icp_unit<MODE, kPersistUnroll>(P, s_nsrc, s_G, nvb, s_ntgt, vb, epoch > 0, T, sys);
         else
-            icp_unit<MODE>(P, st->n_src, st->G, nvb, st->n_tgt, vb, epoch > 0, T, sys);
-        unit_commit<MODE>(P, states, p, vb, nvb, epoch, sys);
+            icp_unit<MODE, kPersistUnroll>(P, st->n_src, st->G, nvb, st->n_tgt, vb, epoch > 0, T, sys);
+        unit_commit<MODE>(P, states, open, p, vb, nvb, refresh != 0, epoch, sys);
     }
 }
 
@@ -908,6 +932,7 @@ __global__ __launch_bounds__(kIcpBlock) GCA_ICP_OCCUPANCY void k_icp_persist(con
 // Workgroup b runs unit b - unit_first[s] of state s = unit_state[b]; states that are done exit.
 template <int MODE>
 __global__ __launch_bounds__(kIcpBlock) GCA_ICP_OCCUPANCY void k_icp_iter(const PairDesc *__restrict__ pairs, IcpState *states,
+                                                        unsigned long long *open,
                                                         const int32_t *__restrict__ unit_state,
                                                         const int32_t *__restrict__ unit_first)
 {
@@ -924,7 +949,7 @@ __global__ __launch_bounds__(kIcpBlock) GCA_ICP_OCCUPANCY void k_icp_iter(const 
     const PairDesc &P = pairs[p];
     const int nvb = st->nvb;
     icp_unit<MODE>(P, st->n_src, st->G, nvb, st->n_tgt, vb, epoch > 0, T, sys);
-    unit_commit<MODE>(P, states, p, vb, nvb, epoch, sys);
+    unit_commit<MODE>(P, states, open, p, vb, nvb, false, epoch, sys);
 }
 
 // ---- resident launch: one state, every iteration, no scheduler ---------------------------------
@@ -1342,7 +1367,7 @@ struct StateInit {
 
 // Sizes come from the clouds' device headers, so set-up needs no host round trip.
 __global__ void k_state_init(IcpState *states, const PairDesc *__restrict__ pairs, const StateInit *__restrict__ init,
-                             const double *__restrict__ T0, int n, uint32_t *err)
+                             const double *__restrict__ T0, int n, unsigned long long *open, int all_queues, uint32_t *err)
 {
     const int p = blockIdx.x * blockDim.x + threadIdx.x;
     if (p == 0) *err = 0u;
@@ -1373,6 +1398,7 @@ __global__ void k_state_init(IcpState *states, const PairDesc *__restrict__ pair
         s.q[x].w = w0;
         s.bar[x].w = 0ull;
     }
+    open[p] = I.max_iter <= 0 || !I.open ? w0 : open_word(0, all_queues ? kSubQ : s.nvb);
     s.ticket = 0u;
     s.bar_top = 0u;
 }
@@ -1411,6 +1437,7 @@ struct IcpWork {
     int32_t *unit_state = nullptr;
     int32_t *unit_first = nullptr;
     uint32_t *err = nullptr;
+    unsigned long long *open = nullptr;
     size_t init_off = 0, t0_off = 0;  // from pairs on, in bytes
 };
 
@@ -1419,7 +1446,7 @@ static size_t align256(size_t b) { return (b + 255) & ~size_t(255); }
 static int32_t icp_work(gca_ctx ctx, int n_states, int n_t0, int64_t partial_slots, int64_t nnprev_n,
                         int64_t table_units, IcpWork &w)
 {
-    w.states = (IcpState *)ctx_scratch(ctx, 13, sizeof(IcpState) * n_states + 256, false);
+    w.states = (IcpState *)ctx_scratch(ctx, 13, sizeof(IcpState) * n_states + 256 + sizeof(*w.open) * n_states, false);
     w.partials = (double *)ctx_scratch(ctx, 14, sizeof(double) * kPartStride * std::max<int64_t>(partial_slots, 1), false);
     w.nnprev = (int32_t *)ctx_scratch(ctx, 16, sizeof(int32_t) * std::max<int64_t>(nnprev_n, 1), false);
     if (!w.states || !w.partials || !w.nnprev) return GCA_ERR_OUT_OF_MEMORY;
@@ -1450,6 +1477,7 @@ static int32_t icp_work(gca_ctx ctx, int n_states, int n_t0, int64_t partial_slo
     base += b_us;
     w.unit_first = (int32_t *)base;
     w.err = (uint32_t *)(w.states + n_states);  // read back with the states
+    w.open = (unsigned long long *)((char *)w.err + 256);
     return GCA_OK;
 }
 
@@ -1502,7 +1530,7 @@ template <int MODE>
 static void launch_iter(gca_ctx ctx, const IcpWork &w, int64_t off, int64_t units)
 {
     hipLaunchKernelGGL(k_icp_iter<MODE>, dim3((unsigned)units), dim3(kIcpBlock), 0, ctx->stream, w.pairs, w.states,
-                       w.unit_state + off, w.unit_first);
+                       w.open, w.unit_state + off, w.unit_first);
 }
 
 // ---- registration states: shared set-up ----------------------------------------------------
@@ -1564,27 +1592,27 @@ static void states_describe(int n_pairs, int n_levels, const gca_cloud *srcs, co
 }
 
 template <int MODE>
-static void launch_persist_mode(gca_ctx ctx, const PairDesc *pairs, IcpState *states, int s_first, int n_states,
-                                int refresh, uint32_t *err)
+static void launch_persist_mode(gca_ctx ctx, const PairDesc *pairs, IcpState *states, unsigned long long *open, int s_first,
+                                int n_states, int refresh, uint32_t *err)
 {
-    const int blocks = ctx->tune[GCA_TUNE_ICP_PERSIST_BLOCKS] ? ctx->tune[GCA_TUNE_ICP_PERSIST_BLOCKS] : 2 * ctx->n_cu;
+    const int blocks = ctx->tune[GCA_TUNE_ICP_PERSIST_BLOCKS] ? ctx->tune[GCA_TUNE_ICP_PERSIST_BLOCKS] : kPersistPerCu * ctx->n_cu;
     hipLaunchKernelGGL(k_icp_persist<MODE>, dim3((unsigned)blocks), dim3(kIcpBlock), 0, ctx->stream, pairs, states,
-                       s_first, n_states, refresh, err);
+                       open, s_first, n_states, refresh, err);
 }
 
 // The persistent launch over states [s_first, s_first + n_states) (the chain links of their
 // finishers may open states after the range: those run in a later launch).  refresh: one state,
 // whose sizes the launch takes from its clouds' headers.
-static void launch_persist_any(gca_ctx ctx, int mode, const PairDesc *pairs, IcpState *states, int n_states,
-                               uint32_t *err, int s_first = 0, int refresh = 0)
+static void launch_persist_any(gca_ctx ctx, int mode, const PairDesc *pairs, IcpState *states, unsigned long long *open,
+                               int n_states, uint32_t *err, int s_first = 0, int refresh = 0)
 {
     StageTimer timer(ctx, GCA_STAGE_ICP);
     if (mode == GCA_ACCUM_NAIVE_FP32)
-        launch_persist_mode<GCA_ACCUM_NAIVE_FP32>(ctx, pairs, states, s_first, n_states, refresh, err);
+        launch_persist_mode<GCA_ACCUM_NAIVE_FP32>(ctx, pairs, states, open, s_first, n_states, refresh, err);
     else if (mode == GCA_ACCUM_FP64)
-        launch_persist_mode<GCA_ACCUM_FP64>(ctx, pairs, states, s_first, n_states, refresh, err);
+        launch_persist_mode<GCA_ACCUM_FP64>(ctx, pairs, states, open, s_first, n_states, refresh, err);
     else
-        launch_persist_mode<GCA_ACCUM_COMPENSATED>(ctx, pairs, states, s_first, n_states, refresh, err);
+        launch_persist_mode<GCA_ACCUM_COMPENSATED>(ctx, pairs, states, open, s_first, n_states, refresh, err);
 }
 
 // The resident launch (k_icp_resident) over state s: one workgroup per unit, so it is used only
@@ -1673,7 +1701,7 @@ static int32_t run_states(gca_ctx ctx, int n_pairs, int n_levels, const gca_clou
     memcpy(host + w.t0_off, T0, sizeof(double) * 16 * n_pairs);
     GCA_HIP(hipMemcpyAsync(w.pairs, host, up, hipMemcpyHostToDevice, ctx->stream));
     hipLaunchKernelGGL(k_state_init, dim3((n_states + 63) / 64), dim3(64), 0, ctx->stream, w.states,
-                       (const PairDesc *)w.pairs, (const StateInit *)w.init, (const double *)w.T0, n_states, w.err);
+                       (const PairDesc *)w.pairs, (const StateInit *)w.init, (const double *)w.T0, n_states, w.open, 0, w.err);
     GCA_HIP(hipGetLastError());
 
     const int mode = params[0].accumulate_mode;
@@ -1684,7 +1712,7 @@ static int32_t run_states(gca_ctx ctx, int n_pairs, int n_levels, const gca_clou
         for (int s = 0; s < n_states; ++s) launch_resident_any(ctx, mode, w.pairs, w.states, s, 0, unit_cap, w.err);
         GCA_HIP(hipGetLastError());
     } else if (!per_iter) {
-        launch_persist_any(ctx, mode, w.pairs, w.states, n_states, w.err);
+        launch_persist_any(ctx, mode, w.pairs, w.states, w.open, n_states, w.err);
         GCA_HIP(hipGetLastError());
     } else {
         // unit tables level by level: level l's launches cover the units of its n_pairs states
@@ -1734,6 +1762,7 @@ struct IcpPlan {
     StateInit *init = nullptr;
     double *T0 = nullptr;
     uint32_t *err = nullptr;
+    unsigned long long *open = nullptr;
     IcpState *host_states = nullptr;  // pinned: written by the launch's copy, read after a sync
     uint32_t *host_err = nullptr;
     std::vector<int32_t> tail;
@@ -1800,7 +1829,8 @@ int32_t icp_plan_create(gca_ctx ctx, int n_pairs, int n_levels, const gca_cloud 
     if ((e = hipMalloc(&p->pairs, sizeof(PairDesc) * n_states)) != hipSuccess) return fail(e);
     if ((e = hipMalloc(&p->init, sizeof(StateInit) * n_states)) != hipSuccess) return fail(e);
     if ((e = hipMalloc(&p->T0, sizeof(double) * 16 * n_pairs)) != hipSuccess) return fail(e);
-    if ((e = hipMalloc(&p->err, 256)) != hipSuccess) return fail(e);
+    if ((e = hipMalloc(&p->err, 256 + sizeof(*p->open) * n_states)) != hipSuccess) return fail(e);
+    p->open = (unsigned long long *)((char *)p->err + 256);
     if ((e = hipHostMalloc(&p->host_states, sizeof(IcpState) * n_states)) != hipSuccess) return fail(e);
     if ((e = hipHostMalloc(&p->host_err, 256)) != hipSuccess) return fail(e);
     std::vector<PairDesc> P;
@@ -1821,11 +1851,11 @@ int32_t icp_plan_create(gca_ctx ctx, int n_pairs, int n_levels, const gca_cloud 
 // building of the next state's source: states set up (sizes are provisional), then per state
 // its sizes and one persistent launch over it alone (each on the stream that built its source,
 // after the launch of the state chained before it), then the results.
-int32_t icp_plan_init(gca_ctx ctx, IcpPlan *p)
+int32_t icp_plan_init(gca_ctx ctx, IcpPlan *p, bool sizes_later)
 {
     hipLaunchKernelGGL(k_state_init, dim3((p->n_states + 63) / 64), dim3(64), 0, ctx->stream, p->states,
                        (const PairDesc *)p->pairs, (const StateInit *)p->init, (const double *)p->T0, p->n_states,
-                       p->err);
+                       p->open, sizes_later ? 1 : 0, p->err);
     GCA_HIP(hipGetLastError());
     return GCA_OK;
 }
@@ -1836,7 +1866,7 @@ int32_t icp_plan_persist(gca_ctx ctx, IcpPlan *p, int s)
     if (use_resident(ctx, p->n_pairs, p->unit_cap))
         launch_resident_any(ctx, p->mode, p->pairs, p->states, s, 1, p->unit_cap, p->err);
     else
-        launch_persist_any(ctx, p->mode, p->pairs, p->states, 1, p->err, s, 1);
+        launch_persist_any(ctx, p->mode, p->pairs, p->states, p->open, 1, p->err, s, 1);
     GCA_HIP(hipGetLastError());
     return GCA_OK;
 }
@@ -1873,12 +1903,12 @@ int32_t icp_plan_copy_results(gca_ctx ctx, IcpPlan *p, const uint32_t *extra, ui
 // no allocation, so it can be captured.
 int32_t icp_plan_run(gca_ctx ctx, IcpPlan *p)
 {
-    GCA_TRY(icp_plan_init(ctx, p));
+    GCA_TRY(icp_plan_init(ctx, p, false));
     if (use_resident(ctx, p->n_pairs, p->unit_cap))
         for (int s = 0; s < p->n_states; ++s)
             launch_resident_any(ctx, p->mode, p->pairs, p->states, s, 0, p->unit_cap, p->err);
     else
-        launch_persist_any(ctx, p->mode, p->pairs, p->states, p->n_states, p->err);
+        launch_persist_any(ctx, p->mode, p->pairs, p->states, p->open, p->n_states, p->err);
     GCA_HIP(hipGetLastError());
     return icp_plan_copy_results(ctx, p, nullptr, nullptr);
 }

@@ -192,7 +192,7 @@ int32_t make_plan(gca_pipeline p, int slot)
 int32_t registration_launches(gca_pipeline p, int reg, gca_ctx rc)
 {
     IcpPlan *plan = p->plan[reg];
-    GCA_TRY(icp_plan_init(rc, plan));
+    GCA_TRY(icp_plan_init(rc, plan, true));
     for (int l = 0; l < p->nl; ++l) {
         // the plan reads the target's grid through what it saw at its creation
         if (!icp_plan_target_current(plan, l, p->lvc[prev_slot(p, reg)][l])) return GCA_ERR_DEVICE;
@@ -358,7 +358,7 @@ int32_t enqueue(gca_pipeline p, int slot, int reg, const uint16_t *depth, const 
     if (overlapped) GCA_TRY(enqueue_registration(p, reg));
     // the front end's first kernel also clears this slot's voxel-lattice error word
     GCA_TRY(launch_from_rgbd(ctx, depth, bgr, &p->cam, &p->bil, p->tmin, p->tmax, p->full[slot], err_dev_of(p, slot)));
-    if (plan) GCA_TRY(icp_plan_init(ctx, plan));
+    if (plan) GCA_TRY(icp_plan_init(ctx, plan, true));
     GCA_HIP(hipEventRecord(p->ev_fork, ctx->stream));
     auto build = [&](int l) -> int32_t {
         gca_ctx lc = p->lctx[l];

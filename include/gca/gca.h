@@ -171,7 +171,7 @@ enum {
     GCA_TUNE_ICP_MAX_UNITS = 3,    /* cap on work units (FP64 partials) per pair and iteration, 1..1024 */
     GCA_TUNE_NORMALS_LANES = 4,    /* 1,2,4,8,16,32,64; no effect: the normal and gradient kernels run 8
                                       lanes per query, the fastest for every cloud measured */
-    GCA_TUNE_ICP_PERSIST_BLOCKS = 5, /* workgroups of the persistent ICP launch (0 = 2 per CU), 1..65536 */
+    GCA_TUNE_ICP_PERSIST_BLOCKS = 5, /* workgroups of the persistent ICP launch (0 = 3 per CU), 1..65536 */
     GCA_TUNE_ICP_LAUNCH = 6,       /* 0 = resident launches for one-pair calls, a persistent launch for
                                       several pairs; 1 = one persistent launch per call; 2 = one launch
                                       per iteration; 3 = one resident launch per pair and level.  Every

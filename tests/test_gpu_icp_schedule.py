@@ -1,0 +1,50 @@
+"""The persistent launch's scheduler: many states, few and many work units, few workgroups.  Every
+shape gives the bits of one launch per iteration."""
+import numpy as np
+import pytest
+
+pytestmark = pytest.mark.gpu
+
+
+def _clouds(g, n, seed):
+    r = np.random.default_rng(seed)
+    x = r.uniform(-0.3, 0.3, (n, 3))
+    x[:, 2] = 1.0 + 0.1 * np.sin(5 * x[:, 0]) * np.cos(4 * x[:, 1])
+    c = 0.5 + 0.4 * np.sin(9 * x)
+    src = (x + [0.004, -0.003, 0.005]).astype(np.float32)
+    s, t = g.PointCloud.from_numpy(src, c.astype(np.float32)), g.PointCloud.from_numpy(x.astype(np.float32), c.astype(np.float32))
+    t.estimate_normals(0.1, 30)
+    t.compute_color_gradient(0.1, 0)
+    return s, t
+
+
+@pytest.mark.parametrize("pairs,levels,tune", [
+    (2, 1, {}),                                            # two states
+    (90, 3, {}),                                           # 270 states: more than one read of open words
+    (90, 3, {"icp_persist_blocks": 1}),                    # one workgroup serves them all
+    (7, 2, {"icp_max_units": 1}),                          # one sub-queue in use
+    (7, 2, {"icp_lanes_batch": 64, "icp_max_units": 9}),   # one sub-queue of two units
+    (40, 2, {"icp_lanes_batch": 64, "icp_max_units": 200, "icp_persist_blocks": 2000}),
+])
+def test_persistent_launch_equals_one_launch_per_iteration(pairs, levels, tune):
+    import cuda_3d_amd as g
+
+    ctx = g.default_context()
+    made = [_clouds(g, n, n) for n in (1, 40, 700, 1500)]
+    src = [[made[(k + l) % 4][0] for l in range(levels)] for k in range(pairs)]
+    tgt = [[made[(k + l) % 4][1] for l in range(levels)] for k in range(pairs)]
+    params = [g.icp_params((5, 9, 1)[l], 0.1) for l in range(levels)]
+    T0 = np.tile(np.eye(4), (pairs, 1, 1))
+    T0[:, 0, 3] = np.linspace(-0.01, 0.01, pairs)
+    got = {}
+    try:
+        ctx.set_tuning(**tune)
+        for launch in (1, 2):
+            ctx.set_tuning(icp_launch=launch)
+            T, reps = g.batch_multiscale_icp(src, tgt, params, T0, [0.1] * levels)
+            got[launch] = T, [[(r.iterations, r.n_correspondences, r.rmse) for r in row] for row in reps]
+    finally:
+        ctx.set_tuning(icp_launch=0, **{k: 0 for k in tune})
+    np.testing.assert_array_equal(got[1][0], got[2][0])
+    assert got[1][1] == got[2][1]
+    assert any(r[0] > 1 for row in got[1][1] for r in row)
