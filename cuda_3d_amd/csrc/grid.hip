@@ -210,13 +210,6 @@ int32_t grid_gather_attributes(gca_ctx ctx, gca_cloud c)
 
 constexpr int kQUnroll = 4;  // candidates in flight per lane
 
-// The query's own column of cells, kept within box b.
-__device__ __forceinline__ void own_column(const GridDesc &g, float4 q, const Box &b, int &ix, int &iy)
-{
-    ix = min(max(grid_cell(q.x, g.origin[0], g.cell, g.dims[0]), b.lo[0]), b.hi[0]);
-    iy = min(max(grid_cell(q.y, g.origin[1], g.cell, g.dims[1]), b.lo[1]), b.hi[1]);
-}
-
 // Points within the radius of q, counted by a group of lanes (the count is on all of them); the
 // walk begins with the query's own column, where most of them are, and ends once the count
 // exceeds `limit`.
@@ -235,7 +228,7 @@ __device__ __forceinline__ uint32_t group_count(const GridView &v, float4 q, int
         for (int m = 1; m < gs; m <<= 1) all += __shfl_xor(all, m, kWave);
         return all <= limit;
     };
-    own_column(v.g, q, b, ix, iy);
+    own_column(v.g, q.x, q.y, b, ix, iy);
     group_walk_column<kQUnroll>(v, b, ix, iy, g, gs, test, sum);
     if (all <= limit) group_walk_box<kQUnroll>(v, b, g, gs, ix, iy, test, sum);
     return all;
@@ -246,7 +239,8 @@ __device__ __forceinline__ uint32_t group_count(const GridView &v, float4 q, int
 // there bounds the box of the rest, which for clouds that overlap is a few cells instead of 27
 // (kBoxRel / kBoxAbs cover the rounding of the distance and of the cell arithmetic, so the box
 // holds every point at most that far away: the result is that of the full search).
-// Bound by the candidates' load latency.  92k queries on 92k points of a 424x240 frame, 3 cm: 69 us;
+// Bound by the candidates' load latency.  92k queries on 92k points of a 424x240 frame, 3 cm: 45 us
+// (66 with each candidate's load waited for by itself and its index loaded at once);
 // 359 us with one thread per query over the whole box.
 constexpr int kNnLanes = 8;
 constexpr double kBoxRel = 1e-9, kBoxAbs = 1e-9;
@@ -264,40 +258,39 @@ __global__ __launch_bounds__(256) void k_nn(const float4 *__restrict__ q, const 
          i += (int)(gridDim.x * blockDim.x / kNnLanes)) {
         const float4 p = q[i];
         double bd = DBL_MAX;
-        int32_t bi = -1;
-        auto better = [&](double d2, int32_t idx) {  // (d2, index) order; -1: none yet
-            if (bi < 0 || key_less(d2, idx, bd, bi)) {
+        int32_t bs = -1;  // slot; the original indices are compared (and loaded) only for ties
+        auto better = [&](double d2, int32_t slot) {
+            if (d2 < bd || (d2 == bd && slot != bs && order[slot] < order[bs])) {
                 bd = d2;
-                bi = idx;
+                bs = slot;
             }
         };
         auto test = [&](uint32_t s, float4 c, bool valid) {
-            if (!valid) return;
             const double d2 = dist2(c.x, c.y, c.z, p.x, p.y, p.z);
-            if (d2 < r2 && d2 <= bd) better(d2, order[s]);
+            if (valid && d2 < r2) better(d2, (int32_t)s);
         };
         auto reduce = [&]() {
             for (int m = 1; m < kNnLanes; m <<= 1) {
                 const double od = __shfl_xor(bd, m, kWave);
-                const int32_t oi = __shfl_xor(bi, m, kWave);
-                if (oi >= 0) better(od, oi);
+                const int32_t os = __shfl_xor(bs, m, kWave);
+                if (os >= 0) better(od, os);
             }
         };
         auto go = [] { return true; };
         Box b;
         int ix, iy;
         if (grid_range(g, p.x, p.y, p.z, b.lo, b.hi)) {
-            own_column(g, p, b, ix, iy);
+            own_column(g, p.x, p.y, b, ix, iy);
             group_walk_column<kQUnroll>(v, b, ix, iy, gl, kNnLanes, test, go);
             reduce();
             // the column was searched over the full box's cells, a superset of what is left of it
-            if (bi < 0 || grid_range_r(g, p.x, p.y, p.z, fmin((double)g.radius, sqrt(bd) * (1.0 + kBoxRel) + kBoxAbs),
+            if (bs < 0 || grid_range_r(g, p.x, p.y, p.z, fmin((double)g.radius, sqrt(bd) * (1.0 + kBoxRel) + kBoxAbs),
                                        b.lo, b.hi)) {
                 group_walk_box<kQUnroll>(v, b, gl, kNnLanes, ix, iy, test, go);
                 reduce();
             }
         }
-        if (gl == 0) out[i] = bi;
+        if (gl == 0) out[i] = bs >= 0 ? order[bs] : -1;
     }
 }
 
@@ -341,7 +334,7 @@ __global__ __launch_bounds__(256) void k_radius_count(const float4 *__restrict__
 
 // The fill collects a query's keys in LDS (wave_collect): one pass over the candidates whatever
 // their number, where an insertion sort in global memory grew with the square of the neighbourhood
-// (11k queries of a 424x240 frame, 3 cm, 30 nearest: 81 us, 134 ms before; the counts 14 us with 16
+// (11k queries of a 424x240 frame, 3 cm, 30 nearest: 66 us, 134 ms before; the counts 10 us with 16
 // lanes per query, 364 us with one).  A list longer than the buffer comes out in blocks of
 // kSelBlock, each pass taking the keys after the last one written.
 constexpr int kFillWaves = 4;
@@ -475,7 +468,7 @@ int32_t launch_grid_cells(gca_ctx ctx, gca_cloud c, int32_t *cells)
 
 // A 1024-thread workgroup flags the 256 points of one compaction block, kOutLanes lanes per point.
 // A point in a dense place is settled by its own column's first candidates, so the lanes' loads in
-// flight are what counts (92k points, 3 cm: 31 us, 161 us with one thread per point).
+// flight are what counts (92k points, 3 cm: 20 us, 161 us with one thread per point).
 constexpr int kOutBlock = 1024;
 constexpr int kOutLanes = 8;
 

@@ -239,7 +239,7 @@ __device__ __forceinline__ void group_store(MomentSum<KIND> &A, int32_t cnt, int
     M.cnt = cnt;
 }
 
-// Sums without a K cap: 27 us for the gradient of 110k points at 2 cm (32 us with 64-bit integer
+// Sums without a K cap: 24 us for the gradient of 110k points at 2 cm (30 us with 64-bit integer
 // sums and a division per cell bound).  Eight lanes per query: 4 and 16 measured 1-2 % and 5 %
 // slower on a 640x480 target at 1 cm, 2 and 4 % on the overlapped odometry of such frames.
 template <int KIND>
@@ -288,7 +288,7 @@ __global__ __launch_bounds__(kNbBlock) void k_moments(const float4 *__restrict__
 // Ties at the threshold are settled by index.  A query with more than kSelCandidates in-radius
 // candidates goes to the overflow list.  Bound half by instruction issue (the walk's tests), half by
 // the latency of the cell bounds and candidates.  110k points of a raw 640x480 frame at 1 cm, the 30
-// nearest of about 50 within 2.5 cm: 37 us and 5 us for the (empty) overflow launch, where adding in
+// nearest of about 50 within 2.5 cm: 31 us and 5 us for the (empty) overflow launch, where adding in
 // the walk and ranking every larger neighbourhood by a wavefront of its own took 81 and 75 us.
 // LDS: 32 groups x 96 candidates x 12 bytes (36 KB, four workgroups per CU), 16 bytes with PAIR.
 constexpr int kSelCandidates = 96;
