@@ -35,6 +35,7 @@
 
 #include "gca_device.hpp"
 #include "gca_internal.hpp"
+#include "neighbours.hpp"
 
 namespace gca {
 
@@ -98,6 +99,20 @@ struct IcpState {
     alignas(256) uint32_t pad_end;
 };
 
+// A pointer read from memory (a PairDesc) or passed to a function that is not inlined is a generic
+// one to the compiler, whose loads wait for LDS and memory alike; these say what it points at (by way
+// of an integer: a cast of the pointer itself is folded away).
+template <class T>
+__device__ __forceinline__ T *global_ptr(T *p)
+{
+    return (T *)(__attribute__((address_space(1))) T *)(uintptr_t)p;
+}
+template <class T>
+__device__ __forceinline__ T *lds_ptr(T *p)
+{
+    return (T *)(__attribute__((address_space(3))) T *)(uintptr_t)p;
+}
+
 struct PairDesc {
     const float4 *src;
     const CloudHdr *src_hdr;
@@ -117,6 +132,24 @@ struct PairDesc {
     int32_t unit_cap;    // cap on work units per iteration
     int32_t lanes[3];    // lanes per query for n < 16384, n < 49152, larger
 };
+
+__device__ __forceinline__ PairDesc global_pair(const PairDesc &Q)
+{
+    PairDesc P = Q;
+    P.src = global_ptr(P.src);
+    P.src_hdr = global_ptr(P.src_hdr);
+    P.tgt_hdr = global_ptr(P.tgt_hdr);
+    P.start = global_ptr(P.start);
+    P.order = global_ptr(P.order);
+    P.sxyzi = global_ptr(P.sxyzi);
+    P.nrm = global_ptr(P.nrm);
+    P.grad = global_ptr(P.grad);
+    P.snrm = global_ptr(P.snrm);
+    P.sgrad = global_ptr(P.sgrad);
+    P.partials = global_ptr(P.partials);
+    P.nnprev = global_ptr(P.nnprev);
+    return P;
+}
 
 // Launch-shape rules shared by host and device: the unit partition fixes the summation order, so
 // it must come out the same wherever it is computed.
@@ -456,8 +489,8 @@ __device__ __forceinline__ void sum_partials(const double *partials, int n, doub
 
 // ---- nearest neighbour ----------------------------------------------------------------------
 // Lanes g = 0..G-1 of a group search one query: lane g scans candidates g, g + G, ... of the
-// flattened candidate space, then the group reduces by shuffles.  The result is the sorted slot
-// of argmin (d2, original index) over target points with d2 < r^2 (FP64 d2), or -1.
+// flattened candidate space (group_walk_box), then the group reduces by shuffles.  The result is the
+// sorted slot of argmin (d2, original index) over target points with d2 < r^2 (FP64 d2), or -1.
 //
 // Warm start: `sp` is the slot matched in the previous iteration.  Its distance under the
 // current pose bounds the answer, so only cells overlapping the box of half-width sqrt(d2_sp)
@@ -465,7 +498,6 @@ __device__ __forceinline__ void sum_partials(const double *partials, int n, doub
 // of the cell arithmetic, so the box always contains every point with d2 <= d2_sp and the
 // result is exactly that of the full search.  Ties in d2 compare original indices, which are
 // loaded only then.
-constexpr int kMaxRuns = 9;
 constexpr int kUnroll = 4, kPersistUnroll = 8;  // candidates in flight per lane
 constexpr double kWarmRel = 1e-9, kWarmAbs = 1e-9;
 
@@ -485,6 +517,7 @@ template <int U>
 __device__ __forceinline__ int32_t nn_group(const PairDesc &P, float qx, float qy, float qz, int g, int G,
                                             int32_t sp)
 {
+    const GridView v = make_view(P.g, P.start, P.order, P.sxyzi);
     const double r2 = (double)P.g.radius * (double)P.g.radius;
     double bd = DBL_MAX;
     int32_t bs = -1;
@@ -498,64 +531,13 @@ __device__ __forceinline__ int32_t nn_group(const PairDesc &P, float qx, float q
             box = fmin(box, sqrt(d2) * (1.0 + kWarmRel) + kWarmAbs);
         }
     }
-    int32_t lo[3], hi[3];
-    if (grid_range_r(P.g, qx, qy, qz, box, lo, hi)) {
-        const int nry = hi[1] - lo[1] + 1;
-        const int nruns = (hi[0] - lo[0] + 1) * nry;
-        if (nruns <= kMaxRuns) {
-            // bounds of all (ix, iy) runs up front, then one flattened walk with U
-            // independent loads in flight per lane
-            uint32_t rs[kMaxRuns], cum[kMaxRuns + 1];
-#pragma unroll
-            for (int r = 0; r < kMaxRuns; ++r) {
-                uint32_t a = 0, b = 0;
-                if (r < nruns) {
-                    const int ix = lo[0] + r / nry, iy = lo[1] + r % nry;
-                    const int64_t row = ((int64_t)ix * P.g.dims[1] + iy) * P.g.dims[2];
-                    a = P.start[row + lo[2]];
-                    b = P.start[row + hi[2] + 1];
-                }
-                rs[r] = a;
-                cum[r + 1] = b > a ? b - a : 0u;  // a start table never decreases
-            }
-            cum[0] = 0;
-#pragma unroll
-            for (int r = 0; r < kMaxRuns; ++r) cum[r + 1] += cum[r];
-            const uint32_t total = cum[kMaxRuns];
-            for (uint32_t f0 = g; f0 < total; f0 += G * U) {
-                uint32_t sl[U];
-                float4 c[U];
-#pragma unroll
-                for (int u = 0; u < U; ++u) {
-                    const uint32_t f = f0 + u * G;
-                    uint32_t s = 0xffffffffu;
-                    if (f < total) {
-                        s = rs[0] + f;
-#pragma unroll
-                        for (int r = 1; r < kMaxRuns; ++r)
-                            if (f >= cum[r]) s = rs[r] + (f - cum[r]);
-                        c[u] = P.sxyzi[s];
-                    }
-                    sl[u] = s;
-                }
-#pragma unroll
-                for (int u = 0; u < U; ++u) {
-                    if (sl[u] == 0xffffffffu) continue;
-                    nn_consider(P, dist2(c[u].x, c[u].y, c[u].z, qx, qy, qz), (int32_t)sl[u], r2, bd, bs);
-                }
-            }
-        } else {
-            // cell smaller than the radius (not produced by grid_build): plain run walk
-            for (int32_t ix = lo[0]; ix <= hi[0]; ++ix)
-                for (int32_t iy = lo[1]; iy <= hi[1]; ++iy) {
-                    const int64_t row = ((int64_t)ix * P.g.dims[1] + iy) * P.g.dims[2];
-                    const uint32_t s0 = P.start[row + lo[2]], s1 = P.start[row + hi[2] + 1];
-                    for (uint32_t s = s0 + g; s < s1; s += G) {
-                        const float4 c = P.sxyzi[s];
-                        nn_consider(P, dist2(c.x, c.y, c.z, qx, qy, qz), (int32_t)s, r2, bd, bs);
-                    }
-                }
-        }
+    Box b;
+    if (grid_range_r(P.g, qx, qy, qz, box, b.lo, b.hi)) {
+        auto test = [&](uint32_t s, float4 c, bool valid) {
+            if (valid) nn_consider(P, dist2(c.x, c.y, c.z, qx, qy, qz), (int32_t)s, r2, bd, bs);
+        };
+        auto go = [] { return true; };
+        group_walk_box<U>(v, b, g, G, -1, -1, test, go);
     }
     for (int m = 1; m < G; m <<= 1) {
         const double od = __shfl_xor(bd, m, kWave);
@@ -661,60 +643,90 @@ __device__ __forceinline__ double euler_elem(int t, const double *trig, const do
     }
 }
 
-// Epoch finish of state p (whole workgroup, run by the workgroup that took the last ticket):
-// fixed-order FP64 sum of the unit partials, LDL^T solve, Euler increment, T <- dT T, the
-// stopping rule of color_icp.cu:216-228, then the hand-over: the next epoch of this state, or
-// the pose to the next level of the chain (all_queues: its sizes are not known yet, the launch that
-// runs it masks the open word).  A failed solve takes the identity step (which also
-// satisfies the stopping rule), as the reference does.
-__device__ __noinline__ void icp_finish(IcpState *states, unsigned long long *open, int p, uint32_t epoch,
-                                        const double *partials, int nvb, bool all_queues, double *sys, bool naive)
+// What one iteration's end works on, in LDS.
+struct PoseStep {
+    double sys[kPartStride];
+    double Tc[16], Tn[16], dT[16], xi[6], trig[6];
+    double conv_rot, conv_t2;
+    int ok, conv;
+};
+
+// LDL^T solve of sys, Euler increment, Tn <- dT Tc and the stopping rule of color_icp.cu:216-228, by
+// one wavefront (LDS hand-overs inside it need no barrier).  A failed solve takes the identity step
+// (which also satisfies the stopping rule), as the reference does.  Not inlined: the constants of
+// sincos alone took some 20 registers through the whole iteration loop of the resident launch, which
+// then spilled in the search.
+__device__ __noinline__ void pose_step(PoseStep *step)
 {
+    PoseStep &S = *lds_ptr(step);
+    const int t = lane_id();
+    if (t == 0) {
+        double xi[6];
+        S.ok = solve6(S.sys, S.sys + 21, xi) ? 1 : 0;
+#pragma unroll
+        for (int k = 0; k < 6; ++k) S.xi[k] = xi[k];
+    }
+    wave_lds_sync();
+    if (t < 3) {
+        double sn, cs;
+        sincos(S.xi[t], &sn, &cs);
+        S.trig[2 * t] = sn;
+        S.trig[2 * t + 1] = cs;
+    }
+    wave_lds_sync();
+    if (t < 16) S.dT[t] = euler_elem(t, S.trig, S.xi);
+    wave_lds_sync();
+    if (t < 16) {
+        const int i = t >> 2, j = t & 3;
+        const double *dT = S.dT, *Tc = S.Tc;
+        S.Tn[t] = ((dT[4 * i] * Tc[j] + dT[4 * i + 1] * Tc[4 + j]) + dT[4 * i + 2] * Tc[8 + j]) + dT[4 * i + 3] * Tc[12 + j];
+    } else if (t == 16) {
+        const double *dT = S.dT;
+        const double cos_t = 0.5 * (dT[0] + dT[5] + dT[10] - 1.0);
+        const double tt = (dT[3] * dT[3] + dT[7] * dT[7]) + dT[11] * dT[11];
+        S.conv = cos_t >= 1.0 - S.conv_rot && tt <= S.conv_t2 ? 1 : 0;
+    }
+}
+
+// Epoch finish of state p (whole workgroup, run by the workgroup that took the last ticket):
+// fixed-order FP64 sum of the unit partials, the pose step, then the hand-over: the next epoch of
+// this state, or the pose to the next level of the chain (all_queues: its sizes are not known yet,
+// the launch that runs it masks the open word).
+__device__ __noinline__ void icp_finish(IcpState *states, unsigned long long *open, int p, uint32_t epoch,
+                                        const double *partials, int nvb, bool all_queues, PoseStep *step, bool naive)
+{
+    states = global_ptr(states);
+    open = global_ptr(open);
+    partials = global_ptr(partials);
     IcpState *st = states + p;
-    __shared__ double Tc[16], Tn[16], dT[16], xi[6], trig[6];
-    __shared__ double f_crot, f_ct2;
-    __shared__ int f_iter, f_max, f_fail, f_next, f_ok, f_done;
+    PoseStep &S = *lds_ptr(step);
+    __shared__ int f_iter, f_max, f_fail, f_next, f_done;
     const int t = threadIdx.x;
     // state fields load alongside the partial sums (coherent: the previous epoch's finisher may
     // have run on another XCD)
     if (t >= 64 && t < 80) {
-        Tc[t - 64] = load_coherent(&st->T[t - 64]);
+        S.Tc[t - 64] = load_coherent(&st->T[t - 64]);
     } else if (t == 80) {
         f_iter = load_coherent(&st->iter);
         f_max = load_coherent(&st->max_iter);
         f_fail = load_coherent(&st->solver_failures);
         f_next = load_coherent(&st->next);
-        f_crot = load_coherent(&st->conv_rot);
-        f_ct2 = load_coherent(&st->conv_t2);
+        S.conv_rot = load_coherent(&st->conv_rot);
+        S.conv_t2 = load_coherent(&st->conv_t2);
     }
-    sum_partials(partials, nvb, sys, naive);  // after the acquire in unit_commit
-    if (t == 0) f_ok = solve6(sys, sys + 21, xi) ? 1 : 0;
-    __syncthreads();
-    if (t < 3) {
-        double s, c;
-        sincos(xi[t], &s, &c);
-        trig[2 * t] = s;
-        trig[2 * t + 1] = c;
-    }
-    __syncthreads();
-    if (t < 16) dT[t] = euler_elem(t, trig, xi);
+    sum_partials(partials, nvb, S.sys, naive);  // after the acquire in unit_commit
+    if (t < kWave) pose_step(step);
     __syncthreads();
     if (t < 16) {
-        const int i = t >> 2, j = t & 3;
-        const double v =
-            ((dT[4 * i] * Tc[j] + dT[4 * i + 1] * Tc[4 + j]) + dT[4 * i + 2] * Tc[8 + j]) + dT[4 * i + 3] * Tc[12 + j];
-        Tn[t] = v;
-        store_coherent(&st->T[t], v);
+        store_coherent(&st->T[t], S.Tn[t]);
     } else if (t >= 32 && t < 32 + kNSys) {
-        st->sys[t - 32] = sys[t - 32];
+        st->sys[t - 32] = S.sys[t - 32];
     } else if (t == 64) {
         const int it = f_iter + 1;
-        const double cos_t = 0.5 * (dT[0] + dT[5] + dT[10] - 1.0);
-        const double tt = (dT[3] * dT[3] + dT[7] * dT[7]) + dT[11] * dT[11];
-        const bool conv = cos_t >= 1.0 - f_crot && tt <= f_ct2;
+        const bool conv = S.conv != 0;
         const bool done = conv || it >= f_max;
         store_coherent(&st->iter, it);
-        if (!f_ok) store_coherent(&st->solver_failures, f_fail + 1);
+        if (!S.ok) store_coherent(&st->solver_failures, f_fail + 1);
         if (conv) st->converged = 1;
         if (done) {
             st->done = 1;
@@ -724,7 +736,7 @@ __device__ __noinline__ void icp_finish(IcpState *states, unsigned long long *op
         f_done = done ? 1 : 0;
     }
     __syncthreads();
-    if (f_done && f_next >= 0 && t < 16) store_coherent(&states[f_next].T[t], Tn[t]);
+    if (f_done && f_next >= 0 && t < 16) store_coherent(&states[f_next].T[t], S.Tn[t]);
     // Release before the queue word opens the next epoch or level: readers on other XCDs load
     // the pose with coherent loads once they see the word.  (A vmcnt wait after the stores is
     // not enough: it does not order them before the word for readers on other XCDs.)
@@ -760,17 +772,17 @@ __device__ __noinline__ void icp_finish(IcpState *states, unsigned long long *op
 // release has little left to write back.
 template <int MODE>
 __device__ __forceinline__ void unit_commit(const PairDesc &P, IcpState *states, unsigned long long *open, int p, int vb,
-                                            int nvb, bool all_queues, uint32_t epoch, double *sys)
+                                            int nvb, bool all_queues, uint32_t epoch, PoseStep &S)
 {
     __shared__ bool last;
-    if (threadIdx.x < kNSys) store_coherent(&P.partials[(int64_t)vb * kPartStride + threadIdx.x], sys[threadIdx.x]);
+    if (threadIdx.x < kNSys) store_coherent(&P.partials[(int64_t)vb * kPartStride + threadIdx.x], S.sys[threadIdx.x]);
     if (threadIdx.x == 0)
         last = __hip_atomic_fetch_add(&states[p].ticket, 1u, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_AGENT) ==
                (uint32_t)(nvb - 1);
     __syncthreads();
     if (!last) return;
     fence_acquire_agent();
-    icp_finish(states, open, p, epoch, P.partials, nvb, all_queues, sys, MODE == GCA_ACCUM_NAIVE_FP32);
+    icp_finish(states, open, p, epoch, P.partials, nvb, all_queues, &S, MODE == GCA_ACCUM_NAIVE_FP32);
 }
 
 // ---- persistent launch: every iteration of every state --------------------------------------
@@ -804,7 +816,7 @@ __global__ __launch_bounds__(kIcpBlock) GCA_PERSIST_OCCUPANCY void k_icp_persist
                                                            int refresh, uint32_t *err)
 {
     __shared__ double T[12];
-    __shared__ double sys[kPartStride];
+    __shared__ PoseStep S;
     __shared__ int s_pick, s_alive, s_vb;
     __shared__ uint32_t s_epoch, s_pick_epoch;
     __shared__ int s_nsrc, s_ntgt, s_G, s_nvb;
@@ -918,13 +930,13 @@ __global__ __launch_bounds__(kIcpBlock) GCA_PERSIST_OCCUPANCY void k_icp_persist
         }
         idle = 0;
         home = p - s_first;
-        const PairDesc &P = pairs[p];
+        const PairDesc P = global_pair(pairs[p]);
         const int nvb = refresh ? s_nvb : st->nvb;
         if (refresh)
-            icp_unit<MODE, kPersistUnroll>(P, s_nsrc, s_G, nvb, s_ntgt, vb, epoch > 0, T, sys);
+            icp_unit<MODE, kPersistUnroll>(P, s_nsrc, s_G, nvb, s_ntgt, vb, epoch > 0, T, S.sys);
         else
-            icp_unit<MODE, kPersistUnroll>(P, st->n_src, st->G, nvb, st->n_tgt, vb, epoch > 0, T, sys);
-        unit_commit<MODE>(P, states, open, p, vb, nvb, refresh != 0, epoch, sys);
+            icp_unit<MODE, kPersistUnroll>(P, st->n_src, st->G, nvb, st->n_tgt, vb, epoch > 0, T, S.sys);
+        unit_commit<MODE>(P, states, open, p, vb, nvb, refresh != 0, epoch, S);
     }
 }
 
@@ -937,7 +949,7 @@ __global__ __launch_bounds__(kIcpBlock) GCA_ICP_OCCUPANCY void k_icp_iter(const 
                                                         const int32_t *__restrict__ unit_first)
 {
     __shared__ double T[12];
-    __shared__ double sys[kPartStride];
+    __shared__ PoseStep S;
     const int p = __builtin_amdgcn_readfirstlane(unit_state[blockIdx.x]);
     IcpState *st = states + p;
     if (st->done) return;
@@ -946,10 +958,10 @@ __global__ __launch_bounds__(kIcpBlock) GCA_ICP_OCCUPANCY void k_icp_iter(const 
     if (threadIdx.x < 12) T[threadIdx.x] = st->T[threadIdx.x];
     if (threadIdx.x == 0 && vb == 0 && epoch == 0) st->t_start = wall_clock64();
     __syncthreads();
-    const PairDesc &P = pairs[p];
+    const PairDesc P = global_pair(pairs[p]);
     const int nvb = st->nvb;
-    icp_unit<MODE>(P, st->n_src, st->G, nvb, st->n_tgt, vb, epoch > 0, T, sys);
-    unit_commit<MODE>(P, states, open, p, vb, nvb, false, epoch, sys);
+    icp_unit<MODE>(P, st->n_src, st->G, nvb, st->n_tgt, vb, epoch > 0, T, S.sys);
+    unit_commit<MODE>(P, states, open, p, vb, nvb, false, epoch, S);
 }
 
 // ---- resident launch: one state, every iteration, no scheduler ---------------------------------
@@ -968,6 +980,11 @@ __global__ __launch_bounds__(kIcpBlock) GCA_ICP_OCCUPANCY void k_icp_iter(const 
 // most two per CU (the occupancy allows four); kernels running beside it only delay it, as their
 // workgroups end and free the slots the rest need.  A wait beyond the spin limit flags the error
 // word instead of hanging.
+// An iteration of 354 workgroups (11k points at 2 cm) takes 16 us: the unit 5.5 (search 3.3), the
+// barrier 5 of which about 3 are the wait for the slowest unit, the sum 3, the pose step 2.2.  (19 us
+// with loads that wait for each other, generic pointers and the pose step inlined.  Waiting for the
+// 8 group counters instead of a top counter cost 4 us per iteration: 8 polled lines per workgroup
+// slow the arrivals.)
 __device__ __forceinline__ uint32_t load_coherent_u32(const uint32_t *p)
 {
     return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
@@ -1018,14 +1035,12 @@ __global__ __launch_bounds__(kIcpBlock) GCA_ICP_OCCUPANCY void k_icp_resident(co
                                                                                IcpState *states, int s, int refresh,
                                                                                uint32_t *err)
 {
-    __shared__ double Tc[16], Tn[16], dT[16], xi[6], trig[6];
-    __shared__ double sys[kPartStride];
-    __shared__ int f_ok, f_done, f_stop;
-    __shared__ double f_crot, f_ct2;
+    __shared__ PoseStep S;
+    __shared__ int f_stop;
     __shared__ int f_max, f_next, f_iter0, f_fail0;
     __shared__ int s_nsrc, s_ntgt, s_G, s_nvb;
     IcpState *st = states + s;
-    const PairDesc &P = pairs[s];
+    const PairDesc P = global_pair(pairs[s]);
     const int t = threadIdx.x;
     if (t == 0) {
         int ns, nt, G, nvb;
@@ -1048,8 +1063,8 @@ __global__ __launch_bounds__(kIcpBlock) GCA_ICP_OCCUPANCY void k_icp_resident(co
         f_next = st->next;
         f_iter0 = st->iter;
         f_fail0 = st->solver_failures;
-        f_crot = st->conv_rot;
-        f_ct2 = st->conv_t2;
+        S.conv_rot = st->conv_rot;
+        S.conv_t2 = st->conv_t2;
         f_stop = st->done;
         if (refresh && blockIdx.x == 0) {
             st->n_src = ns;
@@ -1058,7 +1073,7 @@ __global__ __launch_bounds__(kIcpBlock) GCA_ICP_OCCUPANCY void k_icp_resident(co
             st->nvb = nvb;
         }
     } else if (t >= 64 && t < 80) {
-        Tc[t - 64] = st->T[t - 64];
+        S.Tc[t - 64] = st->T[t - 64];
     }
     __syncthreads();
     const int nvb = s_nvb;
@@ -1074,8 +1089,8 @@ __global__ __launch_bounds__(kIcpBlock) GCA_ICP_OCCUPANCY void k_icp_resident(co
     int iter = f_iter0, fails = f_fail0;
     for (uint32_t e = 0;; ++e) {
         double *bank = P.partials + (size_t)(e & 1u) * (size_t)P.unit_cap * kPartStride;
-        icp_unit<MODE>(P, s_nsrc, s_G, nvb, s_ntgt, vb, iter > 0, Tc, sys);
-        if (t < kNSys) store_coherent(&bank[(int64_t)vb * kPartStride + t], sys[t]);
+        icp_unit<MODE>(P, s_nsrc, s_G, nvb, s_ntgt, vb, iter > 0, S.Tc, S.sys);
+        if (t < kNSys) store_coherent(&bank[(int64_t)vb * kPartStride + t], S.sys[t]);
         if (t == 0) {
             const unsigned long long old =
                 __hip_atomic_fetch_add(&st->bar[grp].w, 1ull, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_AGENT);
@@ -1094,48 +1109,29 @@ __global__ __launch_bounds__(kIcpBlock) GCA_ICP_OCCUPANCY void k_icp_resident(co
         }
         __syncthreads();
         if (f_stop) return;
-        sum_partials_coherent(bank, nvb, sys, MODE == GCA_ACCUM_NAIVE_FP32);
-        if (t == 0) f_ok = solve6(sys, sys + 21, xi) ? 1 : 0;
-        __syncthreads();
-        if (t < 3) {
-            double sn, cs;
-            sincos(xi[t], &sn, &cs);
-            trig[2 * t] = sn;
-            trig[2 * t + 1] = cs;
-        }
-        __syncthreads();
-        if (t < 16) dT[t] = euler_elem(t, trig, xi);
-        __syncthreads();
-        if (t < 16) {
-            const int i = t >> 2, j = t & 3;
-            Tn[t] = ((dT[4 * i] * Tc[j] + dT[4 * i + 1] * Tc[4 + j]) + dT[4 * i + 2] * Tc[8 + j]) + dT[4 * i + 3] * Tc[12 + j];
-        } else if (t == 64) {
-            const double cos_t = 0.5 * (dT[0] + dT[5] + dT[10] - 1.0);
-            const double tt = (dT[3] * dT[3] + dT[7] * dT[7]) + dT[11] * dT[11];
-            const bool conv = cos_t >= 1.0 - f_crot && tt <= f_ct2;
-            f_done = (conv || iter + 1 >= f_max) ? (conv ? 2 : 1) : 0;
-        }
+        sum_partials_coherent(bank, nvb, S.sys, MODE == GCA_ACCUM_NAIVE_FP32);
+        if (t < kWave) pose_step(&S);
         __syncthreads();
         ++iter;
-        if (!f_ok) ++fails;
-        if (t < 16) Tc[t] = Tn[t];
-        const int done = f_done;
+        if (!S.ok) ++fails;
+        const bool conv = S.conv != 0, done = conv || iter >= f_max;
         if (done && vb == 0) {
             if (t < 16) {
-                st->T[t] = Tn[t];
-                if (f_next >= 0) states[f_next].T[t] = Tn[t];
+                st->T[t] = S.Tn[t];
+                if (f_next >= 0) states[f_next].T[t] = S.Tn[t];
             } else if (t >= 32 && t < 32 + kNSys) {
-                st->sys[t - 32] = sys[t - 32];
+                st->sys[t - 32] = S.sys[t - 32];
             } else if (t == 64) {
                 st->iter = iter;
                 st->solver_failures = fails;
-                st->converged = done == 2 ? 1 : 0;
+                st->converged = conv ? 1 : 0;
                 st->done = 1;
                 st->t_done = wall_clock64();
             }
         }
-        __syncthreads();  // Tc is read by the next unit; f_done is rewritten by the next finish
         if (done) return;
+        if (t < 16) S.Tc[t] = S.Tn[t];
+        __syncthreads();  // Tc is read by the next unit
     }
 }
 
