@@ -29,8 +29,14 @@ namespace gca {
 constexpr int kRowSeg = 256;
 constexpr int kMaxR = 15;
 constexpr int kStageBatch = 8;  // staging loads in flight per thread
-constexpr int kWrLds = 4096;    // longest range-weight table staged in LDS (32 KB)
-static_assert(sizeof(double) * ((2 * kMaxR + 1) * (2 * kMaxR + 1) + kWrLds) +
+constexpr int kWrLds = 4096;    // range weights staged in LDS at most (32 KB)
+// Range weights of each adaptive step staged in LDS: differences of up to 12 cm, beyond which a tap
+// lies across a depth edge; the six whole tables are 160 KB.  With 128 of each the spatial and range
+// weights of a step fit one load per thread.
+constexpr int kAdaptiveNear = 128;
+constexpr int kAdaptiveWs = 1 + 9 + 25 + 49 + 81 + 121;
+static_assert(121 + kAdaptiveNear < kRowSeg, "a step's weights are staged by one load per thread");
+static_assert(sizeof(double) * ((2 * kMaxR + 1) * (2 * kMaxR + 1) + kWrLds + 1) +
                       sizeof(uint16_t) * (2 * kMaxR + 1) * (kRowSeg + 2 * kMaxR) <= 60 * 1024,
               "the pixel kernel's dynamic LDS must stay within a workgroup's 64 KB");
 
@@ -68,6 +74,88 @@ __device__ __forceinline__ void point_records(float X, float Y, float Z, uint32_
     orgb = make_float4(rr, g, b, 0.0f);
 }
 
+// The weighted mean's sums over the taps of one pixel, in raster order (FP64).  A weight is the
+// product of a spatial and a range weight from the tables in LDS; a range weight at or beyond the
+// `near` entries kept there comes from the full table in memory (0 beyond its end).  A tap out of
+// frame or without depth has weight 0: adding it leaves both sums as they are.
+// The taps of a row are read together, then the far ones (a row across a depth edge) together, then
+// added.  Bound by the taps' vector instructions: 1280x720 with the adaptive filter (up to 11x11 taps)
+// 68 us, 87 with each tap's reads waited for by itself and its tables in memory, 84 with them in LDS
+// but a division per staged depth and two more instructions per tap.
+struct Taps {
+    const uint16_t *row;  // the pixel in the LDS tile
+    int cols;
+    uint32_t d0;
+    const double *ws, *wr;  // wr[near] = 0
+    uint32_t near;
+    const double *far;
+    uint32_t len;
+};
+
+template <int N>
+__device__ __forceinline__ void row_taps(const Taps &t, const uint16_t *row, const double *ws, double &sw, double &swd)
+{
+    uint32_t dn[N], diff[N], most = 0;
+    double w[N];
+#pragma unroll
+    for (int k = 0; k < N; ++k) dn[k] = row[k];
+#pragma unroll
+    for (int k = 0; k < N; ++k) {
+        diff[k] = __usad(t.d0, dn[k], 0u);
+        most = max(most, dn[k] ? diff[k] : 0u);
+        w[k] = t.wr[dn[k] ? min(diff[k], t.near) : t.near];
+    }
+    if (most >= t.near) {
+        double g[N];
+#pragma unroll
+        for (int k = 0; k < N; ++k) g[k] = t.far[min(diff[k], t.len - 1u)];
+#pragma unroll
+        for (int k = 0; k < N; ++k)
+            if (dn[k] && diff[k] >= t.near && diff[k] < t.len) w[k] = g[k];
+    }
+#pragma unroll
+    for (int k = 0; k < N; ++k) {
+        const double v = __dmul_rn(ws[k], w[k]);
+        sw = __dadd_rn(sw, v);
+        swd = __dadd_rn(swd, __dmul_rn(v, (double)dn[k]));
+    }
+}
+
+// RR: the radius r, or -1 for any.
+template <int RR>
+__device__ __forceinline__ void filter_taps(const Taps &t, int r, double &sw, double &swd)
+{
+    const int side = 2 * r + 1;
+#pragma unroll 1  // (all rows at once take 242 registers: 133 us)
+    for (int dy = -r; dy <= r; ++dy) {
+        const uint16_t *row = t.row + dy * t.cols - r;
+        const double *ws = t.ws + (dy + r) * side;
+        if constexpr (RR >= 0) row_taps<2 * RR + 1>(t, row, ws, sw, swd);
+        else
+            for (int k = 0; k < side; ++k) row_taps<1>(t, row + k, ws + k, sw, swd);
+    }
+}
+
+// Column gx of the depth rows y0 .. y0 + rows - 1 into LDS, kStageBatch loads in flight (a loop over
+// the tile's elements divides each by its width: a sixth of the filter's instructions at radius 5).
+__device__ __forceinline__ void stage_column(const uint16_t *__restrict__ depth, int W, int H, int y0, int gx, int rows,
+                                             int cols, uint16_t *out)
+{
+    const bool in = gx >= 0 && gx < W;
+    const int cx = min(max(gx, 0), W - 1);
+    for (int b0 = 0; b0 < rows; b0 += kStageBatch) {
+        uint16_t v[kStageBatch];
+#pragma unroll
+        for (int u = 0; u < kStageBatch; ++u)  // unconditional loads from clamped (in-frame) addresses
+            v[u] = depth[(int64_t)min(max(y0 + b0 + u, 0), H - 1) * W + cx];
+#pragma unroll
+        for (int u = 0; u < kStageBatch; ++u) {
+            const int gy = y0 + b0 + u;
+            if (b0 + u < rows) out[(b0 + u) * cols] = in && gy >= 0 && gy < H ? v[u] : (uint16_t)0;
+        }
+    }
+}
+
 // The pixel work of a workgroup (the row segment x0 .. x0 + 255 of row y): stage the depth rows
 // y-R .. y+R and the weight tables in LDS, then for this thread's pixel the bilateral filter,
 // back-projection, depth -> colour re-projection and BGR sampling in the reference's FP32
@@ -82,7 +170,7 @@ __device__ __forceinline__ bool front_pixel(const uint16_t *__restrict__ depth, 
     extern __shared__ __align__(16) unsigned char front_lds[];
     double *s_ws = reinterpret_cast<double *>(front_lds);
     double *s_wr = s_ws + n_ws;
-    uint16_t *tile = reinterpret_cast<uint16_t *>(s_wr + n_wr);
+    uint16_t *tile = reinterpret_cast<uint16_t *>(s_wr + n_wr + 1);
 
     const int W = fp.W, H = fp.H;
     const int x = x0 + threadIdx.x;
@@ -92,38 +180,39 @@ __device__ __forceinline__ bool front_pixel(const uint16_t *__restrict__ depth, 
 
     // stage rows y-R .. y+R, columns x0-R .. x0+255+R (out of frame -> 0, which the filter
     // skips exactly like the reference skips out-of-frame and zero taps)
-    // (each thread's loads go out kStageBatch at a time before any is written to LDS: one
-    // memory round trip per batch, not per element)
     const int rows = 2 * R + 1, cols = kRowSeg + 2 * R;
-    for (int b0 = 0; b0 < rows * cols; b0 += kRowSeg * kStageBatch) {
-        uint16_t v[kStageBatch];
+    // the thread's own column of the tile, then of the 2 R columns right of them (rows of 2 R)
+    const int gx0 = x0 - R + (int)threadIdx.x;
+    stage_column(depth, W, H, y - R, gx0, rows, cols, tile + threadIdx.x);
+    if ((int)threadIdx.x < 2 * R) stage_column(depth, W, H, y - R, gx0 + kRowSeg, rows, cols, tile + kRowSeg + threadIdx.x);
+    if (fp.mode == GCA_BILATERAL_REFERENCE_ADAPTIVE) {
+        // step q's (2 q + 1)^2 spatial weights and the start of its range table: at most kRowSeg each
+        double w[6];
 #pragma unroll
-        for (int u = 0; u < kStageBatch; ++u) {  // unconditional loads from clamped (in-frame) addresses
-            const int k = b0 + u * kRowSeg + (int)threadIdx.x;
-            const int ry = k / cols, rx = k - ry * cols;
-            const int gy = y - R + ry, gx = x0 - R + rx;
-            const bool in = k < rows * cols && gy >= 0 && gy < H && gx >= 0 && gx < W;
-            const int cy = min(max(gy, 0), H - 1), cx = min(max(gx, 0), W - 1);
-            const uint16_t d = depth[(int64_t)cy * W + cx];
-            v[u] = in ? d : (uint16_t)0;
+        for (int q = 0; q < 6; ++q) {
+            const int side2 = (2 * q + 1) * (2 * q + 1), k = (int)threadIdx.x;
+            w[q] = lut[k < side2 ? fp.ws_off[q] + k : fp.wr_off[q] + min(k - side2, kAdaptiveNear - 1)];
         }
 #pragma unroll
-        for (int u = 0; u < kStageBatch; ++u) {
-            const int k = b0 + u * kRowSeg + (int)threadIdx.x;
-            if (k < rows * cols) tile[k] = v[u];
+        for (int q = 0; q < 6; ++q) {
+            const int side2 = (2 * q + 1) * (2 * q + 1), k = (int)threadIdx.x;
+            if (k < side2) s_ws[q * (2 * q - 1) * (2 * q + 1) / 3 + k] = w[q];
+            else if (k - side2 <= kAdaptiveNear) s_wr[q * (kAdaptiveNear + 1) + k - side2] = k - side2 < kAdaptiveNear ? w[q] : 0.0;
         }
-    }
-    for (int b0 = 0; b0 < n_ws + n_wr; b0 += kRowSeg * kStageBatch) {
-        double w[kStageBatch];
+    } else {
+        if (threadIdx.x == 0) s_wr[n_wr] = 0.0;
+        for (int b0 = 0; b0 < n_ws + n_wr; b0 += kRowSeg * kStageBatch) {
+            double w[kStageBatch];
 #pragma unroll
-        for (int u = 0; u < kStageBatch; ++u) {  // unconditional loads from clamped table indices
-            const int k = min(b0 + u * kRowSeg + (int)threadIdx.x, n_ws + n_wr - 1);
-            w[u] = lut[k < n_ws ? fp.ws_off[0] + k : fp.wr_off[0] + (k - n_ws)];
-        }
+            for (int u = 0; u < kStageBatch; ++u) {  // unconditional loads from clamped table indices
+                const int k = min(b0 + u * kRowSeg + (int)threadIdx.x, n_ws + n_wr - 1);
+                w[u] = lut[k < n_ws ? fp.ws_off[0] + k : fp.wr_off[0] + (k - n_ws)];
+            }
 #pragma unroll
-        for (int u = 0; u < kStageBatch; ++u) {
-            const int k = b0 + u * kRowSeg + (int)threadIdx.x;
-            if (k < n_ws + n_wr) s_ws[k] = w[u];  // s_wr follows s_ws
+            for (int u = 0; u < kStageBatch; ++u) {
+                const int k = b0 + u * kRowSeg + (int)threadIdx.x;
+                if (k < n_ws + n_wr) s_ws[k] = w[u];  // s_wr follows s_ws
+            }
         }
     }
     __syncthreads();
@@ -148,28 +237,30 @@ __device__ __forceinline__ bool front_pixel(const uint16_t *__restrict__ depth, 
                 r = (int)(1.0f * (float)step);
             }
             if (r >= 0) {
-                const int wl = fp.wr_len[s];
-                const int side = 2 * r + 1;
+                Taps t;
+                t.row = &tile[R * cols + threadIdx.x + R];
+                t.cols = cols;
+                t.d0 = d0;
+                t.ws = s_ws;
+                t.wr = s_wr;
+                t.near = (uint32_t)n_wr;
+                if (fp.mode == GCA_BILATERAL_REFERENCE_ADAPTIVE) {
+                    t.ws += s * (2 * s - 1) * (2 * s + 1) / 3;  // (2 q + 1)^2 weights of the steps below
+                    t.wr += s * (kAdaptiveNear + 1);
+                    t.near = (uint32_t)kAdaptiveNear;
+                }
+                t.far = lut + fp.wr_off[s];
+                t.len = (uint32_t)fp.wr_len[s];
                 double sw = 0.0, swd = 0.0;
-                auto taps = [&](const double *ws, const double *wr) {
-                    for (int dy = -r; dy <= r; ++dy) {
-                        const uint16_t *row = &tile[(R + dy) * cols + threadIdx.x + R];
-                        for (int dx = -r; dx <= r; ++dx) {
-                            uint16_t dn = row[dx];
-                            if (!dn) continue;
-                            int diff = abs((int)d0 - (int)dn);
-                            double wrv = diff < wl ? wr[diff] : 0.0;
-                            double w = __dmul_rn(ws[(dy + r) * side + (dx + r)], wrv);
-                            sw = __dadd_rn(sw, w);
-                            swd = __dadd_rn(swd, __dmul_rn(w, (double)dn));
-                        }
-                    }
-                };
-                // two copies of the loop, so each reads its tables with the right instructions
-                if (n_ws > 0)
-                    taps(s_ws, s_wr);
-                else
-                    taps(lut + fp.ws_off[s], lut + fp.wr_off[s]);
+                switch (r) {
+                case 0: filter_taps<0>(t, r, sw, swd); break;
+                case 1: filter_taps<1>(t, r, sw, swd); break;
+                case 2: filter_taps<2>(t, r, sw, swd); break;
+                case 3: filter_taps<3>(t, r, sw, swd); break;
+                case 4: filter_taps<4>(t, r, sw, swd); break;
+                case 5: filter_taps<5>(t, r, sw, swd); break;
+                default: filter_taps<-1>(t, r, sw, swd); break;
+                }
                 f = swd / sw;
             }
             const float z = (float)f * fp.scale;
@@ -202,7 +293,9 @@ __device__ __forceinline__ bool front_pixel(const uint16_t *__restrict__ depth, 
     return valid;
 }
 
-__global__ __launch_bounds__(kRowSeg) void k_rgbd_pixels(const uint16_t *__restrict__ depth,
+// Six wavefronts per SIMD: 640x480 with the 5x5 filter 13.5 us (15.9 at the five that 84 registers
+// leave, 14.4 with eight and spills).
+__global__ __launch_bounds__(kRowSeg) __attribute__((amdgpu_waves_per_eu(6, 8))) void k_rgbd_pixels(const uint16_t *__restrict__ depth,
                                                          const uint8_t *__restrict__ bgr,
                                                          const double *__restrict__ lut, FrontParams fp,
                                                          uint2 *__restrict__ st_pix,
@@ -578,13 +671,18 @@ int32_t launch_from_rgbd(gca_ctx ctx, const uint16_t *depth, const uint8_t *bgr,
     const bool onepass = ctx->tune[GCA_TUNE_FRONTEND] == 1;
     float *bpart = (float *)ctx_scratch(ctx, 20, sizeof(float) * 6 * nblocks, false);
     if (!bpart) return GCA_ERR_OUT_OF_MEMORY;
-    // LDS of the pixel work: weight tables (fixed mode; the range table while it is short)
-    // and the depth tile of the filter's radius
+    // LDS of the pixel work: weight tables (of the range tables the start) and the depth tile of the
+    // filter's radius
     const int R = bil->mode == GCA_BILATERAL_FIXED ? bil->radius : (bil->mode == GCA_BILATERAL_REFERENCE_ADAPTIVE ? 5 : 0);
-    const bool stage = bil->mode == GCA_BILATERAL_FIXED && fp.wr_len[0] <= kWrLds;  // both tables or neither
-    const int n_ws = stage ? (2 * R + 1) * (2 * R + 1) : 0;
-    const int n_wr = stage ? fp.wr_len[0] : 0;
-    const size_t lds = sizeof(double) * (size_t)(n_ws + n_wr) + sizeof(uint16_t) * (size_t)(2 * R + 1) * (kRowSeg + 2 * R);
+    int n_ws = 0, n_wr = 0;
+    if (bil->mode == GCA_BILATERAL_FIXED) {
+        n_ws = (2 * R + 1) * (2 * R + 1);
+        n_wr = std::min(fp.wr_len[0], kWrLds);
+    } else if (bil->mode == GCA_BILATERAL_REFERENCE_ADAPTIVE) {
+        n_ws = kAdaptiveWs;
+        n_wr = 6 * (kAdaptiveNear + 1) - 1;
+    }
+    const size_t lds = sizeof(double) * (size_t)(n_ws + n_wr + 1) + sizeof(uint16_t) * (size_t)(2 * R + 1) * (kRowSeg + 2 * R);
     StageTimer timer(ctx, GCA_STAGE_FRONTEND);
     if (onepass) {
         // look-back words and the segment counter: zeroed once when allocated, then carried
