@@ -249,75 +249,134 @@ void *ctx_scratch(gca_ctx ctx, int slot, size_t bytes, bool zeroed)
 // ---------------------------------------------------------------------------------------
 // utility kernels
 
-__global__ void k_bounds_init(CloudHdr *h)
+// ---- bounding boxes -----------------------------------------------------------------------
+// A kernel that touches every point writes its workgroups' bounds on the side, and a small launch folds
+// them into the header's keys (min from FLT_MAX, max from FLT_MIN as geometry_util.cuh:92).
+// 0.4 M points: 6 us in the transform and 3 for the fold; a pass of its own with 64 workgroups and
+// six atomics each on the header's words took 17 us after an initialising launch of 2.5, and letting
+// the last workgroup fold cost the transform 9 us (every workgroup's release writes back what the
+// kernel has in L2).
+constexpr int kBoundsThreads = 1024, kBoundsBlocks = 256;
+constexpr int kBoundsBatch = 4;  // points in flight per thread
+
+// value a of workgroup b at part[a * kBoundsBlocks + b] (allocated with the ctx: calls that compute
+// bounds may be captured)
+constexpr size_t kBoundsWorkBytes = sizeof(float) * 6 * kBoundsBlocks;
+
+static unsigned bounds_blocks(int64_t cap)
 {
-    for (int a = 0; a < 3; ++a) {
-        h->bmin_key[a] = float_to_key(FLT_MAX);
-        h->bmax_key[a] = float_to_key(FLT_MIN);  // geometry_util.cuh:92 initialises max with FLT_MIN
-    }
+    return (unsigned)std::min<int64_t>(kBoundsBlocks, std::max<int64_t>(1, (cap + kBoundsThreads - 1) / kBoundsThreads));
 }
 
-// Block-reduced AABB, one atomic per block and component.
-__global__ __launch_bounds__(256) void k_bounds_reduce(const float4 *__restrict__ xyzi,
-                                                       CloudHdr *__restrict__ h)
-{
-    __shared__ float smin[3][4], smax[3][4];
-    const int n = h->n;
+struct Bounds {
     float mn[3] = {FLT_MAX, FLT_MAX, FLT_MAX}, mx[3] = {-FLT_MAX, -FLT_MAX, -FLT_MAX};
-    for (int i = blockIdx.x * blockDim.x + threadIdx.x; i < n; i += gridDim.x * blockDim.x) {
-        float4 p = xyzi[i];
-        mn[0] = fminf(mn[0], p.x), mn[1] = fminf(mn[1], p.y), mn[2] = fminf(mn[2], p.z);
-        mx[0] = fmaxf(mx[0], p.x), mx[1] = fmaxf(mx[1], p.y), mx[2] = fmaxf(mx[2], p.z);
+    __device__ __forceinline__ void add(float x, float y, float z)
+    {
+        mn[0] = fminf(mn[0], x), mn[1] = fminf(mn[1], y), mn[2] = fminf(mn[2], z);
+        mx[0] = fmaxf(mx[0], x), mx[1] = fmaxf(mx[1], y), mx[2] = fmaxf(mx[2], z);
     }
+};
+
+// The workgroup's fold of b: value a of thread a < 6.
+__device__ __forceinline__ float bounds_fold(const Bounds &b)
+{
+    __shared__ float red[6][kBoundsThreads / kWave];
     const int w = threadIdx.x / kWave;
+#pragma unroll
     for (int a = 0; a < 3; ++a) {
-        float a0 = wave_min(mn[a]), a1 = wave_max(mx[a]);
-        if (lane_id() == 0) smin[a][w] = a0, smax[a][w] = a1;
+        const float v0 = wave_min(b.mn[a]), v1 = wave_max(b.mx[a]);
+        if (lane_id() == 0) red[a][w] = v0, red[3 + a][w] = v1;
     }
     __syncthreads();
-    if (threadIdx.x < 3) {
-        int a = threadIdx.x;
-        float m0 = smin[a][0], m1 = smax[a][0];
-        for (int k = 1; k < 4; ++k) m0 = fminf(m0, smin[a][k]), m1 = fmaxf(m1, smax[a][k]);
-        if (m0 <= m1 || n > 0) {
-            atomicMin(&h->bmin_key[a], float_to_key(m0));
-            atomicMax(&h->bmax_key[a], float_to_key(m1));
-        }
+    float v = 0.f;
+    if (threadIdx.x < 6) {
+        v = red[threadIdx.x][0];
+        for (int k = 1; k < kBoundsThreads / kWave; ++k)
+            v = threadIdx.x < 3 ? fminf(v, red[threadIdx.x][k]) : fmaxf(v, red[threadIdx.x][k]);
+    }
+    return v;
+}
+
+__device__ __forceinline__ void bounds_store(const Bounds &mine, float *__restrict__ part)
+{
+    const float v = bounds_fold(mine);
+    if (threadIdx.x < 6) part[threadIdx.x * kBoundsBlocks + blockIdx.x] = v;
+}
+
+// One wavefront per value.
+__global__ __launch_bounds__(6 * kWave) void k_bounds_keys(const float *__restrict__ part, int nblk, CloudHdr *__restrict__ h)
+{
+    const int a = (int)threadIdx.x / kWave;
+    float v = a < 3 ? FLT_MAX : FLT_MIN;
+    for (int b = lane_id(); b < nblk; b += kWave) {
+        const float x = part[a * kBoundsBlocks + b];
+        v = a < 3 ? fminf(v, x) : fmaxf(v, x);
+    }
+    v = a < 3 ? wave_min(v) : wave_max(v);
+    if (lane_id() != 0) return;
+    if (a < 3) h->bmin_key[a] = float_to_key(v);
+    else h->bmax_key[a - 3] = float_to_key(v);
+}
+
+static hipError_t bounds_keys(gca_ctx ctx, unsigned nblk, CloudHdr *h)
+{
+    hipLaunchKernelGGL(k_bounds_keys, dim3(1), dim3(6 * kWave), 0, ctx->stream, (const float *)ctx->bounds_work, (int)nblk, h);
+    return hipGetLastError();
+}
+
+// Points at, at + step, ... below n.
+__device__ __forceinline__ void bounds_of(const float4 *xyzi, int64_t n, int64_t at, int64_t step, Bounds &b)
+{
+    for (int64_t i0 = at; i0 < n; i0 += step * kBoundsBatch) {
+        float4 p[kBoundsBatch];
+#pragma unroll
+        for (int u = 0; u < kBoundsBatch; ++u) p[u] = xyzi[min(i0 + u * step, n - 1)];
+#pragma unroll
+        for (int u = 0; u < kBoundsBatch; ++u) b.add(p[u].x, p[u].y, p[u].z);  // past the end: the last point again
     }
 }
 
-__global__ __launch_bounds__(256) void k_transform(float4 *__restrict__ xyzi, float4 *__restrict__ nrm,
-                                                   float4 *__restrict__ grad, const CloudHdr *__restrict__ h,
-                                                   double t00, double t01, double t02, double t03,
-                                                   double t10, double t11, double t12, double t13,
-                                                   double t20, double t21, double t22, double t23,
-                                                   int do_n, int do_g)
+__global__ __launch_bounds__(kBoundsThreads) void k_bounds(const float4 *__restrict__ xyzi, const CloudHdr *__restrict__ h,
+                                                           float *__restrict__ part)
 {
-    const int n = h->n;
-    for (int i = blockIdx.x * blockDim.x + threadIdx.x; i < n; i += gridDim.x * blockDim.x) {
-        float4 p = xyzi[i];
-        double x = p.x, y = p.y, z = p.z;
-        p.x = (float)(((t00 * x + t01 * y) + t02 * z) + t03);
-        p.y = (float)(((t10 * x + t11 * y) + t12 * z) + t13);
-        p.z = (float)(((t20 * x + t21 * y) + t22 * z) + t23);
-        xyzi[i] = p;
-        if (do_n) {
-            float4 v = nrm[i];
-            double a = v.x, b = v.y, c = v.z;
-            v.x = (float)((t00 * a + t01 * b) + t02 * c);
-            v.y = (float)((t10 * a + t11 * b) + t12 * c);
-            v.z = (float)((t20 * a + t21 * b) + t22 * c);
-            nrm[i] = v;
-        }
-        if (do_g) {
-            float4 v = grad[i];
-            double a = v.x, b = v.y, c = v.z;
-            v.x = (float)((t00 * a + t01 * b) + t02 * c);
-            v.y = (float)((t10 * a + t11 * b) + t12 * c);
-            v.z = (float)((t20 * a + t21 * b) + t22 * c);
-            grad[i] = v;
+    Bounds b;
+    bounds_of(xyzi, h->n, (int64_t)blockIdx.x * kBoundsThreads + threadIdx.x, (int64_t)gridDim.x * kBoundsThreads, b);
+    bounds_store(b, part);
+}
+
+// Points (and the normals and gradients there are) moved by T, with the bounds of the moved points.
+__global__ __launch_bounds__(kBoundsThreads) void k_transform(float4 *__restrict__ xyzi, float4 *__restrict__ nrm,
+                                                              float4 *__restrict__ grad, const CloudHdr *__restrict__ h,
+                                                              float *__restrict__ part, double t00, double t01, double t02, double t03,
+                                                              double t10, double t11, double t12, double t13, double t20,
+                                                              double t21, double t22, double t23, int do_n, int do_g)
+{
+    const int n = h->n, step = gridDim.x * kBoundsThreads;
+    auto rotate = [&](float4 v) {
+        const double a = v.x, b = v.y, c = v.z;
+        return make_float4((float)((t00 * a + t01 * b) + t02 * c), (float)((t10 * a + t11 * b) + t12 * c),
+                           (float)((t20 * a + t21 * b) + t22 * c), v.w);
+    };
+    Bounds b;
+    for (int i0 = blockIdx.x * kBoundsThreads + threadIdx.x; i0 < n; i0 += step * kBoundsBatch) {
+        float4 p[kBoundsBatch];
+#pragma unroll
+        for (int u = 0; u < kBoundsBatch; ++u) p[u] = xyzi[(int)min((int64_t)i0 + (int64_t)u * step, (int64_t)n - 1)];
+#pragma unroll
+        for (int u = 0; u < kBoundsBatch; ++u) {
+            if ((int64_t)i0 + (int64_t)u * step >= n) continue;
+            const int i = i0 + u * step;
+            const double x = p[u].x, y = p[u].y, z = p[u].z;
+            p[u].x = (float)(((t00 * x + t01 * y) + t02 * z) + t03);
+            p[u].y = (float)(((t10 * x + t11 * y) + t12 * z) + t13);
+            p[u].z = (float)(((t20 * x + t21 * y) + t22 * z) + t23);
+            xyzi[i] = p[u];
+            if (do_n) nrm[i] = rotate(nrm[i]);
+            if (do_g) grad[i] = rotate(grad[i]);
+            b.add(p[u].x, p[u].y, p[u].z);
         }
     }
+    bounds_store(b, part);
 }
 
 // ---- exclusive scan of uint32: one pass with decoupled look-back ---------------------------
@@ -535,28 +594,23 @@ void cloud_points_changed(gca_cloud c)
     c->grid.attrs_valid = false;
 }
 
-hipError_t bounds_enqueue(gca_ctx ctx, const float4 *xyzi, int64_t cap, CloudHdr *hdr)
-{
-    hipLaunchKernelGGL(k_bounds_init, dim3(1), dim3(1), 0, ctx->stream, hdr);
-    // few blocks: each issues six atomics on the same header words
-    int64_t nb = std::min<int64_t>(64, std::max<int64_t>(1, (cap + 255) / 256));
-    hipLaunchKernelGGL(k_bounds_reduce, dim3((unsigned)nb), dim3(256), 0, ctx->stream, xyzi, hdr);
-    return hipGetLastError();
-}
-
 int32_t launch_bounds(gca_ctx ctx, gca_cloud c)
 {
-    GCA_HIP(bounds_enqueue(ctx, c->xyzi, c->cap, c->hdr));
+    const unsigned nb = bounds_blocks(c->cap);
+    hipLaunchKernelGGL(k_bounds, dim3(nb), dim3(kBoundsThreads), 0, ctx->stream, c->xyzi, c->hdr, ctx->bounds_work);
+    GCA_HIP(hipGetLastError());
+    GCA_HIP(bounds_keys(ctx, nb, c->hdr));
     return GCA_OK;
 }
 
 int32_t launch_transform(gca_ctx ctx, gca_cloud c, const double *T)
 {
-    int64_t nb = std::min<int64_t>(2048, std::max<int64_t>(1, (c->cap + 255) / 256));
-    hipLaunchKernelGGL(k_transform, dim3((unsigned)nb), dim3(256), 0, ctx->stream, c->xyzi, c->nrm,
-                       c->grad, c->hdr, T[0], T[1], T[2], T[3], T[4], T[5], T[6], T[7], T[8], T[9],
-                       T[10], T[11], c->has_normals ? 1 : 0, c->has_gradient ? 1 : 0);
+    const unsigned nb = bounds_blocks(c->cap);
+    hipLaunchKernelGGL(k_transform, dim3(nb), dim3(kBoundsThreads), 0, ctx->stream, c->xyzi, c->nrm, c->grad, c->hdr,
+                       ctx->bounds_work, T[0], T[1], T[2], T[3], T[4], T[5], T[6], T[7], T[8], T[9], T[10], T[11],
+                       c->has_normals ? 1 : 0, c->has_gradient ? 1 : 0);
     GCA_HIP(hipGetLastError());
+    GCA_HIP(bounds_keys(ctx, nb, c->hdr));
     return GCA_OK;
 }
 
@@ -671,7 +725,10 @@ int32_t gca_ctx_create(int32_t device, gca_ctx *out)
         hipEventCreate(&c->ev_a) != hipSuccess || hipEventCreate(&c->ev_b) != hipSuccess ||
         hipHostMalloc((void **)&c->dev_err, sizeof(uint32_t), hipHostMallocDefault) != hipSuccess ||
         hipHostMalloc((void **)&c->pinned, sizeof(double) * gca_ctx_s::kPinnedDoubles, hipHostMallocDefault) !=
-            hipSuccess) {
+            hipSuccess ||
+        hipMalloc((void **)&c->bounds_work, kBoundsWorkBytes) != hipSuccess) {
+        hipFree(c->bounds_work);
+        if (c->pinned) hipHostFree(c->pinned);
         if (c->dev_err) hipHostFree(c->dev_err);
         if (c->stream) hipStreamDestroy(c->stream);
         if (c->ev_a) hipEventDestroy(c->ev_a);
@@ -698,6 +755,7 @@ int32_t gca_ctx_destroy(gca_ctx c)
     for (void *p : c->hdrs.host_slabs) hipHostFree(p);
     if (c->host_buf) hipHostFree(c->host_buf);
     for (hipEvent_t e : c->prof_pool) hipEventDestroy(e);
+    hipFree(c->bounds_work);
     hipFree(c->bitmap);
     hipFree(c->lut);
     hipFree(c->icp_state);
@@ -1015,23 +1073,30 @@ int32_t gca_cloud_copy(gca_ctx ctx, gca_cloud src, gca_cloud dst)
     return GCA_OK;
 }
 
-// dst += src in one launch: the points below nd stay where they are (moved = 0) or are copied to
-// the grown arrays, those from nd on are src's.  nrm null: no normals survive.
-static __global__ __launch_bounds__(256) void k_cloud_append(const float4 *xyzi, const float4 *rgb, const float4 *nrm,
-                                                             const float4 *more_xyzi, const float4 *more_rgb,
-                                                             const float4 *more_nrm, int nd, int total, int moved,
-                                                             float4 *to_xyzi, float4 *to_rgb, float4 *to_nrm,
-                                                             CloudHdr *__restrict__ h)
+// dst += src in one launch, with the bounds of all points: the points below nd stay where they are
+// (moved = 0) or are copied to the grown arrays, those from nd on are src's.  nrm null: no normals
+// survive.
+static __global__ __launch_bounds__(kBoundsThreads) void k_cloud_append(const float4 *xyzi, const float4 *rgb,
+                                                                        const float4 *nrm, const float4 *more_xyzi,
+                                                                        const float4 *more_rgb, const float4 *more_nrm,
+                                                                        int nd, int total, int moved, float4 *to_xyzi,
+                                                                        float4 *to_rgb, float4 *to_nrm,
+                                                                        CloudHdr *__restrict__ h, float *__restrict__ part)
 {
-    const int step = gridDim.x * blockDim.x;
-    for (int i = (moved ? 0 : nd) + blockIdx.x * blockDim.x + threadIdx.x; i < total; i += step) {
+    Bounds b;
+    const int64_t step = (int64_t)gridDim.x * kBoundsThreads, at = (int64_t)blockIdx.x * kBoundsThreads + threadIdx.x;
+    for (int64_t i = at + (moved ? 0 : nd); i < total; i += step) {
         const bool own = i < nd;
-        const int k = own ? i : i - nd;
-        to_xyzi[i] = (own ? xyzi : more_xyzi)[k];
-        to_rgb[i] = (own ? rgb : more_rgb)[k];
+        const int64_t k = own ? i : i - nd;
+        const float4 p = (own ? xyzi : more_xyzi)[k], c = (own ? rgb : more_rgb)[k];
+        to_xyzi[i] = p;
+        to_rgb[i] = c;
         if (nrm) to_nrm[i] = (own ? nrm : more_nrm)[k];
+        b.add(p.x, p.y, p.z);
     }
+    if (!moved) bounds_of(xyzi, nd, at, step, b);
     if (blockIdx.x == 0 && threadIdx.x == 0) h->n = total;
+    bounds_store(b, part);
 }
 
 int32_t gca_cloud_append(gca_ctx ctx, gca_cloud dst, gca_cloud src)
@@ -1056,13 +1121,13 @@ int32_t gca_cloud_append(gca_ctx ctx, gca_cloud dst, gca_cloud src)
                 return st;
             }
         }
-    const unsigned nb = (unsigned)std::min<int64_t>(2048, std::max<int64_t>(1, (total + 255) / 256));
-    hipLaunchKernelGGL(k_cloud_append, dim3(nb), dim3(256), 0, ctx->stream, from[0], from[1], normals ? from[2] : nullptr,
-                       more[0], more[1], more[2], (int)nd, (int)total, cap > dst->cap ? 1 : 0, to[0], to[1], to[2],
-                       dst->hdr);
+    // (get_min_bound / get_max_bound recompute the bounds, point_cloud.cu:107-132)
+    const unsigned nb = bounds_blocks(total);
+    hipLaunchKernelGGL(k_cloud_append, dim3(nb), dim3(kBoundsThreads), 0, ctx->stream, from[0], from[1],
+                       normals ? from[2] : nullptr, more[0], more[1], more[2], (int)nd, (int)total, cap > dst->cap ? 1 : 0,
+                       to[0], to[1], to[2], dst->hdr, ctx->bounds_work);
     hipError_t e = hipGetLastError();
-    // get_min_bound / get_max_bound recompute the bounds (point_cloud.cu:107-132)
-    if (e == hipSuccess) e = bounds_enqueue(ctx, to[0], cap, dst->hdr);
+    if (e == hipSuccess) e = bounds_keys(ctx, nb, dst->hdr);
     const hipError_t es = hipStreamSynchronize(ctx->stream);
     if (e == hipSuccess) e = es;
     if (cap > dst->cap) {
@@ -1301,10 +1366,9 @@ int32_t gca_compute_color_gradient(gca_ctx ctx, gca_cloud c, float radius, int32
 int32_t gca_transform(gca_ctx ctx, gca_cloud c, const double T[16])
 {
     if (!ctx || !c || !T) return GCA_ERR_INVALID_VALUE;
-    GCA_TRY(launch_transform(ctx, c, T));
+    GCA_TRY(launch_transform(ctx, c, T));  // point_cloud.cu:96-100 recomputes the bounds
     const bool n_valid = c->host_valid || c->n_valid;
     cloud_points_changed(c);
-    GCA_TRY(launch_bounds(ctx, c));  // point_cloud.cu:96-100 recomputes the bounds
     c->n_valid = n_valid;
     return GCA_OK;
 }

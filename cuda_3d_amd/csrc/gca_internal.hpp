@@ -156,6 +156,7 @@ struct gca_ctx_s {
     // after the stream has been synchronised
     static constexpr int kPinnedDoubles = 32;
     double *pinned = nullptr;
+    float *bounds_work = nullptr;  // workgroups' bounds on their way to a header
     // pinned host memory for a call's uploads and read-backs, grown on demand (ctx_host_buf); a
     // small read-back into it takes 12 us, into pageable memory 21
     void *host_buf = nullptr;
@@ -340,8 +341,6 @@ int32_t launch_normals_gradient(gca_ctx ctx, gca_cloud c, float radius, int32_t 
                                 bool grid_attrs = false);
 int32_t launch_transform(gca_ctx ctx, gca_cloud c, const double T[16]);
 int32_t launch_bounds(gca_ctx ctx, gca_cloud c);
-// The bounds of hdr->n points (at most cap) into hdr.
-hipError_t bounds_enqueue(gca_ctx ctx, const float4 *xyzi, int64_t cap, CloudHdr *hdr);
 int32_t launch_copy_cloud(gca_ctx ctx, gca_cloud src, gca_cloud dst);
 int32_t launch_upload_finish(gca_ctx ctx, gca_cloud c, int64_t n);
 
