@@ -560,15 +560,26 @@ int32_t cloud_reserve(gca_cloud c, int64_t cap)
     return GCA_OK;
 }
 
-int32_t cloud_sync_header(gca_cloud c)
+int32_t cloud_header_enqueue(gca_cloud c)
 {
-    if (c->host_valid) return GCA_OK;
     GCA_HIP(hipMemcpyAsync(c->ref.host, c->hdr, sizeof(CloudHdr), hipMemcpyDeviceToHost, c->ctx->stream));
-    GCA_HIP(hipStreamSynchronize(c->ctx->stream));
+    return GCA_OK;
+}
+
+int32_t cloud_header_take(gca_cloud c)
+{
     GCA_TRY(ctx_take_device_error(c->ctx));  // a header behind a failed scan is not valid
     c->host_hdr = *c->ref.host;
     c->host_valid = true;
     return GCA_OK;
+}
+
+int32_t cloud_sync_header(gca_cloud c)
+{
+    if (c->host_valid) return GCA_OK;
+    GCA_TRY(cloud_header_enqueue(c));
+    GCA_HIP(hipStreamSynchronize(c->ctx->stream));
+    return cloud_header_take(c);
 }
 
 int32_t cloud_sync_count(gca_ctx ctx, gca_cloud c)

@@ -265,6 +265,9 @@ void dev_array_free(gca_ctx ctx, T *&p, int64_t n, bool idle)
 int32_t ctx_take_device_error(gca_ctx ctx);
 int32_t cloud_reserve(gca_cloud c, int64_t cap);
 int32_t cloud_sync_header(gca_cloud c);  // copies hdr to host (synchronises the stream)
+// The same in two parts, the second once the stream has passed the first.
+int32_t cloud_header_enqueue(gca_cloud c);
+int32_t cloud_header_take(gca_cloud c);
 // host_hdr.n current for a call on ctx's stream: no read-back where the host set the count itself.
 int32_t cloud_sync_count(gca_ctx ctx, gca_cloud c);
 void cloud_host_bounds(gca_cloud c, float mn[3], float mx[3]);

@@ -2270,14 +2270,36 @@ int32_t gca_multiscale_icp(gca_ctx ctx, gca_cloud src_full, gca_cloud tgt_full, 
         gca_cloud *a = &ctx->level_clouds[2 * l], *b = &ctx->level_clouds[2 * l + 1];
         if (!*a) GCA_TRY(gca_cloud_create(ctx, 1, a));
         if (!*b) GCA_TRY(gca_cloud_create(ctx, 1, b));
-        GCA_TRY(gca_voxel_downsample(ctx, src_full, L.voxel_size, *a));
-        GCA_TRY(gca_voxel_downsample(ctx, tgt_full, L.voxel_size, *b));
-        GCA_TRY(gca_estimate_normals(ctx, *b, L.normal_radius, L.normal_max_nn));
-        GCA_TRY(gca_compute_color_gradient(ctx, *b, L.gradient_radius, L.gradient_max_nn));
         cs[l] = *a;
         ct[l] = *b;
         prm[l] = L.icp;
         gr[l] = L.gradient_radius;
+    }
+    // The targets' clouds, their headers on the way to the host, the sources' clouds, then the
+    // targets' grids and attributes: the host lays out the grids while the sources are built, where
+    // level by level the GPU waited for each header's read-back (1280x720, three levels: 30 us).
+    for (int l = 0; l < n_levels; ++l) {
+        GCA_TRY(gca_voxel_downsample(ctx, tgt_full, levels[l].voxel_size, ct[l]));
+        GCA_TRY(cloud_header_enqueue(ct[l]));
+    }
+    GCA_HIP(hipEventRecord(ctx->ev_a, ctx->stream));
+    for (int l = 0; l < n_levels; ++l) GCA_TRY(gca_voxel_downsample(ctx, src_full, levels[l].voxel_size, cs[l]));
+    GCA_HIP(hipEventSynchronize(ctx->ev_a));
+    for (int l = 0; l < n_levels; ++l) {
+        const gca_level_params &L = levels[l];
+        gca_cloud t = ct[l];
+        GCA_TRY(cloud_header_take(t));
+        // the gradient's neighbours are among the normals' unless its radius or cap says otherwise
+        const bool joint = L.normal_max_nn >= 0 && L.gradient_max_nn == 0 && L.gradient_radius > 0.0f &&
+                           L.gradient_radius <= L.normal_radius;
+        if (joint) {
+            GCA_TRY(grid_build(ctx, t, L.normal_radius));
+            GCA_TRY(launch_normals_gradient(ctx, t, L.normal_radius, L.normal_max_nn, L.gradient_radius, true));
+            t->has_normals = t->has_gradient = true;
+        } else {
+            GCA_TRY(gca_estimate_normals(ctx, t, L.normal_radius, L.normal_max_nn));
+            GCA_TRY(gca_compute_color_gradient(ctx, t, L.gradient_radius, L.gradient_max_nn));
+        }
     }
     // the levels in order, each starting from the pose the previous one ends with (one resident
     // launch per level, or one persistent launch over the chain)

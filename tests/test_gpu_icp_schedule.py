@@ -48,3 +48,27 @@ def test_persistent_launch_equals_one_launch_per_iteration(pairs, levels, tune):
     np.testing.assert_array_equal(got[1][0], got[2][0])
     assert got[1][1] == got[2][1]
     assert any(r[0] > 1 for row in got[1][1] for r in row)
+
+
+@pytest.mark.parametrize("normal_r,max_nn,grad_r,grad_nn", [(2.5, 30, 2.0, 0),   # attributes from one walk
+                                                            (2.5, 0, 2.5, 0),    # no cap, equal radii
+                                                            (2.0, 30, 2.5, 0),   # the gradient reaches further
+                                                            (2.5, 30, 2.0, 12)])  # a capped gradient
+def test_multiscale_equals_its_steps(normal_r, max_nn, grad_r, grad_nn):
+    import cuda_3d_amd as g
+
+    src, tgt = _clouds(g, 20000, 5)
+    voxels = (0.05, 0.03, 0.02)
+    levels = [g.level_params(v, normal_radius=normal_r * v, normal_max_nn=max_nn, gradient_radius=grad_r * v,
+                             gradient_max_nn=grad_nn, icp=g.icp_params(6, 2.5 * v)) for v in voxels]
+    T, reps = g.multiscale_icp(src, tgt, levels)
+    pose = np.eye(4)
+    for v, rep in zip(voxels, reps):
+        s, t = src.voxel_grid_down_sample(v), tgt.voxel_grid_down_sample(v)
+        t.estimate_normals(normal_r * v, max_nn)
+        t.compute_color_gradient(grad_r * v, grad_nn)
+        Ts, one = g.batch_multiscale_icp([[s]], [[t]], [g.icp_params(6, 2.5 * v)], pose[None], [grad_r * v])
+        pose = Ts[0]
+        assert (rep.iterations, rep.n_correspondences, rep.rmse) == (one[0][0].iterations, one[0][0].n_correspondences,
+                                                                     one[0][0].rmse)
+    np.testing.assert_array_equal(T, pose)
