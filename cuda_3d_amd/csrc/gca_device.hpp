@@ -25,10 +25,11 @@ __device__ __forceinline__ int xcd_runs(int b, int m)
     return ((i / G) * kXcds + x) * G + i % G;
 }
 
-// Device-scope ordering for the last-block (ticket) pattern.  __threadfence() is a seq_cst
-// fence, which on gfx950 both writes back AND invalidates the XCD's L2: issued by every block
-// it evicts the data the other blocks are still reading.  Writers only need release
-// (write-back); only the block that wins the ticket needs acquire (invalidate).
+// Device-scope ordering for the last-block (ticket) pattern of the registration's epochs.
+// __threadfence() is a seq_cst fence, which on gfx950 both writes back AND invalidates the XCD's
+// L2: issued by every block it evicts the data the other blocks are still reading.  Writers only
+// need release (write-back, itself some microseconds when the block's outputs are dirty in L2);
+// only the block that wins the ticket needs acquire (invalidate).
 __device__ __forceinline__ void fence_release_agent() { __builtin_amdgcn_fence(__ATOMIC_RELEASE, "agent"); }
 __device__ __forceinline__ void fence_acquire_agent() { __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "agent"); }
 

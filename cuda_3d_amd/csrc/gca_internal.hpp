@@ -300,7 +300,6 @@ hipError_t front_launch_update(FrontLaunch *f, hipGraphExec_t exec, hipGraphNode
 // noalloc_setup resolves once per device (noalloc.hip); the library never allocates it.
 constexpr int kNoAllocMaxBlocks = 1024;  // partials of up to this many workgroups
 struct NoAllocScratch {
-    alignas(256) uint32_t ticket;                // last-block ticket, zero between calls
     alignas(256) double partials[kNoAllocMaxBlocks * 32];
 };
 // Device address of `device`'s scratch (resolved on the first call for that device, with the

@@ -1135,15 +1135,14 @@ __global__ __launch_bounds__(kIcpBlock) GCA_ICP_OCCUPANCY void k_icp_resident(co
     }
 }
 
-// Gauss-Newton system for given correspondences (no solve).  ticket: zero at the launch, left at
-// zero; out: the 29 sums (FP64).
+// Gauss-Newton system for given correspondences (no solve): the workgroups' 29 sums (FP64), added in
+// block order by k_gn_fold.
 template <int MODE>
 __global__ __launch_bounds__(kIcpBlock) void k_build_gn(PairDesc P, const float4 *__restrict__ tgt_xyzi,
                                                         const int32_t *__restrict__ nn, double t00, double t01,
                                                         double t02, double t03, double t10, double t11,
                                                         double t12, double t13, double t20, double t21,
-                                                        double t22, double t23, float sl, float sc,
-                                                        uint32_t *ticket, double *out)
+                                                        double t22, double t23, float sl, float sc)
 {
     const double T[12] = {t00, t01, t02, t03, t10, t11, t12, t13, t20, t21, t22, t23};
     const int n = P.src_hdr->n;
@@ -1162,54 +1161,49 @@ __global__ __launch_bounds__(kIcpBlock) void k_build_gn(PairDesc P, const float4
         ++ncorr;
     }
     __shared__ double sys[kPartStride];
-    __shared__ bool last;
     block_partial<MODE>(A, ncorr, 1, kIcpBlock, sys);
     if (threadIdx.x < kNSys) P.partials[(int64_t)blockIdx.x * kPartStride + threadIdx.x] = sys[threadIdx.x];
-    fence_release_agent();
-    __syncthreads();
-    if (threadIdx.x == 0) last = atomicAdd(ticket, 1u) == (uint32_t)(P.nblk - 1);
-    __syncthreads();
-    if (!last) return;
-    fence_acquire_agent();
-    sum_partials(P.partials, P.nblk, sys, MODE == GCA_ACCUM_NAIVE_FP32);
-    if (threadIdx.x < kNSys) out[threadIdx.x] = sys[threadIdx.x];
-    if (threadIdx.x == 0) *ticket = 0u;
 }
 
-__global__ void k_ticket_clear(uint32_t *ticket) { *ticket = 0u; }
+__global__ __launch_bounds__(kIcpBlock) void k_gn_fold(const double *__restrict__ partials, int nblk, int naive,
+                                                       double *__restrict__ out)
+{
+    __shared__ double sys[kPartStride];
+    sum_partials(partials, nblk, sys, naive != 0);
+    if (threadIdx.x < kNSys) out[threadIdx.x] = sys[threadIdx.x];
+}
 
-// k_build_gn over given partials (nblk workgroups' worth), ticket and output, on ctx's stream.
+// k_build_gn over given partials (nblk workgroups' worth) and its fold, on ctx's stream.
 static void launch_build_gn(gca_ctx ctx, const PairDesc &P, const float4 *tgt_xyzi, const int32_t *nn, const double *T,
-                            float lambda, int32_t mode, uint32_t *ticket, double *out)
+                            float lambda, int32_t mode, double *out)
 {
     const float sl = sqrtf(lambda), sc = sqrtf(1.0f - lambda);
     const dim3 g((unsigned)P.nblk), b(kIcpBlock);
     if (mode == GCA_ACCUM_NAIVE_FP32)
         hipLaunchKernelGGL(k_build_gn<GCA_ACCUM_NAIVE_FP32>, g, b, 0, ctx->stream, P, tgt_xyzi, nn, T[0], T[1], T[2],
-                           T[3], T[4], T[5], T[6], T[7], T[8], T[9], T[10], T[11], sl, sc, ticket, out);
+                           T[3], T[4], T[5], T[6], T[7], T[8], T[9], T[10], T[11], sl, sc);
     else if (mode == GCA_ACCUM_FP64)
         hipLaunchKernelGGL(k_build_gn<GCA_ACCUM_FP64>, g, b, 0, ctx->stream, P, tgt_xyzi, nn, T[0], T[1], T[2], T[3],
-                           T[4], T[5], T[6], T[7], T[8], T[9], T[10], T[11], sl, sc, ticket, out);
+                           T[4], T[5], T[6], T[7], T[8], T[9], T[10], T[11], sl, sc);
     else
         hipLaunchKernelGGL(k_build_gn<GCA_ACCUM_COMPENSATED>, g, b, 0, ctx->stream, P, tgt_xyzi, nn, T[0], T[1], T[2],
-                           T[3], T[4], T[5], T[6], T[7], T[8], T[9], T[10], T[11], sl, sc, ticket, out);
+                           T[3], T[4], T[5], T[6], T[7], T[8], T[9], T[10], T[11], sl, sc);
+    hipLaunchKernelGGL(k_gn_fold, dim3(1), b, 0, ctx->stream, (const double *)P.partials, P.nblk,
+                       mode == GCA_ACCUM_NAIVE_FP32 ? 1 : 0, out);
 }
 
-// ---- generic FP64 block sums with last-block finish (residuals, objective) -----------------
-// A block's sums go out write-through and wavefront 0, which stored them, takes the ticket with a
-// release, so no other wavefront's stores are flushed for it.  The last block reads kFinishRows
-// blocks' sums at a time with all its threads, then one thread per value adds them from LDS in
-// block order: the adjoint of 100k points 105 -> 19 us, the residuals of 92k 105 -> 16 us (one
-// thread per value reading them from memory as well: a round trip per block).
-constexpr int kFinishRows = 128;
+// ---- generic FP64 block sums (residuals, objective) ----------------------------------------
+// A workgroup's sums go to its row, and a second launch adds the rows in block order: kFoldRows of
+// them are read at a time with all threads, then one thread per value adds them from LDS.  A last
+// workgroup that added them needed every workgroup to release what it wrote, which writes back the
+// outputs that L2 holds: the adjoint of 100k points 20 us, now 7 + 5; the residuals of 92k 16 us,
+// now 5 + 4 (105 us each with one thread per value reading the rows from memory).
+constexpr int kFoldRows = 512, kFoldThreads = 1024;
 
 template <int NV>
-__device__ __forceinline__ void sum_finish(double (&v)[NV], double *partials, int nblk, uint32_t *ticket,
-                                           double *result)
+__device__ __forceinline__ void block_sums(double (&v)[NV], double *__restrict__ partials)
 {
     __shared__ double wv[kIcpBlock / kWave][NV];
-    __shared__ double rows[kFinishRows][NV];
-    __shared__ bool last;
 #pragma unroll
     for (int k = 0; k < NV; ++k) v[k] = wave_sum(v[k]);
     if (lane_id() == 0)
@@ -1218,28 +1212,38 @@ __device__ __forceinline__ void sum_finish(double (&v)[NV], double *partials, in
     if (threadIdx.x < NV) {
         double a = 0.0;
         for (int w = 0; w < kIcpBlock / kWave; ++w) a += wv[w][threadIdx.x];
-        store_coherent(&partials[(int64_t)blockIdx.x * kPartStride + threadIdx.x], a);
+        partials[(int64_t)blockIdx.x * kPartStride + threadIdx.x] = a;
     }
-    static_assert(NV <= kWave, "the ticket's release covers wavefront 0's stores");
-    if (threadIdx.x == 0)
-        last = __hip_atomic_fetch_add(ticket, 1u, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_AGENT) == (uint32_t)(nblk - 1);
-    __syncthreads();
-    if (!last) return;
-    fence_acquire_agent();
+}
+
+template <int NV>
+__global__ __launch_bounds__(kFoldThreads) void k_sums_fold(const double *__restrict__ partials, int nblk,
+                                                         double *__restrict__ result)
+{
+    __shared__ double rows[kFoldRows][NV];
     double a = 0.0;
-    for (int b0 = 0; b0 < nblk; b0 += kFinishRows) {
-        const int nr = min(kFinishRows, nblk - b0);
-        for (int e = threadIdx.x; e < nr * NV; e += kIcpBlock)
-            rows[e / NV][e % NV] = partials[(int64_t)(b0 + e / NV) * kPartStride + e % NV];
+    for (int b0 = 0; b0 < nblk; b0 += kFoldRows) {
+        const int nr = min(kFoldRows, nblk - b0);
+        constexpr int kPer = (kFoldRows * NV + kFoldThreads - 1) / kFoldThreads;
+        double x[kPer];
+#pragma unroll
+        for (int u = 0; u < kPer; ++u) {  // all loads of the rows out before any is stored
+            const int e = min((int)threadIdx.x + u * kFoldThreads, nr * NV - 1);
+            x[u] = partials[(int64_t)(b0 + e / NV) * kPartStride + e % NV];
+        }
+#pragma unroll
+        for (int u = 0; u < kPer; ++u) {
+            const int e = (int)threadIdx.x + u * kFoldThreads;
+            if (e < nr * NV) rows[e / NV][e % NV] = x[u];
+        }
         __syncthreads();
         if (threadIdx.x < NV) {
-#pragma unroll 8
+#pragma unroll 16
             for (int r = 0; r < nr; ++r) a += rows[r][threadIdx.x];
         }
         __syncthreads();
     }
     if (threadIdx.x < NV) result[threadIdx.x] = a;
-    if (threadIdx.x == 0) *ticket = 0u;
 }
 
 // Pose of the residual kernel (the first three rows) and parameters of the objective's adjoint,
@@ -1253,8 +1257,7 @@ struct ObjectiveParams {
 
 __global__ __launch_bounds__(kIcpBlock) void k_residuals(PairDesc P, const float4 *__restrict__ tgt_xyzi,
                                                          const int32_t *__restrict__ nn, Pose34 Tm, float lam,
-                                                         float sl, float sc, int kind, float *__restrict__ out,
-                                                         uint32_t *ticket, double *__restrict__ result)
+                                                         float sl, float sc, int kind, float *__restrict__ out)
 {
     const double *T = Tm.m;
     const int n = P.src_hdr->n;
@@ -1292,15 +1295,14 @@ __global__ __launch_bounds__(kIcpBlock) void k_residuals(PairDesc P, const float
             v[0] += a;
         }
     }
-    sum_finish<1>(v, P.partials, P.nblk, ticket, result);
+    block_sums<1>(v, P.partials);
 }
 
 // Objective E and its adjoint at pose dT(xi) * T with frozen correspondences, all in FP64.
 __global__ __launch_bounds__(kIcpBlock) void k_objective_grad(PairDesc P, const float4 *__restrict__ tgt_xyzi,
                                                               const int32_t *__restrict__ nn,
                                                               ObjectiveParams prm, double lam,
-                                                              float4 *__restrict__ dpts, uint32_t *ticket,
-                                                              double *__restrict__ result)
+                                                              float4 *__restrict__ dpts)
 {
     const double *T = prm.T, *dT = prm.dT, *RzRy = prm.RzRy, *Rx = prm.Rx, *M = prm.M;
     const int n = P.src_hdr->n;
@@ -1347,7 +1349,7 @@ __global__ __launch_bounds__(kIcpBlock) void k_objective_grad(PairDesc P, const 
             dpts[i] = o;
         }
     }
-    sum_finish<7>(v, P.partials, P.nblk, ticket, result);
+    block_sums<7>(v, P.partials);
 }
 
 // ---------------------------------------------------------------------------------------------
@@ -1932,10 +1934,10 @@ int32_t icp_plan_results(gca_ctx ctx, const IcpPlan *p, double *T_out, gca_icp_r
     return GCA_OK;
 }
 
-// Set-up of the single-pair kernels over given correspondences: no launch and no copy.  The ticket
-// is zero from its allocation on and left at zero by every launch; a launch's last block stores
-// the sums into the ctx's pinned memory, so a stream synchronisation is all it takes to read them.
-static int32_t single_pair(gca_ctx ctx, gca_cloud src, gca_cloud tgt, PairDesc &P, uint32_t **ticket)
+// Set-up of the single-pair kernels over given correspondences: no launch and no copy.  The fold
+// stores the sums into the ctx's pinned memory, so a stream synchronisation is all it takes to read
+// them.
+static int32_t single_pair(gca_ctx ctx, gca_cloud src, gca_cloud tgt, PairDesc &P)
 {
     GCA_TRY(cloud_sync_count(ctx, src));
     P = PairDesc{};
@@ -1946,8 +1948,7 @@ static int32_t single_pair(gca_ctx ctx, gca_cloud src, gca_cloud tgt, PairDesc &
     P.grad = tgt->grad;
     P.nblk = icp_blocks(src->host_hdr.n);
     P.partials = (double *)ctx_scratch(ctx, 14, sizeof(double) * kPartStride * P.nblk, false);
-    *ticket = (uint32_t *)ctx_scratch(ctx, 9, 256, true);
-    return P.partials && *ticket ? GCA_OK : GCA_ERR_OUT_OF_MEMORY;
+    return P.partials ? GCA_OK : GCA_ERR_OUT_OF_MEMORY;
 }
 
 }  // namespace gca
@@ -1964,9 +1965,8 @@ int32_t gca_build_gauss_newton(gca_ctx ctx, gca_cloud src, gca_cloud tgt, const 
     if (lambda > 1.0f || !(lambda >= 0.0f) || mode < 0 || mode > 2) return GCA_ERR_INVALID_VALUE;  // .cu:438-441
     if (!tgt->has_normals || !tgt->has_gradient) return GCA_ERR_NOT_READY;                       // .cu:449-452
     PairDesc P;
-    uint32_t *ticket;
-    GCA_TRY(single_pair(ctx, src, tgt, P, &ticket));
-    launch_build_gn(ctx, P, tgt->xyzi, nn_dev, T, lambda, mode, ticket, ctx->pinned);
+    GCA_TRY(single_pair(ctx, src, tgt, P));
+    launch_build_gn(ctx, P, tgt->xyzi, nn_dev, T, lambda, mode, ctx->pinned);
     GCA_HIP(hipGetLastError());
     GCA_HIP(hipStreamSynchronize(ctx->stream));
     memcpy(out, ctx->pinned, sizeof(double) * kNSys);
@@ -1994,8 +1994,7 @@ int32_t gca_build_gauss_newton_noalloc(gca_ctx ctx, gca_cloud src, gca_cloud tgt
     P.grad = tgt->grad;
     P.partials = sc->partials;
     P.nblk = nb;
-    hipLaunchKernelGGL(k_ticket_clear, dim3(1), dim3(1), 0, ctx->stream, &sc->ticket);
-    launch_build_gn(ctx, P, tgt->xyzi, nn_dev, T, lambda, mode, &sc->ticket, out_dev);
+    launch_build_gn(ctx, P, tgt->xyzi, nn_dev, T, lambda, mode, out_dev);
     GCA_HIP(hipGetLastError());
     return GCA_OK;
 }
@@ -2007,13 +2006,14 @@ int32_t gca_compute_residuals(gca_ctx ctx, gca_cloud src, gca_cloud tgt, const i
     if (lambda > 1.0f || !(lambda >= 0.0f)) return GCA_ERR_INVALID_VALUE;
     if (!tgt->has_normals || !tgt->has_gradient) return GCA_ERR_NOT_READY;
     PairDesc P;
-    uint32_t *ticket;
-    GCA_TRY(single_pair(ctx, src, tgt, P, &ticket));
+    GCA_TRY(single_pair(ctx, src, tgt, P));
     Pose34 pose;
     memcpy(pose.m, T, sizeof(pose.m));
     const float sl = sqrtf(lambda), sc = sqrtf(1.0f - lambda);
     hipLaunchKernelGGL(k_residuals, dim3((unsigned)P.nblk), dim3(kIcpBlock), 0, ctx->stream, P, tgt->xyzi, nn_dev, pose,
-                       lambda, sl, sc, kind, out_dev, ticket, ctx->pinned);
+                       lambda, sl, sc, kind, out_dev);
+    hipLaunchKernelGGL(k_sums_fold<1>, dim3(1), dim3(kFoldThreads), 0, ctx->stream, (const double *)P.partials, P.nblk,
+                       ctx->pinned);
     GCA_HIP(hipGetLastError());
     GCA_HIP(hipStreamSynchronize(ctx->stream));
     if (sum) *sum = ctx->pinned[0];
@@ -2319,8 +2319,7 @@ int32_t gca_color_icp_objective_grad(gca_ctx ctx, gca_cloud src, gca_cloud tgt, 
     if (lambda > 1.0f || !(lambda >= 0.0f)) return GCA_ERR_INVALID_VALUE;
     if (!tgt->has_normals || !tgt->has_gradient) return GCA_ERR_NOT_READY;
     PairDesc P;
-    uint32_t *ticket;
-    GCA_TRY(single_pair(ctx, src, tgt, P, &ticket));
+    GCA_TRY(single_pair(ctx, src, tgt, P));
     ObjectiveParams prm;
     memcpy(prm.T, T, sizeof(prm.T));
     const double ca = cos(xi[0]), sa = sin(xi[0]), cb = cos(xi[1]), sb = sin(xi[1]), cc = cos(xi[2]), sc = sin(xi[2]);
@@ -2337,7 +2336,9 @@ int32_t gca_color_icp_objective_grad(gca_ctx ctx, gca_cloud src, gca_cloud tgt, 
         for (int j = 0; j < 3; ++j)
             prm.M[3 * i + j] = (dTv[4 * i] * T[j] + dTv[4 * i + 1] * T[4 + j]) + dTv[4 * i + 2] * T[8 + j];
     hipLaunchKernelGGL(k_objective_grad, dim3((unsigned)P.nblk), dim3(kIcpBlock), 0, ctx->stream, P, tgt->xyzi, nn_dev, prm,
-                       (double)lambda, (float4 *)dpts_dev, ticket, ctx->pinned);
+                       (double)lambda, (float4 *)dpts_dev);
+    hipLaunchKernelGGL(k_sums_fold<7>, dim3(1), dim3(kFoldThreads), 0, ctx->stream, (const double *)P.partials, P.nblk,
+                       ctx->pinned);
     GCA_HIP(hipGetLastError());
     GCA_HIP(hipStreamSynchronize(ctx->stream));
     if (E) *E = ctx->pinned[0];

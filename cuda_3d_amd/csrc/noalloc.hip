@@ -2,12 +2,12 @@
 //
 // gca_build_gauss_newton_noalloc (icp.hip) runs the Gauss-Newton build of
 // gca_build_gauss_newton for callers that cannot allocate (code under HIP graph capture, serving
-// loops): its workgroup partials and last-block ticket live in `scratch`, a file-scope device
-// array of fixed size that every device holds until the process ends.  Host code never passes the
-// array's name to a kernel: in host code it is a stand-in, not a device address.  The address is
-// resolved once per device, with that device current, by hipGetSymbolAddress, and kept per device;
-// kernels receive that address.  Every call on a device shares its array: calls that overlap on
-// one device (two streams, two threads) race, and the ticket is cleared at the start of each call.
+// loops): its workgroup partials live in `scratch`, a file-scope device array of fixed size that
+// every device holds until the process ends.  Host code never passes the array's name to a kernel:
+// in host code it is a stand-in, not a device address.  The address is resolved once per device,
+// with that device current, by hipGetSymbolAddress, and kept per device; kernels receive that
+// address.  Every call on a device shares its array: calls that overlap on one device (two streams,
+// two threads) race.
 #include <hip/hip_runtime.h>
 
 #include <mutex>
