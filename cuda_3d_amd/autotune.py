@@ -46,7 +46,7 @@ def space(n_cu: int) -> Dict[str, List[int]]:
         "icp_lanes_medium": [1, 2, 4, 8, 16],
         "icp_lanes_large": [1, 2, 4, 8, 16],
         "icp_max_units": [64, 128, 256, 512, 1024],
-        "icp_persist_blocks": [n_cu // 2, n_cu, 2 * n_cu, 4 * n_cu, 8 * n_cu],
+        "icp_persist_blocks": [n_cu // 2, n_cu, 2 * n_cu, 3 * n_cu, 4 * n_cu, 8 * n_cu],
         "icp_lanes_batch": [1, 2, 4, 8],
         "grid_cell": [4, 5, 6, 8],
     }
@@ -63,10 +63,11 @@ STAGES_OF = {
     "grid_cell": ("grid", "normals", "gradient", "icp"),
 }
 # knobs a workload does not exercise (one-pair calls never read the batch lanes, the batch
-# never reads the one-pair lanes or the normals shape)
+# never reads the one-pair lanes; the normal and gradient kernels have one shape, so nothing reads
+# their lanes)
 UNUSED_BY = {
-    "frame": ("icp_lanes_batch",),
-    "frame_overlapped": ("icp_lanes_batch", "icp_persist_blocks"),
+    "frame": ("icp_lanes_batch", "normals_lanes"),
+    "frame_overlapped": ("icp_lanes_batch", "icp_persist_blocks", "normals_lanes"),
     "batch": ("normals_lanes", "icp_lanes_small", "icp_lanes_medium", "icp_lanes_large", "grid_cell"),
 }
 
