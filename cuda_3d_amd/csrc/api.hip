@@ -246,6 +246,34 @@ void *ctx_scratch(gca_ctx ctx, int slot, size_t bytes, bool zeroed)
     return ctx->scratch[slot];
 }
 
+void *lane_scratch(gca_ctx ctx, int lane, int slot, size_t bytes, bool zeroed)
+{
+    // the slots that the voxel, scan and joint normals jobs use
+    constexpr int kSlots[] = {6, 7, 15, 17, 18, 19, 22, 23, 24};
+    constexpr int n = sizeof(kSlots) / sizeof(kSlots[0]);
+    static_assert(gca_ctx_s::kLaneSlots + (kMaxJobs - 1) * n <= gca_ctx_s::kScratchSlots, "lane slots");
+    if (lane == 0) return ctx_scratch(ctx, slot, bytes, zeroed);
+    if (lane < 0 || lane >= kMaxJobs) return nullptr;
+    for (int k = 0; k < n; ++k)
+        if (kSlots[k] == slot) return ctx_scratch(ctx, gca_ctx_s::kLaneSlots + (lane - 1) * n + k, bytes, zeroed);
+    return nullptr;
+}
+
+void ctx_lanes_release(gca_ctx ctx)
+{
+    hipStreamSynchronize(ctx->stream);
+    for (int s = gca_ctx_s::kLaneSlots; s < gca_ctx_s::kScratchSlots; ++s) {
+        hipFree(ctx->scratch[s]);
+        ctx->scratch[s] = nullptr;
+        ctx->scratch_bytes[s] = 0;
+        ctx->scratch_zeroed[s] = false;
+    }
+    for (int l = 1; l < kMaxJobs; ++l) {
+        hipFree(ctx->bitmap[l].p);
+        ctx->bitmap[l] = {};
+    }
+}
+
 // ---------------------------------------------------------------------------------------
 // utility kernels
 
@@ -475,14 +503,14 @@ __global__ __launch_bounds__(BLOCK) void k_scan_onepass(Jobs<ScanJob, N> J)
 bool scan_wide(int64_t n) { return (n + 256 * kScanPer - 1) / (256 * kScanPer) > kScanWideFrom; }
 
 int32_t scan_job(gca_ctx ctx, const uint32_t *in, uint32_t *out, int64_t n, uint32_t *total_dev, bool wide,
-                 ScanJob *job)
+                 ScanJob *job, int lane)
 {
     const int64_t chunk = (wide ? 1024 : 256) * kScanPer;
     int64_t nchunks = (n + chunk - 1) / chunk;
     if (nchunks < 1) nchunks = 1;
     if (nchunks > 1024 * 64) return GCA_ERR_INVALID_VALUE;
-    unsigned long long *flags = (unsigned long long *)ctx_scratch(ctx, 15, sizeof(unsigned long long) * nchunks, true);
-    ScanCtl *ctl = (ScanCtl *)ctx_scratch(ctx, 23, sizeof(ScanCtl), true);
+    unsigned long long *flags = (unsigned long long *)lane_scratch(ctx, lane, 15, sizeof(unsigned long long) * nchunks, true);
+    ScanCtl *ctl = (ScanCtl *)lane_scratch(ctx, lane, 23, sizeof(ScanCtl), true);
     if (!flags || !ctl) return GCA_ERR_OUT_OF_MEMORY;
     *job = ScanJob{in, n, (int32_t)nchunks, 0, flags, ctl, out, total_dev, out + n, ctx->dev_err};
     return GCA_OK;
@@ -672,6 +700,22 @@ int32_t grid_build(gca_ctx ctx, gca_cloud c, float radius, bool exact)
     return GCA_OK;
 }
 
+int32_t grid_build_levels(gca_ctx ctx, const gca_cloud *cs, const float *r, int n)
+{
+    const int32_t q = ctx->tune[GCA_TUNE_GRID_CELL] <= 4 ? 0 : ctx->tune[GCA_TUNE_GRID_CELL];
+    gca_ctx ctxs[kMaxJobs];
+    GridDesc ds[kMaxJobs];
+    if (n < 1 || n > kMaxJobs) return GCA_ERR_INVALID_VALUE;
+    for (int j = 0; j < n; ++j) {
+        GCA_TRY(cloud_sync_header(cs[j]));
+        float mn[3], mx[3];
+        cloud_host_bounds(cs[j], mn, mx);
+        grid_params(mn, mx, r[j], &ds[j], q);
+        ctxs[j] = ctx;
+    }
+    return launch_grid_levels(ctx, ctxs, cs, ds, n, false);
+}
+
 // Events are recorded on the launching ctx's stream; the record is kept by the owner's profiler
 // (a frame pipeline's level ctxs report to the pipeline's ctx).
 StageTimer::StageTimer(gca_ctx c, int stage) : ctx(c), owner(c->prof_owner ? c->prof_owner : c)
@@ -767,7 +811,7 @@ int32_t gca_ctx_destroy(gca_ctx c)
     if (c->host_buf) hipHostFree(c->host_buf);
     for (hipEvent_t e : c->prof_pool) hipEventDestroy(e);
     hipFree(c->bounds_work);
-    hipFree(c->bitmap);
+    for (gca_ctx_s::Bitmap &b : c->bitmap) hipFree(b.p);
     hipFree(c->lut);
     hipFree(c->icp_state);
     hipFree(c->partials);

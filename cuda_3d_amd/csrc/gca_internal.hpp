@@ -145,7 +145,8 @@ struct gca_ctx_s {
     hipStream_t stream = nullptr;
     hipEvent_t ev_a = nullptr, ev_b = nullptr;
     // scratch buffers owned by the ctx, grown on demand
-    static constexpr int kScratchSlots = 48;
+    // (the slots from kLaneSlots on are the further lanes' of calls that build several clouds at once)
+    static constexpr int kLaneSlots = 48, kScratchSlots = 80;
     void *scratch[kScratchSlots] = {nullptr};
     size_t scratch_bytes[kScratchSlots] = {0};
     bool scratch_zeroed[kScratchSlots] = {false};
@@ -166,9 +167,11 @@ struct gca_ctx_s {
     int n_cu = 0;         // compute units of the device (persistent launch sizing)
     int wall_khz = 0;     // rate of the device wall clock (wall_clock64)
     // persistent bitmap of the voxel downsampler (kept all-zero between calls)
-    uint32_t *bitmap = nullptr;
-    int64_t bitmap_words = 0;
-    bool bitmap_dirty = false;
+    struct Bitmap {
+        uint32_t *p = nullptr;
+        int64_t words = 0;
+        bool dirty = false;
+    } bitmap[gca::kMaxJobs];
     // bilateral weight tables (FP64, host-computed), keyed by their parameters
     double *lut = nullptr;
     size_t lut_bytes = 0;
@@ -240,6 +243,10 @@ namespace gca {
 // Internal helpers implemented in api.hip -------------------------------------------------
 int32_t hip_status(hipError_t e);
 void *ctx_scratch(gca_ctx ctx, int slot, size_t bytes, bool zeroed);
+// The same for lane `lane` (< kMaxJobs) of a launch over several clouds of one ctx; lane 0 is slot
+// itself.  ctx_lanes_release gives the further lanes' scratch and bitmaps back.
+void *lane_scratch(gca_ctx ctx, int lane, int slot, size_t bytes, bool zeroed);
+void ctx_lanes_release(gca_ctx ctx);
 // Pinned host memory of the ctx; its content is the calling entry point's until that returns.
 void *ctx_host_buf(gca_ctx ctx, size_t bytes);
 // Buffers of clouds and grids (BufferPool).  dev_free: bytes as allocated; idle = device_idle()
@@ -312,6 +319,8 @@ int32_t launch_from_rgbd(gca_ctx ctx, const uint16_t *depth, const uint8_t *bgr,
                          const gca_camera *cam, const gca_bilateral *bil, float tmin, float tmax,
                          gca_cloud out, uint32_t *clear_word = nullptr);
 int32_t launch_voxel(gca_ctx ctx, gca_cloud in, float voxel, gca_cloud out);
+// The same cloud at n voxel sizes (n <= kMaxJobs), each kernel once for all of them.
+int32_t launch_voxel_sizes(gca_ctx ctx, gca_cloud in, const float *voxel, const gca_cloud *out, int n);
 // No host round trip: the lattice is computed on the device; the bitmap scan covers max_bits
 // cells (a lattice beyond that flags *err and gives an empty output); scratch by capacity.
 int32_t launch_voxel_planned(gca_ctx ctx, gca_cloud in, float voxel, gca_cloud out, double max_bits,
@@ -395,7 +404,7 @@ struct ScanJob {
 };
 bool scan_wide(int64_t n);
 int32_t scan_job(gca_ctx ctx, const uint32_t *in, uint32_t *out, int64_t n, uint32_t *total_dev, bool wide,
-                 ScanJob *job);
+                 ScanJob *job, int lane = 0);
 // jobs[0, nj) in one launch on stream (nj <= kMaxJobs, all of one kind).
 int32_t scan_launch(hipStream_t stream, const ScanJob *jobs, int nj, bool popcount, bool wide);
 
@@ -412,13 +421,18 @@ struct VoxelLevelJob {
 };
 int32_t launch_voxel_levels(gca_ctx launch, const VoxelLevelJob *jobs, int nj);
 // Counted grids (the voxel finalize did the count pass).
-int32_t launch_grid_levels(gca_ctx launch, const gca_ctx *ctxs, const gca_cloud *cs, const GridDesc *ds, int nj);
+int32_t launch_grid_levels(gca_ctx launch, const gca_ctx *ctxs, const gca_cloud *cs, const GridDesc *ds, int nj,
+                           bool counted = true);
+// Grids of n clouds (headers on the host) of one ctx, the radius r[j] each, as grid_build makes them.
+int32_t grid_build_levels(gca_ctx ctx, const gca_cloud *cs, const float *r, int n);
 struct NormalsLevelJob {
     gca_ctx ctx;
     gca_cloud c;
     float radius;
     int32_t max_nn;
     float gradient_radius;  // <= radius
+    int lane = 0;           // of ctx's scratch: jobs of one ctx take different ones
+    int64_t n = 0;          // the cloud's points where the host knows them (0: up to its capacity)
 };
 // launch_normals_gradient(..., grid_attrs = true) per level.
 int32_t launch_normals_gradient_levels(gca_ctx launch, const NormalsLevelJob *jobs, int nj);

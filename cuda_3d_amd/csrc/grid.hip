@@ -24,12 +24,22 @@
 
 namespace gca {
 
-__global__ __launch_bounds__(256) void k_grid_count(const float4 *__restrict__ xyzi,
-                                                    const CloudHdr *__restrict__ hdr, GridDesc g,
-                                                    uint32_t *__restrict__ count,
-                                                    uint32_t *__restrict__ cell_of)
+struct CountArgs {
+    const float4 *xyzi;
+    const CloudHdr *hdr;
+    GridDesc g;
+    uint32_t *count, *cell_of;
+};
+
+template <int N>
+__global__ __launch_bounds__(256) void k_grid_count(Jobs<CountArgs, N> J)
 {
-    const int n = hdr->n;
+    const CountArgs &A = J.a[N == 1 ? 0 : blockIdx.y];
+    const float4 *__restrict__ xyzi = A.xyzi;
+    uint32_t *__restrict__ count = A.count;
+    uint32_t *__restrict__ cell_of = A.cell_of;
+    const GridDesc g = A.g;
+    const int n = A.hdr->n;
     for (int i = blockIdx.x * blockDim.x + threadIdx.x; i < n; i += gridDim.x * blockDim.x) {
         float4 p = xyzi[i];
         int32_t cx = grid_cell(p.x, g.origin[0], g.cell, g.dims[0]);
@@ -129,8 +139,8 @@ int32_t launch_grid_build(gca_ctx ctx, gca_cloud c, const GridDesc &d, bool coun
     const unsigned nb = (unsigned)std::min<int64_t>(4096, std::max<int64_t>(1, (c->cap + 255) / 256));
     StageTimer timer(ctx, GCA_STAGE_GRID);
     if (!counted) {
-        hipLaunchKernelGGL(k_grid_count, dim3(nb), dim3(256), 0, ctx->stream, c->xyzi, c->hdr, d, G.count,
-                           G.cell_of);
+        const Jobs<CountArgs, 1> ct{{{c->xyzi, c->hdr, d, G.count, G.cell_of}}};
+        hipLaunchKernelGGL(k_grid_count<1>, dim3(nb), dim3(256), 0, ctx->stream, ct);
         GCA_HIP(hipGetLastError());
     }
     GCA_TRY(exclusive_scan_u32(ctx, G.count, G.start, d.ncells, nullptr));
@@ -143,7 +153,8 @@ int32_t launch_grid_build(gca_ctx ctx, gca_cloud c, const GridDesc &d, bool coun
     return GCA_OK;
 }
 
-int32_t launch_grid_levels(gca_ctx launch, const gca_ctx *ctxs, const gca_cloud *cs, const GridDesc *ds, int nj)
+int32_t launch_grid_levels(gca_ctx launch, const gca_ctx *ctxs, const gca_cloud *cs, const GridDesc *ds, int nj,
+                           bool counted)
 {
     if (nj < 1 || nj > kMaxJobs) return GCA_ERR_INVALID_VALUE;
     bool wide = false;
@@ -152,16 +163,21 @@ int32_t launch_grid_levels(gca_ctx launch, const gca_ctx *ctxs, const gca_cloud 
         wide = wide || scan_wide(ds[j].ncells);
     }
     ScanJob scans[kMaxJobs];
+    Jobs<CountArgs, kMaxJobs> ct{};
     Jobs<ScatterArgs, kMaxJobs> sc{};
     unsigned nb = 1;
     for (int j = 0; j < nj; ++j) {
         const Grid &G = cs[j]->grid;
-        GCA_TRY(scan_job(ctxs[j], G.count, G.start, ds[j].ncells, nullptr, wide, &scans[j]));
+        int lane = 0;  // a lane of its ctx's scratch each
+        for (int k = 0; k < j; ++k) lane += ctxs[k] == ctxs[j];
+        GCA_TRY(scan_job(ctxs[j], G.count, G.start, ds[j].ncells, nullptr, wide, &scans[j], lane));
+        ct.a[j] = CountArgs{cs[j]->xyzi, cs[j]->hdr, ds[j], G.count, G.cell_of};
         sc.a[j] = ScatterArgs{cs[j]->xyzi, cs[j]->hdr, G.count, G.start, G.cell_of, G.order, G.sxyzi};
         nb = std::max(nb, (unsigned)std::min<int64_t>(4096, std::max<int64_t>(1, (cs[j]->cap + 255) / 256)));
     }
     {
         StageTimer timer(launch, GCA_STAGE_GRID);
+        if (!counted) hipLaunchKernelGGL(k_grid_count<kMaxJobs>, dim3(nb, (unsigned)nj), dim3(256), 0, launch->stream, ct);
         GCA_TRY(scan_launch(launch->stream, scans, nj, false, wide));
         hipLaunchKernelGGL(k_grid_scatter<kMaxJobs>, dim3(nb, (unsigned)nj), dim3(256), 0, launch->stream, sc);
         GCA_HIP(hipGetLastError());

@@ -671,7 +671,7 @@ struct PairJobs {
 };
 
 static int32_t pair_prepare(gca_ctx ctx, gca_cloud c, float radius, int32_t K, float gradient_radius, bool grid_attrs,
-                            PairJobs *pj)
+                            int lane, int64_t n, PairJobs *pj)
 {
     if (!(gradient_radius <= radius)) return GCA_ERR_INVALID_VALUE;
     Grid &G = c->grid;
@@ -679,11 +679,11 @@ static int32_t pair_prepare(gca_ctx ctx, gca_cloud c, float radius, int32_t K, f
         GCA_TRY(dev_array(c->ctx, &G.snrm, G.cap_pts));
         GCA_TRY(dev_array(c->ctx, &G.sgrad, G.cap_pts));
     }
-    const int64_t cap = std::max<int64_t>(c->cap, 1);
-    Moments *mom = (Moments *)ctx_scratch(ctx, 17, sizeof(Moments) * cap, false);
-    int32_t *ovf = (int32_t *)ctx_scratch(ctx, 18, sizeof(int32_t) * cap, false);
-    uint32_t *ovf_n = (uint32_t *)ctx_scratch(ctx, 19, 256, true);  // zero, re-armed by k_solve_pair
-    Moments *mom_g = (Moments *)ctx_scratch(ctx, 24, sizeof(Moments) * cap, false);
+    const int64_t cap = std::max<int64_t>(n > 0 ? n : c->cap, 1);
+    Moments *mom = (Moments *)lane_scratch(ctx, lane, 17, sizeof(Moments) * cap, false);
+    int32_t *ovf = (int32_t *)lane_scratch(ctx, lane, 18, sizeof(int32_t) * cap, false);
+    uint32_t *ovf_n = (uint32_t *)lane_scratch(ctx, lane, 19, 256, true);  // zero, re-armed by k_solve_pair
+    Moments *mom_g = (Moments *)lane_scratch(ctx, lane, 24, sizeof(Moments) * cap, false);
     if (!mom || !ovf || !ovf_n || !mom_g) return GCA_ERR_OUT_OF_MEMORY;
     const GridDesc d = query_desc(G, radius);
     const double rg = (double)gradient_radius;
@@ -736,7 +736,7 @@ int32_t launch_normals_gradient(gca_ctx ctx, gca_cloud c, float radius, int32_t 
                                 bool grid_attrs)
 {
     PairJobs pj;
-    GCA_TRY(pair_prepare(ctx, c, radius, K, gradient_radius, grid_attrs, &pj));
+    GCA_TRY(pair_prepare(ctx, c, radius, K, gradient_radius, grid_attrs, 0, 0, &pj));
     {
         StageTimer timer(ctx, GCA_STAGE_NORMALS);
         GCA_TRY(pair_launch<1>(ctx->stream, &pj, 1));
@@ -751,7 +751,7 @@ int32_t launch_normals_gradient_levels(gca_ctx launch, const NormalsLevelJob *jo
     PairJobs pj[kMaxJobs];
     for (int j = 0; j < nj; ++j)
         GCA_TRY(pair_prepare(jobs[j].ctx, jobs[j].c, jobs[j].radius, jobs[j].max_nn, jobs[j].gradient_radius, true,
-                             &pj[j]));
+                             jobs[j].lane, jobs[j].n, &pj[j]));
     {
         StageTimer timer(launch, GCA_STAGE_NORMALS);
         GCA_TRY(pair_launch<kMaxJobs>(launch->stream, pj, nj));

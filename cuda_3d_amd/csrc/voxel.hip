@@ -483,35 +483,38 @@ struct VoxelJobs {
 // popcount scan over `words` bitmap words (>= the lattice's); enqueues nothing but a first-use
 // clear of the bitmap on ctx's stream.
 static int32_t voxel_prepare(gca_ctx ctx, gca_cloud in, float voxel, gca_cloud out, int64_t n_cap, int64_t words,
-                             double max_bits, uint32_t *err, const GridCount *gc, bool wide, VoxelJobs *vj)
+                             double max_bits, uint32_t *err, const GridCount *gc, bool wide, int lane,
+                             VoxelJobs *vj)
 {
-    if (ctx->bitmap_words < words || ctx->bitmap_dirty) {
+    gca_ctx_s::Bitmap &bm = ctx->bitmap[lane];
+    if (bm.words < words || bm.dirty) {
         GCA_HIP(hipStreamSynchronize(ctx->stream));
-        if (ctx->bitmap_words < words) {
-            hipFree(ctx->bitmap);
-            ctx->bitmap = nullptr;
-            ctx->bitmap_words = 0;
+        if (bm.words < words) {
+            hipFree(bm.p);
+            bm.p = nullptr;
+            bm.words = 0;
             int64_t want = std::max<int64_t>(words + words / 4, 1 << 16);
-            GCA_TRY(dev_array(ctx, &ctx->bitmap, want));
-            ctx->bitmap_words = want;
+            GCA_TRY(dev_array(ctx, &bm.p, want));
+            bm.words = want;
         }
-        GCA_HIP(hipMemsetAsync(ctx->bitmap, 0, sizeof(uint32_t) * ctx->bitmap_words, ctx->stream));
-        ctx->bitmap_dirty = false;
+        GCA_HIP(hipMemsetAsync(bm.p, 0, sizeof(uint32_t) * bm.words, ctx->stream));
+        bm.dirty = false;
     }
     const int64_t nc = std::max<int64_t>(n_cap, 1);
-    uint32_t *word_pre = (uint32_t *)ctx_scratch(ctx, 6, sizeof(uint32_t) * (words + 1), false);
-    unsigned long long *acc = (unsigned long long *)ctx_scratch(ctx, 7, sizeof(unsigned long long) * kVoxRec * nc, true);
-    VoxelParams *vp = (VoxelParams *)ctx_scratch(ctx, 22, sizeof(VoxelParams), false);
+    uint32_t *word_pre = (uint32_t *)lane_scratch(ctx, lane, 6, sizeof(uint32_t) * (words + 1), false);
+    unsigned long long *acc =
+        (unsigned long long *)lane_scratch(ctx, lane, 7, sizeof(unsigned long long) * kVoxRec * nc, true);
+    VoxelParams *vp = (VoxelParams *)lane_scratch(ctx, lane, 22, sizeof(VoxelParams), false);
     if (!word_pre || !acc || !vp) return GCA_ERR_OUT_OF_MEMORY;
-    GCA_TRY(scan_job(ctx, ctx->bitmap, word_pre, words, (uint32_t *)&out->hdr->n, wide, &vj->scan));
+    GCA_TRY(scan_job(ctx, bm.p, word_pre, words, (uint32_t *)&out->hdr->n, wide, &vj->scan, lane));
     // grid widths in multiples of 8: workgroups go to the 8 XCDs by linear id mod 8, so in an
     // all-levels launch (level = blockIdx.y) the levels' workgroups on the same points then share
     // an XCD and its L2, and the points are fetched from HBM once rather than once per level
     vj->nb = (unsigned)((std::min<int64_t>(4096, (nc + 255) / 256) + 7) / 8 * 8);
     vj->nb_acc = (unsigned)((std::min<int64_t>(4096, (nc + kVoxChunk - 1) / kVoxChunk) + 7) / 8 * 8);
-    vj->mark = MarkArgs{in->xyzi, in->hdr, voxel, max_bits, vp, err, ctx->bitmap};
-    vj->accum = AccumArgs{in->xyzi, in->rgb, in->hdr, vp, ctx->bitmap, word_pre, acc};
-    vj->fin = FinalArgs{acc, in->hdr, out->hdr, ctx->bitmap, out->xyzi, out->rgb, gc ? gc->d : GridDesc{},
+    vj->mark = MarkArgs{in->xyzi, in->hdr, voxel, max_bits, vp, err, bm.p};
+    vj->accum = AccumArgs{in->xyzi, in->rgb, in->hdr, vp, bm.p, word_pre, acc};
+    vj->fin = FinalArgs{acc, in->hdr, out->hdr, bm.p, out->xyzi, out->rgb, gc ? gc->d : GridDesc{},
                         gc ? gc->count : nullptr, gc ? gc->cell_of : nullptr};
     return GCA_OK;
 }
@@ -550,26 +553,25 @@ static int32_t voxel_enqueue(gca_ctx ctx, gca_cloud in, float voxel, gca_cloud o
 {
     const bool wide = scan_wide(words);
     VoxelJobs vj;
-    GCA_TRY(voxel_prepare(ctx, in, voxel, out, n_cap, words, max_bits, err, gc, wide, &vj));
-    ctx->bitmap_dirty = true;  // until the whole sequence is enqueued
+    GCA_TRY(voxel_prepare(ctx, in, voxel, out, n_cap, words, max_bits, err, gc, wide, 0, &vj));
+    ctx->bitmap[0].dirty = true;  // until the whole sequence is enqueued
     {
         StageTimer timer(ctx, GCA_STAGE_VOXEL);
         GCA_TRY(voxel_launch<1>(ctx->stream, &vj, 1, wide));
     }
-    ctx->bitmap_dirty = false;
+    ctx->bitmap[0].dirty = false;
     cloud_points_changed(out);
     return GCA_OK;
 }
 
-int32_t launch_voxel(gca_ctx ctx, gca_cloud in, float voxel, gca_cloud out)
+// The lattice of `in` (its header on the host) and its number of cells.
+static int32_t voxel_lattice(gca_cloud in, float voxel, VoxelParams &vp, double &nbits)
 {
-    GCA_TRY(cloud_sync_header(in));
     const int64_t n = in->host_hdr.n;
     float mn[3], mx[3];
     cloud_host_bounds(in, mn, mx);
-    VoxelParams vp{};
     vp.voxel = voxel;
-    double nbits = 1.0;
+    nbits = 1.0;
     for (int a = 0; a < 3; ++a) {  // the same FP32 formulas as voxel_params_of
         const float ext = mx[a] - mn[a];
         if (n > 0 && (double)voxel * (double)INT_MAX < (double)ext)  // point_cloud.cu:213-218
@@ -578,9 +580,63 @@ int32_t launch_voxel(gca_ctx ctx, gca_cloud in, float voxel, gca_cloud out)
         vp.dims[a] = n > 0 ? (int64_t)floorf(ext / voxel) + 1 : 1;
         nbits *= (double)vp.dims[a];
     }
+    return GCA_OK;
+}
+
+int32_t launch_voxel(gca_ctx ctx, gca_cloud in, float voxel, gca_cloud out)
+{
+    GCA_TRY(cloud_sync_header(in));
+    const int64_t n = in->host_hdr.n;
+    VoxelParams vp{};
+    double nbits;
+    GCA_TRY(voxel_lattice(in, voxel, vp, nbits));
     GCA_TRY(cloud_reserve(out, std::max<int64_t>(n, 1)));
     if (ctx->tune[GCA_TUNE_VOXEL] == 2 || nbits > kVoxelMaxBits) return voxel_sort_enqueue(ctx, in, vp, out, (int)n);
     return voxel_enqueue(ctx, in, voxel, out, n, ((int64_t)nbits + 31) / 32, kVoxelMaxBits, nullptr);
+}
+
+// All sizes in one launch a phase where every lattice is the bitmap's and their bits together are no
+// more than one call may take; else (and where the lanes' scratch cannot be had) a call each.
+int32_t launch_voxel_sizes(gca_ctx ctx, gca_cloud in, const float *voxel, const gca_cloud *out, int n)
+{
+    if (n < 1 || n > kMaxJobs) return GCA_ERR_INVALID_VALUE;
+    GCA_TRY(cloud_sync_header(in));
+    const int64_t np = std::max<int64_t>(in->host_hdr.n, 1);
+    int64_t words[kMaxJobs];
+    double all = 0.0;
+    bool wide = false;
+    for (int j = 0; j < n; ++j) {
+        VoxelParams vp{};
+        double nbits;
+        GCA_TRY(voxel_lattice(in, voxel[j], vp, nbits));
+        all += nbits;
+        words[j] = nbits > kVoxelMaxBits ? 0 : ((int64_t)nbits + 31) / 32;
+        wide = wide || scan_wide(words[j]);
+    }
+    bool together = n > 1 && ctx->tune[GCA_TUNE_VOXEL] != 2 && all <= kVoxelMaxBits;
+    VoxelJobs vj[kMaxJobs];
+    for (int j = 0; j < n && together; ++j) {
+        GCA_TRY(cloud_reserve(out[j], np));
+        const int32_t st = voxel_prepare(ctx, in, voxel[j], out[j], in->host_hdr.n, words[j], kVoxelMaxBits, nullptr,
+                                         nullptr, wide, j, &vj[j]);
+        together = st != GCA_ERR_OUT_OF_MEMORY;
+        if (together) GCA_TRY(st);
+        else ctx_lanes_release(ctx);
+    }
+    if (!together) {
+        for (int j = 0; j < n; ++j) GCA_TRY(launch_voxel(ctx, in, voxel[j], out[j]));
+        return GCA_OK;
+    }
+    for (int j = 0; j < n; ++j) ctx->bitmap[j].dirty = true;  // until the whole sequence is enqueued
+    {
+        StageTimer timer(ctx, GCA_STAGE_VOXEL);
+        GCA_TRY(voxel_launch<kMaxJobs>(ctx->stream, vj, n, wide));
+    }
+    for (int j = 0; j < n; ++j) {
+        ctx->bitmap[j].dirty = false;
+        cloud_points_changed(out[j]);
+    }
+    return GCA_OK;
 }
 
 int32_t launch_voxel_planned(gca_ctx ctx, gca_cloud in, float voxel, gca_cloud out, double max_bits, uint32_t *err,
@@ -604,15 +660,15 @@ int32_t launch_voxel_levels(gca_ctx launch, const VoxelLevelJob *jobs, int nj)
     for (int j = 0; j < nj; ++j) {
         const VoxelLevelJob &J = jobs[j];
         GCA_TRY(cloud_reserve(J.out, std::max<int64_t>(J.in->cap, 1)));
-        GCA_TRY(voxel_prepare(J.ctx, J.in, J.voxel, J.out, J.in->cap, words[j], J.max_bits, J.err, &J.gc, wide, &vj[j]));
-        J.ctx->bitmap_dirty = true;
+        GCA_TRY(voxel_prepare(J.ctx, J.in, J.voxel, J.out, J.in->cap, words[j], J.max_bits, J.err, &J.gc, wide, 0, &vj[j]));
+        J.ctx->bitmap[0].dirty = true;
     }
     {
         StageTimer timer(launch, GCA_STAGE_VOXEL);
         GCA_TRY(voxel_launch<kMaxJobs>(launch->stream, vj, nj, wide));
     }
     for (int j = 0; j < nj; ++j) {
-        jobs[j].ctx->bitmap_dirty = false;
+        jobs[j].ctx->bitmap[0].dirty = false;
         cloud_points_changed(jobs[j].out);
     }
     return GCA_OK;

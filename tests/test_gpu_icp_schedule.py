@@ -72,3 +72,43 @@ def test_multiscale_equals_its_steps(normal_r, max_nn, grad_r, grad_nn):
         assert (rep.iterations, rep.n_correspondences, rep.rmse) == (one[0][0].iterations, one[0][0].n_correspondences,
                                                                      one[0][0].rmse)
     np.testing.assert_array_equal(T, pose)
+
+
+@pytest.mark.parametrize("n,sizes,kinds,tune", [
+    (20000, (0.04,), "j", {}),                                    # one level: no shared launch
+    (20000, (0.08, 0.03), "jj", {}),                              # the smallest one
+    (20000, (0.09, 0.06, 0.04, 0.02), "jjjj", {}),                # a full one
+    (20000, (0.1, 0.08, 0.06, 0.05, 0.03), "jjjjj", {}),          # ... and one level over
+    (20000, (0.08, 0.05, 0.03), "jsj", {}),                       # a level with walks of its own between
+    (20000, (0.08, 0.05, 0.03), "sjj", {"grid_cell": 6}),
+    (20000, (0.08, 0.05, 0.03), "jjj", {"voxel": 2}),             # the sorted path, size by size
+    (20000, (0.08, 0.05, 0.00001), "jjj", {}),                    # a lattice beyond the bitmap
+    (1, (0.08, 0.05, 0.03), "jjj", {}),
+    (40, (0.3, 0.1), "jj", {}),
+])
+def test_multiscale_levels_built_together_equal_single_ones(n, sizes, kinds, tune):
+    import cuda_3d_amd as g
+
+    ctx = g.default_context()
+    src, tgt = _clouds(g, n, 9)
+    radii = [max(v, 0.02) for v in sizes]
+    levels = [g.level_params(v, normal_radius=2.5 * r, normal_max_nn=30, gradient_radius=(2.0 if k == "j" else 3.0) * r,
+                             gradient_max_nn=0, icp=g.icp_params(4, 2.5 * r)) for v, r, k in zip(sizes, radii, kinds)]
+    old = ctx.get_tuning()
+    try:
+        ctx.set_tuning(**tune)
+        for _ in range(2):  # the second call reuses the first one's scratch
+            T, reps = g.multiscale_icp(src, tgt, levels)
+            pose = np.eye(4)
+            for v, r, k, rep in zip(sizes, radii, kinds, reps):
+                s, t = src.voxel_grid_down_sample(v), tgt.voxel_grid_down_sample(v)
+                t.estimate_normals(2.5 * r, 30)
+                t.compute_color_gradient((2.0 if k == "j" else 3.0) * r, 0)
+                Ts, one = g.batch_multiscale_icp([[s]], [[t]], [g.icp_params(4, 2.5 * r)], pose[None],
+                                                 [(2.0 if k == "j" else 3.0) * r])
+                pose = Ts[0]
+                assert (rep.iterations, rep.n_correspondences, rep.rmse) == (
+                    one[0][0].iterations, one[0][0].n_correspondences, one[0][0].rmse)
+            np.testing.assert_array_equal(T, pose)
+    finally:
+        ctx.set_tuning(**old)
