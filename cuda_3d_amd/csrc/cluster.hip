@@ -12,26 +12,26 @@
 // Here the components come from a lock-free union-find on the device:
 //   1. chain    size[i] = 0; parent[i] = the first point of i's run of consecutive indices whose
 //               neighbours are linked (raster and lattice order put most neighbours side by side),
-//               within the workgroup; a run's first point takes the point before it if linked, so
-//               parents only decrease and the chains stay short: no atomics, no search
+//               within the workgroup; a run's first point takes the point before it if linked: no
+//               atomics, no search
 //   2. pairs    every point and the few before it in cell order, if linked, are joined; snapshot:
 //               each point's root, in cell order, and the most frequent root of a sample (`big`)
 //   3. hook     the points outside the big component link their root with that of every linked
 //               neighbour of another snapshot component.  An edge inside a component is already
 //               there, and one into the big component is seen from its other end, so the bulk of
-//               a scene takes no part.  A root is only ever linked to a smaller one by
-//               compare-and-swap, so every tree's root is its component's lowest index, which is
-//               the reference's seed.  Linked: the radius search's own predicate, squared FP64
+//               a scene takes no part.  Linked: the radius search's own predicate, squared FP64
 //               distance < r^2, and for the residual form the residual gate
 //   4. compress parent[i] = root (a read-only walk, then a store to the point's own entry),
-//               size[root] += 1 (one atomic per wave and root run)
-//   5. cut      only for components above max_cluster_size (listed by k_cc_over): the
+//               size[root] += 1 and low[root] = min(i) (one atomic per wave and root run); lowest:
+//               the component's lowest index, which is the reference's seed, becomes its root
+//   5. cut      only for components above max_cluster_size (listed by k_cc_lowest): the
 //               reference's truncated searches, replayed exactly on the device (k_cc_truncate),
 //               re-root the component's points on the seeds of the pieces it is cut into
 //   6. rank     kept roots (size >= min) are numbered by an exclusive scan in index order
 //   7. label    label[i] = number of its root's cluster, or -1
-// Parent pointers only ever decrease and always name an ancestor, so the path-halving stores in
-// find() may race with the compare-and-swaps without losing a link.
+// A root is only ever linked, by compare-and-swap, under a point of lower rank (cc_rank) that was a
+// root, so links form no cycle; parent pointers always name an ancestor, so the path-halving stores
+// in find() may race with the compare-and-swaps without losing a link.
 //
 // Neighbour lists are visited in the radius search's canonical order, (squared distance,
 // index), where the reference visits them in its grid-cell order; only the pieces of a cut
@@ -53,9 +53,9 @@ namespace {
 
 constexpr int kCcBlock = 256;
 
-// Workgroup scope lets the load hit L1.  A stale parent is still an ancestor and pointers only
-// decrease, so walks on stale values end, and every link is validated by an agent-scope
-// compare-and-swap; each failed one strictly lowers the larger of the two roots.
+// Workgroup scope lets the load hit L1.  A stale parent is still an ancestor and every step goes
+// towards the root, so walks on stale values end, and every link is validated by an agent-scope
+// compare-and-swap; each failed one strictly lowers the rank of the higher of the two roots.
 __device__ __forceinline__ int32_t cc_load(int32_t *p)
 {
     return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
@@ -87,16 +87,25 @@ __device__ __forceinline__ int32_t cc_root(int32_t *parent, int32_t x)
     return x;
 }
 
+// Which of two roots stays one: a mix of the index's bits (a bijection, so never a tie).  By index
+// alone the rows of an image hang under one another one by one, and the walks grow with the image
+// (289k points at 1 cm: pairs and hook 88 + 76 us by index, 38 + 44 by rank).
+__device__ __forceinline__ uint32_t cc_rank(int32_t x)
+{
+    const uint32_t m = (uint32_t)x * 2654435769u;
+    return m ^ m >> 15;
+}
+
 // Links the trees of u and v (any nodes of them; the point's own root is passed in).
 __device__ __forceinline__ void cc_union(int32_t *parent, int32_t u, int32_t v)
 {
     while (u != v) {
-        if (u > v) {
+        if (cc_rank(u) > cc_rank(v)) {
             const int32_t t = u;
             u = v;
             v = t;
         }
-        int32_t expect = v;  // link the larger root under the smaller one
+        int32_t expect = v;  // link the root of higher rank under the other one
         if (__hip_atomic_compare_exchange_strong(parent + v, &expect, u, __ATOMIC_RELAXED, __ATOMIC_RELAXED,
                                                  __HIP_MEMORY_SCOPE_AGENT))
             return;
@@ -120,7 +129,7 @@ constexpr int kCcWide = 1024;
 __global__ __launch_bounds__(kCcWide) void k_cc_chain(const CloudHdr *__restrict__ h, const float4 *__restrict__ xyzi,
                                                      const float *__restrict__ res, double r2,
                                                      int32_t *__restrict__ parent, uint32_t *__restrict__ size,
-                                                     uint32_t *__restrict__ oversized)
+                                                     int32_t *__restrict__ low, uint32_t *__restrict__ oversized)
 {
     __shared__ int32_t last[kCcWide / kWave];  // per wavefront: its last run's first point, -1 if it has none
     const int n = h->n;
@@ -142,6 +151,7 @@ __global__ __launch_bounds__(kCcWide) void k_cc_chain(const CloudHdr *__restrict
     for (int v = w; head < 0;) head = last[--v];  // the workgroup's first point starts a run
     parent[i] = threadIdx.x == 0 && linked ? i - 1 : head;
     size[i] = 0;
+    low[i] = INT_MAX;
 }
 
 __device__ __forceinline__ void cc_link(int32_t *parent, int32_t &ri, int32_t j)
@@ -224,11 +234,10 @@ __global__ __launch_bounds__(kCcSample) void k_cc_big(const CloudHdr *__restrict
 
 // Hook: kCcLanes lanes per point outside the big component (points in cell order), each lane a share of the point's
 // candidates from the 27 cells around it.  Between two points outside the big component the later
-// one in cell order takes the edge; the components, and their roots (each root is its component's
-// lowest original index), do not depend on which end links it.  The whole labelling is bound by the
-// union-find's dependent loads and contended compare-and-swaps: 92k points of a 424x240 frame at
-// 2 cm 101 us plain and 183 us gated, where hooking every edge of every point took 270 us for either
-// (the hook itself 73 -> 58 us on average once the loads of a walk go out together).
+// one in cell order takes the edge; the components do not depend on which end links it.  The whole
+// labelling is bound by the union-find's dependent loads and contended compare-and-swaps: 92k points of
+// a 424x240 frame at 2 cm 91 us plain and 171 us gated, where hooking every edge of every point took
+// 270 us for either; 289k points of a 640x480 frame at 1 cm 121 us (568 every edge).
 constexpr int kCcLanes = 8;
 constexpr int kCcUnroll = 4;
 
@@ -274,15 +283,17 @@ __global__ __launch_bounds__(kCcBlock) void k_cc_hook(const CloudHdr *__restrict
 // The big component's points are counted per workgroup (its count takes one atomic a workgroup
 // instead of one a wavefront: same-address atomics queue), the others' per wavefront and root.
 __global__ __launch_bounds__(kCcWide) void k_cc_compress(const CloudHdr *__restrict__ h, int32_t *parent,
-                                                        uint32_t *__restrict__ size, const int32_t *__restrict__ big_p)
+                                                        uint32_t *__restrict__ size, int32_t *__restrict__ low,
+                                                        const int32_t *__restrict__ big_p)
 {
     __shared__ uint32_t s_count;
-    __shared__ int32_t s_big;
+    __shared__ int32_t s_big, s_low;
     const int n = h->n;
     const int i = blockIdx.x * kCcWide + threadIdx.x;
     const bool on = i < n;
     if (threadIdx.x == 0) {
         s_count = 0u;
+        s_low = INT_MAX;
         s_big = n > 0 ? cc_root(parent, *big_p) : -1;
     }
     const int32_t r = on ? cc_root(parent, i) : -1;
@@ -290,36 +301,57 @@ __global__ __launch_bounds__(kCcWide) void k_cc_compress(const CloudHdr *__restr
     const int32_t big = s_big;
     if (on) __hip_atomic_store(parent + i, r, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     const uint64_t in_big = __ballot(on && r == big);
-    if (lane_id() == 0 && in_big) atomicAdd(&s_count, (uint32_t)__popcll(in_big));
-    // lanes sharing a root add once: the lowest such lane adds the run's count
+    if (lane_id() == 0 && in_big) {
+        atomicAdd(&s_count, (uint32_t)__popcll(in_big));
+        atomicMin(&s_low, i + __ffsll((long long)in_big) - 1);
+    }
+    // lanes sharing a root add once: the lowest such lane, whose index is their lowest
     uint64_t pending = __ballot(on && r != big);
     while (pending) {
         const int leader = __ffsll((long long)pending) - 1;
         const int32_t lr = __shfl(r, leader);
         const uint64_t same = __ballot(on && r == lr);
-        if (lane_id() == leader) atomicAdd(size + lr, (uint32_t)__popcll(same));
+        if (lane_id() == leader) {
+            atomicAdd(size + lr, (uint32_t)__popcll(same));
+            atomicMin(low + lr, i);
+        }
         pending &= ~same;
     }
     __syncthreads();
-    if (threadIdx.x == 0 && s_count) atomicAdd(size + big, s_count);
+    if (threadIdx.x == 0 && s_count) {
+        atomicAdd(size + big, s_count);
+        atomicMin(low + big, s_low);
+    }
 }
 
-// Components above max_size: one job each (root, size) for the truncated searches; *n_jobs counts
-// them (the jobs' order does not matter: each cut is independent of the others).
 struct CutJob {
     int32_t root, size, base;  // base: the job's region of the queue buffer (set on the host)
     int32_t pad;
 };
 
-__global__ __launch_bounds__(kCcBlock) void k_cc_over(const CloudHdr *__restrict__ h, const int32_t *__restrict__ parent,
-                                                     const uint32_t *__restrict__ size, uint32_t max_size,
-                                                     CutJob *__restrict__ jobs, uint32_t *__restrict__ n_jobs)
+// Each component takes its lowest index as its root: every point's entry (read and written by its
+// own thread only) and the size, which moves from the union-find's root.  Components above max_size:
+// one job each (root, size) for the truncated searches; *n_jobs counts them (the jobs' order does not
+// matter: each cut is independent of the others).
+__global__ __launch_bounds__(kCcBlock) void k_cc_lowest(const CloudHdr *__restrict__ h, int32_t *__restrict__ parent,
+                                                       uint32_t *__restrict__ size, const int32_t *__restrict__ low,
+                                                       uint32_t max_size, CutJob *__restrict__ jobs,
+                                                       uint32_t *__restrict__ n_jobs)
 {
     const int n = h->n;
     const int i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= n || parent[i] != i || size[i] <= max_size) return;
+    if (i >= n) return;
+    const int32_t r = parent[i], m = low[r];
+    parent[i] = m;
+    if (r != i) return;
+    const uint32_t sz = size[i];
+    if (m != i) {
+        size[m] = sz;
+        size[i] = 0;
+    }
+    if (sz <= max_size) return;
     const uint32_t k = atomicAdd(n_jobs, 1u);
-    jobs[k] = CutJob{i, (int32_t)size[i], 0, 0};
+    jobs[k] = CutJob{m, (int32_t)sz, 0, 0};
 }
 
 // Claim words of the truncated searches: kUnvisited, kVisited, or the key (queue position + 1,
@@ -534,16 +566,18 @@ int32_t launch_euclidean_clustering(gca_ctx ctx, gca_cloud c, float tolerance, u
     int32_t *snap = (int32_t *)ctx_scratch(ctx, 11, sizeof(int32_t) * (size_t)c->cap, false);
     float *sres = res ? (float *)ctx_scratch(ctx, 12, sizeof(float) * (size_t)c->cap, false) : nullptr;
     int32_t *big = (int32_t *)ctx_scratch(ctx, 46, 256, false);
-    if (!snap || !big || (res && !sres)) return GCA_ERR_OUT_OF_MEMORY;
+    int32_t *low = (int32_t *)ctx_scratch(ctx, 9, sizeof(int32_t) * (size_t)c->cap, false);
+    if (!snap || !big || !low || (res && !sres)) return GCA_ERR_OUT_OF_MEMORY;
     const double r2 = (double)tolerance * (double)tolerance;
     const dim3 wide((unsigned)std::max<int64_t>(1, (c->cap + kCcWide - 1) / kCcWide));
-    hipLaunchKernelGGL(k_cc_chain, wide, dim3(kCcWide), 0, ctx->stream, c->hdr, c->xyzi, res, r2, label, size, counts_dev + 1);
+    hipLaunchKernelGGL(k_cc_chain, wide, dim3(kCcWide), 0, ctx->stream, c->hdr, c->xyzi, res, r2, label, size, low,
+                       counts_dev + 1);
     // Every second point and its predecessor connect the rows that a cell holds; the residual gate
     // lets about a third of the neighbours through, so it takes more pairs before a scene's bulk
-    // holds together.  Pairs / hook of a 424x240 frame at 2 cm: 23 / 39 us plain (every fourth: 19 /
-    // 54), gated 55 / 89 us with four predecessors of every point (two of every point 40 / 163,
-    // six 139 / 81).
-    const int step = res ? 1 : 2, back = res ? 4 : 1;
+    // holds together.  Pairs / hook of a 424x240 frame at 2 cm: 19 / 36 us plain (every fourth: 16 /
+    // 53), gated 51 / 79 us with three predecessors of every point (two 38 / 118, four 70 / 67); at
+    // 640x480 gated 93 / 276 (two 73 / 387, four 120 / 236).
+    const int step = res ? 1 : 2, back = res ? 3 : 1;
     const dim3 grid_pairs((unsigned)std::max<int64_t>(1, (c->cap / step * back + back + kCcBlock - 1) / kCcBlock));
     hipLaunchKernelGGL(k_cc_pairs, grid_pairs, block, 0, ctx->stream, c->hdr, G.sxyzi, G.order, res, r2, step, back, label);
     hipLaunchKernelGGL(k_cc_snapshot, grid, block, 0, ctx->stream, c->hdr, G.order, res, label, snap, sres);
@@ -551,8 +585,10 @@ int32_t launch_euclidean_clustering(gca_ctx ctx, gca_cloud c, float tolerance, u
     const dim3 grid_hook((unsigned)std::max<int64_t>(1, (c->cap * kCcLanes + kCcBlock - 1) / kCcBlock));
     hipLaunchKernelGGL(k_cc_hook, grid_hook, block, 0, ctx->stream, c->hdr, G.desc, G.start, G.sxyzi, G.order,
                        (const int32_t *)snap, (const float *)sres, (const int32_t *)big, label);
-    hipLaunchKernelGGL(k_cc_compress, wide, dim3(kCcWide), 0, ctx->stream, c->hdr, label, size, (const int32_t *)big);
-    hipLaunchKernelGGL(k_cc_over, grid, block, 0, ctx->stream, c->hdr, label, size, max_size, jobs, counts_dev + 1);
+    hipLaunchKernelGGL(k_cc_compress, wide, dim3(kCcWide), 0, ctx->stream, c->hdr, label, size, low,
+                       (const int32_t *)big);
+    hipLaunchKernelGGL(k_cc_lowest, grid, block, 0, ctx->stream, c->hdr, label, size, (const int32_t *)low, max_size, jobs,
+                       counts_dev + 1);
     GCA_HIP(hipGetLastError());
     GCA_HIP(hipMemcpyAsync(ctx->pinned, counts_dev + 1, sizeof(uint32_t), hipMemcpyDeviceToHost, ctx->stream));
     GCA_HIP(hipStreamSynchronize(ctx->stream));

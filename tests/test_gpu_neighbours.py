@@ -140,3 +140,28 @@ def test_components(ctx, kind, n, r):
             assert len(got) == len(want)
             for a, b in zip(got, want):
                 np.testing.assert_array_equal(a, np.sort(b))
+
+
+@pytest.mark.parametrize("n,reverse,mx", [(1, False, 0), (63, True, 0), (1025, False, 0), (1025, True, 0),
+                                          (6000, None, 0), (6000, None, 40)])
+def test_clusters_are_numbered_by_their_lowest_point(ctx, n, reverse, mx):
+    """Long chains in ascending, descending and shuffled order: the union-find's root is any of a
+    component's points, the seed its lowest (and a capped search starts there)."""
+    import cuda_3d_amd as g
+    import oracle as O
+
+    r = np.random.default_rng(n)
+    k = np.arange(n)
+    x = np.stack([0.009 * (k // 5), 0.1 * (k % 5), np.ones(n)], 1).astype(np.float32)  # five chains side by side
+    x = x[::-1].copy() if reverse else x if reverse is False else x[r.permutation(n)]
+    pc = g.PointCloud.from_numpy(x, np.zeros_like(x), ctx=ctx)
+    pc.set_normals(np.zeros_like(x))
+    xyzi = pc.download_xyzi()
+    res = (0.001 * r.integers(0, 4, n)).astype(np.float32)
+    for residual in (None, res):
+        want = O.euclidean_clustering(xyzi, 0.01, 1, mx or n, residual=residual)
+        got = (pc.euclidean_clustering(0.01, 1, mx or n) if residual is None else
+               pc.icp_residual_segmentation(0.01, residual, 1, mx or n))
+        assert len(got) == len(want)
+        for a, b in zip(got, want):
+            np.testing.assert_array_equal(a, np.sort(b))
