@@ -1,0 +1,59 @@
+"""libgca.so's host code on a stand-in runtime (cpp/host_runtime.cpp): sizes it lays out and what it
+does where memory ends.  No GPU, and the kernels do nothing, so device-made counts are zero."""
+import os
+import subprocess
+import sys
+
+import pytest
+
+ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
+
+PRELUDE = """
+import sys
+sys.modules["torch"] = None  # it would bring a HIP runtime of its own
+import ctypes as C
+import numpy as np
+import cuda_3d_amd as g
+from cuda_3d_amd import _lib as L
+rt = C.CDLL(sys.argv[1])
+rt.host_runtime_budget.argtypes = [C.c_size_t]
+rt.host_runtime_live.restype = C.c_size_t
+MiB = 1 << 20
+ctx = g.default_context()
+def cloud(n, seed=0):
+    r = np.random.default_rng(seed)
+    return g.PointCloud.from_numpy(r.uniform(-1, 1, (n, 3)), r.uniform(0, 1, (n, 3)))
+"""
+
+
+@pytest.fixture(scope="module")
+def runtime(tmp_path_factory):
+    so = tmp_path_factory.mktemp("rt") / "libhost_runtime.so"
+    rocm = os.environ.get("ROCM_PATH", "/opt/rocm")
+    subprocess.run(["g++", "-O1", "-std=c++17", "-shared", "-fPIC", "-D__HIP_PLATFORM_AMD__", "-I", f"{rocm}/include",
+                    os.path.join(ROOT, "tests", "cpp", "host_runtime.cpp"), "-o", str(so)], check=True)
+    return str(so)
+
+
+def _run(runtime, body):
+    preload = [runtime] + [p for p in [os.environ.get("LD_PRELOAD")] if p]
+    r = subprocess.run([sys.executable, "-c", PRELUDE + body, runtime], cwd=ROOT, capture_output=True, text=True, timeout=300,
+                       env=dict(os.environ, LD_PRELOAD=":".join(preload)))
+    assert r.returncode == 0, r.stdout + r.stderr
+    return r.stdout
+
+
+def test_grid_of_an_empty_cloud_is_one_cell(runtime):
+    """An empty cloud's bounds are the fold's start values, lowest above highest."""
+    out = _run(runtime, """
+for q in (0, 6):
+    ctx.set_tuning(grid_cell=q)
+    for radius in (1e-3, 0.05, 1.0, 1e30):
+        e, cells = g.PointCloud(), np.zeros(3, np.int32)
+        dims, edge = np.zeros(3, np.int32), C.c_float()
+        L.check(L.lib.gca_grid_cells(ctx.handle, e.handle, radius, cells.ctypes.data_as(C.c_void_p), None, C.byref(edge),
+                                     dims.ctypes.data_as(C.c_void_p)), "gca_grid_cells")
+        print(q, radius, dims.tolist())
+        assert dims.tolist() == [1, 1, 1] and edge.value == np.float32(radius)
+""")
+    assert out.count("[1, 1, 1]") == 8
