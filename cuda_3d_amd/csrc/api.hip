@@ -667,8 +667,9 @@ void grid_params(const float bmin[3], const float bmax[3], float r, GridDesc *d,
         double total = 1.0;
         for (int a = 0; a < 3; ++a) {
             float q = (top[a] - d->origin[a]) / s;
-            // (q < 0: an empty cloud, whose lowest bound lies above its highest)
-            d->dims[a] = (q < 2.0e9f) ? (q > 0.0f ? (int32_t)q : 0) + 1 : 2000000000;
+            // (q < 0: an empty cloud, whose lowest bound lies above its highest; not a number: infinite
+            // bounds, once the edge is infinite too)
+            d->dims[a] = q >= 2.0e9f ? 2000000000 : (q > 0.0f ? (int32_t)q : 0) + 1;
             total *= (double)d->dims[a];
         }
         if (total <= (double)kGridCellCap) break;

@@ -1,5 +1,5 @@
 """Neighbour calls and registrations with an empty cloud on either side: no neighbours, no points, the
-initial pose."""
+initial pose; and with points that no grid holds."""
 import numpy as np
 import pytest
 
@@ -44,3 +44,18 @@ def test_registration(ctx, levels):
         T, reps = g.multiscale_icp(src, tgt, lv, T0)
         np.testing.assert_array_equal(T, T0)
         assert all(r.n_correspondences == 0 for r in reps)
+
+
+@pytest.mark.parametrize("far", [[np.inf, 0, 0], [0, -np.inf, 0], [np.inf, -np.inf, np.inf], [3e38, 0, -3e38]])
+def test_points_beyond_any_grid(ctx, far):
+    """A cloud with a point at (or near) infinity: one cell holds everything, the answers are the others'."""
+    import cuda_3d_amd as g
+
+    _, some = _clouds(ctx)
+    x = some.download()[0]
+    with_far = np.concatenate([x[:100], np.float32([far]), x[100:]])
+    ref = g.PointCloud.from_numpy(with_far, np.full_like(with_far, 0.5), ctx=ctx)
+    want = g.PointCloud.nn_search(some, some, 0.05)
+    np.testing.assert_array_equal(g.PointCloud.nn_search(some, ref, 0.05), want + (want >= 100))
+    want = some.radius_outlier_removal(0.05, 1).download()[0]
+    np.testing.assert_array_equal(ref.radius_outlier_removal(0.05, 1).download()[0], want)

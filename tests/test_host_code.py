@@ -37,7 +37,7 @@ def runtime(tmp_path_factory):
 
 def _run(runtime, body):
     preload = [runtime] + [p for p in [os.environ.get("LD_PRELOAD")] if p]
-    r = subprocess.run([sys.executable, "-c", PRELUDE + body, runtime], cwd=ROOT, capture_output=True, text=True, timeout=300,
+    r = subprocess.run([sys.executable, "-c", PRELUDE + body, runtime], cwd=ROOT, capture_output=True, text=True, timeout=60,
                        env=dict(os.environ, LD_PRELOAD=":".join(preload)))
     assert r.returncode == 0, r.stdout + r.stderr
     return r.stdout
@@ -57,3 +57,22 @@ for q in (0, 6):
         assert dims.tolist() == [1, 1, 1] and edge.value == np.float32(radius)
 """)
     assert out.count("[1, 1, 1]") == 8
+
+
+@pytest.mark.parametrize("lowest,highest", [(0.0, float("inf")), (float("-inf"), 1.0), (float("-inf"), float("inf")),
+                                            (-3e38, 3e38)])
+def test_grid_of_a_cloud_with_infinite_bounds_ends(runtime, lowest, highest):
+    """The cell edge doubles until the cells are few enough, or it is infinite."""
+    _run(runtime, f"""
+pc = cloud(4)
+hdr = (C.c_uint32 * 7).from_address(pc.device_arrays()[4])  # count, lowest and highest as ordered keys
+def key(f):
+    u = int(np.float32(f).view(np.uint32))
+    return ~u & 0xffffffff if u >> 31 else u | 0x80000000
+lowest, highest = float("{lowest}"), float("{highest}")
+hdr[1:4], hdr[4:7] = [key(lowest)] * 3, [key(highest)] * 3
+cells, dims = np.zeros((4, 3), np.int32), np.zeros(3, np.int32)
+L.check(L.lib.gca_grid_cells(ctx.handle, pc.handle, 0.05, cells.ctypes.data_as(C.c_void_p), None, None,
+                             dims.ctypes.data_as(C.c_void_p)), "gca_grid_cells")
+assert (dims >= 1).all() and dims.astype(float).prod() <= 1 << 25
+""")
