@@ -753,7 +753,8 @@ __device__ __noinline__ void icp_finish(IcpState *states, unsigned long long *op
                 __hip_atomic_store(&states[f_next].q[t].w, 0ull, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
         }
     }
-    // A workgroup that sees an open word before the claim words only loses a claim.
+    // The open word may land before the claim words or after them: a workgroup that sees it first
+    // only loses a claim, and one that claims first waits for it (k_icp_persist).
     if (t == kSubQ) {
         const unsigned long long w =
             f_done ? (unsigned long long)kEpochDone << 32 : open_word(epoch + 1, nvb);
@@ -790,9 +791,12 @@ __device__ __forceinline__ void unit_commit(const PairDesc &P, IcpState *states,
 // states at a time), pick the first state with unclaimed units in round-robin order from the state
 // last served and, in it, the sub-queue nearest to the workgroup's own, claim a unit with one
 // atomic, run it.  The claim of a sub-queue's last unit takes its bit out of the open word before
-// the unit runs, so before the epoch can end.  A workgroup only waits (sleep + re-poll)
-// when every unit of every open epoch is claimed, i.e. held by running workgroups, so progress
-// never depends on how many workgroups are resident.  Exits when every state is done.
+// the unit runs, so before the epoch can end.  A claim in a later epoch than the scan saw may come
+// before that epoch's open word: it waits for the word (its finisher's next store) first, or the
+// word would land with the bit of an empty sub-queue in it, which no claim takes out any more and
+// which workgroups would go on trying for the rest of the epoch.  A workgroup only waits (sleep +
+// re-poll) when every unit of every open epoch is claimed, i.e. held by running workgroups, so
+// progress never depends on how many workgroups are resident.  Exits when every state is done.
 // (Reading the claim words themselves, 64 of them at a time, took a workgroup without work 24
 // dependent reads for the 192 states of 64 pairs on three levels: a lone state's iteration then
 // lasted 57 us, most of it the wait until somebody came past its open epoch again.  Claiming first
@@ -914,8 +918,16 @@ __global__ __launch_bounds__(kIcpBlock) GCA_PERSIST_OCCUPANCY void k_icp_persist
             const bool ok = e < kEpochWait && c < subq_units(refresh ? s_nvb : st->nvb, x);
             s_vb = ok ? subq_unit(refresh ? s_nvb : st->nvb, x, (int)c) : -1;
             s_epoch = e;
-            if (ok && c + 1 == subq_units(refresh ? s_nvb : st->nvb, x))
+            if (ok && c + 1 == subq_units(refresh ? s_nvb : st->nvb, x)) {
+                // (epoch e lasts until this unit is done, so the word stays at e once it is there)
+                for (uint32_t spins = 0; e != s_pick_epoch && spins <= kSpinLimit; ++spins) {
+                    const unsigned long long w = __hip_atomic_load(&open[p], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+                    if ((uint32_t)(w >> 32) == e) break;
+                    __builtin_amdgcn_s_sleep(1);
+                    if (spins == kSpinLimit) atomicOr(err, 1u);
+                }
                 __hip_atomic_fetch_and(&open[p], ~(1ull << x), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            }
             if (ok && e == 0 && c == 0 && x == 0) st->t_start = wall_clock64();  // unit 0 of the first epoch
         } else if (threadIdx.x >= kWave && threadIdx.x < kWave + 12) {
             T[threadIdx.x - kWave] = load_coherent(&st->T[threadIdx.x - kWave]);
@@ -923,7 +935,13 @@ __global__ __launch_bounds__(kIcpBlock) GCA_PERSIST_OCCUPANCY void k_icp_persist
         __syncthreads();
         const int vb = s_vb;
         const uint32_t epoch = s_epoch;
-        if (vb < 0) continue;  // lost the race for the last unit: poll again
+        if (vb < 0) {  // lost the race for the last unit: poll again (a bounded number of times in a row)
+            if (++idle > kSpinLimit) {
+                if (threadIdx.x == 0) atomicOr(err, 1u);
+                break;
+            }
+            continue;
+        }
         if (epoch != s_pick_epoch) {
             if (threadIdx.x < 12) T[threadIdx.x] = load_coherent(&st->T[threadIdx.x]);
             __syncthreads();

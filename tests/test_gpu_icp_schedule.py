@@ -112,3 +112,30 @@ def test_multiscale_levels_built_together_equal_single_ones(n, sizes, kinds, tun
             np.testing.assert_array_equal(T, pose)
     finally:
         ctx.set_tuning(**old)
+
+
+@pytest.mark.parametrize("blocks", [2, 3, 5, 7, 9])
+@pytest.mark.parametrize("pairs,levels,units", [(1, 2, 3), (3, 3, 8), (12, 1, 40)])
+def test_fewer_workgroups_than_sub_queues(blocks, pairs, levels, units):
+    """Sub-queues that no workgroup has as its own, through many epochs: a workgroup that comes late to
+    one is not held up there."""
+    import cuda_3d_amd as g
+
+    ctx = g.default_context()
+    made = [_clouds(g, n, n) for n in (300, 1500)]
+    src = [[made[(k + l) % 2][0] for l in range(levels)] for k in range(pairs)]
+    tgt = [[made[(k + l) % 2][1] for l in range(levels)] for k in range(pairs)]
+    params = [g.icp_params(40, 0.1, conv_rotation=-1.0)] * levels  # never converged: every iteration runs
+    T0 = np.tile(np.eye(4), (pairs, 1, 1))
+    got = {}
+    try:
+        ctx.set_tuning(icp_persist_blocks=blocks, icp_max_units=units, icp_lanes_batch=16, icp_lanes_small=16)
+        for launch in (1, 2):
+            ctx.set_tuning(icp_launch=launch)
+            T, reps = g.batch_multiscale_icp(src, tgt, params, T0, [0.1] * levels)
+            got[launch] = T, [[(r.iterations, r.n_correspondences, r.rmse) for r in row] for row in reps]
+    finally:
+        ctx.set_tuning(icp_launch=0, icp_persist_blocks=0, icp_max_units=0, icp_lanes_batch=0, icp_lanes_small=0)
+    np.testing.assert_array_equal(got[1][0], got[2][0])
+    assert got[1][1] == got[2][1]
+    assert all(r[0] == 40 for row in got[1][1] for r in row)
