@@ -184,7 +184,7 @@ try {
         P.used.reserve((P.slabs.size() + 1) * HdrPool::kPer);
         HdrSlot *d = nullptr;
         CloudHdr *h = nullptr;
-        int32_t st = dev_alloc(ctx, (void **)&d, sizeof(HdrSlot) * HdrPool::kPer);
+        int32_t st = dev_alloc(ctx, (void **)&d, (sizeof(HdrSlot) + sizeof(BoundsWork)) * HdrPool::kPer);
         if (st == GCA_OK && hipHostMalloc((void **)&h, sizeof(CloudHdr) * HdrPool::kPer, hipHostMallocDefault) != hipSuccess)
             st = GCA_ERR_OUT_OF_MEMORY;
         if (st == GCA_OK &&
@@ -198,7 +198,8 @@ try {
         }
         P.slabs.push_back(d);
         P.host_slabs.push_back(h);
-        for (int k = 0; k < HdrPool::kPer; ++k) P.ready.push_back(HdrRef{d + k, h + k});
+        BoundsWork *b = (BoundsWork *)(d + HdrPool::kPer);
+        for (int k = 0; k < HdrPool::kPer; ++k) P.ready.push_back(HdrRef{d + k, h + k, b + k});
     }
     *out = P.ready.back();
     P.ready.pop_back();
@@ -284,12 +285,8 @@ void ctx_lanes_release(gca_ctx ctx)
 // six atomics each on the header's words took 17 us after an initialising launch of 2.5, and letting
 // the last workgroup fold cost the transform 9 us (every workgroup's release writes back what the
 // kernel has in L2).
-constexpr int kBoundsThreads = 1024, kBoundsBlocks = 256;
+constexpr int kBoundsThreads = 1024;
 constexpr int kBoundsBatch = 4;  // points in flight per thread
-
-// value a of workgroup b at part[a * kBoundsBlocks + b] (allocated with the ctx: calls that compute
-// bounds may be captured)
-constexpr size_t kBoundsWorkBytes = sizeof(float) * 6 * kBoundsBlocks;
 
 static unsigned bounds_blocks(int64_t cap)
 {
@@ -346,9 +343,10 @@ __global__ __launch_bounds__(6 * kWave) void k_bounds_keys(const float *__restri
     else h->bmax_key[a - 3] = float_to_key(v);
 }
 
-static hipError_t bounds_keys(gca_ctx ctx, unsigned nblk, CloudHdr *h)
+static hipError_t bounds_keys(gca_ctx ctx, unsigned nblk, gca_cloud c)
 {
-    hipLaunchKernelGGL(k_bounds_keys, dim3(1), dim3(6 * kWave), 0, ctx->stream, (const float *)ctx->bounds_work, (int)nblk, h);
+    hipLaunchKernelGGL(k_bounds_keys, dim3(1), dim3(6 * kWave), 0, ctx->stream, (const float *)c->ref.bounds->part, (int)nblk,
+                       c->hdr);
     return hipGetLastError();
 }
 
@@ -636,9 +634,10 @@ void cloud_points_changed(gca_cloud c)
 int32_t launch_bounds(gca_ctx ctx, gca_cloud c)
 {
     const unsigned nb = bounds_blocks(c->cap);
-    hipLaunchKernelGGL(k_bounds, dim3(nb), dim3(kBoundsThreads), 0, ctx->stream, c->xyzi, c->hdr, ctx->bounds_work);
+    hipLaunchKernelGGL(k_bounds, dim3(nb), dim3(kBoundsThreads), 0, ctx->stream, c->xyzi, c->hdr,
+                       c->ref.bounds->part);
     GCA_HIP(hipGetLastError());
-    GCA_HIP(bounds_keys(ctx, nb, c->hdr));
+    GCA_HIP(bounds_keys(ctx, nb, c));
     return GCA_OK;
 }
 
@@ -646,10 +645,10 @@ int32_t launch_transform(gca_ctx ctx, gca_cloud c, const double *T)
 {
     const unsigned nb = bounds_blocks(c->cap);
     hipLaunchKernelGGL(k_transform, dim3(nb), dim3(kBoundsThreads), 0, ctx->stream, c->xyzi, c->nrm, c->grad, c->hdr,
-                       ctx->bounds_work, T[0], T[1], T[2], T[3], T[4], T[5], T[6], T[7], T[8], T[9], T[10], T[11],
+                       c->ref.bounds->part, T[0], T[1], T[2], T[3], T[4], T[5], T[6], T[7], T[8], T[9], T[10], T[11],
                        c->has_normals ? 1 : 0, c->has_gradient ? 1 : 0);
     GCA_HIP(hipGetLastError());
-    GCA_HIP(bounds_keys(ctx, nb, c->hdr));
+    GCA_HIP(bounds_keys(ctx, nb, c));
     return GCA_OK;
 }
 
@@ -782,9 +781,7 @@ int32_t gca_ctx_create(int32_t device, gca_ctx *out)
         hipEventCreate(&c->ev_a) != hipSuccess || hipEventCreate(&c->ev_b) != hipSuccess ||
         hipHostMalloc((void **)&c->dev_err, sizeof(uint32_t), hipHostMallocDefault) != hipSuccess ||
         hipHostMalloc((void **)&c->pinned, sizeof(double) * gca_ctx_s::kPinnedDoubles, hipHostMallocDefault) !=
-            hipSuccess ||
-        hipMalloc((void **)&c->bounds_work, kBoundsWorkBytes) != hipSuccess) {
-        hipFree(c->bounds_work);
+            hipSuccess) {
         if (c->pinned) hipHostFree(c->pinned);
         if (c->dev_err) hipHostFree(c->dev_err);
         if (c->stream) hipStreamDestroy(c->stream);
@@ -812,7 +809,6 @@ int32_t gca_ctx_destroy(gca_ctx c)
     for (void *p : c->hdrs.host_slabs) hipHostFree(p);
     if (c->host_buf) hipHostFree(c->host_buf);
     for (hipEvent_t e : c->prof_pool) hipEventDestroy(e);
-    hipFree(c->bounds_work);
     for (gca_ctx_s::Bitmap &b : c->bitmap) hipFree(b.p);
     hipFree(c->lut);
     hipFree(c->icp_state);
@@ -1182,9 +1178,9 @@ int32_t gca_cloud_append(gca_ctx ctx, gca_cloud dst, gca_cloud src)
     const unsigned nb = bounds_blocks(total);
     hipLaunchKernelGGL(k_cloud_append, dim3(nb), dim3(kBoundsThreads), 0, ctx->stream, from[0], from[1],
                        normals ? from[2] : nullptr, more[0], more[1], more[2], (int)nd, (int)total, cap > dst->cap ? 1 : 0,
-                       to[0], to[1], to[2], dst->hdr, ctx->bounds_work);
+                       to[0], to[1], to[2], dst->hdr, dst->ref.bounds->part);
     hipError_t e = hipGetLastError();
-    if (e == hipSuccess) e = bounds_keys(ctx, nb, dst->hdr);
+    if (e == hipSuccess) e = bounds_keys(ctx, nb, dst);
     const hipError_t es = hipStreamSynchronize(ctx->stream);
     if (e == hipSuccess) e = es;
     if (cap > dst->cap) {

@@ -125,9 +125,17 @@ struct HdrSlot {
     float4 one[4];
     char pad[32];
 };
+// Workgroups' bounds on their way to the header, value a of workgroup b at [a * kBoundsBlocks + b]: a
+// cloud's own, so that calls on different clouds of one ctx share nothing while they are in flight,
+// and allocated with the header, as calls that compute bounds may be captured.
+constexpr int kBoundsBlocks = 256;
+struct BoundsWork {
+    float part[6 * kBoundsBlocks];
+};
 struct HdrRef {
     HdrSlot *dev;
     CloudHdr *host;  // pinned
+    BoundsWork *bounds;
 };
 // Headers by slabs of kPer: ready ones carry an empty cloud's header, used ones are reset together
 // by one launch once kPer / 2 of them have come back.
@@ -157,7 +165,6 @@ struct gca_ctx_s {
     // after the stream has been synchronised
     static constexpr int kPinnedDoubles = 32;
     double *pinned = nullptr;
-    float *bounds_work = nullptr;  // workgroups' bounds on their way to a header
     // pinned host memory for a call's uploads and read-backs, grown on demand (ctx_host_buf); a
     // small read-back into it takes 12 us, into pageable memory 21
     void *host_buf = nullptr;

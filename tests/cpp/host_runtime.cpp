@@ -6,6 +6,7 @@
 #include <cstdlib>
 #include <cstring>
 #include <map>
+#include <string>
 
 namespace {
 std::map<void *, size_t> blocks;
@@ -14,6 +15,8 @@ hipError_t last = hipSuccess;
 dim3 cfg_grid, cfg_block;
 size_t cfg_lds;
 hipStream_t cfg_stream;
+std::map<const void *, std::string> kernels;
+void *bounds_of = nullptr;  // the last k_bounds_keys launch's workgroup bounds
 
 hipError_t alloc(void **p, size_t n)
 {
@@ -29,13 +32,17 @@ hipError_t alloc(void **p, size_t n)
 extern "C" {
 void host_runtime_budget(size_t bytes) { budget = bytes; }
 size_t host_runtime_live() { return live; }
+void *host_runtime_bounds() { return bounds_of; }
 
 void **__hipRegisterFatBinary(const void *)
 {
     static void *handle;
     return &handle;
 }
-void __hipRegisterFunction(void **, const void *, char *, const char *, unsigned, void *, void *, void *, void *, int *) {}
+void __hipRegisterFunction(void **, const void *f, char *, const char *name, unsigned, void *, void *, void *, void *, int *)
+{
+    kernels[f] = name;
+}
 void __hipRegisterVar(void **, void *, char *, char *, int, size_t, int, int) {}
 void __hipUnregisterFatBinary(void **) {}
 hipError_t __hipPushCallConfiguration(dim3 g, dim3 b, size_t lds, hipStream_t s)
@@ -48,7 +55,11 @@ hipError_t __hipPopCallConfiguration(dim3 *g, dim3 *b, size_t *lds, hipStream_t 
     *g = cfg_grid, *b = cfg_block, *lds = cfg_lds, *s = cfg_stream;
     return hipSuccess;
 }
-hipError_t hipLaunchKernel(const void *, dim3, dim3, void **, size_t, hipStream_t) { return hipSuccess; }
+hipError_t hipLaunchKernel(const void *f, dim3, dim3, void **args, size_t, hipStream_t)
+{
+    if (kernels[f].find("k_bounds_keys") != std::string::npos) bounds_of = *(void **)args[0];
+    return hipSuccess;
+}
 
 hipError_t hipGetLastError()
 {

@@ -107,3 +107,36 @@ def test_clouds_of_one_context_on_threads():
     for t in ts:
         t.join()
     assert not bad
+
+
+def test_bounds_of_clouds_on_threads():
+    """Each cloud's bounds are its own while clouds of the same context are made, moved and appended to
+    on other threads."""
+    import cuda_3d_amd as g
+
+    g.default_context()
+    bad = []
+
+    def work(seed):
+        r = np.random.default_rng(seed)
+        T = np.eye(4)
+        T[:3, 3] = 0.5, -0.25, 2.0
+        for k in range(150):
+            n = int(r.integers(1, 9000))
+            x = (r.uniform(-1, 1, (n, 3)) + 10 * seed).astype(np.float32)
+            pc = g.PointCloud.from_numpy(x, np.zeros_like(x))
+            for step in range(3):
+                if step == 1:
+                    pc.transform(T)
+                    x = (x.astype(np.float64) + T[:3, 3]).astype(np.float32)
+                elif step == 2:
+                    pc += pc
+                if not (np.array_equal(pc.get_min_bound(), x.min(0)) and np.array_equal(pc.get_max_bound(), x.max(0))):
+                    bad.append((seed, k, n, step))
+
+    ts = [threading.Thread(target=work, args=(s,)) for s in range(1, 9)]
+    for t in ts:
+        t.start()
+    for t in ts:
+        t.join()
+    assert not bad, (len(bad), bad[:5])

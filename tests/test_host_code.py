@@ -76,3 +76,26 @@ L.check(L.lib.gca_grid_cells(ctx.handle, pc.handle, 0.05, cells.ctypes.data_as(C
                              dims.ctypes.data_as(C.c_void_p)), "gca_grid_cells")
 assert (dims >= 1).all() and dims.astype(float).prod() <= 1 << 25
 """)
+
+
+def test_clouds_do_not_share_the_bounds_in_flight(runtime):
+    """Upload, transform and append fold their workgroups' bounds in a second launch: what the two
+    launches hand over is the cloud's own, whatever is enqueued between them for another cloud."""
+    _run(runtime, """
+rt.host_runtime_bounds.restype = C.c_void_p
+used = []
+T = np.ascontiguousarray(np.eye(4))
+clouds = [cloud(n) for n in (1, 500, 70000)]
+for pc in clouds:
+    mine = set()
+    L.check(L.lib.gca_transform(ctx.handle, pc.handle, T.ctypes.data_as(C.c_void_p)), "gca_transform")
+    mine.add(rt.host_runtime_bounds())
+    L.check(L.lib.gca_cloud_append(ctx.handle, pc.handle, pc.handle), "gca_cloud_append")
+    mine.add(rt.host_runtime_bounds())
+    xyz = np.zeros((3, 3), np.float32)
+    L.check(L.lib.gca_cloud_upload(pc.handle, xyz.ctypes.data_as(C.c_void_p), xyz.ctypes.data_as(C.c_void_p), 3), "upload")
+    mine.add(rt.host_runtime_bounds())
+    assert len(mine) == 1 and None not in mine
+    used += mine
+assert len(set(used)) == len(clouds)
+""")
