@@ -18,6 +18,7 @@ namespace gca {
 
 int32_t hip_status(hipError_t e)
 {
+    (void)hipGetLastError();  // reported here, not by the next launch's check again
     if (e == hipErrorOutOfMemory) return GCA_ERR_OUT_OF_MEMORY;
     return GCA_ERR_DEVICE;
 }
@@ -47,6 +48,24 @@ static void pool_drop(gca_ctx ctx, size_t keep)
     pool_drop_locked(ctx->pool, keep);
 }
 
+// hipMalloc on the current device, tried again without the pool where memory ends.  The runtime keeps
+// a failed call's error until it is asked for, and every launch is followed by that question, so an
+// error that is dealt with here is taken here.
+static hipError_t ctx_malloc(gca_ctx ctx, void **p, size_t bytes)
+{
+    hipError_t e = hipMalloc(p, bytes);
+    if (e == hipErrorOutOfMemory) {
+        (void)hipGetLastError();
+        pool_drop(ctx, 0);
+        e = hipMalloc(p, bytes);
+    }
+    if (e != hipSuccess) {
+        (void)hipGetLastError();
+        *p = nullptr;
+    }
+    return e;
+}
+
 // Steps of an eighth of the power of two below, so at most an eighth of a buffer is slack.
 static size_t pool_class(size_t bytes)
 {
@@ -74,13 +93,8 @@ int32_t dev_alloc(gca_ctx ctx, void **p, size_t bytes)
     int dev = ctx->device;
     GCA_HIP(hipGetDevice(&dev));
     if (dev != ctx->device) GCA_HIP(hipSetDevice(ctx->device));
-    hipError_t e = hipMalloc(p, bytes);
-    if (e == hipErrorOutOfMemory) {
-        pool_drop(ctx, 0);
-        e = hipMalloc(p, bytes);
-    }
+    const hipError_t e = ctx_malloc(ctx, p, bytes);
     if (dev != ctx->device) hipSetDevice(dev);
-    if (e != hipSuccess) *p = nullptr;
     GCA_HIP(e);
     return GCA_OK;
 }
@@ -110,7 +124,7 @@ bool device_idle(gca_ctx ctx)
     if (hipGetDevice(&dev) != hipSuccess) return false;
     if (dev != ctx->device && hipSetDevice(ctx->device) != hipSuccess) return false;
     void *p = nullptr;
-    const bool ok = hipMalloc(&p, 256) == hipSuccess && hipFree(p) == hipSuccess;
+    const bool ok = ctx_malloc(ctx, &p, 256) == hipSuccess && hipFree(p) == hipSuccess;
     if (dev != ctx->device) hipSetDevice(dev);
     return ok;
 }
@@ -126,6 +140,7 @@ void *ctx_host_buf(gca_ctx ctx, size_t bytes)
         ctx->host_buf_bytes = 0;
         const size_t want = (bytes + bytes / 2 + 4095) & ~size_t(4095);
         if (hipHostMalloc(&ctx->host_buf, want, hipHostMallocDefault) != hipSuccess) {
+            (void)hipGetLastError();
             ctx->host_buf = nullptr;
             return nullptr;
         }
@@ -193,6 +208,7 @@ try {
             st = GCA_ERR_DEVICE;
         }
         if (st != GCA_OK) {
+            (void)hipGetLastError();
             hipFree(d);
             return st;
         }
@@ -228,14 +244,7 @@ void *ctx_scratch(gca_ctx ctx, int slot, size_t bytes, bool zeroed)
         size_t want = bytes + bytes / 2;
         want = (want + 255) & ~size_t(255);
         ctx->scratch_bytes[slot] = 0;
-        if (hipMalloc(&ctx->scratch[slot], want) != hipSuccess) {
-            ctx->scratch[slot] = nullptr;
-            pool_drop(ctx, 0);
-            if (hipMalloc(&ctx->scratch[slot], want) != hipSuccess) {
-                ctx->scratch[slot] = nullptr;
-                return nullptr;
-            }
-        }
+        if (ctx_malloc(ctx, &ctx->scratch[slot], want) != hipSuccess) return nullptr;
         ctx->scratch_bytes[slot] = want;
         ctx->scratch_zeroed[slot] = false;
     }

@@ -20,9 +20,17 @@ rt.host_runtime_budget.argtypes = [C.c_size_t]
 rt.host_runtime_live.restype = C.c_size_t
 MiB = 1 << 20
 ctx = g.default_context()
+def key(f):
+    u = int(np.float32(f).view(np.uint32))
+    return ~u & 0xffffffff if u >> 31 else u | 0x80000000
+def bounds(pc, lowest, highest):         # what the kernels would have left
+    hdr = (C.c_uint32 * 7).from_address(pc.device_arrays()[4])
+    hdr[1:4], hdr[4:7] = [key(lowest)] * 3, [key(highest)] * 3
 def cloud(n, seed=0):
     r = np.random.default_rng(seed)
-    return g.PointCloud.from_numpy(r.uniform(-1, 1, (n, 3)), r.uniform(0, 1, (n, 3)))
+    pc = g.PointCloud.from_numpy(r.uniform(-1, 1, (n, 3)), r.uniform(0, 1, (n, 3)))
+    bounds(pc, -1, 1)
+    return pc
 """
 
 
@@ -65,12 +73,7 @@ def test_grid_of_a_cloud_with_infinite_bounds_ends(runtime, lowest, highest):
     """The cell edge doubles until the cells are few enough, or it is infinite."""
     _run(runtime, f"""
 pc = cloud(4)
-hdr = (C.c_uint32 * 7).from_address(pc.device_arrays()[4])  # count, lowest and highest as ordered keys
-def key(f):
-    u = int(np.float32(f).view(np.uint32))
-    return ~u & 0xffffffff if u >> 31 else u | 0x80000000
-lowest, highest = float("{lowest}"), float("{highest}")
-hdr[1:4], hdr[4:7] = [key(lowest)] * 3, [key(highest)] * 3
+bounds(pc, float("{lowest}"), float("{highest}"))
 cells, dims = np.zeros((4, 3), np.int32), np.zeros(3, np.int32)
 L.check(L.lib.gca_grid_cells(ctx.handle, pc.handle, 0.05, cells.ctypes.data_as(C.c_void_p), None, None,
                              dims.ctypes.data_as(C.c_void_p)), "gca_grid_cells")
@@ -98,4 +101,49 @@ for pc in clouds:
     assert len(mine) == 1 and None not in mine
     used += mine
 assert len(set(used)) == len(clouds)
+""")
+
+
+def test_an_allocation_retried_without_the_pool_leaves_no_error(runtime):
+    """The first try fails, the pool goes, the second succeeds: the call does, too, and so does the
+    next one after a call that was refused for good."""
+    _run(runtime, """
+keep, a = cloud(1000), cloud(400_000)
+del a                                    # its arrays are in the pool: 4 of 6.4 MB
+rt.host_runtime_budget(rt.host_runtime_live() + MiB)
+b = cloud(300_000)                       # another size class: no room beside the pool
+assert b.points_number() == 300_000
+try:
+    cloud(2_000_000)
+    raise SystemExit("room for 128 MB?")
+except L.GcaError as e:
+    assert e.status == L.GCA_ERR_OUT_OF_MEMORY
+keep.transform(np.eye(4))
+assert keep.points_number() == 1000
+""")
+
+
+def test_levels_built_one_by_one_where_the_lanes_do_not_fit(runtime):
+    """A multi-scale call that cannot have the scratch of several levels at once still goes through."""
+    _run(runtime, """
+levels = [g.level_params(v, icp=g.icp_params(2, 2.5 * v)) for v in (0.1, 0.06, 0.04)]
+src, tgt = cloud(200_000, 1), cloud(200_000, 2)
+for pc in (src, tgt):
+    for v in (0.1, 0.06, 0.04):
+        pc.voxel_grid_down_sample(v)     # the scratch of one level at a time
+one = rt.host_runtime_live()
+other = g.Context(0)
+tries = []
+for extra in range(0, 200, 5):
+    rt.host_runtime_budget(one + extra * MiB)
+    try:
+        g.multiscale_icp(src, tgt, levels)
+        tries.append(extra)
+        break
+    except L.GcaError as e:
+        assert e.status == L.GCA_ERR_OUT_OF_MEMORY
+rt.host_runtime_budget(1 << 40)
+g.multiscale_icp(src, tgt, levels)       # with all the memory it likes
+print("one level at a time", one / MiB, "succeeds with", tries, "more; together takes", (rt.host_runtime_live() - one) / MiB)
+assert tries and tries[0] <= 150
 """)
