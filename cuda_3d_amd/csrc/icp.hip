@@ -2294,7 +2294,11 @@ static int32_t build_targets(gca_ctx ctx, const gca_level_params *levels, int n,
     NormalsLevelJob jobs[kMaxJobs];
     gca_cloud cl[kMaxJobs];
     float r[kMaxJobs];
-    int nj = 0;
+    int at[kMaxJobs], nj = 0;
+    auto by_itself = [&](int l) -> int32_t {
+        GCA_TRY(gca_estimate_normals(ctx, ct[l], levels[l].normal_radius, levels[l].normal_max_nn));
+        return gca_compute_color_gradient(ctx, ct[l], levels[l].gradient_radius, levels[l].gradient_max_nn);
+    };
     for (int l = 0; l < n; ++l) {
         const gca_level_params &L = levels[l];
         gca_cloud t = ct[l];
@@ -2304,11 +2308,11 @@ static int32_t build_targets(gca_ctx ctx, const gca_level_params *levels, int n,
         if (joint) {
             cl[nj] = t;
             r[nj] = L.normal_radius;
+            at[nj] = l;
             jobs[nj] = NormalsLevelJob{ctx, t, L.normal_radius, L.normal_max_nn, L.gradient_radius, nj, t->host_hdr.n};
             ++nj;
         } else {
-            GCA_TRY(gca_estimate_normals(ctx, t, L.normal_radius, L.normal_max_nn));
-            GCA_TRY(gca_compute_color_gradient(ctx, t, L.gradient_radius, L.gradient_max_nn));
+            GCA_TRY(by_itself(l));
         }
         if (nj == 0 || (nj < kMaxJobs && l + 1 < n)) continue;
         int32_t st = GCA_OK;
@@ -2316,16 +2320,17 @@ static int32_t build_targets(gca_ctx ctx, const gca_level_params *levels, int n,
             st = grid_build_levels(ctx, cl, r, nj);
             if (st == GCA_OK) st = launch_normals_gradient_levels(ctx, jobs, nj);
             if (st == GCA_ERR_OUT_OF_MEMORY) ctx_lanes_release(ctx);
+        } else {
+            st = grid_build(ctx, cl[0], r[0]);
+            if (st == GCA_OK)
+                st = launch_normals_gradient(ctx, cl[0], r[0], jobs[0].max_nn, jobs[0].gradient_radius, true);
         }
-        if (nj == 1 || st == GCA_ERR_OUT_OF_MEMORY) {  // (where the lanes' scratch cannot be had)
-            for (int j = 0; j < nj; ++j) {
-                GCA_TRY(grid_build(ctx, cl[j], r[j]));
-                GCA_TRY(launch_normals_gradient(ctx, cl[j], r[j], jobs[j].max_nn, jobs[j].gradient_radius, true));
-            }
+        if (st == GCA_ERR_OUT_OF_MEMORY) {  // where the scratch of a shared walk cannot be had: a walk each
+            for (int j = 0; j < nj; ++j) GCA_TRY(by_itself(at[j]));
         } else {
             GCA_TRY(st);
+            for (int j = 0; j < nj; ++j) cl[j]->has_normals = cl[j]->has_gradient = true;
         }
-        for (int j = 0; j < nj; ++j) cl[j]->has_normals = cl[j]->has_gradient = true;
         nj = 0;
     }
     return GCA_OK;

@@ -145,5 +145,7 @@ for extra in range(0, 200, 5):
 rt.host_runtime_budget(1 << 40)
 g.multiscale_icp(src, tgt, levels)       # with all the memory it likes
 print("one level at a time", one / MiB, "succeeds with", tries, "more; together takes", (rt.host_runtime_live() - one) / MiB)
-assert tries and tries[0] <= 150
+# level by level, a walk each: the levels' clouds (as large as their inputs here, 3 x 2 x 12.2 MiB),
+# the targets' grids (3 x 10.7) and one level's sums (22.9)
+assert tries and tries[0] <= 135
 """)
