@@ -48,15 +48,29 @@ static void pool_drop(gca_ctx ctx, size_t keep)
     pool_drop_locked(ctx->pool, keep);
 }
 
-// hipMalloc on the current device, tried again without the pool where memory ends.  The runtime keeps
-// a failed call's error until it is asked for, and every launch is followed by that question, so an
-// error that is dealt with here is taken here.
-static hipError_t ctx_malloc(gca_ctx ctx, void **p, size_t bytes)
+// All ctxs of the process: each holds memory that another may need more.
+static std::mutex g_ctxs_m;
+static gca_ctx g_ctxs = nullptr;
+
+static void reclaim(int device)
+{
+    std::lock_guard<std::mutex> lock(g_ctxs_m);
+    for (gca_ctx c = g_ctxs; c; c = c->next) {
+        if (c->device != device) continue;
+        pool_drop(c, 0);
+        hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;  // (a wait would end the capture)
+        if (hipStreamIsCapturing(c->stream, &cap) == hipSuccess && cap == hipStreamCaptureStatusNone) ctx_lanes_release(c);
+    }
+}
+
+// (The runtime keeps a failed call's error until it is asked for, and every launch is followed by that
+// question, so an error that is dealt with here is taken here.)
+hipError_t ctx_malloc(gca_ctx ctx, void **p, size_t bytes)
 {
     hipError_t e = hipMalloc(p, bytes);
     if (e == hipErrorOutOfMemory) {
         (void)hipGetLastError();
-        pool_drop(ctx, 0);
+        reclaim(ctx->device);
         e = hipMalloc(p, bytes);
     }
     if (e != hipSuccess) {
@@ -74,10 +88,15 @@ static size_t pool_class(size_t bytes)
     return (bytes + step - 1) / step * step;
 }
 
+static bool pool_keeps(size_t bytes)
+{
+    return bytes >= BufferPool::kSmall && pool_class(bytes) <= BufferPool::kLimit / 4;
+}
+
 int32_t dev_alloc(gca_ctx ctx, void **p, size_t bytes)
 {
     *p = nullptr;
-    if (bytes >= BufferPool::kSmall) {
+    if (pool_keeps(bytes)) {
         bytes = pool_class(bytes);
         BufferPool &P = ctx->pool;
         std::lock_guard<std::mutex> lock(P.m);
@@ -104,7 +123,7 @@ void dev_free(gca_ctx ctx, void *p, size_t bytes, bool idle)
     if (!p) return;
     BufferPool &P = ctx->pool;
     const size_t cls = pool_class(bytes);
-    if (!idle || bytes < BufferPool::kSmall || cls > BufferPool::kLimit / 4) {
+    if (!idle || !pool_keeps(bytes)) {
         hipFree(p);
         return;
     }
@@ -124,7 +143,8 @@ bool device_idle(gca_ctx ctx)
     if (hipGetDevice(&dev) != hipSuccess) return false;
     if (dev != ctx->device && hipSetDevice(ctx->device) != hipSuccess) return false;
     void *p = nullptr;
-    const bool ok = ctx_malloc(ctx, &p, 256) == hipSuccess && hipFree(p) == hipSuccess;
+    const bool ok = hipMalloc(&p, 256) == hipSuccess && hipFree(p) == hipSuccess;
+    if (!ok) (void)hipGetLastError();
     if (dev != ctx->device) hipSetDevice(dev);
     return ok;
 }
@@ -271,7 +291,12 @@ void *lane_scratch(gca_ctx ctx, int lane, int slot, size_t bytes, bool zeroed)
 
 void ctx_lanes_release(gca_ctx ctx)
 {
-    hipStreamSynchronize(ctx->stream);
+    int free = 0;
+    if (!ctx->lanes.compare_exchange_strong(free, 2)) return;
+    bool held = false;
+    for (int s = gca_ctx_s::kLaneSlots; s < gca_ctx_s::kScratchSlots; ++s) held = held || ctx->scratch[s];
+    for (int l = 1; l < kMaxJobs; ++l) held = held || ctx->bitmap[l].p;
+    if (held) hipStreamSynchronize(ctx->stream);
     for (int s = gca_ctx_s::kLaneSlots; s < gca_ctx_s::kScratchSlots; ++s) {
         hipFree(ctx->scratch[s]);
         ctx->scratch[s] = nullptr;
@@ -282,6 +307,7 @@ void ctx_lanes_release(gca_ctx ctx)
         hipFree(ctx->bitmap[l].p);
         ctx->bitmap[l] = {};
     }
+    ctx->lanes.store(0);
 }
 
 // ---------------------------------------------------------------------------------------
@@ -801,6 +827,11 @@ int32_t gca_ctx_create(int32_t device, gca_ctx *out)
     }
     *c->dev_err = 0u;
     c->noalloc_scratch = noalloc_setup(device);  // this device's static scratch (no allocation)
+    {
+        std::lock_guard<std::mutex> lock(g_ctxs_m);
+        c->next = g_ctxs;
+        g_ctxs = c;
+    }
     *out = c;
     return GCA_OK;
 }
@@ -808,6 +839,14 @@ int32_t gca_ctx_create(int32_t device, gca_ctx *out)
 int32_t gca_ctx_destroy(gca_ctx c)
 {
     if (!c) return GCA_ERR_INVALID_VALUE;
+    {
+        std::lock_guard<std::mutex> lock(g_ctxs_m);
+        for (gca_ctx *at = &g_ctxs; *at; at = &(*at)->next)
+            if (*at == c) {
+                *at = c->next;
+                break;
+            }
+    }
     hipSetDevice(c->device);
     hipStreamSynchronize(c->stream);
     for (int i = 0; i < 16; ++i)

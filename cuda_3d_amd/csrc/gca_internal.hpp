@@ -11,6 +11,7 @@
 
 #include <hip/hip_runtime.h>
 
+#include <atomic>
 #include <cstdint>
 #include <cstring>
 #include <mutex>
@@ -155,6 +156,7 @@ struct gca_ctx_s {
     // scratch buffers owned by the ctx, grown on demand
     // (the slots from kLaneSlots on are the further lanes' of calls that build several clouds at once)
     static constexpr int kLaneSlots = 48, kScratchSlots = 80;
+    std::atomic<int> lanes{0};  // the further lanes: 0 free to be given back, 1 in use (LanesInUse), 2 going
     void *scratch[kScratchSlots] = {nullptr};
     size_t scratch_bytes[kScratchSlots] = {0};
     bool scratch_zeroed[kScratchSlots] = {false};
@@ -171,6 +173,7 @@ struct gca_ctx_s {
     size_t host_buf_bytes = 0;
     gca::BufferPool pool;
     gca::HdrPool hdrs;
+    gca_ctx_s *next = nullptr;  // in the list of all ctxs (ctx_malloc)
     int n_cu = 0;         // compute units of the device (persistent launch sizing)
     int wall_khz = 0;     // rate of the device wall clock (wall_clock64)
     // persistent bitmap of the voxel downsampler (kept all-zero between calls)
@@ -251,9 +254,22 @@ namespace gca {
 int32_t hip_status(hipError_t e);
 void *ctx_scratch(gca_ctx ctx, int slot, size_t bytes, bool zeroed);
 // The same for lane `lane` (< kMaxJobs) of a launch over several clouds of one ctx; lane 0 is slot
-// itself.  ctx_lanes_release gives the further lanes' scratch and bitmaps back.
+// itself.  ctx_lanes_release gives the further lanes' scratch and bitmaps back, unless they are in use:
+// from the first lane_scratch of a launch until it is enqueued.
 void *lane_scratch(gca_ctx ctx, int lane, int slot, size_t bytes, bool zeroed);
 void ctx_lanes_release(gca_ctx ctx);
+struct LanesInUse {
+    gca_ctx ctx;
+    explicit LanesInUse(gca_ctx c) : ctx(c)
+    {
+        for (int free = 0; !ctx->lanes.compare_exchange_weak(free, 1); free = 0) {
+        }
+    }
+    ~LanesInUse() { ctx->lanes.store(0); }
+};
+// hipMalloc on the current device, ctx's.  Where memory ends, what the device's ctxs only keep for
+// reuse (their pools, the further lanes not in use) goes back first.
+hipError_t ctx_malloc(gca_ctx ctx, void **p, size_t bytes);
 // Pinned host memory of the ctx; its content is the calling entry point's until that returns.
 void *ctx_host_buf(gca_ctx ctx, size_t bytes);
 // Buffers of clouds and grids (BufferPool).  dev_free: bytes as allocated; idle = device_idle()

@@ -1839,13 +1839,13 @@ int32_t icp_plan_create(gca_ctx ctx, int n_pairs, int n_levels, const gca_cloud 
         return hip_status(e);
     };
     hipError_t e;
-    if ((e = hipMalloc(&p->states, sizeof(IcpState) * n_states)) != hipSuccess) return fail(e);
-    if ((e = hipMalloc(&p->partials, sizeof(double) * kPartStride * n_states * 2 * unit_cap)) != hipSuccess) return fail(e);
-    if ((e = hipMalloc(&p->nnprev, sizeof(int32_t) * std::max<int64_t>(nn_off[n_states], 1))) != hipSuccess) return fail(e);
-    if ((e = hipMalloc(&p->pairs, sizeof(PairDesc) * n_states)) != hipSuccess) return fail(e);
-    if ((e = hipMalloc(&p->init, sizeof(StateInit) * n_states)) != hipSuccess) return fail(e);
-    if ((e = hipMalloc(&p->T0, sizeof(double) * 16 * n_pairs)) != hipSuccess) return fail(e);
-    if ((e = hipMalloc(&p->err, 256 + sizeof(*p->open) * n_states)) != hipSuccess) return fail(e);
+    if ((e = ctx_malloc(ctx, (void **)&p->states, sizeof(IcpState) * n_states)) != hipSuccess) return fail(e);
+    if ((e = ctx_malloc(ctx, (void **)&p->partials, sizeof(double) * kPartStride * n_states * 2 * unit_cap)) != hipSuccess) return fail(e);
+    if ((e = ctx_malloc(ctx, (void **)&p->nnprev, sizeof(int32_t) * std::max<int64_t>(nn_off[n_states], 1))) != hipSuccess) return fail(e);
+    if ((e = ctx_malloc(ctx, (void **)&p->pairs, sizeof(PairDesc) * n_states)) != hipSuccess) return fail(e);
+    if ((e = ctx_malloc(ctx, (void **)&p->init, sizeof(StateInit) * n_states)) != hipSuccess) return fail(e);
+    if ((e = ctx_malloc(ctx, (void **)&p->T0, sizeof(double) * 16 * n_pairs)) != hipSuccess) return fail(e);
+    if ((e = ctx_malloc(ctx, (void **)&p->err, 256 + sizeof(*p->open) * n_states)) != hipSuccess) return fail(e);
     p->open = (unsigned long long *)((char *)p->err + 256);
     if ((e = hipHostMalloc(&p->host_states, sizeof(IcpState) * n_states)) != hipSuccess) return fail(e);
     if ((e = hipHostMalloc(&p->host_err, 256)) != hipSuccess) return fail(e);
@@ -2317,8 +2317,11 @@ static int32_t build_targets(gca_ctx ctx, const gca_level_params *levels, int n,
         if (nj == 0 || (nj < kMaxJobs && l + 1 < n)) continue;
         int32_t st = GCA_OK;
         if (nj > 1) {
-            st = grid_build_levels(ctx, cl, r, nj);
-            if (st == GCA_OK) st = launch_normals_gradient_levels(ctx, jobs, nj);
+            {
+                LanesInUse lanes(ctx);
+                st = grid_build_levels(ctx, cl, r, nj);
+                if (st == GCA_OK) st = launch_normals_gradient_levels(ctx, jobs, nj);
+            }
             if (st == GCA_ERR_OUT_OF_MEMORY) ctx_lanes_release(ctx);
         } else {
             st = grid_build(ctx, cl[0], r[0]);

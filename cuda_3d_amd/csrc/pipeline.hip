@@ -713,7 +713,7 @@ int32_t gca_pipeline_create(gca_ctx ctx, const gca_camera *cam, const gca_bilate
         st = gca_cloud_create(p->ctx, cap, &p->full[s]);
         for (int l = 0; l < n_levels && st == GCA_OK; ++l) st = gca_cloud_create(p->ctx, cap, &p->lvc[s][l]);
     }
-    if (st == GCA_OK && hipMalloc(&p->err_dev, 256) != hipSuccess) st = GCA_ERR_OUT_OF_MEMORY;
+    if (st == GCA_OK && ctx_malloc(p->ctx, (void **)&p->err_dev, 256) != hipSuccess) st = GCA_ERR_OUT_OF_MEMORY;
     if (st == GCA_OK && hipHostMalloc(&p->err_host, 256) != hipSuccess) st = GCA_ERR_OUT_OF_MEMORY;
     if (st == GCA_OK) memset(p->err_host, 0, 256);
     if (st != GCA_OK) {

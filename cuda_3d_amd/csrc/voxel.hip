@@ -595,13 +595,34 @@ int32_t launch_voxel(gca_ctx ctx, gca_cloud in, float voxel, gca_cloud out)
     return voxel_enqueue(ctx, in, voxel, out, n, ((int64_t)nbits + 31) / 32, kVoxelMaxBits, nullptr);
 }
 
+static int32_t voxel_together(gca_ctx ctx, gca_cloud in, const float *voxel, const int64_t *words, bool wide,
+                              const gca_cloud *out, int n)
+{
+    LanesInUse lanes(ctx);
+    VoxelJobs vj[kMaxJobs];
+    for (int j = 0; j < n; ++j) {
+        GCA_TRY(cloud_reserve(out[j], std::max<int64_t>(in->host_hdr.n, 1)));
+        GCA_TRY(voxel_prepare(ctx, in, voxel[j], out[j], in->host_hdr.n, words[j], kVoxelMaxBits, nullptr, nullptr, wide, j,
+                              &vj[j]));
+    }
+    for (int j = 0; j < n; ++j) ctx->bitmap[j].dirty = true;  // until the whole sequence is enqueued
+    {
+        StageTimer timer(ctx, GCA_STAGE_VOXEL);
+        GCA_TRY(voxel_launch<kMaxJobs>(ctx->stream, vj, n, wide));
+    }
+    for (int j = 0; j < n; ++j) {
+        ctx->bitmap[j].dirty = false;
+        cloud_points_changed(out[j]);
+    }
+    return GCA_OK;
+}
+
 // All sizes in one launch a phase where every lattice is the bitmap's and their bits together are no
 // more than one call may take; else (and where the lanes' scratch cannot be had) a call each.
 int32_t launch_voxel_sizes(gca_ctx ctx, gca_cloud in, const float *voxel, const gca_cloud *out, int n)
 {
     if (n < 1 || n > kMaxJobs) return GCA_ERR_INVALID_VALUE;
     GCA_TRY(cloud_sync_header(in));
-    const int64_t np = std::max<int64_t>(in->host_hdr.n, 1);
     int64_t words[kMaxJobs];
     double all = 0.0;
     bool wide = false;
@@ -613,29 +634,12 @@ int32_t launch_voxel_sizes(gca_ctx ctx, gca_cloud in, const float *voxel, const 
         words[j] = nbits > kVoxelMaxBits ? 0 : ((int64_t)nbits + 31) / 32;
         wide = wide || scan_wide(words[j]);
     }
-    bool together = n > 1 && ctx->tune[GCA_TUNE_VOXEL] != 2 && all <= kVoxelMaxBits;
-    VoxelJobs vj[kMaxJobs];
-    for (int j = 0; j < n && together; ++j) {
-        GCA_TRY(cloud_reserve(out[j], np));
-        const int32_t st = voxel_prepare(ctx, in, voxel[j], out[j], in->host_hdr.n, words[j], kVoxelMaxBits, nullptr,
-                                         nullptr, wide, j, &vj[j]);
-        together = st != GCA_ERR_OUT_OF_MEMORY;
-        if (together) GCA_TRY(st);
-        else ctx_lanes_release(ctx);
+    if (n > 1 && ctx->tune[GCA_TUNE_VOXEL] != 2 && all <= kVoxelMaxBits) {
+        const int32_t st = voxel_together(ctx, in, voxel, words, wide, out, n);
+        if (st != GCA_ERR_OUT_OF_MEMORY) return st;
+        ctx_lanes_release(ctx);
     }
-    if (!together) {
-        for (int j = 0; j < n; ++j) GCA_TRY(launch_voxel(ctx, in, voxel[j], out[j]));
-        return GCA_OK;
-    }
-    for (int j = 0; j < n; ++j) ctx->bitmap[j].dirty = true;  // until the whole sequence is enqueued
-    {
-        StageTimer timer(ctx, GCA_STAGE_VOXEL);
-        GCA_TRY(voxel_launch<kMaxJobs>(ctx->stream, vj, n, wide));
-    }
-    for (int j = 0; j < n; ++j) {
-        ctx->bitmap[j].dirty = false;
-        cloud_points_changed(out[j]);
-    }
+    for (int j = 0; j < n; ++j) GCA_TRY(launch_voxel(ctx, in, voxel[j], out[j]));
     return GCA_OK;
 }
 

@@ -149,3 +149,74 @@ print("one level at a time", one / MiB, "succeeds with", tries, "more; together 
 # the targets' grids (3 x 10.7) and one level's sums (22.9)
 assert tries and tries[0] <= 135
 """)
+
+
+def test_memory_kept_for_reuse_gives_way(runtime):
+    """What a context only keeps for its next calls (buffers of clouds that are gone, the scratch of a
+    multi-scale call's further levels) is there for whatever does not fit otherwise: its own clouds, a
+    batch plan, another context, a pipeline's."""
+    _run(runtime, """
+def level(n):
+    s, t = cloud(n, 3), cloud(n, 4)
+    t.estimate_normals(0.1, 30)
+    t.compute_color_gradient(0.1, 0)
+    return s, t
+pairs = [level(2000) for _ in range(40)]
+prm = [g.icp_params(3, 0.1)]
+def plan():
+    return g.BatchPlan([[s] for s, _ in pairs], [[t] for _, t in pairs], prm, np.tile(np.eye(4), (40, 1, 1)), [0.1])
+def pipeline():
+    cam, bil, h = g.make_camera(640, 480, 615.0, 615.0, 320, 240), g.bilateral(), C.c_void_p()
+    lv = (L.LevelParams * 3)(*[g.level_params(v) for v in (0.04, 0.02, 0.01)])
+    L.check(L.lib.gca_pipeline_create(ctx.handle, C.byref(cam), C.byref(bil), 0.2, 3.5, 3, lv, C.byref(h)), "pipeline")
+    return h
+def taken(make):
+    rt.host_runtime_budget(1 << 40)
+    before = rt.host_runtime_live()
+    made = make()
+    size = rt.host_runtime_live() - before
+    if isinstance(made, C.c_void_p):
+        L.lib.gca_pipeline_destroy(made)
+    elif hasattr(made, "close"):
+        made.close()
+    return size
+levels = [g.level_params(v, icp=g.icp_params(2, 2.5 * v)) for v in (0.1, 0.06, 0.04)]
+src, tgt = cloud(400_000, 1), cloud(400_000, 2)
+g.multiscale_icp(src, tgt, levels)       # its scratch stays
+plan().close()                           # (so that the calls below find their small buffers)
+other = g.Context(0)
+wanted = {"cloud": lambda: cloud(600_000),
+          "plan": plan,
+          "other": lambda: g.PointCloud(other, 600_000),
+          "pipeline": pipeline}
+sizes = {k: taken(f) for k, f in wanted.items()}
+for kept in ("pool", "lanes"):
+    for k, make in wanted.items():
+        rt.host_runtime_budget(1 << 40)
+        if kept == "pool":
+            bulk = [cloud(1_500_000) for _ in range(6)]
+            del bulk
+        else:
+            g.multiscale_icp(src, tgt, levels)
+        full = rt.host_runtime_live()
+        rt.host_runtime_budget(full + sizes[k] // 4)  # a quarter of what it takes, the rest is kept memory
+        made = make()
+        print(kept, k, sizes[k] / MiB, full / MiB, "->", rt.host_runtime_live() / MiB)
+        assert rt.host_runtime_live() <= full + sizes[k] // 4
+        if k == "pipeline":
+            L.lib.gca_pipeline_destroy(made)
+        del made
+""")
+
+
+def test_large_arrays_take_what_they_hold(runtime):
+    """Buffers too large for the pool are not rounded up to its classes."""
+    _run(runtime, """
+cloud(1)
+for n in (9_000_001, 17_300_000):        # 137 and 264 MiB an array
+    before = rt.host_runtime_live()
+    pc = g.PointCloud(ctx, n)
+    assert rt.host_runtime_live() - before == 4 * 16 * n
+    del pc
+    assert rt.host_runtime_live() == before
+""")
