@@ -14,23 +14,25 @@
 //               neighbours are linked (raster and lattice order put most neighbours side by side),
 //               within the workgroup; a run's first point takes the point before it if linked: no
 //               atomics, no search
-//   2. pairs    every point and the few before it in cell order, if linked, are joined; snapshot:
-//               each point's root, in cell order, and the most frequent root of a sample (`big`)
-//   3. hook     the points outside the big component link their root with that of every linked
+//   2. pairs    (clouds large and dense enough for it, hook_direct) every point and the few before it in
+//               cell order, if linked, are joined; snapshot: each point's root, in cell order, and the most
+//               frequent root of a sample (`big`), if it is that of half the sample
+//   3. hook     with a big component: the points outside it link their root with that of every linked
 //               neighbour of another snapshot component.  An edge inside a component is already
 //               there, and one into the big component is seen from its other end, so the bulk of
-//               a scene takes no part.  Linked: the radius search's own predicate, squared FP64
-//               distance < r^2, and for the residual form the residual gate
+//               a scene takes no part.  Else every point does so with the neighbours before it in cell
+//               order.  Linked: the radius search's own predicate, squared FP64 distance < r^2, and for the
+//               residual form the residual gate
 //   4. compress parent[i] = root (a read-only walk, then a store to the point's own entry),
-//               size[root] += 1 and low[root] = min(i) (one atomic per wave and root run); lowest:
-//               the component's lowest index, which is the reference's seed, becomes its root
+//               size[root] += 1 and, after links by rank, low[root] = min(i) (one atomic per wave and root
+//               run); lowest: the component's lowest index, the reference's seed, becomes its root
 //   5. cut      only for components above max_cluster_size (listed by k_cc_lowest): the
 //               reference's truncated searches, replayed exactly on the device (k_cc_truncate),
 //               re-root the component's points on the seeds of the pieces it is cut into
 //   6. rank     kept roots (size >= min) are numbered by an exclusive scan in index order
 //   7. label    label[i] = number of its root's cluster, or -1
-// A root is only ever linked, by compare-and-swap, under a point of lower rank (cc_rank) that was a
-// root, so links form no cycle; parent pointers always name an ancestor, so the path-halving stores
+// A root is only ever linked, by compare-and-swap, under a point of lower rank (cc_rank; without pairs of
+// lower index, so that the root is the lowest point) that was a root, so links form no cycle; parent pointers always name an ancestor, so the path-halving stores
 // in find() may race with the compare-and-swaps without losing a link.
 //
 // Neighbour lists are visited in the radius search's canonical order, (squared distance,
@@ -96,11 +98,13 @@ __device__ __forceinline__ uint32_t cc_rank(int32_t x)
     return m ^ m >> 15;
 }
 
-// Links the trees of u and v (any nodes of them; the point's own root is passed in).
+// Links the trees of u and v (any nodes of them; the point's own root is passed in).  LOWEST: by index, so
+// that a tree's root is its lowest point.
+template <bool LOWEST>
 __device__ __forceinline__ void cc_union(int32_t *parent, int32_t u, int32_t v)
 {
     while (u != v) {
-        if (cc_rank(u) > cc_rank(v)) {
+        if (LOWEST ? u > v : cc_rank(u) > cc_rank(v)) {
             const int32_t t = u;
             u = v;
             v = t;
@@ -129,13 +133,17 @@ constexpr int kCcWide = 1024;
 __global__ __launch_bounds__(kCcWide) void k_cc_chain(const CloudHdr *__restrict__ h, const float4 *__restrict__ xyzi,
                                                      const float *__restrict__ res, double r2,
                                                      int32_t *__restrict__ parent, uint32_t *__restrict__ size,
-                                                     int32_t *__restrict__ low, uint32_t *__restrict__ oversized)
+                                                     int32_t *__restrict__ low, int32_t *__restrict__ big,
+                                                     uint32_t *__restrict__ oversized)
 {
     __shared__ int32_t last[kCcWide / kWave];  // per wavefront: its last run's first point, -1 if it has none
     const int n = h->n;
     const int lane = lane_id(), w = threadIdx.x / kWave;
     const int i = blockIdx.x * kCcWide + threadIdx.x;
-    if (i == 0) *oversized = 0;
+    if (i == 0) {
+        *oversized = 0;
+        *big = -1;
+    }
     bool linked = false;
     if (i > 0 && i < n) {
         const float4 p = xyzi[i], q = xyzi[i - 1];
@@ -151,16 +159,17 @@ __global__ __launch_bounds__(kCcWide) void k_cc_chain(const CloudHdr *__restrict
     for (int v = w; head < 0;) head = last[--v];  // the workgroup's first point starts a run
     parent[i] = threadIdx.x == 0 && linked ? i - 1 : head;
     size[i] = 0;
-    low[i] = INT_MAX;
+    if (low) low[i] = INT_MAX;
 }
 
+template <bool LOWEST>
 __device__ __forceinline__ void cc_link(int32_t *parent, int32_t &ri, int32_t j)
 {
     const int32_t rj = cc_find(parent, j);
     if (rj != ri) {
         ri = cc_find(parent, ri);  // short walk: ri was a root not long ago
         if (rj != ri) {
-            cc_union(parent, ri, rj);  // a compare-and-swap only for distinct roots
+            cc_union<LOWEST>(parent, ri, rj);  // a compare-and-swap only for distinct roots
             ri = cc_find(parent, ri);
         }
     }
@@ -180,7 +189,7 @@ __global__ __launch_bounds__(kCcBlock) void k_cc_pairs(const CloudHdr *__restric
     if (!(dist2(p.x, p.y, p.z, q.x, q.y, q.z) < r2) || !residual_gate(res, i, j)) return;
     if (cc_load(parent + i) == cc_load(parent + j)) return;  // most pairs: joined already
     int32_t ri = cc_find(parent, i);
-    cc_link(parent, ri, j);
+    cc_link<false>(parent, ri, j);
 }
 
 // Each point's root, in cell order, and its residual likewise (what the hook reads per candidate).
@@ -198,8 +207,10 @@ __global__ __launch_bounds__(kCcBlock) void k_cc_snapshot(const CloudHdr *__rest
     if (res) sres[s] = res[i];
 }
 
-// The most frequent root among kCcSample points spread over the cloud (a tie: the lowest).  Any
-// answer is right; a good one lets the hook leave out most points.
+// The most frequent root among kCcSample points spread over the cloud (a tie: the lowest), or -1 if it is
+// not half of them: the hook then takes each edge from one end, where leaving out a big component's points
+// makes it look at the others' edges from both.  Any answer is right; a good one lets the hook leave out
+// most points.
 constexpr int kCcSample = 1024;
 
 __global__ __launch_bounds__(kCcSample) void k_cc_big(const CloudHdr *__restrict__ h, const int32_t *__restrict__ snap,
@@ -217,7 +228,8 @@ __global__ __launch_bounds__(kCcSample) void k_cc_big(const CloudHdr *__restrict
     __syncthreads();
     if (n > 0) {
         const int32_t r = snap[(int64_t)t * n / kCcSample];
-        uint32_t e = ((uint32_t)r * 2654435761u) >> 21;
+        // (not the multiplier of cc_rank: roots are of low rank, and would all fall into few entries)
+        uint32_t e = ((uint32_t)r * 0x85ebca6bu) >> 21;
         for (;;) {  // the table is never full
             const int32_t old = atomicCAS(&key[e], -1, r);
             if (old == -1 || old == r) break;
@@ -226,21 +238,28 @@ __global__ __launch_bounds__(kCcSample) void k_cc_big(const CloudHdr *__restrict
         atomicAdd(&cnt[e], 1u);
     }
     __syncthreads();
+    unsigned long long mine = 0ull;
     for (int e = t; e < 2 * kCcSample; e += kCcSample)
-        if (cnt[e]) atomicMax(&best, ((unsigned long long)cnt[e] << 32) | (uint32_t)(INT_MAX - key[e]));
+        if (cnt[e]) mine = max(mine, ((unsigned long long)cnt[e] << 32) | (uint32_t)(INT_MAX - key[e]));
+    for (int m = 1; m < kWave; m <<= 1) mine = max(mine, (unsigned long long)__shfl_xor(mine, m, kWave));
+    if (lane_id() == 0) atomicMax(&best, mine);  // (one a wavefront: a thousand of them queue for 40 us)
     __syncthreads();
-    if (t == 0) *big = INT_MAX - (int32_t)(uint32_t)best;
+    if (t == 0) *big = 2 * (uint32_t)(best >> 32) >= kCcSample ? INT_MAX - (int32_t)(uint32_t)best : -1;
 }
 
 // Hook: kCcLanes lanes per point outside the big component (points in cell order), each lane a share of the point's
 // candidates from the 27 cells around it.  Between two points outside the big component the later
-// one in cell order takes the edge; the components do not depend on which end links it.  The whole
+// one in cell order takes the edge, and without one the walk ends at the point's own slot (and loads the
+// neighbours' roots with them: 300k points in clusters of 150, 285 -> 240 us); the components do not depend
+// on which end links an edge.  DIRECT: no pairs and no snapshot came before, each
+// point stands for itself (snap is the cell order, sres the residuals by index).  The whole
 // labelling is bound by the union-find's dependent loads and contended compare-and-swaps: 92k points of
 // a 424x240 frame at 2 cm 91 us plain and 171 us gated, where hooking every edge of every point took
-// 270 us for either; 289k points of a 640x480 frame at 1 cm 121 us (568 every edge).
+// 270 us for either; 289k points of a 640x480 frame at 1 cm 127 us (568 every edge).
 constexpr int kCcLanes = 8;
 constexpr int kCcUnroll = 4;
 
+template <bool DIRECT>
 __global__ __launch_bounds__(kCcBlock) void k_cc_hook(const CloudHdr *__restrict__ h, GridDesc g,
                                                      const uint32_t *__restrict__ start,
                                                      const float4 *__restrict__ sxyzi,
@@ -253,15 +272,23 @@ __global__ __launch_bounds__(kCcBlock) void k_cc_hook(const CloudHdr *__restrict
     const int gl = (int)threadIdx.x & (kCcLanes - 1);
     const int s = (int)((blockIdx.x * blockDim.x + threadIdx.x) / kCcLanes);  // the group's point
     if (s >= n) return;  // the whole group
-    const int32_t big = *big_p, mine = snap[s];
+    const int32_t big = DIRECT ? -1 : *big_p, mine = snap[s];
     if (mine == big) return;
     const GridView v = make_view(g, start, order, sxyzi);
     const double r2 = (double)g.radius * (double)g.radius;
     const float4 p = sxyzi[s];
-    const float res = sres ? sres[s] : 0.f;
+    const float res = sres ? sres[DIRECT ? mine : s] : 0.f;
     Box b;
     if (!grid_range(g, p.x, p.y, p.z, b.lo, b.hi)) return;
     int32_t ri = cc_find(parent, mine);
+    if (big < 0) {
+        group_walk_box<kCcUnroll, 3, true>(v, b, gl, kCcLanes, -1, -1, [&](uint32_t t, float4 q, bool valid, int32_t other) {
+            if (!valid || other == mine || !(dist2(q.x, q.y, q.z, p.x, p.y, p.z) < r2)) return;
+            if (sres && !residual_close(res, sres[DIRECT ? other : (int32_t)t])) return;
+            cc_link<DIRECT>(parent, ri, other);
+        }, [] { return true; }, (uint32_t)s, snap);
+        return;
+    }
     // once this component is part of the big one (by this point's doing or another's), its other
     // edges into the big one are done with; likewise a second edge into the component just joined
     bool joined = ri == cc_find(parent, big);
@@ -271,7 +298,7 @@ __global__ __launch_bounds__(kCcBlock) void k_cc_hook(const CloudHdr *__restrict
         const int32_t other = snap[t];
         if (other == mine || other == done || (other == big ? joined : t > (uint32_t)s)) return;
         if (sres && !residual_close(res, sres[t])) return;
-        cc_link(parent, ri, other);
+        cc_link<false>(parent, ri, other);
         done = other;
         joined |= other == big;
     }, [&] {
@@ -294,7 +321,7 @@ __global__ __launch_bounds__(kCcWide) void k_cc_compress(const CloudHdr *__restr
     if (threadIdx.x == 0) {
         s_count = 0u;
         s_low = INT_MAX;
-        s_big = n > 0 ? cc_root(parent, *big_p) : -1;
+        s_big = *big_p < 0 ? -1 : cc_root(parent, *big_p);
     }
     const int32_t r = on ? cc_root(parent, i) : -1;
     __syncthreads();
@@ -313,14 +340,14 @@ __global__ __launch_bounds__(kCcWide) void k_cc_compress(const CloudHdr *__restr
         const uint64_t same = __ballot(on && r == lr);
         if (lane_id() == leader) {
             atomicAdd(size + lr, (uint32_t)__popcll(same));
-            atomicMin(low + lr, i);
+            if (low) atomicMin(low + lr, i);
         }
         pending &= ~same;
     }
     __syncthreads();
     if (threadIdx.x == 0 && s_count) {
         atomicAdd(size + big, s_count);
-        atomicMin(low + big, s_low);
+        atomicMin(low + big, s_low);  // (with a big component there is low)
     }
 }
 
@@ -341,7 +368,7 @@ __global__ __launch_bounds__(kCcBlock) void k_cc_lowest(const CloudHdr *__restri
     const int n = h->n;
     const int i = blockIdx.x * blockDim.x + threadIdx.x;
     if (i >= n) return;
-    const int32_t r = parent[i], m = low[r];
+    const int32_t r = parent[i], m = low ? low[r] : r;
     parent[i] = m;
     if (r != i) return;
     const uint32_t sz = size[i];
@@ -548,6 +575,21 @@ __global__ __launch_bounds__(kCcBlock) void k_cc_label(const CloudHdr *__restric
     label[i] = kept[r] ? (int32_t)rank[r] : -1;
 }
 
+// Whether the hook takes every edge at once.  Pairs, snapshot and the search for a big component cost three
+// launches, 20 to 30 us, and pay where a component of most points spares the hook its bulk: in larger clouds
+// whose points lie close (their number per column of cells along the grid's shortest side tells, for the
+// surfaces that a camera sees).  us a labelling, every edge at once / pairs first, plain then gated; rendered
+// frames: 80x60 at 2 cm 73 / 100, 73 / 97; 160x120 at 1, 2 and 4 cm (0.3, 1.1 and 4 points a column) 80 / 106,
+// 92 / 106, 190 / 98, gated 78 / 101, 92 / 105, 130 / 107; 240x180 at 1 and 2 cm (0.6 and 2.4) 92 / 113, 229 / 115,
+// gated 91 / 113, 126 / 109; 320x240 at 1 cm (1.1) 172 / 122, gated 108 / 114; 640x480 at 5 mm (1.1) 415 / 277,
+// gated 298 / 216.  16k points scattered on a surface at 2 cm (3 a column): 237 / 130, gated 89 / 106.
+bool hook_direct(const GridDesc &g, int64_t n, bool gated)
+{
+    int64_t d[3] = {g.dims[0], g.dims[1], g.dims[2]};
+    std::sort(d, d + 3);
+    return n < (gated ? 20000 : 12000) || 4 * n < 3 * d[1] * d[2];
+}
+
 }  // namespace
 
 int32_t launch_euclidean_clustering(gca_ctx ctx, gca_cloud c, float tolerance, uint32_t min_size,
@@ -563,28 +605,35 @@ int32_t launch_euclidean_clustering(gca_ctx ctx, gca_cloud c, float tolerance, u
     CutJob *jobs = (CutJob *)ctx_scratch(ctx, 28, sizeof(CutJob) * (size_t)std::max<int64_t>(c->cap, 1), false);
     if (!size || !kept || !bcnt || !boff || !jobs) return GCA_ERR_OUT_OF_MEMORY;
     const dim3 grid((unsigned)nb), block(kCcBlock);
-    int32_t *snap = (int32_t *)ctx_scratch(ctx, 11, sizeof(int32_t) * (size_t)c->cap, false);
-    float *sres = res ? (float *)ctx_scratch(ctx, 12, sizeof(float) * (size_t)c->cap, false) : nullptr;
     int32_t *big = (int32_t *)ctx_scratch(ctx, 46, 256, false);
-    int32_t *low = (int32_t *)ctx_scratch(ctx, 9, sizeof(int32_t) * (size_t)c->cap, false);
-    if (!snap || !big || !low || (res && !sres)) return GCA_ERR_OUT_OF_MEMORY;
+    const bool direct = hook_direct(G.desc, c->host_hdr.n, res != nullptr);
+    int32_t *low = direct ? nullptr : (int32_t *)ctx_scratch(ctx, 9, sizeof(int32_t) * (size_t)c->cap, false);
+    if (!big || (!direct && !low)) return GCA_ERR_OUT_OF_MEMORY;
     const double r2 = (double)tolerance * (double)tolerance;
     const dim3 wide((unsigned)std::max<int64_t>(1, (c->cap + kCcWide - 1) / kCcWide));
-    hipLaunchKernelGGL(k_cc_chain, wide, dim3(kCcWide), 0, ctx->stream, c->hdr, c->xyzi, res, r2, label, size, low,
+    hipLaunchKernelGGL(k_cc_chain, wide, dim3(kCcWide), 0, ctx->stream, c->hdr, c->xyzi, res, r2, label, size, low, big,
                        counts_dev + 1);
-    // Every second point and its predecessor connect the rows that a cell holds; the residual gate
-    // lets about a third of the neighbours through, so it takes more pairs before a scene's bulk
-    // holds together.  Pairs / hook of a 424x240 frame at 2 cm: 19 / 36 us plain (every fourth: 16 /
-    // 53), gated 51 / 79 us with three predecessors of every point (two 38 / 118, four 70 / 67); at
-    // 640x480 gated 93 / 276 (two 73 / 387, four 120 / 236).
-    const int step = res ? 1 : 2, back = res ? 3 : 1;
-    const dim3 grid_pairs((unsigned)std::max<int64_t>(1, (c->cap / step * back + back + kCcBlock - 1) / kCcBlock));
-    hipLaunchKernelGGL(k_cc_pairs, grid_pairs, block, 0, ctx->stream, c->hdr, G.sxyzi, G.order, res, r2, step, back, label);
-    hipLaunchKernelGGL(k_cc_snapshot, grid, block, 0, ctx->stream, c->hdr, G.order, res, label, snap, sres);
-    hipLaunchKernelGGL(k_cc_big, dim3(1), dim3(kCcSample), 0, ctx->stream, c->hdr, (const int32_t *)snap, big);
     const dim3 grid_hook((unsigned)std::max<int64_t>(1, (c->cap * kCcLanes + kCcBlock - 1) / kCcBlock));
-    hipLaunchKernelGGL(k_cc_hook, grid_hook, block, 0, ctx->stream, c->hdr, G.desc, G.start, G.sxyzi, G.order,
-                       (const int32_t *)snap, (const float *)sres, (const int32_t *)big, label);
+    if (direct) {
+        hipLaunchKernelGGL(k_cc_hook<true>, grid_hook, block, 0, ctx->stream, c->hdr, G.desc, G.start, G.sxyzi, G.order,
+                           (const int32_t *)G.order, res, (const int32_t *)big, label);
+    } else {
+        int32_t *snap = (int32_t *)ctx_scratch(ctx, 11, sizeof(int32_t) * (size_t)c->cap, false);
+        float *sres = res ? (float *)ctx_scratch(ctx, 12, sizeof(float) * (size_t)c->cap, false) : nullptr;
+        if (!snap || (res && !sres)) return GCA_ERR_OUT_OF_MEMORY;
+        // Every second point and its predecessor connect the rows that a cell holds; the residual gate
+        // lets about a third of the neighbours through, so it takes more pairs before a scene's bulk
+        // holds together.  Pairs / hook of a 424x240 frame at 2 cm: 19 / 36 us plain (every fourth: 16 /
+        // 53), gated 51 / 79 us with three predecessors of every point (two 38 / 118, four 70 / 67); at
+        // 640x480 gated 93 / 276 (two 73 / 387, four 120 / 236).
+        const int step = res ? 1 : 2, back = res ? 3 : 1;
+        const dim3 grid_pairs((unsigned)std::max<int64_t>(1, (c->cap / step * back + back + kCcBlock - 1) / kCcBlock));
+        hipLaunchKernelGGL(k_cc_pairs, grid_pairs, block, 0, ctx->stream, c->hdr, G.sxyzi, G.order, res, r2, step, back, label);
+        hipLaunchKernelGGL(k_cc_snapshot, grid, block, 0, ctx->stream, c->hdr, G.order, res, label, snap, sres);
+        hipLaunchKernelGGL(k_cc_big, dim3(1), dim3(kCcSample), 0, ctx->stream, c->hdr, (const int32_t *)snap, big);
+        hipLaunchKernelGGL(k_cc_hook<false>, grid_hook, block, 0, ctx->stream, c->hdr, G.desc, G.start, G.sxyzi, G.order,
+                           (const int32_t *)snap, (const float *)sres, (const int32_t *)big, label);
+    }
     hipLaunchKernelGGL(k_cc_compress, wide, dim3(kCcWide), 0, ctx->stream, c->hdr, label, size, low,
                        (const int32_t *)big);
     hipLaunchKernelGGL(k_cc_lowest, grid, block, 0, ctx->stream, c->hdr, label, size, (const int32_t *)low, max_size, jobs,

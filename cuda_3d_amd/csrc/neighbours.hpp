@@ -98,12 +98,13 @@ __device__ __forceinline__ void keep_loaded(T &v)
 }
 
 // Run r of the A x A columns from (x0, y0) on: candidates cum[r] .. cum[r + 1], at slot off[r] + f;
-// columns outside the box, and column (sx, sy), are empty.  Cell numbers fit 32 bits (at most
+// columns outside the box, and column (sx, sy), are empty, and so is what lies at slots from `limit` on.
+// Cell numbers fit 32 bits (at most
 // 2^25 cells), and the columns lie a fixed stride apart, so a bound is one 32-bit offset: numbering
 // the columns by division cost more than the walk's distances.
 template <int A>
 __device__ __forceinline__ void block_runs(const uint32_t *__restrict__ start, const GridDesc &g, const Box &b, int x0, int y0,
-                                           int sx, int sy, uint32_t off[A * A], uint32_t cum[A * A + 1])
+                                           int sx, int sy, uint32_t limit, uint32_t off[A * A], uint32_t cum[A * A + 1])
 {
     const uint32_t dy = (uint32_t)g.dims[2], dx = (uint32_t)g.dims[1] * dy;
     const uint32_t len = (uint32_t)(b.hi[2] + 1 - b.lo[2]);
@@ -129,6 +130,7 @@ __device__ __forceinline__ void block_runs(const uint32_t *__restrict__ start, c
         const int x = x0 + r / A, y = y0 + r % A;
         const bool in = x <= b.hi[0] && y <= b.hi[1] && !(x == sx && y == sy);
         off[r] = s0[r];
+        s1[r] = min(s1[r], limit);
         cum[r + 1] = in && s1[r] > s0[r] ? s1[r] - s0[r] : 0u;
     }
     cum[0] = 0;
@@ -142,41 +144,50 @@ __device__ __forceinline__ void block_runs(const uint32_t *__restrict__ start, c
 // The candidates [0, total) at slots slot(f) by a group of gs lanes (a power of two, lanes g = 0 ..
 // gs - 1 of one wavefront), U loads in flight per lane: calls f(slot, point, valid) U times per
 // round on every lane of the group (valid: the lane has a candidate), then more(): false ends the
-// walk (the same answer on the group's lanes).  Returns whether it went to the end.
-template <int U, class S, class F, class M>
+// walk (the same answer on the group's lanes).  Returns whether it went to the end.  With IDS, ids[slot]
+// is loaded with the point and goes to f as well.
+template <int U, bool IDS = false, class S, class F, class M>
 __device__ __forceinline__ bool group_walk(const float4 *__restrict__ sxyzi, uint32_t total, int g, int gs, S &&slot, F &&f,
-                                           M &&more)
+                                           M &&more, const int32_t *__restrict__ ids = nullptr)
 {
     for (uint32_t f0 = 0; f0 < total; f0 += gs * U) {
         float4 c[U];
         uint32_t sl[U];
+        int32_t id[IDS ? U : 1];
 #pragma unroll
         for (int u = 0; u < U; ++u) {
             sl[u] = slot(min(f0 + u * gs + g, total - 1u));  // a lane past the end loads the last one
             c[u] = sxyzi[sl[u]];
+            if constexpr (IDS) id[u] = ids[sl[u]];
         }
 #pragma unroll
         for (int u = 0; u < U; ++u) {
             keep_loaded(c[u].x);
             keep_loaded(c[u].y);
             keep_loaded(c[u].z);
+            if constexpr (IDS) keep_loaded(id[u]);
         }
 #pragma unroll
-        for (int u = 0; u < U; ++u) f(sl[u], c[u], f0 + u * gs + g < total);
+        for (int u = 0; u < U; ++u) {
+            if constexpr (IDS) f(sl[u], c[u], f0 + u * gs + g < total, id[u]);
+            else f(sl[u], c[u], f0 + u * gs + g < total);
+        }
         if (!more()) return false;
     }
     return true;
 }
 
-// The walk over box b (without column (sx, sy)), a block of A x A columns as one flattened range.
-template <int U, int A = 3, class F, class M>
-__device__ __forceinline__ void group_walk_box(const GridView &v, const Box &b, int g, int gs, int sx, int sy, F &&f, M &&more)
+// The walk over box b (without column (sx, sy), and up to slot `limit`), a block of A x A columns as one
+// flattened range.
+template <int U, int A = 3, bool IDS = false, class F, class M>
+__device__ __forceinline__ void group_walk_box(const GridView &v, const Box &b, int g, int gs, int sx, int sy, F &&f, M &&more,
+                                               uint32_t limit = UINT_MAX, const int32_t *__restrict__ ids = nullptr)
 {
     constexpr int kRuns = A * A;
     for (int x0 = b.lo[0]; x0 <= b.hi[0]; x0 += A)
         for (int y0 = b.lo[1]; y0 <= b.hi[1]; y0 += A) {
             uint32_t off[kRuns], cum[kRuns + 1];
-            block_runs<A>(v.start, v.g, b, x0, y0, sx, sy, off, cum);
+            block_runs<A>(v.start, v.g, b, x0, y0, sx, sy, limit, off, cum);
             auto slot = [&](uint32_t fi) {
                 uint32_t o = off[0];
 #pragma unroll
@@ -186,7 +197,7 @@ __device__ __forceinline__ void group_walk_box(const GridView &v, const Box &b, 
                 }
                 return o + fi;
             };
-            if (!group_walk<U>(v.sxyzi, cum[kRuns], g, gs, slot, f, more)) return;
+            if (!group_walk<U, IDS>(v.sxyzi, cum[kRuns], g, gs, slot, f, more, ids)) return;
         }
 }
 

@@ -165,3 +165,44 @@ def test_clusters_are_numbered_by_their_lowest_point(ctx, n, reverse, mx):
         assert len(got) == len(want)
         for a, b in zip(got, want):
             np.testing.assert_array_equal(a, np.sort(b))
+
+
+@pytest.mark.parametrize("n", [11999, 12000, 19999, 20000])
+@pytest.mark.parametrize("kind,r", [("plane", 0.004), ("plane", 0.0012), ("blobs", 0.004), ("halves", 0.004), ("apart", 0.004)])
+def test_components_on_both_sides_of_the_hook_rule(ctx, n, kind, r):
+    """Clouds just below and above the sizes from which pairs and a big component come before the hook
+    (12000, gated 20000), dense and too sparse for them, with one component of most points, with none and
+    with one of about half."""
+    import cuda_3d_amd as g
+    import oracle as O
+
+    rng = np.random.default_rng(n)
+    x = rng.uniform(-0.1, 0.1, (n, 3))
+    x[:, 2] = 1.0 + 1e-4 * rng.normal(size=n)
+    if kind == "blobs":
+        c = np.stack(np.meshgrid(np.arange(-5, 5), np.arange(-5, 5)), -1).reshape(-1, 2) * 0.02
+        x[:, :2] = c[rng.integers(0, 100, n)] + rng.normal(0, 0.001, (n, 2))
+    elif kind == "halves":   # half in one place, the rest in many
+        c = np.stack(np.meshgrid(np.arange(-5, 5), np.arange(-5, 5)), -1).reshape(-1, 2) * 0.02
+        k = n // 2 + (n % 3) - 1
+        x[k:, :2] = c[rng.integers(0, 100, n - k)] + rng.normal(0, 0.001, (n - k, 2)) + 0.5
+    elif kind == "apart":    # nothing is linked: every point is a component
+        w = int(np.ceil(np.sqrt(n)))
+        x[:, 0], x[:, 1] = 0.0041 * (np.arange(n) % w), 0.0041 * (np.arange(n) // w)
+        x = x[rng.permutation(n)]
+    x = x.astype(np.float32)
+    pc = g.PointCloud.from_numpy(x, np.zeros_like(x), ctx=ctx)
+    pc.set_normals(np.zeros_like(x))
+    xyzi = pc.download_xyzi()
+    res = rng.uniform(0, 0.02, n).astype(np.float32)
+    for residual in (None, res):
+        want = O.euclidean_clustering(xyzi, r, 1, n, residual=residual)
+        got = (pc.euclidean_clustering(r, 1, n) if residual is None else pc.icp_residual_segmentation(r, residual, 1, n))
+        assert len(got) == len(want)
+        label = np.full(n, -1)
+        for k, b in enumerate(want):
+            label[b] = k
+        have = np.full(n, -1)
+        for k, a in enumerate(got):
+            have[a] = k
+        np.testing.assert_array_equal(have, label)
