@@ -89,3 +89,9 @@ def test_wall_score_times_runs_after_warm_ones():
 
     ms = autotune.measure_wall(FakeCtx(), run, ("icp",), reps=3, warm=2)
     assert len(ran) == 5 and 0.5 <= ms < 8.0
+
+
+def test_batch_table_keeps_the_partition_of_the_sums():
+    """The unit cap fixes the order in which a batch's sums are added, so a tuned batch's last bits
+    hang on it: it stays where it was for a sweep's 0.3 %."""
+    assert autotune.load(autotune.DEFAULT_TABLE, "batch")["icp_max_units"] == 128
