@@ -1,8 +1,7 @@
 """Launch-shape autotuner for libgca.so (no reference counterpart: the reference takes the
 shapes Thrust picks).
 
-The knobs are the ctx tuning keys (GCA_TUNE_*): lanes per neighbourhood query for normals and
-colour gradients, lanes per correspondence query of the ICP by cloud size (the size of a query's
+The knobs are the ctx tuning keys (GCA_TUNE_*): lanes per correspondence query of the ICP by cloud size (the size of a query's
 lane group within the 256-thread workgroup), the cap on ICP work units per iteration (one FP64
 partial each, one workgroup each in a resident launch), the workgroup count of the persistent ICP
 launch, and the neighbour-grid cell edge (in quarters of the search radius).  None of them
@@ -63,8 +62,8 @@ STAGES_OF = {
     "grid_cell": ("grid", "normals", "gradient", "icp"),
 }
 # knobs a workload does not exercise (one-pair calls never read the batch lanes, the batch
-# never reads the one-pair lanes; the normal and gradient kernels have one shape, so nothing reads
-# their lanes)
+# never reads the one-pair lanes).  normals_lanes: the normal and gradient kernels have one shape, so
+# nothing reads it; the library takes the key and ignores it.
 UNUSED_BY = {
     "frame": ("icp_lanes_batch", "normals_lanes"),
     "frame_overlapped": ("icp_lanes_batch", "icp_persist_blocks", "normals_lanes"),

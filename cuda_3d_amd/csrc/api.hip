@@ -902,7 +902,8 @@ int32_t gca_ctx_set_tuning(gca_ctx c, int32_t key, int32_t value)
     if (key == GCA_TUNE_VOXEL && value > 2) return GCA_ERR_INVALID_VALUE;
     if (key == GCA_TUNE_GRID_CELL && value != 0 && (value < 4 || value > 12)) return GCA_ERR_INVALID_VALUE;
     if (key == GCA_TUNE_NORMALS_LANES && !pow2(value, 64)) return GCA_ERR_INVALID_VALUE;
-    if (c->tune[key] != value) ++c->tune_version;
+    // (a key that no kernel reads is no reason for a pipeline to make its plans and graphs again)
+    if (c->tune[key] != value && key != GCA_TUNE_NORMALS_LANES) ++c->tune_version;
     c->tune[key] = value;
     return GCA_OK;
 }

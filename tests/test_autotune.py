@@ -95,3 +95,11 @@ def test_batch_table_keeps_the_partition_of_the_sums():
     """The unit cap fixes the order in which a batch's sums are added, so a tuned batch's last bits
     hang on it: it stays where it was for a sweep's 0.3 %."""
     assert autotune.load(autotune.DEFAULT_TABLE, "batch")["icp_max_units"] == 128
+
+
+def test_committed_table_holds_no_knob_that_nothing_reads():
+    with open(autotune.DEFAULT_TABLE) as fh:
+        table = json.load(fh)
+    for entry in table.values():
+        assert "normals_lanes" not in entry["tuning"]
+        assert not any(row[1] == "normals_lanes" for row in entry["measurements"])

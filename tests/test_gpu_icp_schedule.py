@@ -139,3 +139,25 @@ def test_fewer_workgroups_than_sub_queues(blocks, pairs, levels, units):
     np.testing.assert_array_equal(got[1][0], got[2][0])
     assert got[1][1] == got[2][1]
     assert all(r[0] == 40 for row in got[1][1] for r in row)
+
+
+def test_a_knob_that_nothing_reads_keeps_the_graphs(ctx):
+    """Setting normals_lanes is accepted and changes nothing: the pipeline's graphs are not captured again."""
+    import cuda_3d_amd as g
+    from cuda_3d_amd import scene
+    from cuda_3d_amd.pipeline import FramePipeline
+
+    (td, tc), (sd, sc), _, cm = scene.frame_pair(5, 160, 120)
+    dev = [(g.device_tensor(d.view(np.int16)), g.device_tensor(c)) for d, c in ((td, tc), (sd, sc))]
+    pipe = FramePipeline(ctx, g.make_camera(160, 120, cm.fx, cm.fy, cm.cx, cm.cy), g.bilateral(), levels=(0.04,), iters=4)
+    captures = []
+    for k in range(16):
+        if k == 8:
+            pipe.ctx.set_tuning(normals_lanes=4)
+            assert pipe.ctx.get_tuning()["normals_lanes"] == 4
+        d, c = dev[k % 2]
+        pipe.step(d.data_ptr(), c.data_ptr())
+        pipe.result()
+        captures.append(pipe.graph_stats()[0])
+    assert captures[7] > 0 and captures[-1] == captures[7]
+    pipe.close()
