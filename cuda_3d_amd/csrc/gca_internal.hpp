@@ -364,7 +364,8 @@ int32_t launch_outlier(gca_ctx ctx, gca_cloud in, float radius, int32_t min_nn, 
 int32_t launch_euclidean_clustering(gca_ctx ctx, gca_cloud c, float tolerance, uint32_t min_size,
                                     uint32_t max_size, int32_t *label, uint32_t *counts_dev,
                                     const float *res = nullptr);
-// Copies normals and colour gradients into the grid's cell order (c->grid.snrm / sgrad).
+// Copies normals and colour gradients into the grid's cell order (c->grid.snrm / sgrad, made by the first).
+int32_t grid_alloc_attributes(gca_cloud c);
 int32_t grid_gather_attributes(gca_ctx ctx, gca_cloud c);
 int32_t launch_normals(gca_ctx ctx, gca_cloud c, float radius, int32_t max_nn);
 int32_t launch_gradient(gca_ctx ctx, gca_cloud c, float radius, int32_t max_nn);

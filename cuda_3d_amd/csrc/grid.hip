@@ -205,15 +205,21 @@ __global__ __launch_bounds__(256) void k_gather_sorted(const CloudHdr *__restric
     }
 }
 
+// The grid's copies of normals and gradients: a call that gets only the first leaves it for the next one.
+int32_t grid_alloc_attributes(gca_cloud c)
+{
+    Grid &G = c->grid;
+    if (!G.snrm) GCA_TRY(dev_array(c->ctx, &G.snrm, G.cap_pts));
+    if (!G.sgrad) GCA_TRY(dev_array(c->ctx, &G.sgrad, G.cap_pts));
+    return GCA_OK;
+}
+
 int32_t grid_gather_attributes(gca_ctx ctx, gca_cloud c)
 {
     Grid &G = c->grid;
     if (!G.valid) return GCA_ERR_NOT_READY;
     if (G.attrs_valid) return GCA_OK;
-    if (!G.snrm) {
-        GCA_TRY(dev_array(c->ctx, &G.snrm, G.cap_pts));
-        GCA_TRY(dev_array(c->ctx, &G.sgrad, G.cap_pts));
-    }
+    GCA_TRY(grid_alloc_attributes(c));
     const unsigned nb = (unsigned)std::min<int64_t>(4096, std::max<int64_t>(1, (c->cap + 255) / 256));
     hipLaunchKernelGGL(k_gather_sorted, dim3(nb), dim3(256), 0, ctx->stream, c->hdr, G.order, c->nrm, c->grad,
                        G.snrm, G.sgrad);

@@ -687,10 +687,7 @@ static int32_t pair_prepare(gca_ctx ctx, gca_cloud c, float radius, int32_t K, f
 {
     if (!(gradient_radius <= radius)) return GCA_ERR_INVALID_VALUE;
     Grid &G = c->grid;
-    if (grid_attrs && !G.snrm) {
-        GCA_TRY(dev_array(c->ctx, &G.snrm, G.cap_pts));
-        GCA_TRY(dev_array(c->ctx, &G.sgrad, G.cap_pts));
-    }
+    if (grid_attrs) GCA_TRY(grid_alloc_attributes(c));
     const int64_t cap = std::max<int64_t>(n > 0 ? n : c->cap, 1);
     Moments *mom = (Moments *)lane_scratch(ctx, lane, 17, sizeof(Moments) * cap, false);
     int32_t *ovf = (int32_t *)lane_scratch(ctx, lane, 18, sizeof(int32_t) * cap, false);

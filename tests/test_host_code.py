@@ -220,3 +220,40 @@ for n in (9_000_001, 17_300_000):        # 137 and 264 MiB an array
     del pc
     assert rt.host_runtime_live() == before
 """)
+
+
+def test_grid_attributes_are_both_there_or_neither(runtime):
+    """A registration that ran out of memory between the target's sorted normals and its sorted
+    gradients finds both on the next try."""
+    _run(runtime, """
+src, a, b = cloud(1000, 1), cloud(200_000, 2), cloud(200_000, 3)
+def target(pc):
+    pc.estimate_normals(0.1, 30)
+    pc.compute_color_gradient(0.1, 0)
+def align(pc):
+    icp = g.ColorICP(3, 0.1, 0.1)
+    icp.set_source_point_cloud(src)
+    icp.set_target_point_cloud(pc)
+    return icp.align()
+def takes(pc):
+    before = rt.host_runtime_live()
+    assert align(pc)
+    return rt.host_runtime_live() - before
+target(a)
+target(b)
+warm = cloud(1000, 4)
+target(warm)
+assert align(warm)                       # the registration's own scratch
+whole = takes(a)
+assert whole >= 2 * 16 * 200_000         # normals and gradients in the grid's order
+base, refused = rt.host_runtime_live(), 0
+for room in range(0, whole + MiB, MiB // 4):
+    rt.host_runtime_budget(base + room)
+    try:
+        assert align(b)
+        break
+    except L.GcaError as e:
+        assert e.status == L.GCA_ERR_OUT_OF_MEMORY
+        refused += 1
+assert refused >= 8 and rt.host_runtime_live() - base == whole
+""")
