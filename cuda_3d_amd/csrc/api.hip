@@ -603,6 +603,26 @@ static void cloud_arrays_free(gca_cloud c, bool idle)
     c->cap = 0;
 }
 
+static void cloud_own_slot(gca_cloud c)
+{
+    c->xyzi = &c->ref.dev->one[0];
+    c->rgb = &c->ref.dev->one[1];
+    c->nrm = &c->ref.dev->one[2];
+    c->grad = &c->ref.dev->one[3];
+    c->cap = 1;
+}
+
+// A cloud whose arrays could not be had again holds no points: its count must not outlive them.
+static void cloud_make_empty(gca_cloud c)
+{
+    cloud_arrays_free(c, false);
+    cloud_own_slot(c);
+    cloud_points_changed(c);
+    c->has_normals = c->has_gradient = false;
+    c->host_hdr = empty_hdr();
+    c->host_valid = hipMemcpy(c->hdr, &c->host_hdr, sizeof(CloudHdr), hipMemcpyHostToDevice) == hipSuccess;
+}
+
 int32_t cloud_reserve(gca_cloud c, int64_t cap)
 {
     if (cap <= c->cap) return GCA_OK;
@@ -613,12 +633,13 @@ int32_t cloud_reserve(gca_cloud c, int64_t cap)
         idle = device_idle(c->ctx);
     }
     cloud_arrays_free(c, idle);
-    GCA_TRY(dev_array(c->ctx, &c->xyzi, cap));
-    GCA_TRY(dev_array(c->ctx, &c->rgb, cap));
-    GCA_TRY(dev_array(c->ctx, &c->nrm, cap));
-    GCA_TRY(dev_array(c->ctx, &c->grad, cap));
-    c->cap = cap;
-    return GCA_OK;
+    int32_t st = dev_array(c->ctx, &c->xyzi, cap);
+    if (st == GCA_OK) st = dev_array(c->ctx, &c->rgb, cap);
+    if (st == GCA_OK) st = dev_array(c->ctx, &c->nrm, cap);
+    if (st == GCA_OK) st = dev_array(c->ctx, &c->grad, cap);
+    if (st == GCA_OK) c->cap = cap;
+    else cloud_make_empty(c);
+    return st;
 }
 
 int32_t cloud_header_enqueue(gca_cloud c)
@@ -957,11 +978,7 @@ int32_t gca_cloud_create(gca_ctx ctx, int64_t capacity, gca_cloud *out)
     c->hdr = &c->ref.dev->h;
     c->host_hdr = empty_hdr();
     c->host_valid = true;
-    c->xyzi = &c->ref.dev->one[0];
-    c->rgb = &c->ref.dev->one[1];
-    c->nrm = &c->ref.dev->one[2];
-    c->grad = &c->ref.dev->one[3];
-    c->cap = 1;
+    cloud_own_slot(c);
     s = cloud_reserve(c, capacity);
     if (s != GCA_OK) {
         gca_cloud_destroy(c);

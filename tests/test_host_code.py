@@ -257,3 +257,21 @@ for room in range(0, whole + MiB, MiB // 4):
         refused += 1
 assert refused >= 8 and rt.host_runtime_live() - base == whole
 """)
+
+
+@pytest.mark.parametrize("room", [0, 5, 9, 14])
+def test_a_cloud_that_could_not_grow_is_empty(runtime, room):
+    """Its old arrays went before the new ones could not all be had: no call may find the old count."""
+    _run(runtime, f"""
+pc, full = cloud(30_000), cloud(400_000)
+pc.estimate_normals(0.1, 30)
+assert pc.points_number() == 30_000
+rt.host_runtime_budget(rt.host_runtime_live() + {room} * MiB)
+status = L.lib.gca_cloud_copy(ctx.handle, full.handle, pc.handle)
+assert status == L.GCA_ERR_OUT_OF_MEMORY
+count = C.c_int32.from_address(pc.device_arrays()[4]).value
+assert (pc.points_number(), count, pc.has_normals()) == (0, 0, False)
+assert all(pc.device_arrays())
+rt.host_runtime_budget(1 << 40)
+L.check(L.lib.gca_cloud_copy(ctx.handle, full.handle, pc.handle), "gca_cloud_copy")
+""")
