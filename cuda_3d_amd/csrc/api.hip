@@ -881,7 +881,6 @@ int32_t gca_ctx_destroy(gca_ctx c)
     for (gca_ctx_s::Bitmap &b : c->bitmap) hipFree(b.p);
     hipFree(c->lut);
     hipFree(c->icp_state);
-    hipFree(c->partials);
     hipEventDestroy(c->ev_a);
     hipEventDestroy(c->ev_b);
     hipStreamDestroy(c->stream);

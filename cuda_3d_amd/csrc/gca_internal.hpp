@@ -191,8 +191,6 @@ struct gca_ctx_s {
     // ICP device state
     void *icp_state = nullptr;
     size_t icp_state_bytes = 0;
-    double *partials = nullptr;
-    size_t partials_bytes = 0;
     // per-level working clouds of the multi-scale driver (created on first use)
     gca_cloud level_clouds[16] = {nullptr};
     // launch-shape tuning (GCA_TUNE_*), 0 = heuristic; the version counts changes (objects that

@@ -1459,15 +1459,15 @@ struct IcpWork {
 
 static size_t align256(size_t b) { return (b + 255) & ~size_t(255); }
 
-static int32_t icp_work(gca_ctx ctx, int n_states, int n_t0, int64_t partial_slots, int64_t nnprev_n,
+static int32_t icp_work(gca_ctx ctx, int n_states, int n_pairs, int64_t partial_slots, int64_t nnprev_n,
                         int64_t table_units, IcpWork &w)
 {
     w.states = (IcpState *)ctx_scratch(ctx, 13, sizeof(IcpState) * n_states + 256 + sizeof(*w.open) * n_states, false);
-    w.partials = (double *)ctx_scratch(ctx, 14, sizeof(double) * kPartStride * std::max<int64_t>(partial_slots, 1), false);
+    w.partials = (double *)ctx_scratch(ctx, 14, sizeof(double) * kPartStride * partial_slots, false);
     w.nnprev = (int32_t *)ctx_scratch(ctx, 16, sizeof(int32_t) * std::max<int64_t>(nnprev_n, 1), false);
     if (!w.states || !w.partials || !w.nnprev) return GCA_ERR_OUT_OF_MEMORY;
     const size_t b_pairs = align256(sizeof(PairDesc) * n_states), b_init = align256(sizeof(StateInit) * n_states),
-                 b_t0 = align256(sizeof(double) * 16 * std::max(n_t0, 4)),
+                 b_t0 = align256(sizeof(double) * 16 * n_pairs),
                  b_us = align256(sizeof(int32_t) * std::max<int64_t>(table_units, 1)),
                  b_uf = align256(sizeof(int32_t) * n_states);
     const size_t need = b_pairs + b_init + b_t0 + b_us + b_uf;
