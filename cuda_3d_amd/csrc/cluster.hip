@@ -91,7 +91,7 @@ __device__ __forceinline__ int32_t cc_root(int32_t *parent, int32_t x)
 
 // Which of two roots stays one: a mix of the index's bits (a bijection, so never a tie).  By index
 // alone the rows of an image hang under one another one by one, and the walks grow with the image
-// (289k points at 1 cm: pairs and hook 88 + 76 us by index, 38 + 44 by rank).
+// (289k points at 1 cm: pairs and hook 88 + 76 us by index, 38 + 49 by rank).
 __device__ __forceinline__ uint32_t cc_rank(int32_t x)
 {
     const uint32_t m = (uint32_t)x * 2654435769u;
@@ -254,8 +254,8 @@ __global__ __launch_bounds__(kCcSample) void k_cc_big(const CloudHdr *__restrict
 // on which end links an edge.  DIRECT: no pairs and no snapshot came before, each
 // point stands for itself (snap is the cell order, sres the residuals by index).  The whole
 // labelling is bound by the union-find's dependent loads and contended compare-and-swaps: 92k points of
-// a 424x240 frame at 2 cm 91 us plain and 171 us gated, where hooking every edge of every point took
-// 270 us for either; 289k points of a 640x480 frame at 1 cm 127 us (568 every edge).
+// a 424x240 frame at 2 cm 97 us plain and 128 us gated, where hooking every edge of every point took
+// 270 us for either; 289k points of a 640x480 frame at 1 cm 125 us (568 every edge).
 constexpr int kCcLanes = 8;
 constexpr int kCcUnroll = 4;
 
@@ -625,7 +625,8 @@ int32_t launch_euclidean_clustering(gca_ctx ctx, gca_cloud c, float tolerance, u
         // lets about a third of the neighbours through, so it takes more pairs before a scene's bulk
         // holds together.  Pairs / hook of a 424x240 frame at 2 cm: 19 / 36 us plain (every fourth: 16 /
         // 53), gated 51 / 79 us with three predecessors of every point (two 38 / 118, four 70 / 67); at
-        // 640x480 gated 93 / 276 (two 73 / 387, four 120 / 236).
+        // 640x480 gated 93 / 276 (two 73 / 387, four 120 / 236).  (Linked by index; by rank, as now, 22 / 35
+        // and 37 / 58.)
         const int step = res ? 1 : 2, back = res ? 3 : 1;
         const dim3 grid_pairs((unsigned)std::max<int64_t>(1, (c->cap / step * back + back + kCcBlock - 1) / kCcBlock));
         hipLaunchKernelGGL(k_cc_pairs, grid_pairs, block, 0, ctx->stream, c->hdr, G.sxyzi, G.order, res, r2, step, back, label);

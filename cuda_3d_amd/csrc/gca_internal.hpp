@@ -104,8 +104,9 @@ struct Jobs {
 // Device buffers given back by clouds and grids, kept for the next ones of the same size class.
 // A HIP allocation of 2 MiB or more takes 17-25 us and its release 60-230 us (below 64 KiB: 0.4 us
 // each), so a call that makes and drops a cloud spends more on them than on its kernels (a copy,
-// transform, append and 1 cm downsample of 0.8 M points: 2280 us with them, 232 us here).  Blocks enter the pool only once the
-// device has been idle since their last use, so the next owner may use them on any stream.
+// transform, append and 8 mm downsample of 1.5 M points: 2360 us with them, 205 us here).  Blocks
+// enter the pool only once the device has been idle since their last use, so the next owner may use
+// them on any stream.  Where memory ends, the pools of all ctxs of the device are emptied (ctx_malloc).
 struct BufferPool {
     static constexpr size_t kSmall = 64 << 10;   // smaller buffers are not kept
     static constexpr size_t kLimit = 512 << 20;  // bytes kept per ctx; the oldest go first

@@ -804,7 +804,7 @@ __device__ __forceinline__ void unit_commit(const PairDesc &P, IcpState *states,
 // epoch is drained adds a failing atomic on a hot claim word.)
 // 4 wavefronts per SIMD (<= 128 VGPRs) for the launches below that need their workgroups resident, so
 // that two of them fit the device at once.  The persistent launch needs none of its workgroups
-// resident and takes the registers (144) that 8 candidates in flight need: three workgroups per CU,
+// resident and takes the registers (167) that 8 candidates in flight need: three workgroups per CU,
 // and as many are launched.  64 pairs of 5k to 200k points, three levels: 8.25 ms with the claim
 // words scanned; 6.57 with the open words, 6.41 with 8 candidates in flight (4: 6.5), 5.92 with three
 // workgroups per CU (four, of which one waits for its turn: 5.92).

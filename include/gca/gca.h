@@ -22,7 +22,14 @@
  *  - Device pointers passed in (depth/colour frames, index buffers) are borrowed: the caller
  *    keeps ownership and must keep them alive until the ctx stream has passed the call.
  *  - Poses are double[16], row-major 4x4 homogeneous matrices.
- *  - One ctx per host thread.  Calls on one ctx are not thread-safe.
+ *  - One ctx per host thread.  Calls on one ctx are not thread-safe.  (Clouds may be made, filled,
+ *    copied, moved, appended to, read and destroyed on several threads at once if no two of them use
+ *    one cloud.)
+ *  - A ctx keeps memory for its next calls: scratch for its largest call so far, buffers of clouds
+ *    that are gone (at most 512 MiB), and after gca_multiscale_icp the scratch of up to three
+ *    further levels (each some 200 bytes per point of the larger cloud and 250 per point of the
+ *    level).  The last two are given back when an allocation of any ctx of the device would fail
+ *    otherwise, everything with the ctx.
  */
 #ifndef GCA_GCA_H
 #define GCA_GCA_H
