@@ -239,13 +239,17 @@ __device__ __forceinline__ void group_store(MomentSum<KIND> &A, int32_t cnt, int
     M.cnt = cnt;
 }
 
-// Sums without a K cap: 24 us for the gradient of 110k points at 2 cm (30 us with 64-bit integer
+// Sums without a K cap, or with one that the buffer of k_moments_sel does not reach (K >= kSelCandidates:
+// it selects nothing then, and sends every larger neighbourhood to a wavefront of its own): queries with
+// more than K neighbours go to the overflow list.  100k points of a surface, 200 neighbours each, K 500:
+// 304 us, 756 by k_moments_sel.  24 us for the gradient of 110k points at 2 cm (30 us with 64-bit integer
 // sums and a division per cell bound).  Eight lanes per query: 4 and 16 measured 1-2 % and 5 %
 // slower on a 640x480 target at 1 cm, 2 and 4 % on the overlapped odometry of such frames.
 template <int KIND>
 __global__ __launch_bounds__(kNbBlock) void k_moments(const float4 *__restrict__ xyzi, const CloudHdr *__restrict__ hdr,
                                                       GridDesc g, const uint32_t *__restrict__ start,
-                                                      const float4 *__restrict__ sxyzi, Moments *__restrict__ mom)
+                                                      const float4 *__restrict__ sxyzi, Moments *__restrict__ mom, int32_t K,
+                                                      int32_t *__restrict__ ovf, uint32_t *__restrict__ ovf_n)
 {
     const GridView v = make_view(g, start, nullptr, sxyzi);
     const int n = hdr->n;
@@ -260,7 +264,9 @@ __global__ __launch_bounds__(kNbBlock) void k_moments(const float4 *__restrict__
         A.zero();
         if (grid_range(g, q.x, q.y, q.z, b.lo, b.hi)) cnt = walk_moments<KIND>(v, b, q, gl, kNbLanes, r2, inv, A);
         cnt = (int32_t)group_sum<kNbLanes>((uint32_t)cnt);
-        if (cnt <= kExactTerms) {
+        if (K > 0 && cnt > K) {
+            if (gl == 0) ovf[atomicAdd(ovf_n, 1u)] = i;
+        } else if (cnt <= kExactTerms) {
             group_store<KIND>(A, cnt, gl, mom[i]);
         } else {
             long long S[9];
@@ -630,12 +636,16 @@ static unsigned grid_for(int64_t items, int per_block, int64_t cap)
     return (unsigned)std::min<int64_t>(cap, std::max<int64_t>(1, (items + per_block - 1) / per_block));
 }
 
-// The sums without a K cap of the cloud of A, on grid d.
+// The sums without selection of the cloud of A, on grid d (K: those with more neighbours go to A's overflow
+// list).
 template <int KIND>
-static void launch_all(dim3 grid, hipStream_t stream, const SelArgs &A, const GridDesc &d, Moments *mom)
+static void launch_all(dim3 grid, hipStream_t stream, const SelArgs &A, const GridDesc &d, Moments *mom, int32_t K)
 {
-    hipLaunchKernelGGL(k_moments<KIND>, grid, dim3(kNbBlock), 0, stream, A.xyzi, A.hdr, d, A.start, A.sxyzi, mom);
+    hipLaunchKernelGGL(k_moments<KIND>, grid, dim3(kNbBlock), 0, stream, A.xyzi, A.hdr, d, A.start, A.sxyzi, mom, K, A.ovf,
+                       A.ovf_n);
 }
+
+static bool selects(int32_t K) { return K > 0 && K < kSelCandidates; }
 
 template <int KIND>
 static int32_t launch_moments_pipeline(gca_ctx ctx, gca_cloud c, float radius, int32_t K, float4 *out)
@@ -650,13 +660,12 @@ static int32_t launch_moments_pipeline(gca_ctx ctx, gca_cloud c, float radius, i
     StageTimer timer(ctx, KIND == 0 ? GCA_STAGE_NORMALS : GCA_STAGE_GRADIENT);
     const dim3 grid(grid_for(cap, kNbBlock / kNbLanes, 4096));
     const Jobs<SelArgs, 1> sj{{{c->xyzi, c->hdr, d, G.start, G.order, G.sxyzi, K, 0, 0.0, mom, nullptr, ovf, ovf_n}}};
+    if (selects(K)) hipLaunchKernelGGL((k_moments_sel<KIND, false, 1>), grid, dim3(kNbBlock), 0, ctx->stream, sj);
+    else launch_all<KIND>(grid, ctx->stream, sj.a[0], d, mom, K);
     if (K > 0) {
-        hipLaunchKernelGGL((k_moments_sel<KIND, false, 1>), grid, dim3(kNbBlock), 0, ctx->stream, sj);
         const Jobs<OvfArgs, 1> oj{{{c->xyzi, c->hdr, d, G.start, G.order, G.sxyzi, K, 0, ovf, ovf_n, mom, nullptr, 0.0}}};
         hipLaunchKernelGGL((k_moments_overflow<KIND, 1>), dim3(grid_for(cap, kOvfWaves, 1024)), dim3(kWave * kOvfWaves),
                            0, ctx->stream, oj);
-    } else {
-        launch_all<KIND>(grid, ctx->stream, sj.a[0], d, mom);
     }
     hipLaunchKernelGGL(k_solve<KIND>, dim3(grid_for(cap, kNbBlock, 2048)), dim3(kNbBlock), 0, ctx->stream, c->hdr,
                        (const Moments *)mom, (const float4 *)c->nrm, (double)radius, out, ovf_n);
@@ -707,35 +716,37 @@ static int32_t pair_prepare(gca_ctx ctx, gca_cloud c, float radius, int32_t K, f
 }
 
 // moments, overflow K-selection, solve: each kernel once for all nj calls (blockIdx.y = call), on
-// stream.  A call without a K cap has no selection to share a walk with, so its two sums come from
-// a walk each.
+// stream.  A call that selects nothing in its walk (no K cap, or one beyond the buffer) has nothing to
+// share with the gradient's, so its two sums come from a walk each.
 template <int N>
 static int32_t pair_launch(hipStream_t stream, const PairJobs *pj, int nj)
 {
     Jobs<SelArgs, N> pair{};
     Jobs<OvfArgs, N> ovf{};
     Jobs<SolveArgs, N> solve{};
-    unsigned nb_pair = 1, nb_ovf = 1, nb_solve = 1, nsel = 0;
+    unsigned nb_pair = 1, nb_ovf = 1, nb_solve = 1, nsel = 0, novf = 0;
     for (int j = 0; j < nj; ++j) {
         const SelArgs &A = pj[j].pair;
-        if (A.K > 0) {
-            pair.a[nsel] = A;
-            ovf.a[nsel++] = pj[j].ovf;
+        if (selects(A.K)) {
+            pair.a[nsel++] = A;
             nb_pair = std::max(nb_pair, pj[j].nb_pair);
-            nb_ovf = std::max(nb_ovf, pj[j].nb_ovf);
         } else {
             GridDesc dg = A.g;
             dg.radius = (float)A.rg;
-            launch_all<0>(dim3(pj[j].nb_pair), stream, A, A.g, A.mom);
-            launch_all<1>(dim3(pj[j].nb_pair), stream, A, dg, A.mom_g);
+            launch_all<0>(dim3(pj[j].nb_pair), stream, A, A.g, A.mom, A.K);
+            launch_all<1>(dim3(pj[j].nb_pair), stream, A, dg, A.mom_g, 0);
+        }
+        if (A.K > 0) {
+            ovf.a[novf] = pj[j].ovf;
+            if (!selects(A.K)) ovf.a[novf].mom_g = nullptr;  // (the gradient's sums are complete)
+            ++novf;
+            nb_ovf = std::max(nb_ovf, pj[j].nb_ovf);
         }
         solve.a[j] = pj[j].solve;
         nb_solve = std::max(nb_solve, pj[j].nb_solve);
     }
-    if (nsel > 0) {
-        hipLaunchKernelGGL((k_moments_sel<0, true, N>), dim3(nb_pair, nsel), dim3(kNbBlock), 0, stream, pair);
-        hipLaunchKernelGGL((k_moments_overflow<0, N>), dim3(nb_ovf, nsel), dim3(kWave * kOvfWaves), 0, stream, ovf);
-    }
+    if (nsel > 0) hipLaunchKernelGGL((k_moments_sel<0, true, N>), dim3(nb_pair, nsel), dim3(kNbBlock), 0, stream, pair);
+    if (novf > 0) hipLaunchKernelGGL((k_moments_overflow<0, N>), dim3(nb_ovf, novf), dim3(kWave * kOvfWaves), 0, stream, ovf);
     hipLaunchKernelGGL(k_solve_pair<N>, dim3(nb_solve, (unsigned)nj), dim3(kNbBlock), 0, stream, solve);
     GCA_HIP(hipGetLastError());
     return GCA_OK;
